@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_peval(Scenes sc, Nbr nb, const f
     float df = 0.0f;
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = size_t(k) * N + i;
+        const size_t slot = ell(k, i, N);
         const uint32_t j = nb.ff[slot];
         df += P.V * pG_ff[slot] * dot3(xi - mk(pos[j]), vi - mk(vel[j]));
     }
@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_kbar(Scenes sc, Nbr nb, const fl
     f3 gx = f3z();
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = size_t(k) * N + i;
+        const size_t slot = ell(k, i, N);
         const uint32_t j = nb.ff[slot];
         const float4 xj4 = pos[j];
         const f3 xij = xi - mk(xj4);
@@ -258,7 +258,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_dbar(Scenes sc, Nbr nb, const fl
     f3 accv = f3z(), accx = f3z();
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = size_t(k) * N + i;
+        const size_t slot = ell(k, i, N);
         const uint32_t j = nb.ff[slot];
         const float4 xj4 = pos[j];
         const f3 xij = xi - mk(xj4);
@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_dbar(Scenes sc, Nbr nb, const fl
 }
 
 // ----------------------------------------------------------------- implicit viscosity / ST solve
-// rev[k*N + i] = position of i in the list of its k-th neighbour (the lists are symmetric);
+// rev at entry k of slot i (ell()) = position of i in the list of its k-th neighbour (the lists are symmetric);
 // kEmpty (and *bad = 1) if it is missing.
 __global__ void __launch_bounds__(kBlock) k_adj_rev_index(Scenes sc, Nbr nb, uint32_t* __restrict__ rev, uint32_t* bad) {
     const uint32_t sid = sc.blk_scene[blockIdx.x];
@@ -303,30 +303,33 @@ __global__ void __launch_bounds__(kBlock) k_adj_rev_index(Scenes sc, Nbr nb, uin
     if (i >= sc.P[sid].end) return;
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const uint32_t j = nb.ff[size_t(k) * N + i];
+        const uint32_t j = nb.ff[ell(k, i, N)];
         const uint32_t cj = nb.cff[j];
         uint32_t m = kEmpty;
         for (uint32_t q = 0; q < cj; q++)
-            if (nb.ff[size_t(q) * N + j] == i) {
+            if (nb.ff[ell(q, j, N)] == i) {
                 m = q;
                 break;
             }
         if (m == kEmpty) atomicOr(bad, 1u);
-        rev[size_t(k) * N + i] = m;
+        rev[ell(k, i, N)] = m;
     }
 }
-// cabT[k*N + i] = the coefficients (a_ji, b_ji) of the pair seen from the neighbour j
+// (caT, cbT) at entry k of slot i = the coefficients (a_ji, b_ji) of the pair seen from the neighbour j
 __global__ void __launch_bounds__(kBlock) k_adj_transpose_coeffs(Scenes sc, Nbr nb, const uint32_t* __restrict__ rev,
-                                                               const float2* __restrict__ cab, float2* __restrict__ cabT) {
+                                                               const float* __restrict__ ca, const float* __restrict__ cb,
+                                                               float* __restrict__ caT, float* __restrict__ cbT) {
     const uint32_t sid = sc.blk_scene[blockIdx.x];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t N = sc.N;
     if (i >= sc.P[sid].end) return;
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = size_t(k) * N + i;
+        const size_t slot = ell(k, i, N);
         const uint32_t m = rev[slot];
-        cabT[slot] = m == kEmpty ? make_float2(0.f, 0.f) : cab[size_t(m) * N + nb.ff[slot]];
+        const size_t at = m == kEmpty ? 0 : ell(m, nb.ff[slot], N);
+        caT[slot] = m == kEmpty ? 0.0f : ca[at];
+        cbT[slot] = m == kEmpty ? 0.0f : cb[at];
     }
 }
 
@@ -356,8 +359,9 @@ __global__ void __launch_bounds__(kBlock) k_adj_cg_init(Scenes sc, const float4*
 }
 // Warm start: r = b - A_f^T x0 (x0 packed in recA), p = r into recB, x = x0; partials of r.r
 // at partials[blk] and of b.b at partials[nblk + blk].
-__global__ void __launch_bounds__(kBlock) k_adj_cg_init_warm(Scenes sc, Nbr nb, const float2* __restrict__ cab,
-                                                           const float2* __restrict__ cabT, const float4* __restrict__ recA,
+__global__ void __launch_bounds__(kBlock) k_adj_cg_init_warm(Scenes sc, Nbr nb, const float* __restrict__ ca,
+                                                           const float* __restrict__ cb, const float* __restrict__ caT,
+                                                           const float* __restrict__ cbT, const float4* __restrict__ recA,
                                                            const float4* __restrict__ b, float4* __restrict__ x,
                                                            float4* __restrict__ r, float4* __restrict__ recB,
                                                            double* __restrict__ partials, uint32_t nblk) {
@@ -374,9 +378,9 @@ __global__ void __launch_bounds__(kBlock) k_adj_cg_init_warm(Scenes sc, Nbr nb, 
             f3 acc = f3z();
             const uint32_t c = nb.cff[i];
             for (uint32_t k = 0; k < c; k++) {
-                const size_t slot = size_t(k) * N + i;
+                const size_t slot = ell(k, i, N);
                 const uint32_t j = nb.ff[slot];
-                const float2 ab = cab[slot], abT = cabT[slot];
+                const float2 ab = make_float2(ca[slot], cb[slot]), abT = make_float2(caT[slot], cbT[slot]);
                 const float4 ja = recA[2 * size_t(j)], jb = recA[2 * size_t(j) + 1];
                 const f3 xij = xi - mk(ja);
                 const f3 pj = rec_pv(ja, jb);
@@ -425,8 +429,9 @@ __global__ void __launch_bounds__(kBlock) k_adj_fold_start(Scenes sc, const doub
 
 // (A_f^T p)_i = (1+f) p_i + sum_j [ (a_ij p_i - a_ji p_j) + (b_ij (p_i.x_ij) - b_ji (p_j.x_ij)) x_ij ]
 // and partials of p.Ap, for scenes whose solve is still running.
-__global__ void __launch_bounds__(kBlock) k_adj_cg_applyT(Scenes sc, Nbr nb, const float2* __restrict__ cab,
-                                                        const float2* __restrict__ cabT, const float4* __restrict__ rec,
+__global__ void __launch_bounds__(kBlock) k_adj_cg_applyT(Scenes sc, Nbr nb, const float* __restrict__ ca,
+                                                        const float* __restrict__ cb, const float* __restrict__ caT,
+                                                        const float* __restrict__ cbT, const float4* __restrict__ rec,
                                                         float4* __restrict__ Ap, const SolverDev* st, double* __restrict__ partials) {
     __shared__ double lds[kBlock / 64];
     const uint32_t sid = sc.blk_scene[blockIdx.x];
@@ -441,9 +446,9 @@ __global__ void __launch_bounds__(kBlock) k_adj_cg_applyT(Scenes sc, Nbr nb, con
         f3 acc = f3z();
         const uint32_t c = nb.cff[i];
         for (uint32_t k = 0; k < c; k++) {
-            const size_t slot = size_t(k) * N + i;
+            const size_t slot = ell(k, i, N);
             const uint32_t j = nb.ff[slot];
-            const float2 ab = cab[slot], abT = cabT[slot];
+            const float2 ab = make_float2(ca[slot], cb[slot]), abT = make_float2(caT[slot], cbT[slot]);
             const float4 ja = rec[2 * size_t(j)], jb = rec[2 * size_t(j) + 1];
             const f3 xij = xi - mk(ja);
             const f3 pj = rec_pv(ja, jb);
@@ -551,7 +556,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_cg_grad(Scenes sc, Nbr nb, const
         float gr = 0.0f, gf = 0.0f;
         const uint32_t c = nb.cff[i];
         for (uint32_t k = 0; k < c; k++) {
-            const uint32_t j = nb.ff[size_t(k) * N + i];
+            const uint32_t j = nb.ff[ell(k, i, N)];
             const float4 xj4 = pos[j], vj4 = vin[j];
             const f3 xij = xi - mk(xj4), uij = ui - mk(vj4), pij = si - mk(vstar[j]);
             const float rj = rho[j], fj = fst[j], mj = vj4.w;
@@ -590,7 +595,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_fst(Scenes sc, Nbr nb, const flo
     f3 accv = f3z(), accx = f3z();
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = size_t(k) * N + i;
+        const size_t slot = ell(k, i, N);
         const uint32_t j = nb.ff[slot];
         const float4 vj4 = vin[j], xj4 = pos[j];
         const f3 xij = xi - mk(xj4);
@@ -647,7 +652,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_gvec(Scenes sc, Nbr nb, const fl
     float s = 0.0f;
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = size_t(k) * N + i;
+        const size_t slot = ell(k, i, N);
         const f3 grad = (P.V * pG_ff[slot]) * (xi - mk(pos[nb.ff[slot]]));
         gf = gf + grad;
         s += dot3(grad, grad);
@@ -690,7 +695,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_density(Scenes sc, Nbr nb, const
     f3 acc = f3z();
     const uint32_t c = nb.cff[i];
     for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = size_t(k) * N + i;
+        const size_t slot = ell(k, i, N);
         const uint32_t j = nb.ff[slot];
         const float4 xj4 = pos[j];
         const f3 xij = xi - mk(xj4);
@@ -822,16 +827,17 @@ void adj_dbar(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, con
 void adj_rev_index(const Scenes& sc, const Nbr& nb, uint32_t* rev, uint32_t* bad, hipStream_t s) {
     if (sc.N) launch_k(k_adj_rev_index, nbk(sc.N), kBlock, 0, s, sc, nb, rev, bad);
 }
-void adj_transpose_coeffs(const Scenes& sc, const Nbr& nb, const uint32_t* rev, const float2* cab, float2* cabT, hipStream_t s) {
-    if (sc.N) launch_k(k_adj_transpose_coeffs, nbk(sc.N), kBlock, 0, s, sc, nb, rev, cab, cabT);
+void adj_transpose_coeffs(const Scenes& sc, const Nbr& nb, const uint32_t* rev, const float* ca, const float* cb, float* caT, float* cbT,
+                          hipStream_t s) {
+    if (sc.N) launch_k(k_adj_transpose_coeffs, nbk(sc.N), kBlock, 0, s, sc, nb, rev, ca, cb, caT, cbT);
 }
 void adj_cg_init(const Scenes& sc, const float4* pos, const float4* b, float4* x, float4* r, float4* rec, double* partials,
                  hipStream_t s) {
     if (sc.N) launch_k(k_adj_cg_init, nbk(sc.N), kBlock, 0, s, sc, pos, b, x, r, rec, partials);
 }
-void adj_cg_applyT(const Scenes& sc, const Nbr& nb, const float2* cab, const float2* cabT, const float4* rec, float4* Ap,
+void adj_cg_applyT(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* rec, float4* Ap,
                    const SolverDev* st, double* partials, hipStream_t s) {
-    if (sc.N) launch_k(k_adj_cg_applyT, nbk(sc.N), kBlock, 0, s, sc, nb, cab, cabT, rec, Ap, st, partials);
+    if (sc.N) launch_k(k_adj_cg_applyT, nbk(sc.N), kBlock, 0, s, sc, nb, ca, cb, caT, cbT, rec, Ap, st, partials);
 }
 void adj_cg_grad(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vin, const float4* vstar,
                  const float* rho, const float* fst, const float4* lam, float4* avin, float4* ax, float* rbar, float* fbar,
@@ -870,9 +876,9 @@ void adj_unpermute(uint32_t n, const uint32_t* src, const float4* ax, const floa
                    float4* av_out, float4* al_out, hipStream_t s) {
     if (n) launch_k(k_adj_unpermute, nbk(n), kBlock, 0, s, n, src, ax, av, al, ax_out, av_out, al_out);
 }
-void adj_cg_init_warm(const Scenes& sc, const Nbr& nb, const float2* cab, const float2* cabT, const float4* recA,
+void adj_cg_init_warm(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* recA,
                       const float4* b, float4* x, float4* r, float4* recB, double* partials, hipStream_t s) {
-    if (sc.N) launch_k(k_adj_cg_init_warm, nbk(sc.N), kBlock, 0, s, sc, nb, cab, cabT, recA, b, x, r, recB, partials, nbk(sc.N));
+    if (sc.N) launch_k(k_adj_cg_init_warm, nbk(sc.N), kBlock, 0, s, sc, nb, ca, cb, caT, cbT, recA, b, x, r, recB, partials, nbk(sc.N));
 }
 void adj_fold_start(const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, hipStream_t s) {
     if (sc.N) launch_k(k_adj_fold_start, sc.S, kBlock, 0, s, sc, partials, nbk(sc.N), st, active, tol);

@@ -231,7 +231,7 @@ struct mps_ctx {
     DBuf<float4> adx, adv, adx2, adv2, aux4, gvec, avin, lam, lam2;
     bool lam_valid = false;  // lam holds the later step's transposed solution (warm start)
     DBuf<float> abar, rbar, dbar, fbar, fstr;
-    DBuf<float2> cabT;
+    DBuf<float> caT, cbT;  // (a_ji, b_ji) per list entry
     DBuf<double> acc_mu, acc_sig;
     // fluid: pos = (x, y, z, r), vel = (vx, vy, vz, m)
     DBuf<float4> pos, vel, color, cgb, cgx, cgr, cgAp, jprev, jt[3], jcand, tmp4;
@@ -275,8 +275,8 @@ struct mps_ctx {
     bool coupled() const { return cfg.couple_scenes != 0 && S > 1; }
     // per neighbour slot: G_ij (ff, fb) for the pressure solves, a_ij / b_ij for the CG operator
     DBuf<float> pairG_ff, pairG_fb;
-    DBuf<float2> pairAB;  // (a_ij, b_ij) of the implicit viscosity operator
-    DBuf<float> pairA;    // a_ij alone, when A.p recomputes b_ij (cfg.cg_stream_coeffs == 0)
+    DBuf<float> pairA;    // a_ij of the implicit viscosity operator
+    DBuf<float> pairB;    // b_ij, unless A.p recomputes it (cfg.cg_stream_coeffs == 0)
     DBuf<float> irho;     // 1/rho per slot for that recomputation
     // block halos of the fluid lists for A.p (halo.hip): sorted distinct neighbour slots per
     // workgroup, their count, and every list entry as a 16-bit position in its block's halo
@@ -922,7 +922,13 @@ struct mps_ctx {
         if (!pairs_valid) density_alpha(mps::launch::kDoPairs);
     }
     // Block halos of the fluid lists for the halo-staged kernels (pressure solves, A.p)
-    mps::Halo halo() const { return mps::Halo{halo_idx.p, halo_n.p, nb16.p}; }
+    mps::Halo halo() const { return mps::Halo{halo_idx.p, halo_n.p, nb16.p, use_deep()}; }
+    // Whether the staged kernels run their deep forms: when the last list build had more than one
+    // workgroup in a thousand with a halo over the shallow depth (or as cfg.cg_halo_depth says).
+    bool use_deep() const {
+        const uint64_t nb = (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
+        return cfg.cg_halo_depth == 2 || (cfg.cg_halo_depth == 0 && uint64_t(deep_halos) * 1000u > nb);
+    }
     void ensure_halo() {
         if (halo_valid) return;
         const size_t m = std::max<uint32_t>(N, 1);
@@ -982,6 +988,7 @@ struct mps_ctx {
                 key.push_back(u(q));
             key.push_back(u(tol));
             key.push_back(lmin);
+            key.push_back(hl.deep);
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
                     T_(df ? K_EVAL_DF : K_EVAL_CD, [&] {
@@ -1050,28 +1057,25 @@ struct mps_ctx {
         mps::launch::CgOperator op;
         op.recompute = cfg.cg_stream_coeffs ? 0 : 1;
         op.cubic = cubic();
-        {  // halo depth of the streamed operator (the last list build's halos decide when asked to)
-            const uint64_t nb = (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
-            op.deep = !op.recompute && (cfg.cg_halo_depth == 2 || (cfg.cg_halo_depth == 0 && uint64_t(deep_halos) * 1000u > nb));
-        }
+        op.deep = !op.recompute && use_deep();
+        pairA.reserve(size_t(Kff) * m);
+        op.ca = pairA.p;
         if (op.recompute) {
-            pairA.reserve(size_t(Kff) * m);
             irho.reserve(m);
-            op.ca = pairA.p;
             op.vel = vel.p;
             op.rho = rho.p;
             op.irho = irho.p;
         } else {
-            pairAB.reserve(size_t(Kff) * m);
-            op.cab = pairAB.p;
+            pairB.reserve(size_t(Kff) * m);
+            op.cb = pairB.p;
         }
         v3x.reserve(m); v3r.reserve(m); v3Ap.reserve(m); v3p.reserve(m); v3q.reserve(m);
         ensure_halo();
         const mps::Halo hl = halo();
         T_(K_ST_FACTOR, [&] { mps::launch::st_factor(P, nbr(), hl, pos.p, vel.p, pairG_ff.p, fst.p, cgx.p, stream); });
         T_(K_CG_SETUP, [&] {
-            mps::launch::cg_setup(cubic(), P, nbr(), hl, pos.p, vel.p, rho.p, fst.p, op.recompute ? pairA.p : nullptr,
-                                  op.recompute ? nullptr : pairAB.p, cgb.p, op.recompute ? irho.p : nullptr, stream);
+            mps::launch::cg_setup(cubic(), P, nbr(), hl, pos.p, vel.p, rho.p, fst.p, pairA.p,
+                                  op.recompute ? nullptr : pairB.p, cgb.p, op.recompute ? irho.p : nullptr, stream);
         });
         mps::launch::solver_reset(sd, S, act, stream);
         const double tol = cfg.cg_tol;
@@ -1117,7 +1121,7 @@ struct mps_ctx {
         while (it <= cap && !done) {
             const uint32_t chunk = chunk_len(it, pred[2], cap - it + 1);
             std::vector<uint64_t> key = key_base(3, chunk, P, nbr());
-            for (const void* q : {(const void*)op.cab, (const void*)op.ca, (const void*)op.vel, (const void*)op.rho,
+            for (const void* q : {(const void*)op.cb, (const void*)op.ca, (const void*)op.vel, (const void*)op.rho,
                                   (const void*)op.irho, (const void*)pos.p, (const void*)pbuf(it - 1), (const void*)pbuf(it),
                                   (const void*)v3Ap.p, (const void*)v3r.p, (const void*)v3x.p, (const void*)sd,
                                   (const void*)partials.p, (const void*)act, (const void*)hl.idx, (const void*)hl.n,
@@ -1356,7 +1360,7 @@ struct mps_ctx {
         if (lam_valid) {
             cgrecA.reserve(2 * std::max<uint32_t>(N, 1));
             mps::launch::cg_pack(N, p0, lam.p, cgrecA.p, stream);
-            mps::launch::adj_cg_init_warm(P, nb, pairAB.p, cabT.p, cgrecA.p, adv.p, cgx.p, cgr.p, cgrecB.p, partials.p,
+            mps::launch::adj_cg_init_warm(P, nb, pairA.p, pairB.p, caT.p, cbT.p, cgrecA.p, adv.p, cgx.p, cgr.p, cgrecB.p, partials.p,
                                           stream);
             mps::launch::adj_fold_start(P, partials.p, sd, act, tol, stream);
         } else {
@@ -1369,14 +1373,14 @@ struct mps_ctx {
         while (it <= cap && !done) {
             const uint32_t chunk = chunk_len(it, pred_adj, cap - it + 1);
             std::vector<uint64_t> key = key_base(4, chunk, P, nb);
-            for (const void* q : {(const void*)pairAB.p, (const void*)cabT.p, (const void*)cgrecB.p, (const void*)cgAp.p,
+            for (const void* q : {(const void*)pairA.p, (const void*)pairB.p, (const void*)caT.p, (const void*)cbT.p, (const void*)cgrecB.p, (const void*)cgAp.p,
                                   (const void*)cgx.p, (const void*)cgr.p, (const void*)sd, (const void*)partials.p,
                                   (const void*)act})
                 key.push_back(u(q));
             key.push_back(u(tol));
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
-                    mps::launch::adj_cg_applyT(P, nb, pairAB.p, cabT.p, cgrecB.p, cgAp.p, sd, partials.p, stream);
+                    mps::launch::adj_cg_applyT(P, nb, pairA.p, pairB.p, caT.p, cbT.p, cgrecB.p, cgAp.p, sd, partials.p, stream);
                     mps::launch::fold_cg(1, P, partials.p, sd, act, tol, stream);
                     mps::launch::cg_update(P, cgx.p, cgr.p, cgrecB.p, cgAp.p, sd, partials.p, stream);
                     mps::launch::fold_cg(2, P, partials.p, sd, act, tol, stream);
@@ -1429,14 +1433,15 @@ struct mps_ctx {
         {  // the implicit viscosity / surface-tension solve
             const float4* vin = T.snaps[T.df_last].p;
             const float4* vst = T.snaps[T.cg_out].p;
-            pairAB.reserve(size_t(T.Kff) * m); cabT.reserve(size_t(T.Kff) * m); rev.reserve(size_t(T.Kff) * m);
+            pairA.reserve(size_t(T.Kff) * m); pairB.reserve(size_t(T.Kff) * m);
+            caT.reserve(size_t(T.Kff) * m); cbT.reserve(size_t(T.Kff) * m); rev.reserve(size_t(T.Kff) * m);
             cgrecB.reserve(2 * m);
             mps::launch::st_factor(P, nb, mps::Halo{}, T.pos.p, vin, pairG_ff.p, fstr.p, cgx.p, stream);
-            mps::launch::cg_setup(cubic(), P, nb, mps::Halo{}, T.pos.p, vin, rho.p, fstr.p, nullptr, pairAB.p, cgb.p, nullptr,
+            mps::launch::cg_setup(cubic(), P, nb, mps::Halo{}, T.pos.p, vin, rho.p, fstr.p, pairA.p, pairB.p, cgb.p, nullptr,
                                   stream);
             mps::launch::zero_words(d_flags + 2, 1, stream);
             mps::launch::adj_rev_index(P, nb, rev.p, d_flags + 2, stream);
-            mps::launch::adj_transpose_coeffs(P, nb, rev.p, pairAB.p, cabT.p, stream);
+            mps::launch::adj_transpose_coeffs(P, nb, rev.p, pairA.p, pairB.p, caT.p, cbT.p, stream);
             adj_solveT(nb, T.pos.p);
             lam.reserve(m);
             HIPCHK(hipMemcpyAsync(lam.p, cgx.p, sizeof(float4) * N, hipMemcpyDeviceToDevice, stream));
@@ -2213,21 +2218,23 @@ struct mps_ctx {
         }
     }
     // CSR in reference order from slot-order ELL lists; fluid neighbour slots are mapped to
-    // reference indices (map_ids), boundary neighbours are already reference indices.
+    // reference indices (groups), boundary neighbours are already reference indices.
     std::vector<uint32_t> csr_idx_fluid(const uint32_t* cnt) {
         std::vector<uint32_t> c = down(cnt, N), iv = down(inv.p, Nref), idx(size_t(Nref) + 1, 0u);
         for (uint32_t i = 0; i < Nref; i++) idx[i + 1] = idx[i] + c[iv[i]];
         return idx;
     }
-    std::vector<uint32_t> csr_nei_fluid(const uint32_t* nbrs, const uint32_t* cnt, uint32_t K, bool map_ids) {
+    std::vector<uint32_t> csr_nei_fluid(const uint32_t* nbrs, const uint32_t* cnt, uint32_t K, bool groups) {
         std::vector<uint32_t> c = down(cnt, N), iv = down(inv.p, Nref), pm = down(perm.p, N);
         std::vector<uint32_t> ell = down(nbrs, size_t(K) * N);
         std::vector<uint32_t> out;
         for (uint32_t i = 0; i < Nref; i++) {
             const uint32_t sl = iv[i];
             for (uint32_t k = 0; k < c[sl]; k++) {
-                const uint32_t j = ell[size_t(k) * N + sl];
-                out.push_back(map_ids ? pm[j] : j);
+                // fluid lists keep four entries of a slot side by side (ell()), wall lists are columns
+                const size_t at = groups ? (size_t(k >> 2) * N + sl) * 4 + (k & 3u) : size_t(k) * N + sl;
+                const uint32_t j = ell[at];
+                out.push_back(groups ? pm[j] : j);
             }
         }
         return out;
@@ -2442,7 +2449,7 @@ struct mps_ctx {
         bobj.release(); bS4.release();
         partials.release();
         arrive.release();
-        pairG_ff.release(); pairG_fb.release(); pairAB.release(); pairA.release(); irho.release(); halo_idx.release(); halo_n.release(); nb16.release(); nstat.release(); cgrecA.release(); cgrecB.release();
+        pairG_ff.release(); pairG_fb.release(); pairA.release(); pairB.release(); irho.release(); halo_idx.release(); halo_n.release(); nb16.release(); nstat.release(); cgrecA.release(); cgrecB.release();
         if (copy_stream) (void)hipStreamSynchronize(copy_stream);
         for (ReadbackSlot& sl : rb) {
             sl.buf.release();
@@ -2458,7 +2465,7 @@ struct mps_ctx {
         ck_end.release();
         perm0.release(); d_L.release(); rev.release(); gobs.release(); adx.release(); adv.release(); adx2.release(); adv2.release();
         aux4.release(); gvec.release(); avin.release(); abar.release(); rbar.release(); dbar.release(); fbar.release();
-        fstr.release(); cabT.release(); acc_mu.release(); acc_sig.release(); lam.release(); lam2.release();
+        fstr.release(); caT.release(); cbT.release(); acc_mu.release(); acc_sig.release(); lam.release(); lam2.release();
         if (d_active) (void)hipFree(d_active);
         if (h_active) (void)hipHostFree(h_active);
         for (const Rec& r : recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }

@@ -15,6 +15,12 @@ namespace dev {
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 constexpr int kBlock = 256;  // 4 wave64s per workgroup for particle-parallel kernels
 
+// Place of entry k of slot i in the fluid neighbour lists and in every array stored per entry of
+// them (N slots): the entries 4g .. 4g+3 of a slot lie side by side, groups of all slots after one
+// another, so a lane can load or store four entries at once (16 bytes of slots) and a wave still
+// touches contiguous memory.
+__device__ __forceinline__ size_t ell(uint32_t k, uint32_t i, uint32_t N) { return (size_t(k >> 2) * N + i) * 4u + (k & 3u); }
+
 // --------------------------------------------------------------------- float3 helpers
 struct f3 {
     float x, y, z;

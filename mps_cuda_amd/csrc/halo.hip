@@ -56,18 +56,29 @@ __global__ void __launch_bounds__(kBlock) k_halo_build(Scenes sc, Nbr nb, uint32
     // insert; stop as soon as the block is known to exceed the limit. The count is checked
     // before every insert, so each thread adds at most one key after the count passes the
     // limit: the table holds at most limit + kBlock keys, never fills, and every probe ends.
-    // List entries are loaded kBatch at a time so their latency overlaps.
+    // List entries are loaded kBatch at a time (two groups of four) so their latency overlaps.
     constexpr uint32_t kBatch = 8;
+    const uint4* ff4 = reinterpret_cast<const uint4*>(nb.ff);
+    auto load = [&](uint32_t k0, uint32_t (&jb)[kBatch]) {
+#pragma unroll
+        for (uint32_t g = 0; g < kBatch / 4; g++) {
+            if (k0 + 4 * g < c) {
+                const uint4 v = ff4[size_t(k0 / 4 + g) * N + i];
+                jb[4 * g] = v.x;
+                jb[4 * g + 1] = v.y;
+                jb[4 * g + 2] = v.z;
+                jb[4 * g + 3] = v.w;
+            }
+        }
+    };
     bool over = false;
     for (uint32_t k0 = 0; k0 < c && !over; k0 += kBatch) {
         uint32_t jb[kBatch];
-#pragma unroll
-        for (uint32_t q = 0; q < kBatch; q++)
-            jb[q] = k0 + q < c ? nb.ff[size_t(k0 + q) * N + i] : kNoKey;
+        load(k0, jb);
 #pragma unroll
         for (uint32_t q = 0; q < kBatch; q++) {
+            if (k0 + q >= c) break;
             const uint32_t j = jb[q];
-            if (j == kNoKey) break;
             if (*(volatile uint32_t*)&cnt > limit) {
                 over = true;
                 break;
@@ -136,12 +147,15 @@ __global__ void __launch_bounds__(kBlock) k_halo_build(Scenes sc, Nbr nb, uint32
     __syncthreads();
     for (uint32_t k0 = 0; k0 < c; k0 += kBatch) {
         uint32_t jb[kBatch];
+        load(k0, jb);
 #pragma unroll
-        for (uint32_t q = 0; q < kBatch; q++)
-            if (k0 + q < c) jb[q] = nb.ff[size_t(k0 + q) * N + i];
+        for (uint32_t g = 0; g < kBatch / 4; g++) {
+            uint32_t p[4];
 #pragma unroll
-        for (uint32_t q = 0; q < kBatch; q++)
-            if (k0 + q < c) n16[size_t(k0 + q) * N + i] = at[halo_find(key, jb[q])];
+            for (uint32_t q = 0; q < 4; q++) p[q] = k0 + 4 * g + q < c ? at[halo_find(key, jb[4 * g + q])] : 0u;
+            if (k0 + 4 * g < c)  // four positions at once (0 past the end of the list)
+                reinterpret_cast<uint2*>(n16)[size_t(k0 / 4 + g) * N + i] = make_uint2(p[0] | p[1] << 16, p[2] | p[3] << 16);
+        }
     }
 }
 

@@ -7,13 +7,15 @@
 //     keep ascending particle id — the order the reference's neighbour lists depend on;
 //   * cell start/end tables cleared incrementally (only cells occupied last step), plus a
 //     copy of the positions in key order so the 27-cell scan reads contiguous memory;
-//   * one search pass per particle (no count/scan/fill double scan): fluid neighbour ids go
-//     to column-major ELL storage nbr[k*N + i] (a wave reads 256 contiguous bytes per k),
-//     the boundary-boundary list to rows of K slots (it is read once, when the walls move),
+//   * one search pass per particle (no count/scan/fill double scan): fluid neighbours go to ELL
+//     storage in groups of four entries per slot (ell(), device_common.hpp), the wall neighbours
+//     to column-major ELL storage nbr[k*N + i], the boundary-boundary list to rows of K slots (it is read once, when the walls move),
 //     the per-particle count to cnt[i]; overflow past the capacity is counted and reported
 //     so the host can grow the capacity and search again;
 //   * the fluid search stages a workgroup's candidates in LDS, row by row, so that each
 //     particle walks its 27 cells as 9 contiguous runs (k_neighbors_fluid).
+#include <type_traits>
+
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -295,7 +297,7 @@ __global__ void __launch_bounds__(kBlock) k_cell_table(const uint32_t* __restric
 // Neighbour when |x_i - x_j| < (4 r_i + 4 r_j) * 0.5, self excluded when SELF.
 // The 27 (start, end) pairs are loaded up front, so their latencies overlap instead of
 // adding up cell after cell; candidates are read two at a time for the same reason. Lists
-// are written column-major (out[k*stride + i]) when COLS, else as rows of K slots.
+// are written in the layout LAYOUT.
 // Neighbour test of the reference: |x_i - x_j| < (h_i + h_j) / 2 with h = 4 r.
 // sqrt is monotone and correctly rounded: far from the cut-off the squared distance decides;
 // near it the exact test of the reference runs.
@@ -337,7 +339,17 @@ __device__ __forceinline__ uint32_t hit_bits4(const float4& xi, float thr, float
     return in;
 }
 
-template <bool SELF, bool COLS>
+// Where a search puts its lists: rows of K slots (out[i*K + k]), columns (out[k*stride + i]) or
+// groups of four entries (ell()).
+enum ListLayout { kRows, kCols, kGroups };
+template <int LAYOUT>
+__device__ __forceinline__ size_t list_at(uint32_t k, uint32_t i, uint32_t K, uint32_t stride) {
+    if constexpr (LAYOUT == kRows) return size_t(i) * K + k;
+    else if constexpr (LAYOUT == kCols) return size_t(k) * stride + i;
+    else return ell(k, i, stride);
+}
+
+template <bool SELF, int LAYOUT>
 __device__ __forceinline__ uint32_t search_cells(float4 xi, uint32_t i, const HashGeom& g, const uint32_t* __restrict__ start,
                                                  const uint32_t* __restrict__ end, const uint32_t* __restrict__ ids,
                                                  const float4* __restrict__ spos, uint32_t* __restrict__ out, uint32_t K,
@@ -349,7 +361,7 @@ __device__ __forceinline__ uint32_t search_cells(float4 xi, uint32_t i, const Ha
         if (within(xi, ri, q)) {
             const uint32_t j = ids ? ids[s] : s;
             if (!(SELF && j == i)) {
-                if (k < K) out[COLS ? size_t(k) * stride + i : size_t(i) * K + k] = j;
+                if (k < K) out[list_at<LAYOUT>(k, i, K, stride)] = j;
                 k++;
             }
         }
@@ -484,8 +496,9 @@ __device__ __forceinline__ unsigned long long block_scan_u64(unsigned long long 
 
 // The hits among staged candidates [lo, hi) in order: four candidates per step (hit_bits4,
 // the threshold of equal radii), a hit mask per 32 candidates, then the hits' ids (held in w) as
-// list entries cnt, cnt + 1, ... (column-major, stride N; entries past K are counted only).
+// list entries cnt, cnt + 1, ... (entries past K are counted only).
 // `self` is the particle's own staged index, which is not a neighbour (any value >= hi: none).
+template <int LAYOUT>
 __device__ __forceinline__ void walk_run(const float4* cand, uint32_t lo, uint32_t hi, const float4& xi, float thr, float t2lo,
                                          float t2hi, uint32_t self, uint32_t* __restrict__ out, uint32_t K, uint32_t N,
                                          uint32_t i, uint32_t& cnt) {
@@ -504,7 +517,7 @@ __device__ __forceinline__ void walk_run(const float4* cand, uint32_t lo, uint32
         while (m) {
             const uint32_t b = static_cast<uint32_t>(__builtin_ctz(m));
             m &= m - 1u;
-            if (cnt < K) out[size_t(cnt) * N + i] = __float_as_uint(cand[c0 + b].w);
+            if (cnt < K) out[list_at<LAYOUT>(cnt, i, K, N)] = __float_as_uint(cand[c0 + b].w);
             cnt++;
         }
     }
@@ -688,28 +701,28 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __rest
             for (uint32_t probe = 0; probe < kSrchRowHash && rkey[h] != k; probe++) h = (h + 1u) & (kSrchRowHash - 1u);
             return rkey[h] == k ? rbase[h] + static_cast<uint32_t>(p.x + dx - rxlo[h]) : kNoRow;
         };
-        auto rows = [&](const uint16_t* eo, float thr, uint32_t self, uint32_t* out, uint32_t K, uint32_t& cnt) {
+        auto rows = [&](auto layout, const uint16_t* eo, float thr, uint32_t self, uint32_t* out, uint32_t K, uint32_t& cnt) {
             const float t2 = thr * thr, t2lo = t2 * 0.9999f, t2hi = t2 * 1.0001f;
             for (int r = 0; r < 9; r++) {
                 const uint32_t e = cell_of(-1, p.y + r % 3 - 1, p.z + r / 3 - 1);
                 if (e == kNoRow) continue;  // not reached: every row of a run was registered
-                walk_run(cand, eo[e], eo[e + 3u], xi, thr, t2lo, t2hi, self, out, K, N, i, cnt);
+                walk_run<decltype(layout)::value>(cand, eo[e], eo[e + 3u], xi, thr, t2lo, t2hi, self, out, K, N, i, cnt);
             }
         };
         if (!(mix & 1u)) {
             const uint32_t eh = cell_of(0, p.y, p.z);
             const uint32_t self = eh == kNoRow ? kNoRow : efo[eh] + (i - efs[eh]);
-            rows(efo, (ri + ri) * 0.5f, self, nff, Kff, a);
+            rows(std::integral_constant<int, kGroups>{}, efo, (ri + ri) * 0.5f, self, nff, Kff, a);
         } else {
-            a = search_cells<true, true>(xi, i, g, fstart, fend, fl.id, fl.spos, nff, Kff, N);
+            a = search_cells<true, kGroups>(xi, i, g, fstart, fend, fl.id, fl.spos, nff, Kff, N);
         }
         if (bd.n) {
             if (staged && tb == 0u) {
                 b = 0u;  // no wall particle in any cell of the block
             } else if (!(mix & 2u)) {
-                rows(ebo, (ri + rw * 4.0f) * 0.5f, kNoRow, nfb, Kfb, b);
+                rows(std::integral_constant<int, kCols>{}, ebo, (ri + rw * 4.0f) * 0.5f, kNoRow, nfb, Kfb, b);
             } else {
-                b = search_cells<false, true>(xi, i, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N);
+                b = search_cells<false, kCols>(xi, i, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N);
             }
         }
     }
@@ -729,7 +742,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_boundary(const float4* __r
     uint32_t a = 0u;
     if (i < B) {
         const size_t base = scene ? size_t(scene[i]) * C : 0;
-        a = search_cells<true, false>(pos[i], i, g, bd.start + base, bd.end + base, bd.id, bd.spos, nbb, Kbb, B);
+        a = search_cells<true, kRows>(pos[i], i, g, bd.start + base, bd.end + base, bd.id, bd.spos, nbb, Kbb, B);
         cbb[i] = a;
     }
     const uint32_t cnt[1] = {a};
@@ -753,7 +766,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_ref(const float4* __restri
         for (uint32_t t = 0; t < sc.S; t++) {
             if (t == sid) continue;
             const uint32_t at = k < Kfr ? k : Kfr;  // entries past the capacity are counted, not written
-            k += search_cells<false, true>(xi, i, g, fl.start + size_t(t) * C, fl.end + size_t(t) * C, nullptr, fl.spos,
+            k += search_cells<false, kCols>(xi, i, g, fl.start + size_t(t) * C, fl.end + size_t(t) * C, nullptr, fl.spos,
                                            nfr + size_t(at) * N, Kfr - at, N);
         }
     }

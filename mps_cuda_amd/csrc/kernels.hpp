@@ -80,7 +80,9 @@ struct Scenes {
     uint32_t S;                 // scenes
 };
 
-// Column-major ELL neighbour lists: nbr[k*N + i], k < cnt[i]. fr/cfr: the ref lists into the
+// ELL neighbour lists, k < cnt[i]: the fluid list ff, and every array stored per entry of it, keeps
+// groups of four entries of a slot side by side (ell(), device_common.hpp; capacities are multiples
+// of 4); the wall list fb and the ref list fr are column-major, nbr[k*N + i]. fr/cfr: the ref lists into the
 // other scenes when the scenes are coupled fluid objects (null otherwise).
 struct Nbr {
     const uint32_t* ff;
@@ -97,7 +99,7 @@ constexpr uint32_t kMaxWallObjects = 4;
 
 // Block halos of the fluid-fluid lists (halo.hip): for workgroup b of slots, idx[b*kHaloCap + t]
 // (t < n[b]) are the distinct neighbour slots in ascending order and nb16[k*N + i] is the
-// position of nff[k*N + i] in its block's list. n[b] > kHaloCap: not staged (use nff).
+// position of nff's entry in its block's list (same place). n[b] > kHaloCap: not staged (use nff).
 // Each staged kernel stages the halos up to its own LDS depth and gathers deeper ones from
 // global memory. A.p comes in two depths: kHaloShallow (five workgroups per CU) and kHaloCap
 // (four); the deep one pays once a few blocks in a thousand have halos over kHaloShallow.
@@ -107,6 +109,7 @@ struct Halo {
     const uint32_t* idx;
     const uint32_t* n;
     const uint16_t* nb16;
+    bool deep = false;  // enough halos are over kHaloShallow for the kernels' deep forms
 };
 
 namespace launch {
@@ -215,9 +218,9 @@ void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, 
                     hipStream_t s);
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
                float4* cgx, hipStream_t s);
-// pair coefficients of the implicit operator: a_ij into ca and/or (a_ij, b_ij) into cab (either may be null)
+// pair coefficients of the implicit operator: a_ij into ca, b_ij into cb (may be null)
 void cg_setup(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* rho,
-              const float* fst, float* ca, float2* cab, float4* cgb, float* irho, hipStream_t s);
+              const float* fst, float* ca, float* cb, float4* cgb, float* irho, hipStream_t s);
 // The adjoint's transposed solve keeps p in 32-byte records with the position:
 // rec[2i] = (x, y, z, p.x), rec[2i+1] = (p.y, p.z, 0, 0)
 void cg_pack(uint32_t N, const float4* pos, const float4* x0, float4* rec, hipStream_t s);
@@ -225,14 +228,14 @@ void cg_pack(uint32_t N, const float4* pos, const float4* x0, float4* rec, hipSt
 // mode 0: A x0 with f = 0 (x0 from the float4 array x0), then r = b - A x0, pout = r, x = x0, partial r.r;
 // mode 1: p = r + beta pprev (r in rr, beta from the record), A p with f into Ap, p into pout,
 // partial p.Ap. Halo records are staged in LDS (kHaloCap).
-// The implicit operator's coefficients: streamed (a_ij, b_ij) pairs (cab), or a_ij (ca) with
-// b_ij recomputed from positions, masses (vel.w) and 1/rho (irho) of the CG set-up.
+// The implicit operator's coefficients per list entry: a_ij (ca), and b_ij streamed too (cb) or
+// recomputed from positions, masses (vel.w) and 1/rho (irho) of the CG set-up.
 struct CgOperator {
     int recompute = 0;
     int cubic = 1;
     int deep = 0;  // the streamed operator stages halos up to kHaloCap (else kHaloShallow)
-    const float2* cab = nullptr;
     const float* ca = nullptr;
+    const float* cb = nullptr;
     const float4* vel = nullptr;
     const float* rho = nullptr;
     const float* irho = nullptr;
@@ -315,10 +318,11 @@ void adj_dbar(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, con
               const float* bvol, const float4* bvel, const float* pG_ff, const float* pG_fb, const float* dbar, const uint32_t* L, uint32_t it,
               float4* av, float4* ax, hipStream_t s);
 void adj_rev_index(const Scenes& sc, const Nbr& nb, uint32_t* rev, uint32_t* bad, hipStream_t s);
-void adj_transpose_coeffs(const Scenes& sc, const Nbr& nb, const uint32_t* rev, const float2* cab, float2* cabT, hipStream_t s);
+void adj_transpose_coeffs(const Scenes& sc, const Nbr& nb, const uint32_t* rev, const float* ca, const float* cb, float* caT, float* cbT,
+                          hipStream_t s);
 void adj_cg_init(const Scenes& sc, const float4* pos, const float4* b, float4* x, float4* r, float4* rec, double* partials,
                  hipStream_t s);
-void adj_cg_applyT(const Scenes& sc, const Nbr& nb, const float2* cab, const float2* cabT, const float4* rec, float4* Ap,
+void adj_cg_applyT(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* rec, float4* Ap,
                    const SolverDev* st, double* partials, hipStream_t s);
 // partials: 2 * ceil(N / kBlock) doubles (mubar, sigmabar per workgroup)
 void adj_cg_grad(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vin, const float4* vstar, const float* rho,
@@ -335,7 +339,7 @@ void adj_density(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, 
 void adj_unpermute(uint32_t n, const uint32_t* src, const float4* ax, const float4* av, const float4* al, float4* ax_out,
                    float4* av_out, float4* al_out, hipStream_t s);
 // warm start of A_f^T lambda = b from x0 (packed in recA with the positions): partials of r.r and b.b
-void adj_cg_init_warm(const Scenes& sc, const Nbr& nb, const float2* cab, const float2* cabT, const float4* recA,
+void adj_cg_init_warm(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* recA,
                       const float4* b, float4* x, float4* r, float4* recB, double* partials, hipStream_t s);
 void adj_fold_start(const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, hipStream_t s);
 // adx[s] += gx[perm[s]], adv[s] += gv[perm[s]] (gx, gv: n_ref x 3 floats in reference order; gv may be

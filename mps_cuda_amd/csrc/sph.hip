@@ -1,7 +1,7 @@
 // sph.hip — DFSPH / implicit viscosity / advection kernels for gfx950.
 //
-// One thread per particle walks its column-major ELL neighbour lists (fluid then
-// boundary), accumulating in registers in the reference's order, so a per-particle
+// One thread (or, in small grids, four lanes) per particle walks its ELL neighbour lists (fluid
+// then boundary), accumulating in registers in the reference's order, so a per-particle
 // result equals (0 + fluid sum) + boundary sum exactly as the reference's two kernels and
 // AtomicAdd produce it. Passes that the reference splits into several kernels over the
 // same neighbour list are fused (density + alpha + gravity; delta + stiffness + error
@@ -27,31 +27,41 @@ namespace mps {
 namespace dev {
 
 __device__ __forceinline__ uint32_t nbr_ff(const Nbr& nb, uint32_t k, uint32_t i, uint32_t N) {
-    return nb.ff[size_t(k) * N + i];
+    return nb.ff[ell(k, i, N)];
 }
 __device__ __forceinline__ uint32_t nbr_fb(const Nbr& nb, uint32_t k, uint32_t i, uint32_t N) {
     return nb.fb[size_t(k) * N + i];
 }
 
 // Walks the wall list of slot i in list order, kWallBatch entries at a time: the batch's
-// indices are loaded together, then gather(j, slot) fetches each entry's wall record, and only
-// then does use(k, j, slot, record) consume them in order. A batch costs about one dependent
-// memory latency instead of two per entry.
+// indices are loaded together, then gather(j, entry) fetches each entry's wall record, and only
+// then does use(true, entry, record) consume them in order. A batch costs about one dependent
+// memory latency instead of two per entry. With a quad per slot (Q = 4) lane part l handles the
+// batch's entry l, and use(false, ...) is called in the lanes past the list's end, whose term has
+// to be +0.
 constexpr uint32_t kWallBatch = 4;
-template <class Gather, class Use>
-__device__ __forceinline__ void walk_walls(const Nbr& nb, uint32_t i, uint32_t N, uint32_t cb, Gather&& gather, Use&& use) {
+template <int Q, class Gather, class Use>
+__device__ __forceinline__ void walk_walls(const Nbr& nb, uint32_t i, uint32_t l, uint32_t N, uint32_t cb, Gather&& gather, Use&& use) {
     using Rec = decltype(gather(0u, size_t(0)));
     for (uint32_t k0 = 0; k0 < cb; k0 += kWallBatch) {
-        uint32_t j[kWallBatch];
+        if constexpr (Q == 4) {
+            const bool in = k0 + l < cb;
+            const uint32_t k = in ? k0 + l : k0;
+            const size_t entry = size_t(k) * N + i;
+            const Rec w = gather(nbr_fb(nb, k, i, N), entry);
+            use(in, entry, w);
+        } else {
+            uint32_t j[kWallBatch];
 #pragma unroll
-        for (uint32_t q = 0; q < kWallBatch; q++) j[q] = k0 + q < cb ? nbr_fb(nb, k0 + q, i, N) : 0u;
-        Rec w[kWallBatch];
+            for (uint32_t q = 0; q < kWallBatch; q++) j[q] = k0 + q < cb ? nbr_fb(nb, k0 + q, i, N) : 0u;
+            Rec w[kWallBatch];
 #pragma unroll
-        for (uint32_t q = 0; q < kWallBatch; q++)
-            if (k0 + q < cb) w[q] = gather(j[q], size_t(k0 + q) * N + i);
+            for (uint32_t q = 0; q < kWallBatch; q++)
+                if (k0 + q < cb) w[q] = gather(j[q], size_t(k0 + q) * N + i);
 #pragma unroll
-        for (uint32_t q = 0; q < kWallBatch; q++)
-            if (k0 + q < cb) use(k0 + q, j[q], size_t(k0 + q) * N + i, w[q]);
+            for (uint32_t q = 0; q < kWallBatch; q++)
+                if (k0 + q < cb) use(true, size_t(k0 + q) * N + i, w[q]);
+        }
     }
 }
 
@@ -115,57 +125,240 @@ __device__ __forceinline__ double fold(const double* __restrict__ partials, uint
     return block_sum_d(s, lds);
 }
 
-// Fluid-fluid list entries each thread keeps in flight in the halo-staged kernels (their
-// occupancy is bounded by LDS, so registers are free for it). The 16-bit halo positions are
-// read with ordinary loads: they are reused by every solver iteration and stay in the
-// memory-side cache, while the larger per-pair coefficient streams are read non-temporally.
-constexpr uint32_t kListBatch = 4;       // once-per-step walks (density/alpha, ST factor, CG setup)
-constexpr uint32_t kListBatchSolve = 2;  // solver iterations (DF/CD evaluate and apply, A.p): measured best
-// A.p loads its first entries before staging the halo (a multiple of kListBatchSolve). Measured
-// on the 1M dam break, one run: 4 / 8 / 12 / 16 entries give 89.3 / 86.5 / 89.3 / 94.1 us per A.p.
-constexpr uint32_t kListPrefetchApply = 8;
-constexpr uint32_t kListBatchAp = kListBatchSolve;  // A.p's entries in flight after the prefetch
-// The entries the DF/CD evaluation and the pressure apply load before their halo staging (a
-// multiple of kListBatchSolve). Measured on the 1M dam break, one run: the evaluation takes
-// 91 / 75 / 88 us with 2 / 4 / 8.
-constexpr uint32_t kListPrefetchEval = 4;
-constexpr uint32_t kListPrefetchPressure = 4;
-static_assert(kListPrefetchEval % kListBatchSolve == 0 && kListPrefetchPressure % kListBatchSolve == 0,
-              "the batches after the prefetch stay aligned");
-static_assert(kListPrefetchApply % kListBatchAp == 0, "the batches after the prefetch stay aligned");
-
-// Calls body(t, s) for every halo record t < H (s = its slot), with R slots per thread loaded
-// ahead so the bodies' loads can be in flight together.
-template <uint32_t R, typename F>
-__device__ __forceinline__ void for_halo(const uint32_t* __restrict__ hs, uint32_t H, F&& body) {
-    for (uint32_t t0 = threadIdx.x; t0 < H; t0 += R * blockDim.x) {
-        uint32_t s[R];
-#pragma unroll
-        for (uint32_t q = 0; q < R; q++) {
-            const uint32_t t = t0 + q * blockDim.x;
-            s[q] = t < H ? hs[t] : 0u;
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < R; q++) {
-            const uint32_t t = t0 + q * blockDim.x;
-            if (t < H) body(t, s[q]);
-        }
-    }
-}
-
 // Halo count of workgroup blk: > kHaloCap (not staged) when there are no halos (hl.n null: the
 // adjoint's kernels run on its taped lists).
 __device__ __forceinline__ uint32_t halo_count(const Halo& hl, uint32_t blk) { return hl.n ? hl.n[blk] : kHaloCap + 1u; }
 
+// ---- walks of the fluid lists
+// The fluid lists, and everything stored per list entry, keep the four entries 4g .. 4g+3 of a
+// slot side by side (ell(), device_common.hpp). With one lane per slot (Q = 1) a lane loads a group
+// of four at once: 8 bytes of halo positions, 16 of G_ij, 16 each of a_ij and b_ij. Against one
+// entry per load (columns, two entries in flight) a walk waits for a quarter of the round trips and
+// issues a quarter of the loads and addresses: A.p 25 -> 15 us at 45k particles (66 neighbours each),
+// 85 -> 70 us at 525k (61), 76 -> 73 us at 1M (31; there the stream itself is the bound, and the
+// unused entries of the last groups cost 5 % more bytes). With a quad per slot
+// (Q = 4) lane part l of the quad takes entry 4g + l of every group, and the group's four terms
+// are added to the running sum one after the other, in list order, by every lane of the quad
+// (add_quad): a sum has the same bits in both forms. An entry past the end of the list
+// contributes +0 there; the sums start at +0 (or a positive term), and x + 0 = x, x - 0 = x for
+// every value that such a sum can take.
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+template <int L>
+__device__ __forceinline__ float quad_lane(float v) {  // the value of lane L of the quad, by DPP
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), L * 0x55, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float add_quad(float s, float t) {
+    return (((s + quad_lane<0>(t)) + quad_lane<1>(t)) + quad_lane<2>(t)) + quad_lane<3>(t);
+}
+__device__ __forceinline__ f3 add_quad(f3 s, f3 t) { return {add_quad(s.x, t.x), add_quad(s.y, t.y), add_quad(s.z, t.z)}; }
+
+__device__ __forceinline__ float sub_quad(float s, float t) {
+    return (((s - quad_lane<0>(t)) - quad_lane<1>(t)) - quad_lane<2>(t)) - quad_lane<3>(t);
+}
+__device__ __forceinline__ f3 sub_quad(f3 s, f3 t) { return {sub_quad(s.x, t.x), sub_quad(s.y, t.y), sub_quad(s.z, t.z)}; }
+template <int Q, class T>
+__device__ __forceinline__ T add_lanes(T s, T t) {
+    if constexpr (Q == 4) return add_quad(s, t);
+    else return s + t;
+}
+template <int Q, class T>
+__device__ __forceinline__ T sub_lanes(T s, T t) {
+    if constexpr (Q == 4) return sub_quad(s, t);
+    else return s - t;
+}
+// block_partial of a workgroup with a quad per slot (`v` counts in lane part 0): the slots'
+// values are put back one per lane of the first kBlock / 64 waves and reduced there in
+// block_sum_d's order, so the partial has the same bits.
+template <int Q, bool COH = false>
+__device__ __forceinline__ void slot_partial(double v, double* __restrict__ partials, uint32_t blk) {
+    if constexpr (Q == 1) {
+        block_partial<COH>(v, partials, blk);
+    } else {
+        static_assert(!COH, "the persistent solver runs one lane per slot");
+        __shared__ double pv[kBlock];
+        __shared__ double ws[kBlock / 64];
+        if (threadIdx.x % Q == 0) pv[threadIdx.x / Q] = v;
+        __syncthreads();
+        if (threadIdx.x < kBlock) {
+            double s = pv[threadIdx.x];
+            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+            if ((threadIdx.x & 63u) == 0) ws[threadIdx.x >> 6] = s;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double s = 0.0;
+            for (int w = 0; w < kBlock / 64; w++) s += ws[w];
+            partials[blk] = s;
+        }
+    }
+}
+
+// The neighbours named by one group (Q = 1) or by this lane's entry of it (Q = 4): positions in
+// the block's halo (STAGED) or slots.
+template <int Q, bool STAGED>
+struct GroupIdx;
+template <>
+struct GroupIdx<1, true> {
+    uint2 w;
+    __device__ __forceinline__ void load(const Nbr&, const Halo& hl, size_t group, uint32_t) {
+        w = reinterpret_cast<const uint2*>(hl.nb16)[group];
+    }
+    __device__ __forceinline__ uint32_t at(int e) const { return e < 2 ? (e ? w.x >> 16 : w.x & 0xFFFFu) : (e == 3 ? w.y >> 16 : w.y & 0xFFFFu); }
+};
+template <>
+struct GroupIdx<1, false> {
+    v4u w;
+    __device__ __forceinline__ void load(const Nbr& nb, const Halo&, size_t group, uint32_t) {
+        w = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(nb.ff) + group);
+    }
+    __device__ __forceinline__ uint32_t at(int e) const { return w[e]; }
+};
+template <bool STAGED>
+struct GroupIdx<4, STAGED> {
+    uint32_t w;
+    __device__ __forceinline__ void load(const Nbr& nb, const Halo& hl, size_t group, uint32_t l) {
+        if constexpr (STAGED) w = hl.nb16[4 * group + l];
+        else w = __builtin_nontemporal_load(nb.ff + 4 * group + l);
+    }
+    __device__ __forceinline__ uint32_t at(int) const { return w; }
+};
+// A float stored per entry, streamed with non-temporal loads; GroupAB: two such arrays. (The
+// coefficients a_ij and b_ij are two arrays and not pairs, so that each of a lane's 16-byte loads
+// belongs to a contiguous kilobyte of the wave: with pairs, two loads touch every line, and the
+// line is fetched twice.)
+template <int Q>
+struct GroupVal {
+    typename std::conditional<Q == 1, v4f, float>::type v;
+    __device__ __forceinline__ void load(const float* p, const float*, size_t group, uint32_t l) {
+        if constexpr (Q == 1) v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p) + group);
+        else v = __builtin_nontemporal_load(p + 4 * group + l);
+    }
+    __device__ __forceinline__ float at(int e) const {
+        if constexpr (Q == 1) return v[e];
+        else return v;
+    }
+};
+template <int Q>
+struct GroupAB {
+    GroupVal<Q> a, b;
+    __device__ __forceinline__ void load(const float* pa, const float* pb, size_t group, uint32_t l) {
+        a.load(pa, nullptr, group, l);
+        b.load(pb, nullptr, group, l);
+    }
+};
+struct NoVal {
+    __device__ __forceinline__ void load(const float*, const float*, size_t, uint32_t) {}
+};
+
+// Groups requested before the halo staging, and halo records that a thread stages per pass. A.p
+// at 1M particles (31 neighbours each), one run: 1 group and 2 records 73.3 us, 2 and 2 74.7,
+// 1 and 4 75.8, 2 and 4 77.0 (with 4 records the evaluation and the density are 1-3 us faster).
+constexpr int kPreApply = 1, kPreEval = 1, kPrePressure = 1;  // one lane per slot
+constexpr int kPreQuad = 8;                                   // a quad per slot
+template <int Q>
+constexpr uint32_t kHaloLoads = Q == 1 ? 4 : 2;
+constexpr uint32_t kHaloLoadsApply = 2;
+
+// A walk over the c entries of one slot: whole groups in order, one being loaded ahead of the one
+// in use, then the rest (c % 4). begin() requests the first PRE groups and the rest, so that these
+// loads run beside the halo staging between begin() and run(). full(group number, indices, values)
+// and rest(group number, indices, values, c % 4) consume them.
+template <int Q, bool STAGED, class Val, int PRE>
+struct Walk {
+    using Idx = GroupIdx<Q, STAGED>;
+    Idx ip[PRE], ir;
+    Val vp[PRE], vr;
+    const Nbr& nb;
+    const Halo& hl;
+    const float *val, *val2;  // the arrays that Val reads
+    uint32_t i, l, N, gf, nr;
+    __device__ __forceinline__ Walk(const Nbr& nb, const Halo& hl, const float* val, const float* val2, uint32_t i, uint32_t l,
+                                    uint32_t N, uint32_t c)
+        : nb(nb), hl(hl), val(val), val2(val2), i(i), l(l), N(N), gf(c >> 2), nr(c & 3u) {
+#pragma unroll
+        for (uint32_t g = 0; g < PRE; g++)
+            if (g < gf) get(g, ip[g], vp[g]);
+        if (nr) get(gf, ir, vr);
+    }
+    __device__ __forceinline__ void get(uint32_t g, Idx& x, Val& v) const {
+        const size_t group = size_t(g) * N + i;
+        x.load(nb, hl, group, l);
+        v.load(val, val2, group, l);
+    }
+    template <class Full, class Rest>
+    __device__ __forceinline__ void run(Full&& full, Rest&& rest) {
+        Idx xn;
+        Val vn;
+        if (PRE < gf) get(PRE, xn, vn);
+#pragma unroll
+        for (uint32_t g = 0; g < PRE; g++)
+            if (g < gf) full(g, ip[g], vp[g]);
+        for (uint32_t g = PRE; g < gf; g++) {
+            const Idx x = xn;
+            const Val v = vn;
+            if (g + 1 < gf) get(g + 1, xn, vn);
+            full(g, x, v);
+        }
+        if (nr) rest(gf, ir, vr, nr);
+    }
+};
+
+// What every halo-staged kernel requests first: these loads depend on the workgroup's number
+// alone, so the kernel waits for two memory latencies (these, then what they lead to) and not for
+// one per lookup. The first halo slots are read before the halo's size is known (a row always has
+// kHaloCap words); padding slots have a list length of 0.
+template <int Q, uint32_t R>
+struct BlockHead {
+    static constexpr uint32_t kThreads = Q * kBlock;
+    uint32_t i, l, c, H;
+    const uint32_t* hs;
+    uint32_t sh[R];
+    __device__ __forceinline__ BlockHead(uint32_t blk, uint32_t N, const uint32_t* cff, const Halo& hl) {
+        i = blk * kBlock + threadIdx.x / Q;
+        l = threadIdx.x % Q;
+        c = i < N ? cff[i] : 0u;
+        H = halo_count(hl, blk);
+        hs = hl.idx + size_t(blk) * kHaloCap;
+#pragma unroll
+        for (uint32_t q = 0; q < R; q++) {
+            const uint32_t t = threadIdx.x + q * kThreads;
+            sh[q] = hl.n && t < kHaloCap ? hs[t] : 0u;
+        }
+    }
+    // store(t, load(s)) for every halo record t < H (s = its slot): R records per thread and
+    // pass, all their loads before the first LDS store (past the halo's end a thread loads slot 0
+    // and stores nothing).
+    template <class Load, class Store>
+    __device__ __forceinline__ void stage(Load&& load, Store&& store) const {
+        using Rec = decltype(load(0u));
+        for (uint32_t t0 = threadIdx.x; t0 < H; t0 += R * kThreads) {
+            Rec rec[R];
+#pragma unroll
+            for (uint32_t q = 0; q < R; q++) {
+                const uint32_t t = t0 + q * kThreads;
+                rec[q] = load(t < H ? (t0 == threadIdx.x ? sh[q] : hs[t]) : 0u);
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < R; q++) {
+                const uint32_t t = t0 + q * kThreads;
+                if (t < H) store(t, rec[q]);
+            }
+        }
+    }
+};
+
 // LDS staging depth (records per workgroup, <= kHaloCap) of each halo-staged kernel: with wide
 // records the depth decides how many workgroups share a CU's 160 KiB. A block with a deeper halo
-// gathers from global memory instead, with the same results. On the 1M dam break:
-// DF/CD evaluation, 24-byte records: 1104 -> 26.5 KB, six per CU (1264: five), 90 -> 82 us;
-// CG setup, 36-byte records: 1104 -> 39.7 KB, four per CU (1264: three), 213 -> 191 us;
-// A.p, 24-byte records: kHaloShallow = 1264 -> 30.3 KB, five per CU (1136, six per CU, was
-// slower: its blocks over the depth cost more than a sixth workgroup gains), or kHaloCap when the
-// host sees enough deeper halos (kernels.hpp).
-constexpr uint32_t kStageEval = 1104;
+// gathers from global memory instead, with the same results. A.p and the DF/CD evaluation
+// (24-byte records) stage kHaloShallow = 1264 records (30.3 KB, five workgroups per CU) or, when
+// the host sees enough deeper halos (Halo::deep), kHaloCap = 1536 (36.9 KB, four): near rest
+// density a block's halo holds ~1400 slots, and gathering them costs the evaluation 198 us
+// instead of 54 (525k particles at 0.95 of the rest density). The CG setup (36-byte records)
+// stages 1104 (39.7 KB, four per CU) or, with deep halos, runs its quad form at kHaloCap (54 KB:
+// 260 -> 160 us there). The quad forms of all three stage kHaloCap.
+constexpr uint32_t kStageEval = kHaloShallow;
 constexpr uint32_t kStageSetup = 1104;
 constexpr uint32_t kStageAp = kHaloShallow;
 constexpr uint32_t kStageDensity = kHaloShallow, kStageST = kHaloShallow, kStagePApply = kHaloShallow;
@@ -253,77 +446,114 @@ __global__ void __launch_bounds__(kBlock) k_boundary_volume_obj(const float4* __
 // ComputeDFSPHFactor_kernel ff/fb + Final (MPSSPHDFSPHUtil.cuh:10-137),
 // ApplyGravity + UpdateVelocity (MPSAdvectUtil.cuh:8-34).
 // Also stores G_ij per neighbour slot (pG_ff, pG_fb) when kDoPairs is set.
-template <bool CUBIC, bool REF, bool BOBJ>
-__global__ void __launch_bounds__(kBlock) k_density_alpha(int flags, Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
+template <bool CUBIC, bool REF, bool BOBJ, int Q>
+__global__ void __launch_bounds__(Q * kBlock) k_density_alpha(int flags, Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                         float4* __restrict__ vel, const float4* __restrict__ bpos,
                                                         const float* __restrict__ bvol, float* __restrict__ rho,
                                                         float* __restrict__ alpha, float4* __restrict__ color,
                                                         float* __restrict__ pG_ff, float* __restrict__ pG_fb) {
+    static_assert(Q == 1 || !(REF || BOBJ), "coupled scenes and wall objects run one lane per slot");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const uint32_t sid = sc.blk_scene[blk];
-    const StepParams P = sc.P[sid];
-    const uint32_t i = blk * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
-    const bool live = i < P.end;
+    const uint32_t N = sc.N;
     const bool dens = flags & launch::kDoDensity, alph = flags & launch::kDoAlpha;
     const bool pairs = flags & launch::kDoPairs;
     const bool walk = dens || alph || pairs;
-    const uint32_t c = live && walk ? nb.cff[i] : 0u;
     // the block's halo positions in LDS (see k_cg_apply)
     __shared__ float4 la[kStageDensity];
-    const uint32_t H = halo_count(hl, blk);
-    const bool staged = walk && H <= kStageDensity;
-    constexpr uint32_t U = kListBatch;
-    uint32_t jn[U];
-    auto fetch = [&](uint32_t k0) {
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            if (k0 + q < c) {
-                const size_t slot = size_t(k0 + q) * N + i;
-                jn[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-            }
-        }
-    };
-    fetch(0);
-    if (staged) {
-        const uint32_t* hs = hl.idx + size_t(blk) * kHaloCap;
-        for_halo<4>(hs, H, [&](uint32_t t, uint32_t s) { la[t] = pos[s]; });
-        __syncthreads();
-    }
-    if (!live) return;
-    const float4 xi4 = pos[i];
+    BlockHead<Q, kHaloLoads<Q>> hd(blk, N, nb.cff, hl);
+    const uint32_t i = hd.i, l = hd.l, c = walk ? hd.c : 0u;
+    const uint32_t cb = walk && i < N ? nb.cfb[i] : 0u;
+    const float4 xi4 = i < N ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t sid = sc.blk_scene[blk];
+    const StepParams P = sc.P[sid];
+    const bool live = i < P.end;
     const f3 xi = mk(xi4);
     const float hi = xi4.w * 4.0f;
     const float invHi = 1.0f / hi;
     float sf = dens ? P.V * Wk<CUBIC>(0.0f, invHi) : 0.0f;
     f3 gf{0.f, 0.f, 0.f};
     float s = 0.0f;
-    if (walk) {
-        auto pair = [&](uint32_t k, float4 xj4) {
-            const f3 xij = xi - mk(xj4);
-            const float dist = len3(xij);
-            if (dens) sf += P.V * Wk<CUBIC>(dist, invHi);
-            if (alph || pairs) {
-                const float G = Gk<CUBIC>(dist, invHi);
-                if (pairs) pG_ff[size_t(k) * N + i] = G;
-                const f3 grad = (P.V * G) * xij;
-                gf = gf + grad;
-                s += dot3(grad, grad);
-            }
-        };
-        for (uint32_t k = 0; k < c; k += U) {
-            uint32_t j[U];
-#pragma unroll
-            for (uint32_t q = 0; q < U; q++) j[q] = jn[q];
-            if (k + U < c) fetch(k + U);
-            if (staged) {
-#pragma unroll
-                for (uint32_t q = 0; q < U; q++)
-                    if (k + q < c) pair(k + q, la[j[q]]);
-            } else {
-                for (uint32_t q = 0; q < U && k + q < c; q++) pair(k + q, pos[j[q]]);
-            }
+    // terms of one pair; W, G, grad and its square
+    struct Term {
+        float w, G, s2;
+        f3 g;
+    };
+    auto term = [&](f3 xj) -> Term {
+        Term t{0.f, 0.f, 0.f, {0.f, 0.f, 0.f}};
+        const f3 xij = xi - xj;
+        const float dist = len3(xij);
+        if (dens) t.w = P.V * Wk<CUBIC>(dist, invHi);
+        if (alph || pairs) {
+            t.G = Gk<CUBIC>(dist, invHi);
+            t.g = (P.V * t.G) * xij;
+            t.s2 = dot3(t.g, t.g);
         }
+        return t;
+    };
+    auto walk_fluid = [&](auto staged) {
+        constexpr bool STAGED = decltype(staged)::value;
+        Walk<Q, STAGED, NoVal, 1> wk(nb, hl, nullptr, nullptr, i, l, N, live ? c : 0u);
+        if constexpr (STAGED) {
+            hd.stage([&](uint32_t j) { return pos[j]; }, [&](uint32_t t, const float4& x) { la[t] = x; });
+            __syncthreads();
+        }
+        auto at = [&](uint32_t j) { return mk(STAGED ? la[j] : pos[j]); };
+        wk.run(
+            [&](uint32_t g, const auto& x, const NoVal&) {
+                const size_t group = size_t(g) * N + i;
+                if constexpr (Q == 1) {
+                    f3 xj[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) xj[e] = at(x.at(e));
+                    v4f G;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const Term t = term(xj[e]);
+                        sf += t.w;
+                        gf = gf + t.g;
+                        s += t.s2;
+                        G[e] = t.G;
+                    }
+                    if (pairs) reinterpret_cast<v4f*>(pG_ff)[group] = G;
+                } else {
+                    const Term t = term(at(x.at(0)));
+                    sf = add_quad(sf, t.w);
+                    gf = add_quad(gf, t.g);
+                    s = add_quad(s, t.s2);
+                    if (pairs) pG_ff[4 * group + l] = t.G;
+                }
+            },
+            [&](uint32_t g, const auto& x, const NoVal&, uint32_t n) {
+                const size_t group = size_t(g) * N + i;
+                if constexpr (Q == 1) {
+#pragma unroll
+                    for (int e = 0; e < 3; e++) {
+                        if (e < int(n)) {
+                            const Term t = term(at(x.at(e)));
+                            sf += t.w;
+                            gf = gf + t.g;
+                            s += t.s2;
+                            if (pairs) pG_ff[4 * group + e] = t.G;
+                        }
+                    }
+                } else {
+                    Term t{0.f, 0.f, 0.f, {0.f, 0.f, 0.f}};
+                    if (l < n) {
+                        t = term(at(x.at(0)));
+                        if (pairs) pG_ff[4 * group + l] = t.G;
+                    }
+                    sf = add_quad(sf, t.w);
+                    gf = add_quad(gf, t.g);
+                    s = add_quad(s, t.s2);
+                }
+            });
+    };
+    if (walk) {
+        if (hd.H <= kStageDensity) walk_fluid(std::true_type{});
+        else walk_fluid(std::false_type{});
+    }
+    if (!live) return;
+    if (walk) {
         float sb = 0.0f;
         f3 gb{0.f, 0.f, 0.f};
         float sbo[kMaxWallObjects] = {0.f, 0.f, 0.f, 0.f};  // per wall object (BOBJ)
@@ -333,30 +563,28 @@ __global__ void __launch_bounds__(kBlock) k_density_alpha(int flags, Scenes sc, 
             float vb;
             uint32_t o;
         };
-        walk_walls(nb, i, N, nb.cfb[i],
+        walk_walls<Q>(nb, i, l, N, cb,
                    [&](uint32_t j, size_t) { return WallRec{bpos[j], bvol[j], BOBJ ? nb.fbo[j] : 0u}; },
-                   [&](uint32_t, uint32_t, size_t slot, const WallRec& w) {
+                   [&](bool in, size_t slot, const WallRec& w) {
             const f3 xij = xi - mk(w.x);
             const float dist = len3(xij);
             const float vb = w.vb;
+            float wk = 0.0f, G = 0.0f;
+            f3 gg{0.f, 0.f, 0.f};
+            if (in) {
+                if (dens) wk = vb * Wk<CUBIC>(dist, invHi);
+                if (alph || pairs) {
+                    G = Gk<CUBIC>(dist, invHi);
+                    gg = (vb * G) * xij;
+                    if (pairs) pG_fb[slot] = G;
+                }
+            }
             if constexpr (BOBJ) {
-                if (dens) {
-                    const float wk = vb * Wk<CUBIC>(dist, invHi);
-                    at_obj(sbo, w.o, [&](float& a) { a += wk; });
-                }
-                if (alph || pairs) {
-                    const float G = Gk<CUBIC>(dist, invHi);
-                    if (pairs) pG_fb[slot] = G;
-                    const f3 gg = (vb * G) * xij;
-                    at_obj(gbo, w.o, [&](f3& a) { a = a + gg; });
-                }
+                at_obj(sbo, w.o, [&](float& a) { a += wk; });
+                at_obj(gbo, w.o, [&](f3& a) { a = a + gg; });
             } else {
-                if (dens) sb += vb * Wk<CUBIC>(dist, invHi);
-                if (alph || pairs) {
-                    const float G = Gk<CUBIC>(dist, invHi);
-                    if (pairs) pG_fb[slot] = G;
-                    gb = gb + (vb * G) * xij;
-                }
+                sb = add_lanes<Q>(sb, wk);
+                gb = add_lanes<Q>(gb, gg);
             }
         });
         // ((own + each ref object's sum, in scene order) + walls), as the reference's Sub
@@ -413,12 +641,12 @@ __global__ void __launch_bounds__(kBlock) k_density_alpha(int flags, Scenes sc, 
                 d += sb;
             }
             const float r = d * P.rho0;
-            rho[i] = r;
+            if (l == 0) rho[i] = r;
             const float ratio = r / P.rho0;
             const float blue = fminf(fmaxf(1.0f - ratio, 0.0f), 1.0f);
             const float green = fminf(fmaxf(ratio < 1.0f ? ratio : 1.0f - (ratio - 1.0f), 0.0f), 1.0f);
             const float red = fminf(fmaxf(ratio - 1.0f, 0.0f), 1.0f);
-            color[i] = make_float4(red, green, blue, 1.0f);
+            if (l == 0) color[i] = make_float4(red, green, blue, 1.0f);
         }
         if (alph) {
             if constexpr (BOBJ) {
@@ -429,10 +657,10 @@ __global__ void __launch_bounds__(kBlock) k_density_alpha(int flags, Scenes sc, 
                 g = g + gb;
             }
             a += dot3(g, g);
-            alpha[i] = a > kEps ? 1.0f / a : 0.0f;
+            if (l == 0) alpha[i] = a > kEps ? 1.0f / a : 0.0f;
         }
     }
-    if (flags & launch::kDoGravity) {
+    if (l == 0 && (flags & launch::kDoGravity)) {
         float4 v4 = vel[i];
         const float m = v4.w;
         const f3 F = f3{0.f, 0.f, 0.f} + f3{P.gx, P.gy, P.gz} * m;
@@ -452,99 +680,84 @@ __global__ void __launch_bounds__(kBlock) k_density_alpha(int flags, Scenes sc, 
 // alpha pass. Each workgroup publishes its sum of positive errors for k_fold_pressure.
 // The records of the block's halo (x_j, v_j) are staged in LDS (see k_cg_apply); the pairs
 // are summed in list order on both paths.
-template <bool DF, bool REF, bool CUBIC, bool BOBJ>
-__global__ void __launch_bounds__(kBlock) k_pressure_eval(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
+template <bool DF, bool REF, bool CUBIC, bool BOBJ, int Q, bool DEEP>
+__global__ void __launch_bounds__(Q * kBlock) k_pressure_eval(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                         const float4* __restrict__ vel, const float4* __restrict__ bpos,
                                                         const float* __restrict__ bvol, const float4* __restrict__ bvel,
                                                         const float* __restrict__ rho, const float* __restrict__ alpha,
                                                         const float* __restrict__ pG_ff, const float* __restrict__ pG_fb,
                                                         float* __restrict__ kappa, float* __restrict__ delta,
                                                         const SolverDev* st, double* __restrict__ partials) {
+    static_assert(Q == 1 || !(REF || BOBJ), "coupled scenes and wall objects run one lane per slot");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t N = sc.N;
+    constexpr uint32_t kDepth = DEEP ? kHaloCap : kStageEval;
+    __shared__ float4 la[kDepth];
+    __shared__ float2 lb[kDepth];
+    BlockHead<Q, kHaloLoads<Q>> hd(blk, N, nb.cff, hl);
+    const uint32_t i = hd.i, l = hd.l;
+    const bool in = i < N;
+    const uint32_t cb = in ? nb.cfb[i] : 0u;
+    const float4 xi4 = in ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const f3 vi = in ? mk(vel[i]) : f3{0.f, 0.f, 0.f};
+    const float rhoi = in ? rho[i] : 0.0f, alphai = in ? alpha[i] : 0.0f;
     const uint32_t sid = sc.blk_scene[blk];
-    const StepParams P = sc.P[sid];
     if (st[sid].done) return;  // this scene's loop has finished
-    const uint32_t i = blk * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
+    const StepParams P = sc.P[sid];
     const bool live = i < P.end;
-    const uint32_t c = live ? nb.cff[i] : 0u;
-    __shared__ float4 la[kStageEval];
-    __shared__ float2 lb[kStageEval];
-    const uint32_t H = hl.n[blk];
-    const bool staged = H <= kStageEval;
-    constexpr uint32_t U = kListBatchSolve;
-    uint32_t jn[U];
-    float gn[U];
-    auto fetch = [&](uint32_t k0) {
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            if (k0 + q < c) {
-                const size_t slot = size_t(k0 + q) * N + i;
-                jn[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-                gn[q] = __builtin_nontemporal_load(pG_ff + slot);
+    const f3 xi = mk(xi4);
+    float df = 0.0f;
+    using Val = GroupVal<Q>;
+    auto walk_fluid = [&](auto staged) {
+        constexpr bool STAGED = decltype(staged)::value;
+        Walk<Q, STAGED, Val, Q == 1 ? kPreEval : kPreQuad> wk(nb, hl, pG_ff, nullptr, i, l, N, hd.c);
+        struct Rec {
+            f3 x, v;
+        };
+        if constexpr (STAGED) {
+            hd.stage([&](uint32_t j) { return Rec{mk(pos[j]), mk(vel[j])}; },
+                     [&](uint32_t t, const Rec& r) {
+                         la[t] = make_float4(r.x.x, r.x.y, r.x.z, r.v.x);
+                         lb[t] = make_float2(r.v.y, r.v.z);
+                     });
+            __syncthreads();
+        }
+        auto at = [&](uint32_t j) -> Rec {
+            if constexpr (STAGED) {
+                const float4 a = la[j];
+                const float2 b = lb[j];
+                return {mk(a), {a.w, b.x, b.y}};
+            } else {
+                return {mk(pos[j]), mk(vel[j])};
             }
-        }
-    };
-    // the first kPre entries are loaded before the halo staging, as in A.p
-    constexpr uint32_t kPre = kListPrefetchEval;
-    uint32_t jp[kPre];
-    float gp[kPre];
+        };
+        auto term = [&](float G, const Rec& r) { return P.V * G * dot3(xi - r.x, vi - r.v); };
+        wk.run(
+            [&](uint32_t, const auto& x, const Val& G) {
+                if constexpr (Q == 1) {
+                    Rec r[4];
 #pragma unroll
-    for (uint32_t q = 0; q < kPre; q++) {
-        if (q < c) {
-            const size_t slot = size_t(q) * N + i;
-            jp[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-            gp[q] = __builtin_nontemporal_load(pG_ff + slot);
-        }
-    }
-    if (staged) {
-        const uint32_t* hs = hl.idx + size_t(blk) * kHaloCap;
-        for_halo<4>(hs, H, [&](uint32_t t, uint32_t s) {
-            const float4 x = pos[s], v = vel[s];
-            la[t] = make_float4(x.x, x.y, x.z, v.x);
-            lb[t] = make_float2(v.y, v.z);
-        });
-        __syncthreads();
-    }
+                    for (int e = 0; e < 4; e++) r[e] = at(x.at(e));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) df += term(G.at(e), r[e]);
+                } else {
+                    df = add_quad(df, term(G.at(0), at(x.at(0))));
+                }
+            },
+            [&](uint32_t, const auto& x, const Val& G, uint32_t n) {
+                if constexpr (Q == 1) {
+#pragma unroll
+                    for (int e = 0; e < 3; e++)
+                        if (e < int(n)) df += term(G.at(e), at(x.at(e)));
+                } else {
+                    df = add_quad(df, l < n ? term(G.at(0), at(x.at(0))) : 0.0f);
+                }
+            });
+    };
+    if (hd.H <= kDepth) walk_fluid(std::true_type{});
+    else walk_fluid(std::false_type{});
     double epos = 0.0;
     if (live) {
-        const f3 xi = mk(pos[i]), vi = mk(vel[i]);
-        float df = 0.0f;
-        if (kPre < c) fetch(kPre);
-#pragma unroll
-        for (uint32_t q = 0; q < kPre; q++) {
-            if (q < c) {
-                if (staged) {
-                    const float4 a = la[jp[q]];
-                    const float2 b = lb[jp[q]];
-                    df += P.V * gp[q] * dot3(xi - mk(a), vi - f3{a.w, b.x, b.y});
-                } else {
-                    df += P.V * gp[q] * dot3(xi - mk(pos[jp[q]]), vi - mk(vel[jp[q]]));
-                }
-            }
-        }
-        for (uint32_t k = kPre; k < c; k += U) {
-            uint32_t j[U];
-            float G[U];
-#pragma unroll
-            for (uint32_t q = 0; q < U; q++) {
-                j[q] = jn[q];
-                G[q] = gn[q];
-            }
-            if (k + U < c) fetch(k + U);
-            if (staged) {
-#pragma unroll
-                for (uint32_t q = 0; q < U; q++) {
-                    if (k + q < c) {
-                        const float4 a = la[j[q]];
-                        const float2 b = lb[j[q]];
-                        df += P.V * G[q] * dot3(xi - mk(a), vi - f3{a.w, b.x, b.y});
-                    }
-                }
-            } else {
-                for (uint32_t q = 0; q < U && k + q < c; q++) df += P.V * G[q] * dot3(xi - mk(pos[j[q]]), vi - mk(vel[j[q]]));
-            }
-        }
         float db = 0.0f;
         float dbo[kMaxWallObjects] = {0.f, 0.f, 0.f, 0.f};
         struct WallRec {
@@ -552,24 +765,21 @@ __global__ void __launch_bounds__(kBlock) k_pressure_eval(Scenes sc, Nbr nb, Hal
             float vb, G;
             uint32_t o;
         };
-        walk_walls(nb, i, N, nb.cfb[i],
+        walk_walls<Q>(nb, i, l, N, cb,
                    [&](uint32_t j, size_t slot) {
                        return WallRec{bpos[j], bvel[j], bvol[j], pG_fb[slot], BOBJ ? nb.fbo[j] : 0u};
                    },
-                   [&](uint32_t, uint32_t, size_t, const WallRec& w) {
+                   [&](bool in, size_t, const WallRec& w) {
             const f3 xij = xi - mk(w.x);
             const f3 vij = vi - mk(w.v);
-            if constexpr (BOBJ) {
-                const float t = w.vb * w.G * dot3(xij, vij);
-                at_obj(dbo, w.o, [&](float& a) { a += t; });
-            } else {
-                db += w.vb * w.G * dot3(xij, vij);
-            }
+            const float t = in ? w.vb * w.G * dot3(xij, vij) : 0.0f;
+            if constexpr (BOBJ) at_obj(dbo, w.o, [&](float& a) { a += t; });
+            else db = add_lanes<Q>(db, t);
         });
         float d = 0.0f;
         d += df;
         if constexpr (REF) {  // ComputeDensityDelta ref (MPSSPHDFSPHUtil.cuh:177-216): one sum per ref object
-            const float invHi = 1.0f / (pos[i].w * 4.0f);
+            const float invHi = 1.0f / (xi4.w * 4.0f);
             const uint32_t cr = nb.cfr[i];
             uint32_t cur = kEmpty;
             float Vt = 0.0f, dr = 0.0f;
@@ -595,24 +805,26 @@ __global__ void __launch_bounds__(kBlock) k_pressure_eval(Scenes sc, Nbr nb, Hal
         } else {
             d += db;
         }
-        delta[i] = d;
         float e;
         if (DF) {
             const float a = d * P.dt;
-            const float b = rho[i] / P.rho0 + P.dt * d - 0.8f;
+            const float b = rhoi / P.rho0 + P.dt * d - 0.8f;
             e = a < b ? a : b;
         } else {
-            e = rho[i] / P.rho0 + P.dt * d - 1.0f;
+            e = rhoi / P.rho0 + P.dt * d - 1.0f;
         }
         if (e > 0.0f) {
             epos = double(e);
-            e *= alpha[i] / (P.dt * P.dt);
+            e *= alphai / (P.dt * P.dt);
         } else {
             e = 0.0f;
         }
-        kappa[i] = e;
+        if (l == 0) {
+            delta[i] = d;
+            kappa[i] = e;
+        }
     }
-    block_partial(epos, partials, blk);
+    slot_partial<Q>(epos, partials, blk);
 }
 
 // Mean positive error and the loop decision of the DF/CD drivers
@@ -673,93 +885,73 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_pressure_joint(Scenes sc,
 
 // ApplyDFSPH_kernel ff/fb + ApplyDFSPHFinal_kernel (MPSSPHDFSPHUtil.cuh:342-468) + UpdateVelocity.
 // The halo's (x_j, kappa_j) are staged in LDS (see k_cg_apply).
-template <bool REF, bool CUBIC, bool BOBJ>
-__global__ void __launch_bounds__(kBlock) k_pressure_apply(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
+template <bool REF, bool CUBIC, bool BOBJ, int Q>
+__global__ void __launch_bounds__(Q * kBlock) k_pressure_apply(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                          float4* __restrict__ vel, const float4* __restrict__ bpos,
                                                          const float* __restrict__ bvol, const float* __restrict__ pG_ff,
                                                          const float* __restrict__ pG_fb, const float* __restrict__ kappa,
                                                          const SolverDev* st) {
+    static_assert(Q == 1 || !(REF || BOBJ), "coupled scenes and wall objects run one lane per slot");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const uint32_t sid = sc.blk_scene[blk];
-    const StepParams P = sc.P[sid];
-    if (st[sid].done) return;
-    const uint32_t i = blk * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
-    const bool live = i < P.end;
-    const uint32_t c = live ? nb.cff[i] : 0u;
+    const uint32_t N = sc.N;
     __shared__ float4 la[kStagePApply];
-    const uint32_t H = hl.n[blk];
-    const bool staged = H <= kStagePApply;
-    constexpr uint32_t U = kListBatchSolve;
-    uint32_t jn[U];
-    float gn[U];
-    auto fetch = [&](uint32_t k0) {
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            if (k0 + q < c) {
-                const size_t slot = size_t(k0 + q) * N + i;
-                jn[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-                gn[q] = __builtin_nontemporal_load(pG_ff + slot);
-            }
-        }
-    };
-    // the first kPre entries are loaded before the halo staging, as in A.p
-    constexpr uint32_t kPre = kListPrefetchPressure;
-    uint32_t jp[kPre];
-    float gp[kPre];
-#pragma unroll
-    for (uint32_t q = 0; q < kPre; q++) {
-        if (q < c) {
-            const size_t slot = size_t(q) * N + i;
-            jp[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-            gp[q] = __builtin_nontemporal_load(pG_ff + slot);
-        }
-    }
-    if (staged) {
-        const uint32_t* hs = hl.idx + size_t(blk) * kHaloCap;
-        for_halo<4>(hs, H, [&](uint32_t t, uint32_t s) {
-            const float4 x = pos[s];
-            la[t] = make_float4(x.x, x.y, x.z, kappa[s]);
-        });
-        __syncthreads();
-    }
-    if (!live) return;
-    const f3 xi = mk(pos[i]);
-    const float pi = kappa[i];
+    BlockHead<Q, kHaloLoads<Q>> hd(blk, N, nb.cff, hl);
+    const uint32_t i = hd.i, l = hd.l;
+    const bool in = i < N;
+    const uint32_t cb = in ? nb.cfb[i] : 0u;
+    const float4 xi4 = in ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 vi4 = in ? vel[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float pi = in ? kappa[i] : 0.0f;
+    const uint32_t sid = sc.blk_scene[blk];
+    if (st[sid].done) return;
+    const StepParams P = sc.P[sid];
+    const bool live = i < P.end;
+    const f3 xi = mk(xi4);
     f3 ff{0.f, 0.f, 0.f};
-    if (kPre < c) fetch(kPre);
-#pragma unroll
-    for (uint32_t q = 0; q < kPre; q++) {
-        if (q < c) {
-            if (staged) {
-                const float4 a = la[jp[q]];
-                ff = ff - 0.5f * P.V * (pi + a.w) * gp[q] * (xi - mk(a));
-            } else {
-                ff = ff - 0.5f * P.V * (pi + kappa[jp[q]]) * gp[q] * (xi - mk(pos[jp[q]]));
-            }
+    using Val = GroupVal<Q>;
+    auto walk_fluid = [&](auto staged) {
+        constexpr bool STAGED = decltype(staged)::value;
+        Walk<Q, STAGED, Val, Q == 1 ? kPrePressure : kPreQuad> wk(nb, hl, pG_ff, nullptr, i, l, N, hd.c);
+        auto rec = [&](uint32_t j) {
+            const float4 x = pos[j];
+            return make_float4(x.x, x.y, x.z, kappa[j]);
+        };
+        if constexpr (STAGED) {
+            hd.stage(rec, [&](uint32_t t, const float4& r) { la[t] = r; });
+            __syncthreads();
         }
-    }
-    for (uint32_t k = kPre; k < c; k += U) {
-        uint32_t j[U];
-        float G[U];
+        auto at = [&](uint32_t j) -> float4 {
+            if constexpr (STAGED) return la[j];
+            else return rec(j);
+        };
+        auto term = [&](float G, const float4& a) { return 0.5f * P.V * (pi + a.w) * G * (xi - mk(a)); };
+        wk.run(
+            [&](uint32_t, const auto& x, const Val& G) {
+                if constexpr (Q == 1) {
+                    float4 r[4];
 #pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            j[q] = jn[q];
-            G[q] = gn[q];
-        }
-        if (k + U < c) fetch(k + U);
-        if (staged) {
+                    for (int e = 0; e < 4; e++) r[e] = at(x.at(e));
 #pragma unroll
-            for (uint32_t q = 0; q < U; q++) {
-                if (k + q < c) {
-                    const float4 a = la[j[q]];
-                    ff = ff - 0.5f * P.V * (pi + a.w) * G[q] * (xi - mk(a));
+                    for (int e = 0; e < 4; e++) ff = ff - term(G.at(e), r[e]);
+                } else {
+                    ff = sub_quad(ff, term(G.at(0), at(x.at(0))));
                 }
-            }
-        } else {
-            for (uint32_t q = 0; q < U && k + q < c; q++) ff = ff - 0.5f * P.V * (pi + kappa[j[q]]) * G[q] * (xi - mk(pos[j[q]]));
-        }
-    }
+            },
+            [&](uint32_t, const auto& x, const Val& G, uint32_t n) {
+                if constexpr (Q == 1) {
+#pragma unroll
+                    for (int e = 0; e < 3; e++)
+                        if (e < int(n)) ff = ff - term(G.at(e), at(x.at(e)));
+                } else {
+                    f3 t{0.f, 0.f, 0.f};
+                    if (l < n) t = term(G.at(0), at(x.at(0)));
+                    ff = sub_quad(ff, t);
+                }
+            });
+    };
+    if (hd.H <= kStagePApply) walk_fluid(std::true_type{});
+    else walk_fluid(std::false_type{});
+    if (!live) return;
     f3 fb{0.f, 0.f, 0.f};
     f3 fbo[kMaxWallObjects] = {};
     struct WallRec {
@@ -767,18 +959,19 @@ __global__ void __launch_bounds__(kBlock) k_pressure_apply(Scenes sc, Nbr nb, Ha
         float vb, G;
         uint32_t o;
     };
-    walk_walls(nb, i, N, nb.cfb[i],
+    walk_walls<Q>(nb, i, l, N, cb,
                [&](uint32_t j, size_t slot) { return WallRec{bpos[j], bvol[j], pG_fb[slot], BOBJ ? nb.fbo[j] : 0u}; },
-               [&](uint32_t, uint32_t, size_t, const WallRec& w) {
+               [&](bool in, size_t, const WallRec& w) {
         const f3 xij = xi - mk(w.x);
-        const f3 fij = 0.5f * w.vb * pi * w.G * xij;
+        f3 fij{0.f, 0.f, 0.f};
+        if (in) fij = 0.5f * w.vb * pi * w.G * xij;
         if constexpr (BOBJ) at_obj(fbo, w.o, [&](f3& a) { a = a - fij; });
-        else fb = fb - fij;
+        else fb = sub_lanes<Q>(fb, fij);
     });
     f3 F{0.f, 0.f, 0.f};
     F = F + ff;
     if constexpr (REF) {  // ApplyDFSPH ref (MPSSPHDFSPHUtil.cuh:379-418): one sum per ref object
-        const float invHi = 1.0f / (pos[i].w * 4.0f);
+        const float invHi = 1.0f / (xi4.w * 4.0f);
         const uint32_t cr = nb.cfr[i];
         uint32_t cur = kEmpty;
         float Vt = 0.0f;
@@ -804,10 +997,10 @@ __global__ void __launch_bounds__(kBlock) k_pressure_apply(Scenes sc, Nbr nb, Ha
     } else {
         F = F + fb;
     }
-    float4 v4 = vel[i];
+    float4 v4 = vi4;
     const float m = v4.w;
     F = m * F;
-    if (m > 1.0e-10f) {
+    if (l == 0 && m > 1.0e-10f) {
         const float cdt = P.dt / m;
         v4.x = v4.x + cdt * F.x;
         v4.y = v4.y + cdt * F.y;
@@ -819,73 +1012,74 @@ __global__ void __launch_bounds__(kBlock) k_pressure_apply(Scenes sc, Nbr nb, Ha
 // ----------------------------------------------------------------- viscosity + surface tension CG
 // ComputeSurfaceTensionFactor_kernel (MPSSPHNonPressureUtil.cuh:425-465) with the stored
 // G_ij; also x0 = v (the copy into pPredictVel, MPSSPHNonPressureUtil.cu:144-147).
-__global__ void __launch_bounds__(kBlock) k_st_factor(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
+template <int Q>
+__global__ void __launch_bounds__(Q * kBlock) k_st_factor(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                     const float4* __restrict__ vel, const float* __restrict__ pG_ff,
                                                     float* __restrict__ fst, float4* __restrict__ cgx) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const uint32_t sid = sc.blk_scene[blk];
-    const StepParams P = sc.P[sid];
-    const uint32_t i = blk * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
-    const bool live = i < P.end;
-    const uint32_t c = live ? nb.cff[i] : 0u;
+    const uint32_t N = sc.N;
     // the block's halo (x_j, v_j, m_j) in LDS (see k_cg_apply)
     __shared__ float4 la[kStageST], lb[kStageST];
-    const uint32_t H = halo_count(hl, blk);
-    const bool staged = H <= kStageST;
-    constexpr uint32_t U = kListBatch;
-    uint32_t jn[U];
-    float gn[U];
-    auto fetch = [&](uint32_t k0) {
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            if (k0 + q < c) {
-                const size_t slot = size_t(k0 + q) * N + i;
-                jn[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-                gn[q] = __builtin_nontemporal_load(pG_ff + slot);
-            }
-        }
-    };
-    fetch(0);
-    if (staged) {
-        const uint32_t* hs = hl.idx + size_t(blk) * kHaloCap;
-        for_halo<4>(hs, H, [&](uint32_t t, uint32_t s) {
-            const float4 x = pos[s], v = vel[s];
-            la[t] = make_float4(x.x, x.y, x.z, v.x);
-            lb[t] = make_float4(v.y, v.z, v.w, 0.0f);
-        });
-        __syncthreads();
-    }
-    if (!live) return;
-    const float4 vi4 = vel[i];
-    const f3 xi = mk(pos[i]), vi = mk(vi4);
+    BlockHead<Q, kHaloLoads<Q>> hd(blk, N, nb.cff, hl);
+    const uint32_t i = hd.i, l = hd.l;
+    const bool in = i < N;
+    const float4 xi4 = in ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 vi4 = in ? vel[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool live = i < sc.P[sc.blk_scene[blk]].end;
+    const f3 xi = mk(xi4), vi = mk(vi4);
     float d = 0.0f;
-    for (uint32_t k = 0; k < c; k += U) {
-        uint32_t j[U];
-        float G[U];
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            j[q] = jn[q];
-            G[q] = gn[q];
+    using Val = GroupVal<Q>;
+    auto walk_fluid = [&](auto staged) {
+        constexpr bool STAGED = decltype(staged)::value;
+        Walk<Q, STAGED, Val, 1> wk(nb, hl, pG_ff, nullptr, i, l, N, hd.c);
+        struct Rec {
+            float4 x, v;
+        };
+        if constexpr (STAGED) {
+            hd.stage([&](uint32_t j) { return Rec{pos[j], vel[j]}; },
+                     [&](uint32_t t, const Rec& r) {
+                         la[t] = make_float4(r.x.x, r.x.y, r.x.z, r.v.x);
+                         lb[t] = make_float4(r.v.y, r.v.z, r.v.w, 0.0f);
+                     });
+            __syncthreads();
         }
-        if (k + U < c) fetch(k + U);
-        if (staged) {
+        auto at = [&](uint32_t j) -> Rec {
+            if constexpr (STAGED) {
+                const float4 e = la[j], g = lb[j];
+                return {e, make_float4(e.w, g.x, g.y, g.z)};
+            } else {
+                return {pos[j], vel[j]};
+            }
+        };
+        auto term = [&](float G, const Rec& r) { return r.v.w * dot3(vi - mk(r.v), G * (xi - mk(r.x))); };
+        wk.run(
+            [&](uint32_t, const auto& x, const Val& G) {
+                if constexpr (Q == 1) {
+                    Rec r[4];
 #pragma unroll
-            for (uint32_t q = 0; q < U; q++) {
-                if (k + q < c) {
-                    const float4 e = la[j[q]], g = lb[j[q]];
-                    d += g.z * dot3(vi - f3{e.w, g.x, g.y}, G[q] * (xi - mk(e)));
+                    for (int e = 0; e < 4; e++) r[e] = at(x.at(e));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) d += term(G.at(e), r[e]);
+                } else {
+                    d = add_quad(d, term(G.at(0), at(x.at(0))));
                 }
-            }
-        } else {
-            for (uint32_t q = 0; q < U && k + q < c; q++) {
-                const float4 vj = vel[j[q]];
-                d += vj.w * dot3(vi - mk(vj), G[q] * (xi - mk(pos[j[q]])));
-            }
-        }
+            },
+            [&](uint32_t, const auto& x, const Val& G, uint32_t n) {
+                if constexpr (Q == 1) {
+#pragma unroll
+                    for (int e = 0; e < 3; e++)
+                        if (e < int(n)) d += term(G.at(e), at(x.at(e)));
+                } else {
+                    d = add_quad(d, l < n ? term(G.at(0), at(x.at(0))) : 0.0f);
+                }
+            });
+    };
+    if (hd.H <= kStageST) walk_fluid(std::true_type{});
+    else walk_fluid(std::false_type{});
+    if (live && l == 0) {
+        fst[i] = d;
+        cgx[i] = make_float4(vi4.x, vi4.y, vi4.z, 0.0f);
     }
-    fst[i] = d;
-    cgx[i] = make_float4(vi4.x, vi4.y, vi4.z, 0.0f);
 }
 
 // g_ij of the surface-tension operator (MPSSPHNonPressureUtil.cuh:503-512,563-572)
@@ -904,97 +1098,130 @@ __device__ __forceinline__ float st_g(const StepParams& P, f3 vij, f3 xij, float
 //   c_ij = (0.5(m_i+m_j) (1/rho_j)) Phi(d_ij)   (the reference's (0.5(m_i+m_j)/rho_j) /
 //          (d^2 + 0.01 h_i^2) G_ij / (d + FLT_EPSILON) regrouped, see Phik),
 //   cs_i = dt sigma/m_i, cx = XSPH/dt, cv_i = 10 rho0 mu/rho_i.
-// Writes a_ij (ca) and/or (a_ij, b_ij) (cab), and 1/rho_i per slot (irho) for the A.p that
-// recomputes b_ij.
-template <bool CUBIC>
-__global__ void __launch_bounds__(kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
+// Writes a_ij (ca), b_ij (cb, unless null), and 1/rho_i per slot (irho, unless null) for the A.p
+// that recomputes b_ij.
+template <bool CUBIC, int Q>
+__global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const float* __restrict__ rho,
-                                                   const float* __restrict__ fst, float* __restrict__ ca, float2* __restrict__ cab, float4* __restrict__ cgb,
+                                                   const float* __restrict__ fst, float* __restrict__ ca, float* __restrict__ cb, float4* __restrict__ cgb,
                                                    float* __restrict__ irho) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t N = sc.N;
+    // the block's halo (x_j, v_j, m_j, rho_j, f_j) in LDS (see k_cg_apply)
+    constexpr uint32_t kDepth = Q == 1 ? kStageSetup : kHaloCap;
+    __shared__ float4 la[kDepth], lb[kDepth];
+    __shared__ float lc[kDepth];
+    BlockHead<Q, kHaloLoads<Q>> hd(blk, N, nb.cff, hl);
+    const uint32_t i = hd.i, l = hd.l;
+    const bool in = i < N;
+    const float4 xi4 = in ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 vi4 = in ? vel[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float di = in ? rho[i] : 0.0f, fi = in ? fst[i] : 0.0f;
     const uint32_t sid = sc.blk_scene[blk];
     const StepParams P = sc.P[sid];
-    const uint32_t i = blk * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
     const bool live = i < P.end;
-    const uint32_t c = live ? nb.cff[i] : 0u;
-    // the block's halo (x_j, v_j, m_j, rho_j, f_j) in LDS (see k_cg_apply)
-    __shared__ float4 la[kStageSetup], lb[kStageSetup];
-    __shared__ float lc[kStageSetup];
-    const uint32_t H = halo_count(hl, blk);
-    const bool staged = H <= kStageSetup;
-    constexpr uint32_t U = kListBatch;
-    uint32_t jn[U];
-    auto fetch = [&](uint32_t k0) {
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            if (k0 + q < c) {
-                const size_t slot = size_t(k0 + q) * N + i;
-                jn[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-            }
-        }
-    };
-    fetch(0);
-    if (staged) {
-        const uint32_t* hs = hl.idx + size_t(blk) * kHaloCap;
-        for_halo<4>(hs, H, [&](uint32_t t, uint32_t s) {
-            const float4 x = pos[s], v = vel[s];
-            la[t] = make_float4(x.x, x.y, x.z, v.x);
-            lb[t] = make_float4(v.y, v.z, v.w, rho[s]);
-            lc[t] = fst[s];
-        });
-        __syncthreads();
-    }
-    if (!live) return;
-    const float4 xi4 = pos[i];
-    const float4 vi4 = vel[i];
     const f3 xi = mk(xi4), vi = mk(vi4);
-    const float mi = vi4.w, di = rho[i], fi = fst[i];
+    const float mi = vi4.w;
     const float hi = xi4.w * 4.0f;
     const float invHi = 1.0f / hi;
     const float onePercentHSq = 0.01f * hi * hi;
     const float cs = P.dt * P.sigma / mi;
     const float cx = P.xsph / P.dt;
     const float cv = 10.0f * P.rho0 * P.mu / di;
-    if (irho) irho[i] = 1.0f / di;
     f3 bi{0.f, 0.f, 0.f};
-    auto pair = [&](size_t slot, f3 xj, f3 vj, float mj, float dj, float fj) {
-        const f3 xij = xi - xj;
+    struct Rec {
+        float4 x, v;
+        float rho, f;
+    };
+    struct Term {
+        float a, b;
+        f3 s;
+    };
+    auto term = [&](const Rec& r) -> Term {
+        const float mj = r.v.w, dj = r.rho;
+        const f3 xij = xi - mk(r.x);
         const float dist = len3(xij);
         float mij;
-        const float gij = st_g(P, vi - vj, xij, dist, invHi, mi, mj, di, dj, fi, fj, mij);
+        const float gij = st_g(P, vi - mk(r.v), xij, dist, invHi, mi, mj, di, dj, fi, r.f, mij);
         const float sij = mij * gij;
         const float wij = mj / dj * Wk<CUBIC>(dist, invHi);
-        const float aij = P.dt * (cs * sij + cx * wij);
-        if (ca) ca[slot] = aij;
-        if (cab) {
+        Term t;
+        t.a = P.dt * (cs * sij + cx * wij);
+        t.b = 0.0f;
+        if (cb) {
             const float irhoj = 1.0f / dj;
             const float cij = 0.5f * (mi + mj) * irhoj * Phik<CUBIC>(dist, invHi, onePercentHSq);
-            cab[slot] = make_float2(aij, -P.dt * cv * cij);
+            t.b = -P.dt * cv * cij;
         }
-        bi = bi - sij * xij;
+        t.s = sij * xij;
+        return t;
     };
-    for (uint32_t k = 0; k < c; k += U) {
-        uint32_t j[U];
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) j[q] = jn[q];
-        if (k + U < c) fetch(k + U);
-        if (staged) {
-#pragma unroll
-            for (uint32_t q = 0; q < U; q++) {
-                if (k + q < c) {
-                    const float4 e = la[j[q]], g = lb[j[q]];
-                    pair(size_t(k + q) * N + i, mk(e), f3{e.w, g.x, g.y}, g.z, g.w, lc[j[q]]);
-                }
-            }
-        } else {
-            for (uint32_t q = 0; q < U && k + q < c; q++) {
-                const uint32_t jj = j[q];
-                const float4 vj = vel[jj];
-                pair(size_t(k + q) * N + i, mk(pos[jj]), mk(vj), vj.w, rho[jj], fst[jj]);
-            }
+    auto walk_fluid = [&](auto staged) {
+        constexpr bool STAGED = decltype(staged)::value;
+        Walk<Q, STAGED, NoVal, 1> wk(nb, hl, nullptr, nullptr, i, l, N, hd.c);
+        if constexpr (STAGED) {
+            hd.stage([&](uint32_t j) { return Rec{pos[j], vel[j], rho[j], fst[j]}; },
+                     [&](uint32_t t, const Rec& r) {
+                         la[t] = make_float4(r.x.x, r.x.y, r.x.z, r.v.x);
+                         lb[t] = make_float4(r.v.y, r.v.z, r.v.w, r.rho);
+                         lc[t] = r.f;
+                     });
+            __syncthreads();
         }
-    }
+        auto at = [&](uint32_t j) -> Rec {
+            if constexpr (STAGED) {
+                const float4 e = la[j], g = lb[j];
+                return {e, make_float4(e.w, g.x, g.y, g.z), g.w, lc[j]};
+            } else {
+                return {pos[j], vel[j], rho[j], fst[j]};
+            }
+        };
+        // one entry's coefficients at its place in the list
+        auto put = [&](size_t entry, const Term& t) {
+            ca[entry] = t.a;
+            if (cb) cb[entry] = t.b;
+        };
+        wk.run(
+            [&](uint32_t g, const auto& x, const NoVal&) {
+                const size_t group = size_t(g) * N + i;
+                if constexpr (Q == 1) {
+                    Term t[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        t[e] = term(at(x.at(e)));
+                        bi = bi - t[e].s;
+                    }
+                    reinterpret_cast<v4f*>(ca)[group] = v4f{t[0].a, t[1].a, t[2].a, t[3].a};
+                    if (cb) reinterpret_cast<v4f*>(cb)[group] = v4f{t[0].b, t[1].b, t[2].b, t[3].b};
+                } else {
+                    const Term t = term(at(x.at(0)));
+                    put(4 * group + l, t);
+                    bi = sub_quad(bi, t.s);
+                }
+            },
+            [&](uint32_t g, const auto& x, const NoVal&, uint32_t n) {
+                const size_t group = size_t(g) * N + i;
+                if constexpr (Q == 1) {
+#pragma unroll 1
+                    for (int e = 0; e < int(n); e++) {
+                        const Term t = term(at(x.at(e)));
+                        put(4 * group + e, t);
+                        bi = bi - t.s;
+                    }
+                } else {
+                    Term t{0.f, 0.f, {0.f, 0.f, 0.f}};
+                    if (l < n) {
+                        t = term(at(x.at(0)));
+                        put(4 * group + l, t);
+                    }
+                    bi = sub_quad(bi, t.s);
+                }
+            });
+    };
+    if (hd.H <= kDepth) walk_fluid(std::true_type{});
+    else walk_fluid(std::false_type{});
+    if (!live || l != 0) return;
+    if (irho) irho[i] = 1.0f / di;
     const f3 b = (P.dt * P.sigma / mi) * bi + vi;
     cgb[i] = make_float4(b.x, b.y, b.z, 0.0f);
 }
@@ -1032,146 +1259,135 @@ __global__ void __launch_bounds__(kBlock) k_cg_pack(uint32_t N, const float4* __
 // MODE 0: A x0 with f = 0 (x0 in x0) fused with InitCGResidual_kernel (MPSCGKernel.cuh:5-19):
 //         r = b - A x0, pout = r, x = x0, partial sums of r.r.
 // MODE 1: A p with f (r in rr), partial sums of p.Ap (MPSCGKernel.cuh:21-67).
-// One workgroup's share of A.p: block `blk` of scene `sid`, search-direction factor bta.
+// One workgroup's share of A.p: block `blk`. head() gives its scene, whether that scene's loop has
+// finished, and the search-direction factor; it is called once the loads that need none of these
+// are on their way.
 // PCOH: the partial sum is stored device-coherently (a workgroup of the same launch folds it).
-template <int MODE, bool RECOMP, bool CUBIC, bool COH = false, bool PCOH = COH, uint32_t DEPTH = kStageAp>
-__device__ __forceinline__ void cg_apply_block(uint32_t blk, uint32_t sid, float bta, const Scenes& sc, const Nbr& nb,
-                                               const Halo& hl, const float2* __restrict__ cab, const float* __restrict__ ca,
+struct CgHead {
+    uint32_t sid;
+    bool done;
+    float beta;
+};
+template <int MODE, bool RECOMP, bool CUBIC, bool COH = false, bool PCOH = COH, uint32_t DEPTH = kStageAp, int Q = 1, class Head>
+__device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const Scenes& sc, const Nbr& nb,
+                                               const Halo& hl, const float* __restrict__ cb, const float* __restrict__ ca,
                                                const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                const float* __restrict__ rho, const float* __restrict__ irho,
                                                const float4* __restrict__ x0, const f3* __restrict__ rr,
                                                const f3* __restrict__ pprev, f3* __restrict__ pout, f3* __restrict__ Ap,
                                                const float4* __restrict__ b, f3* __restrict__ r, f3* __restrict__ x,
                                                double* __restrict__ partials) {
-    const StepParams P = sc.P[sid];
-    const uint32_t i = blk * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
+    const uint32_t N = sc.N;
+    using LB = typename std::conditional<RECOMP, float4, float2>::type;
+    __shared__ float4 la[DEPTH];
+    __shared__ LB lb[DEPTH];
+    BlockHead<Q, kHaloLoadsApply> hd(blk, N, nb.cff, hl);
+    const uint32_t i = hd.i, l = hd.l;
+    const CgHead ch = head();
+    if (ch.done) return;
+    const float bta = ch.beta;
+    const StepParams P = sc.P[ch.sid];
     const bool live = i < P.end;
-    const uint32_t c = live ? nb.cff[i] : 0u;
     // the vector the operator is applied to, at slot j
     auto vec = [&](uint32_t j) -> f3 {
         if (MODE == 0) return mk(x0[j]);
         const f3 a = ld3c<COH>(rr + j), q = ld3c<COH>(pprev + j);
         return {a.x + bta * q.x, a.y + bta * q.y, a.z + bta * q.z};
     };
-    using LB = typename std::conditional<RECOMP, float4, float2>::type;
-    __shared__ float4 la[DEPTH];
-    __shared__ LB lb[DEPTH];
-    const uint32_t H = hl.n[blk];
-    const bool staged = H <= DEPTH;  // same for the whole block
-    using Coef = typename std::conditional<RECOMP, float, float2>::type;
-    auto coef = [&](size_t slot) -> Coef {
+    // b_ij's per-particle factors, as k_cg_setup forms them (RECOMP)
+    float mi = 0.0f, ncv = 0.0f, invHi = 0.0f, h2 = 0.0f;
+    f3 xi{0.f, 0.f, 0.f}, pi{0.f, 0.f, 0.f}, acc{0.f, 0.f, 0.f};
+    // one halo record: (x_j, p_j) and, for RECOMP, (m_j, 1/rho_j)
+    struct Rec {
+        f3 x, p;
+        float m, irho;
+    };
+    auto term = [&](float a, float bb, const Rec& q) -> f3 {
+        const f3 xij = xi - q.x;
+        const f3 pij = pi - q.p;
         if constexpr (RECOMP) {
-            return __builtin_nontemporal_load(ca + slot);
+            const float dist = len3(xij);
+            const float cij = 0.5f * (mi + q.m) * q.irho * Phik<CUBIC>(dist, invHi, h2);
+            const float bij = ncv * cij;
+            return a * pij + (bij * dot3(pij, xij)) * xij;
         } else {
-            const double d = __builtin_nontemporal_load(reinterpret_cast<const double*>(cab + slot));
-            return __builtin_bit_cast(float2, d);
+            return a * pij + (bb * dot3(pij, xij)) * xij;
         }
     };
-    constexpr uint32_t U = kListBatchAp;
-    uint32_t jn[U];
-    Coef abn[U];
-    auto fetch = [&](uint32_t k0) {
-#pragma unroll
-        for (uint32_t q = 0; q < U; q++) {
-            if (k0 + q < c) {
-                const size_t slot = size_t(k0 + q) * N + i;
-                jn[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-                abn[q] = coef(slot);
-            }
-        }
-    };
-    // The first kListPrefetchApply entries are loaded before the halo staging: their stream
-    // overlaps the staging's gathers instead of following them.
-    constexpr uint32_t kPre = kListPrefetchApply;
-    uint32_t jp[kPre];
-    Coef abp[kPre];
-#pragma unroll
-    for (uint32_t q = 0; q < kPre; q++) {
-        if (q < c) {
-            const size_t slot = size_t(q) * N + i;
-            jp[q] = staged ? uint32_t(hl.nb16[slot]) : __builtin_nontemporal_load(nb.ff + slot);
-            abp[q] = coef(slot);
-        }
-    }
-    if (staged) {
-        const uint32_t* hs = hl.idx + size_t(blk) * kHaloCap;
-        for_halo<4>(hs, H, [&](uint32_t t, uint32_t s) {
-            const float4 xs = pos[s];
-            const f3 v = vec(s);
-            la[t] = make_float4(xs.x, xs.y, xs.z, v.x);
-            if constexpr (RECOMP) lb[t] = make_float4(v.y, v.z, vel[s].w, irho[s]);
-            else lb[t] = make_float2(v.y, v.z);
-        });
-        __syncthreads();
-    }
-    double part = 0.0;
-    if (live) {
-        const float4 xi4 = pos[i];
-        const f3 xi = mk(xi4);
-        const f3 pi = vec(i);
-        // b_ij's per-particle factors, as k_cg_setup forms them
-        float mi = 0.0f, ncv = 0.0f, invHi = 0.0f, h2 = 0.0f;
-        if constexpr (RECOMP) {
-            mi = vel[i].w;
-            const float cv = 10.0f * P.rho0 * P.mu / rho[i];
-            ncv = -P.dt * cv;
-            const float hi = xi4.w * 4.0f;
-            invHi = 1.0f / hi;
-            h2 = 0.01f * hi * hi;
-        }
-        f3 acc{0.f, 0.f, 0.f};
-        // one pair: record (xj, pj) and, for RECOMP, (mj, 1/rho_j)
-        auto pair = [&](Coef ab, f3 xj, f3 pj, float mj, float irhoj) {
-            const f3 xij = xi - xj;
-            const f3 pij = pi - pj;
+    using Val = typename std::conditional<RECOMP, GroupVal<Q>, GroupAB<Q>>::type;
+    auto walk_fluid = [&](auto staged) {
+        constexpr bool STAGED = decltype(staged)::value;
+        // the first groups are loaded before the halo staging: their stream overlaps the
+        // staging's gathers instead of following them
+        Walk<Q, STAGED, Val, Q == 1 ? kPreApply : kPreQuad> wk(nb, hl, ca, cb, i, l, N, hd.c);
+        auto rec = [&](uint32_t j) -> Rec {
+            const float4 xj = pos[j];
+            if constexpr (RECOMP) return {mk(xj), vec(j), vel[j].w, irho[j]};
+            else return {mk(xj), vec(j), 0.0f, 0.0f};
+        };
+        if (live) {
+            const float4 xi4 = pos[i];
+            xi = mk(xi4);
+            pi = vec(i);
             if constexpr (RECOMP) {
-                const float dist = len3(xij);
-                const float cij = 0.5f * (mi + mj) * irhoj * Phik<CUBIC>(dist, invHi, h2);
-                const float bij = ncv * cij;
-                acc = acc + (ab * pij + (bij * dot3(pij, xij)) * xij);
+                mi = vel[i].w;
+                const float cv = 10.0f * P.rho0 * P.mu / rho[i];
+                ncv = -P.dt * cv;
+                const float hi = xi4.w * 4.0f;
+                invHi = 1.0f / hi;
+                h2 = 0.01f * hi * hi;
+            }
+        }
+        if constexpr (STAGED) {
+            hd.stage(rec, [&](uint32_t t, const Rec& q) {
+                la[t] = make_float4(q.x.x, q.x.y, q.x.z, q.p.x);
+                if constexpr (RECOMP) lb[t] = make_float4(q.p.y, q.p.z, q.m, q.irho);
+                else lb[t] = make_float2(q.p.y, q.p.z);
+            });
+            __syncthreads();
+        }
+        auto at = [&](uint32_t j) -> Rec {
+            if constexpr (STAGED) {
+                const float4 a = la[j];
+                const LB e = lb[j];
+                if constexpr (RECOMP) return {mk(a), {a.w, e.x, e.y}, e.z, e.w};
+                else return {mk(a), {a.w, e.x, e.y}, 0.0f, 0.0f};
             } else {
-                (void)mj;
-                (void)irhoj;
-                acc = acc + (ab.x * pij + (ab.y * dot3(pij, xij)) * xij);
+                return rec(j);
             }
         };
-        auto pair_lds = [&](Coef ab, uint32_t t) {
-            const float4 a = la[t];
-            const LB e = lb[t];
-            if constexpr (RECOMP) pair(ab, mk(a), f3{a.w, e.x, e.y}, e.z, e.w);
-            else pair(ab, mk(a), f3{a.w, e.x, e.y}, 0.0f, 0.0f);
+        auto entry = [&](const Val& v, int e, const Rec& q) -> f3 {
+            if constexpr (RECOMP) return term(v.at(e), 0.0f, q);
+            else return term(v.a.at(e), v.b.at(e), q);
         };
-        auto pair_glb = [&](Coef ab, uint32_t j) {
-            if constexpr (RECOMP) pair(ab, mk(pos[j]), vec(j), vel[j].w, irho[j]);
-            else pair(ab, mk(pos[j]), vec(j), 0.0f, 0.0f);
-        };
-        if (kPre < c) fetch(kPre);
-        // the prefetched entries, then batches, all in list order
+        wk.run(
+            [&](uint32_t, const auto& jx, const Val& v) {
+                if constexpr (Q == 1) {
+                    Rec q[4];
 #pragma unroll
-        for (uint32_t q = 0; q < kPre; q++) {
-            if (q < c) {
-                if (staged) pair_lds(abp[q], jp[q]);
-                else pair_glb(abp[q], jp[q]);
-            }
-        }
-        for (uint32_t k = kPre; k < c; k += U) {
-            uint32_t j[U];
-            Coef ab[U];
+                    for (int e = 0; e < 4; e++) q[e] = at(jx.at(e));
 #pragma unroll
-            for (uint32_t q = 0; q < U; q++) {
-                j[q] = jn[q];
-                ab[q] = abn[q];
-            }
-            if (k + U < c) fetch(k + U);
-            if (staged) {
+                    for (int e = 0; e < 4; e++) acc = acc + entry(v, e, q[e]);
+                } else {
+                    acc = add_quad(acc, entry(v, 0, at(jx.at(0))));
+                }
+            },
+            [&](uint32_t, const auto& jx, const Val& v, uint32_t n) {
+                if constexpr (Q == 1) {
 #pragma unroll
-                for (uint32_t q = 0; q < U; q++)
-                    if (k + q < c) pair_lds(ab[q], j[q]);
-            } else {  // halo over the limit: gather from global memory
-                for (uint32_t q = 0; q < U && k + q < c; q++) pair_glb(ab[q], j[q]);
-            }
-        }
+                    for (int e = 0; e < 3; e++)
+                        if (e < int(n)) acc = acc + entry(v, e, at(jx.at(e)));
+                } else {
+                    f3 t{0.f, 0.f, 0.f};
+                    if (l < n) t = entry(v, 0, at(jx.at(0)));
+                    acc = add_quad(acc, t);
+                }
+            });
+    };
+    if (hd.H <= DEPTH) walk_fluid(std::true_type{});  // the same for the whole block
+    else walk_fluid(std::false_type{});               // halo over the limit: gather from global memory
+    double part = 0.0;
+    if (live && l == 0) {
         const float f = MODE == 0 ? 0.0f : P.cg_factor;
         const f3 o = pi * (1.0f + f) + acc;
         if (MODE == 0) {
@@ -1187,11 +1403,11 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, uint32_t sid, float
             part = double(pi.x * o.x) + double(pi.y * o.y) + double(pi.z * o.z);
         }
     }
-    block_partial<PCOH>(part, partials, blk);
+    slot_partial<Q, PCOH>(part, partials, blk);
 }
 
-template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false>
-__global__ void __launch_bounds__(kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl, const float2* __restrict__ cab,
+template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1>
+__global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl, const float* __restrict__ cb,
                                                    const float* __restrict__ ca, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const float* __restrict__ rho,
                                                    const float* __restrict__ irho, const float4* __restrict__ x0,
@@ -1200,11 +1416,13 @@ __global__ void __launch_bounds__(kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl,
                                                    const float4* __restrict__ b, f3* __restrict__ r, f3* __restrict__ x,
                                                    const SolverDev* st, double* __restrict__ partials) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const uint32_t sid = sc.blk_scene[blk];
-    if (MODE == 1 && st[sid].done) return;
-    const float bta = MODE == 1 ? st[sid].beta : 0.0f;
-    cg_apply_block<MODE, RECOMP, CUBIC, false, false, DEEP ? kHaloCap : kStageAp>(
-        blk, sid, bta, sc, nb, hl, cab, ca, pos, vel, rho, irho, x0, rr, pprev, pout, Ap, b, r, x, partials);
+    auto head = [&]() -> CgHead {
+        const uint32_t sid = sc.blk_scene[blk];
+        if (MODE == 0) return {sid, false, 0.0f};
+        return {sid, st[sid].done != 0u, st[sid].beta};
+    };
+    cg_apply_block<MODE, RECOMP, CUBIC, false, false, DEEP ? kHaloCap : kStageAp, Q>(
+        blk, head, sc, nb, hl, cb, ca, pos, vel, rho, irho, x0, rr, pprev, pout, Ap, b, r, x, partials);
 }
 
 // Scalars of CGSolver (MPSSolver.cuh:31-65). MODE 0: r.r of the initial residual and the
@@ -1421,7 +1639,7 @@ __device__ __forceinline__ bool grid_barrier(GridSync* gs, uint32_t nwg, uint32_
 // after iteration cap. Partial sums alternate between two buffers, so a fold never reads a
 // buffer that the next phase writes. Results are those of the chunked launches bit for bit.
 template <bool RECOMP, bool CUBIC, bool COH>
-__global__ void __launch_bounds__(kBlock) k_cg_persistent(Scenes sc, Nbr nb, Halo hl, const float2* __restrict__ cab,
+__global__ void __launch_bounds__(kBlock) k_cg_persistent(Scenes sc, Nbr nb, Halo hl, const float* __restrict__ cb,
                                                         const float* __restrict__ ca, const float4* __restrict__ pos,
                                                         const float4* __restrict__ vel, const float* __restrict__ rho,
                                                         const float* __restrict__ irho, f3* __restrict__ r,
@@ -1444,7 +1662,7 @@ __global__ void __launch_bounds__(kBlock) k_cg_persistent(Scenes sc, Nbr nb, Hal
         f3* pprev = (k & 1u) ? pbuf0 : pbuf1;  // p of iteration k - 1 (p_0 = r in pbuf0)
         f3* pout = (k & 1u) ? pbuf1 : pbuf0;
         if (!done)
-            cg_apply_block<1, RECOMP, CUBIC, COH>(blk, sid, beta, sc, nb, hl, cab, ca, pos, vel, rho, irho, nullptr, r, pprev,
+            cg_apply_block<1, RECOMP, CUBIC, COH>(blk, [&]() -> CgHead { return {sid, false, beta}; }, sc, nb, hl, cb, ca, pos, vel, rho, irho, nullptr, r, pprev,
                                                   pout, Ap, nullptr, nullptr, nullptr, partA);
         if (!grid_barrier<COH>(gs, nwg, spin)) return;
         if (threadIdx.x == 0) running_s = __hip_atomic_load(active, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1533,7 +1751,7 @@ __device__ __forceinline__ void fold_in_last_workgroup(const Scenes& sc, uint32_
 }
 // k_cg_apply<1> + k_fold_cg<1> in one launch
 template <bool RECOMP, bool CUBIC>
-__global__ void __launch_bounds__(kBlock) k_cg_apply_fold(Scenes sc, Nbr nb, Halo hl, const float2* __restrict__ cab,
+__global__ void __launch_bounds__(kBlock) k_cg_apply_fold(Scenes sc, Nbr nb, Halo hl, const float* __restrict__ cb,
                                                         const float* __restrict__ ca, const float4* __restrict__ pos,
                                                         const float4* __restrict__ vel, const float* __restrict__ rho,
                                                         const float* __restrict__ irho, const f3* __restrict__ rr,
@@ -1543,7 +1761,7 @@ __global__ void __launch_bounds__(kBlock) k_cg_apply_fold(Scenes sc, Nbr nb, Hal
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t sid = sc.blk_scene[blk];
     if (st[sid].done) return;
-    cg_apply_block<1, RECOMP, CUBIC, false, true>(blk, sid, st[sid].beta, sc, nb, hl, cab, ca, pos, vel, rho, irho, nullptr, rr,
+    cg_apply_block<1, RECOMP, CUBIC, false, true>(blk, [&]() -> CgHead { return {sid, false, st[sid].beta}; }, sc, nb, hl, cb, ca, pos, vel, rho, irho, nullptr, rr,
                                                   pprev, pout, Ap, nullptr, nullptr, nullptr, partials);
     fold_in_last_workgroup<1>(sc, sid, blk, partials, st, nullptr, 0.0, arrive);
 }
@@ -1840,6 +2058,15 @@ __global__ void __launch_bounds__(kBlock) k_pack_readback_f64(uint32_t n, const 
 namespace launch {
 using namespace dev;
 static inline unsigned nb_(size_t n) { return unsigned((n + kBlock - 1) / kBlock); }
+// Which form of a list walk a launch takes. With few workgroups the chip is idle and a walk is a
+// chain of latencies, which a quad per slot cuts to a quarter; with many, the one-lane form moves
+// more bytes per instruction. Measured (us, quad / one lane), dam break: 128 workgroups: A.p 7.5 /
+// 8.3, evaluation 8.2 / 11.5, CG setup 16 / 23, density 15 / 26; 349: A.p 17 / 12.5, evaluation
+// 11.6 / 14.6, setup 28 / 36, density 25 / 31; 649: A.p 26 / 17, evaluation 18.5 / 17.0. So A.p, the
+// pressure apply and the ST factor take a quad up to one workgroup per CU, the evaluation, the
+// density and the CG setup up to two.
+constexpr unsigned kQuadOnePerCu = 256, kQuadTwoPerCu = 512;
+static inline bool quad(const Scenes& sc, unsigned most) { return nb_(sc.N) <= most; }
 
 void boundary_sum(int cubic, const float4* bpos, uint32_t B, const uint32_t* nbb, uint32_t Kbb, const uint32_t* cbb, float* S,
                   hipStream_t s) {
@@ -1863,12 +2090,17 @@ void density_alpha(int cubic, int flags, const Scenes& sc, const Nbr& nb, const 
                    const float4* bpos, const float* bvol, float* rho, float* alpha, float4* color, float* pG_ff,
                    float* pG_fb, hipStream_t s) {
     if (!sc.N) return;
-    using K = decltype(&k_density_alpha<false, false, false>);
-    static constexpr K tab[8] = {k_density_alpha<false, false, false>, k_density_alpha<false, false, true>,
-                                 k_density_alpha<false, true, false>,  k_density_alpha<false, true, true>,
-                                 k_density_alpha<true, false, false>,  k_density_alpha<true, false, true>,
-                                 k_density_alpha<true, true, false>,   k_density_alpha<true, true, true>};
+    using K = decltype(&k_density_alpha<false, false, false, 1>);
+    static constexpr K tab[8] = {k_density_alpha<false, false, false, 1>, k_density_alpha<false, false, true, 1>,
+                                 k_density_alpha<false, true, false, 1>,  k_density_alpha<false, true, true, 1>,
+                                 k_density_alpha<true, false, false, 1>,  k_density_alpha<true, false, true, 1>,
+                                 k_density_alpha<true, true, false, 1>,   k_density_alpha<true, true, true, 1>};
     const K k = tab[(cubic ? 4 : 0) | (nb.fr ? 2 : 0) | (nb.fbo ? 1 : 0)];
+    if (!nb.fr && !nb.fbo && hl.n && quad(sc, kQuadTwoPerCu)) {
+        launch_k(cubic ? k_density_alpha<true, false, false, 4> : k_density_alpha<false, false, false, 4>, nb_(sc.N), 4 * kBlock, 0, s,
+                 flags, sc, nb, hl, pos, vel, bpos, bvol, rho, alpha, color, pG_ff, pG_fb);
+        return;
+    }
     launch_k(k, nb_(sc.N), kBlock, 0, s, flags, sc, nb, hl, pos, vel, bpos, bvol, rho, alpha, color, pG_ff, pG_fb);
 }
 void pressure_eval(int cubic, int df, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel,
@@ -1879,17 +2111,27 @@ void pressure_eval(int cubic, int df, const Scenes& sc, const Nbr& nb, const Hal
     const unsigned g = nb_(sc.N);
     // the ref sums evaluate G_ij themselves (the stored G covers the own and wall lists only);
     // `cubic` matters for the ref instances only
-    using K = decltype(&k_pressure_eval<true, false, false, false>);
+    using K = decltype(&k_pressure_eval<true, false, false, false, 1, false>);
     static constexpr K tab[16] = {
-        k_pressure_eval<false, false, false, false>, k_pressure_eval<false, false, false, true>,
-        k_pressure_eval<false, false, false, false>, k_pressure_eval<false, false, false, true>,
-        k_pressure_eval<false, true, false, false>,  k_pressure_eval<false, true, false, true>,
-        k_pressure_eval<false, true, true, false>,   k_pressure_eval<false, true, true, true>,
-        k_pressure_eval<true, false, false, false>,  k_pressure_eval<true, false, false, true>,
-        k_pressure_eval<true, false, false, false>,  k_pressure_eval<true, false, false, true>,
-        k_pressure_eval<true, true, false, false>,   k_pressure_eval<true, true, false, true>,
-        k_pressure_eval<true, true, true, false>,    k_pressure_eval<true, true, true, true>};
+        k_pressure_eval<false, false, false, false, 1, false>, k_pressure_eval<false, false, false, true, 1, false>,
+        k_pressure_eval<false, false, false, false, 1, false>, k_pressure_eval<false, false, false, true, 1, false>,
+        k_pressure_eval<false, true, false, false, 1, false>,  k_pressure_eval<false, true, false, true, 1, false>,
+        k_pressure_eval<false, true, true, false, 1, false>,   k_pressure_eval<false, true, true, true, 1, false>,
+        k_pressure_eval<true, false, false, false, 1, false>,  k_pressure_eval<true, false, false, true, 1, false>,
+        k_pressure_eval<true, false, false, false, 1, false>,  k_pressure_eval<true, false, false, true, 1, false>,
+        k_pressure_eval<true, true, false, false, 1, false>,   k_pressure_eval<true, true, false, true, 1, false>,
+        k_pressure_eval<true, true, true, false, 1, false>,    k_pressure_eval<true, true, true, true, 1, false>};
     const K k = tab[(df ? 8 : 0) | (nb.fr ? 4 : 0) | (cubic ? 2 : 0) | (nb.fbo ? 1 : 0)];
+    if (!nb.fr && !nb.fbo && quad(sc, kQuadTwoPerCu)) {
+        launch_k(df ? k_pressure_eval<true, false, false, false, 4, true> : k_pressure_eval<false, false, false, false, 4, true>, g, 4 * kBlock, 0, s,
+                 sc, nb, hl, pos, vel, bpos, bvol, bvel, rho, alpha, pG_ff, pG_fb, kappa, delta, st, partials);
+        return;
+    }
+    if (!nb.fr && !nb.fbo && hl.deep) {
+        launch_k(df ? k_pressure_eval<true, false, false, false, 1, true> : k_pressure_eval<false, false, false, false, 1, true>, g, kBlock, 0, s,
+                 sc, nb, hl, pos, vel, bpos, bvol, bvel, rho, alpha, pG_ff, pG_fb, kappa, delta, st, partials);
+        return;
+    }
     launch_k(k, g, kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, bvel, rho, alpha, pG_ff, pG_fb, kappa, delta, st, partials);
 }
 void fold_pressure(const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, uint32_t lmin,
@@ -1902,23 +2144,31 @@ void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, 
                     const float* bvol, const float* pG_ff, const float* pG_fb, const float* kappa, const SolverDev* st,
                     hipStream_t s) {
     if (!sc.N) return;
-    using K = decltype(&k_pressure_apply<false, false, false>);
-    static constexpr K tab[8] = {k_pressure_apply<false, false, false>, k_pressure_apply<false, false, true>,
-                                 k_pressure_apply<false, false, false>, k_pressure_apply<false, false, true>,
-                                 k_pressure_apply<true, false, false>,  k_pressure_apply<true, false, true>,
-                                 k_pressure_apply<true, true, false>,   k_pressure_apply<true, true, true>};
+    using K = decltype(&k_pressure_apply<false, false, false, 1>);
+    static constexpr K tab[8] = {k_pressure_apply<false, false, false, 1>, k_pressure_apply<false, false, true, 1>,
+                                 k_pressure_apply<false, false, false, 1>, k_pressure_apply<false, false, true, 1>,
+                                 k_pressure_apply<true, false, false, 1>,  k_pressure_apply<true, false, true, 1>,
+                                 k_pressure_apply<true, true, false, 1>,   k_pressure_apply<true, true, true, 1>};
     const K k = tab[(nb.fr ? 4 : 0) | (cubic ? 2 : 0) | (nb.fbo ? 1 : 0)];
+    if (!nb.fr && !nb.fbo && quad(sc, kQuadOnePerCu)) {
+        launch_k(k_pressure_apply<false, false, false, 4>, nb_(sc.N), 4 * kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb,
+                 kappa, st);
+        return;
+    }
     launch_k(k, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb, kappa, st);
 }
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
                float4* cgx, hipStream_t s) {
-    if (sc.N) launch_k(k_st_factor, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
+    if (!sc.N) return;
+    if (hl.n && quad(sc, kQuadOnePerCu)) launch_k(k_st_factor<4>, nb_(sc.N), 4 * kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
+    else launch_k(k_st_factor<1>, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
 }
 void cg_setup(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* rho,
-              const float* fst, float* ca, float2* cab, float4* cgb, float* irho, hipStream_t s) {
+              const float* fst, float* ca, float* cb, float4* cgb, float* irho, hipStream_t s) {
     if (!sc.N) return;
-    if (cubic) launch_k(k_cg_setup<true>, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, rho, fst, ca, cab, cgb, irho);
-    else launch_k(k_cg_setup<false>, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, rho, fst, ca, cab, cgb, irho);
+    const bool q = hl.n && (hl.deep || quad(sc, kQuadTwoPerCu));
+    if (cubic) launch_k(q ? k_cg_setup<true, 4> : k_cg_setup<true, 1>, nb_(sc.N), q ? 4 * kBlock : kBlock, 0, s, sc, nb, hl, pos, vel, rho, fst, ca, cb, cgb, irho);
+    else launch_k(q ? k_cg_setup<false, 4> : k_cg_setup<false, 1>, nb_(sc.N), q ? 4 * kBlock : kBlock, 0, s, sc, nb, hl, pos, vel, rho, fst, ca, cb, cgb, irho);
 }
 void cg_pack(uint32_t N, const float4* pos, const float4* x0, float4* rec, hipStream_t s) {
     if (N) launch_k(k_cg_pack, nb_(N), kBlock, 0, s, N, pos, x0, rec);
@@ -1928,10 +2178,15 @@ void cg_apply(int mode, const CgOperator& op, const Scenes& sc, const Nbr& nb, c
               const SolverDev* st, double* partials, hipStream_t s) {
     if (!sc.N) return;
     const unsigned g = nb_(sc.N);
+    const bool q = !op.recompute && quad(sc, kQuadOnePerCu);
+    const unsigned threads = q ? 4 * kBlock : kBlock;
 #define MPS_CG_APPLY(M, R, C, ...)                                                                                   \
-    launch_k(k_cg_apply<M, R, C, ##__VA_ARGS__>, g, kBlock, 0, s, sc, nb, hl, op.cab, op.ca, pos, op.vel, op.rho, op.irho, \
+    launch_k(k_cg_apply<M, R, C, ##__VA_ARGS__>, g, threads, 0, s, sc, nb, hl, op.cb, op.ca, pos, op.vel, op.rho, op.irho, \
              x0, rr, pprev, pout, Ap, b, r, x, st, partials)
-    if (!op.recompute && op.deep) {
+    if (q) {
+        if (mode == 0) MPS_CG_APPLY(0, false, true, true, 4);
+        else MPS_CG_APPLY(1, false, true, true, 4);
+    } else if (!op.recompute && op.deep) {
         if (mode == 0) MPS_CG_APPLY(0, false, true, true);
         else MPS_CG_APPLY(1, false, true, true);
     } else if (!op.recompute) {
@@ -1951,7 +2206,7 @@ void cg_apply_fold(const CgOperator& op, const Scenes& sc, const Nbr& nb, const 
     if (!sc.N) return;
     const unsigned g = nb_(sc.N);
 #define MPS_CG_APPLY_FOLD(R, C)                                                                                    \
-    launch_k(k_cg_apply_fold<R, C>, g, kBlock, 0, s, sc, nb, hl, op.cab, op.ca, pos, op.vel, op.rho, op.irho, rr, pprev, \
+    launch_k(k_cg_apply_fold<R, C>, g, kBlock, 0, s, sc, nb, hl, op.cb, op.ca, pos, op.vel, op.rho, op.irho, rr, pprev, \
              pout, Ap, st, partials, arrive)
     if (!op.recompute) MPS_CG_APPLY_FOLD(false, true);
     else if (op.cubic) MPS_CG_APPLY_FOLD(true, true);
@@ -1984,7 +2239,7 @@ void cg_persistent(const CgOperator& op, int coherent, const Scenes& sc, const N
                    double* partB, GridSync* gs, uint32_t cap, double tol, uint32_t spin, hipStream_t s) {
     if (!sc.N) return;
     const uint32_t nblk = nb_(sc.N);
-    void* args[] = {const_cast<Scenes*>(&sc), const_cast<Nbr*>(&nb), const_cast<Halo*>(&hl), const_cast<float2**>(&op.cab),
+    void* args[] = {const_cast<Scenes*>(&sc), const_cast<Nbr*>(&nb), const_cast<Halo*>(&hl), const_cast<float**>(&op.cb),
                     const_cast<float**>(&op.ca), const_cast<float4**>(&pos), const_cast<float4**>(&op.vel),
                     const_cast<float**>(&op.rho), const_cast<float**>(&op.irho), &r, &pbuf0, &pbuf1, &Ap, &x, &st, &active,
                     &partA, &partB, &gs, &cap, &tol, &spin};
