@@ -942,6 +942,12 @@ struct mps_ctx {
         halo_valid = true;
     }
 
+    // Workgroups of the largest scene: the number of partial sums that a fold adds.
+    uint32_t most_blocks() const {
+        uint32_t n = 0;
+        for (const SceneHost& h : scenes) n = std::max(n, h.nf);
+        return ((scenes.empty() ? N : n) + mps::dev::kBlock - 1) / mps::dev::kBlock;
+    }
     // number of scenes whose loop `idx` is still running
     uint32_t fetch_active(int idx) {
         HIPCHK(hipMemcpyAsync(&h_active[idx], &d_active[idx], sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
@@ -978,6 +984,8 @@ struct mps_ctx {
         const uint32_t cap = cfg.max_iter;
         uint32_t it = 1;
         bool done = false;
+        const bool fuse = !coupled() && mps::launch::fold_in_consumer(most_blocks());
+        const mps::launch::FoldPressure fp{partials.p, d_active + idx, tol, lmin};
         while (it <= cap && !done) {
             const uint32_t chunk = chunk_len(it, std::max<uint32_t>(pred[idx], lmin + 1), cap - it + 1);
             std::vector<uint64_t> key = key_base(df ? 1 : 2, chunk, P, nbr());
@@ -988,19 +996,20 @@ struct mps_ctx {
                 key.push_back(u(q));
             key.push_back(u(tol));
             key.push_back(lmin);
-            key.push_back(hl.deep);
+            key.push_back(uint64_t(hl.deep) | (uint64_t(fuse) << 1));
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
                     T_(df ? K_EVAL_DF : K_EVAL_CD, [&] {
                         mps::launch::pressure_eval(cubic(), df, P, nbr(), hl, pos.p, vel.p, bpos.p, bvol.p, bvel.p, rho.p, alpha.p,
                                                    pairG_ff.p, pairG_fb.p, kappa.p, delta.p, sd, partials.p, stream);
                     }, false);
-                    T_(K_FOLD, [&] {
-                        mps::launch::fold_pressure(P, partials.p, sd, d_active + idx, tol, lmin, coupled(), stream);
-                    }, false);
+                    if (!fuse)
+                        T_(K_FOLD, [&] {
+                            mps::launch::fold_pressure(P, partials.p, sd, d_active + idx, tol, lmin, coupled(), stream);
+                        }, false);
                     T_(K_APPLY, [&] {
                         mps::launch::pressure_apply(cubic(), P, nbr(), hl, pos.p, vel.p, bpos.p, bvol.p, pairG_ff.p, pairG_fb.p, kappa.p,
-                                                    sd, stream);
+                                                    sd, fuse ? &fp : nullptr, stream);
                     }, false);
                     rec_snap();
                 }
@@ -1021,7 +1030,7 @@ struct mps_ctx {
         }
         if (prof_on) {  // eval and fold 1..min(l,cap), apply 1..l-1 did work (slowest scene)
             kuse[df ? K_EVAL_DF : K_EVAL_CD] += std::min(l, cap);
-            kuse[K_FOLD] += std::min(l, cap);
+            if (!fuse) kuse[K_FOLD] += std::min(l, cap);
             kuse[K_APPLY] += l - 1;
         }
         for (uint32_t q = 0; q < S && q < sstats.size(); q++) {
@@ -1083,7 +1092,7 @@ struct mps_ctx {
         auto pbuf = [&](uint32_t k) { return (k & 1u) ? v3q.p : v3p.p; };
         T_(K_CG_INIT, [&] {
             mps::launch::cg_apply(0, op, P, nbr(), hl, pos.p, cgx.p, nullptr, nullptr, pbuf(0), nullptr, cgb.p, v3r.p,
-                                  v3x.p, sd, partials.p, stream);
+                                  v3x.p, sd, partials.p, nullptr, stream);
         });
         T_(K_FOLD, [&] { mps::launch::fold_cg(0, P, partials.p, sd, act, tol, stream); });
         const uint32_t cap = cfg.cg_max_iter;
@@ -1112,7 +1121,7 @@ struct mps_ctx {
                     mps::launch::solver_reset(sd, S, act, stream);
                     T_(K_CG_INIT, [&] {
                         mps::launch::cg_apply(0, op, P, nbr(), hl, pos.p, cgx.p, nullptr, nullptr, pbuf(0), nullptr, cgb.p,
-                                              v3r.p, v3x.p, sd, partials.p, stream);
+                                              v3r.p, v3x.p, sd, partials.p, nullptr, stream);
                     });
                     T_(K_FOLD, [&] { mps::launch::fold_cg(0, P, partials.p, sd, act, tol, stream); });
                 }
@@ -1130,10 +1139,15 @@ struct mps_ctx {
             key.push_back(u(tol));
             // the allocation-free step keeps the fold launches (their counters would be scratch)
             const bool fold_in = cfg.cg_fold_in_kernel != 0 && !g_no_alloc;
+            // the sums folded by the launches that need them: p.Ap in `partials`, r.r in the next
+            // nblk of them; a chunk ends with a fold launch of its last r.r
+            const bool fuse = !fold_in && !op.recompute && mps::launch::fold_in_consumer(most_blocks());
+            double* part_rr = fuse ? partials.p + nblk : partials.p;
+            const mps::launch::FoldCg fc{part_rr, act, tol};
             uint32_t* arr = fold_in ? arrive_counters() : nullptr;
             key.push_back(fold_in);
             key.push_back(u(arr));
-            key.push_back(uint64_t(op.deep));
+            key.push_back(uint64_t(op.deep) | (uint64_t(fuse) << 1));
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
                     const uint32_t k = it + c;
@@ -1150,13 +1164,14 @@ struct mps_ctx {
                     }
                     T_(K_CG_APPLY, [&] {
                         mps::launch::cg_apply(1, op, P, nbr(), hl, pos.p, nullptr, v3r.p, pbuf(k - 1), pbuf(k), v3Ap.p,
-                                              nullptr, nullptr, nullptr, sd, partials.p, stream);
+                                              nullptr, nullptr, nullptr, sd, partials.p, fuse && c ? &fc : nullptr, stream);
                     }, false);
-                    T_(K_FOLD, [&] { mps::launch::fold_cg(1, P, partials.p, sd, act, tol, stream); }, false);
+                    if (!fuse) T_(K_FOLD, [&] { mps::launch::fold_cg(1, P, partials.p, sd, act, tol, stream); }, false);
                     T_(K_CG_UPDATE, [&] {
-                        mps::launch::cg_update3(P, v3x.p, v3r.p, pbuf(k), v3Ap.p, sd, partials.p, stream);
+                        mps::launch::cg_update3(P, v3x.p, v3r.p, pbuf(k), v3Ap.p, sd, fuse ? partials.p : nullptr, part_rr, stream);
                     }, false);
-                    T_(K_FOLD, [&] { mps::launch::fold_cg(2, P, partials.p, sd, act, tol, stream); }, false);
+                    if (!fuse || c + 1 == chunk)
+                        T_(K_FOLD, [&] { mps::launch::fold_cg(2, P, part_rr, sd, act, tol, stream); }, false);
                 }
             });
             it += chunk;
@@ -1168,7 +1183,8 @@ struct mps_ctx {
         if (prof_on) {  // A.p (with the direction) and the update ran for iterations 1..l-1
             kuse[K_CG_APPLY] += std::min(l - 1, cap);
             kuse[K_CG_UPDATE] += std::min(l - 1, cap);
-            if (!cfg.cg_fold_in_kernel || g_no_alloc) kuse[K_FOLD] += 2 * std::min(l - 1, cap);
+            if ((!cfg.cg_fold_in_kernel || g_no_alloc) && (op.recompute || !mps::launch::fold_in_consumer(most_blocks())))
+                kuse[K_FOLD] += 2 * std::min(l - 1, cap);
         }
         T_(K_COPY_OUT, [&] { mps::launch::copy_vel_out3(P, v3x.p, vel.p, stream); });
         for (uint32_t q = 0; q < S && q < sstats.size(); q++) {

@@ -160,16 +160,55 @@ __device__ __forceinline__ uint32_t grid_zindex(i3 p, const HashGeom& g) {
 }
 
 // --------------------------------------------------------------------- wave/block reductions
-// Sum of a double over the 256-thread block in a fixed tree order; result valid in thread 0.
-__device__ __forceinline__ double block_sum_d(double v, double* lds /*[kBlock/64]*/) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) lds[wave] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0) {
-        for (int w = 0; w < (int)(blockDim.x >> 6); w++) s += lds[w];
+// Sum of a double over the wave in every lane, in the order of the butterfly v += v[lane ^ off],
+// off = 32, 16, 8, 4, 2, 1. The first two steps swap half waves and rows of 16 lanes; after them
+// (and after each further step) the values repeat every `off` lanes of a row, where rotating by
+// `off` reads what lane ^ off holds. No step goes through LDS, as a shuffle does (the sums sit at
+// the end of the latency chain of every solver launch).
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum_d(double v) {
+    {
+        const uint32_t lo = __double2loint(v), hi = __double2hiint(v);
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        v = __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
     }
+    {
+        const uint32_t lo = __double2loint(v), hi = __double2hiint(v);
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        v = __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+    }
+    v += dpp_d<0x128>(v);  // row_ror:8
+    v += dpp_d<0x124>(v);
+    v += dpp_d<0x122>(v);
+    v += dpp_d<0x121>(v);
+    return v;
+}
+// Sum of a double over a workgroup of NW waves in a fixed order (the butterfly within a wave, then
+// the waves in order), valid in every thread. `lds` holds NW values and may be written again only
+// after a further barrier.
+template <int NW>
+__device__ __forceinline__ double block_total(double v, double* lds) {
+    v = wave_sum_d(v);
+    if ((threadIdx.x & 63u) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t[NW];
+#pragma unroll
+    for (int w = 0; w < NW; w++) t[w] = lds[w];
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) s += t[w];
+    return s;
+}
+// The same over a workgroup of kBlock threads; `lds` may be used again at once.
+__device__ __forceinline__ double block_sum_d(double v, double* lds /*[kBlock/64]*/) {
+    const double s = block_total<kBlock / 64>(v, lds);
     __syncthreads();
     return s;
 }

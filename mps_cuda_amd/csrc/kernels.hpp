@@ -48,8 +48,9 @@ struct SolverDev {
     uint32_t done;     // loop finished (converged); later kernels of the chunk exit at once
     uint32_t l;        // reference loop variable when the loop ended (or next iteration)
     uint32_t counter;  // workgroups of the current launch that arrived (folds in the last workgroup)
-    uint32_t pad;
+    uint32_t it;       // pressure loop: the iteration whose evaluation ran last (folds in the consumer)
     double rr;         // CG: r.r of the current residual
+    double rr_prev;    // CG: r.r before the last update (folds in the consumer)
     double pAp;        // CG: p.Ap
     double thr;        // CG: stop when r.r < thr (tol, or -tol * initial r.r when tol < 0)
     float alpha, beta; // CG step scalars (rounded to float like the FP32 reference)
@@ -208,14 +209,24 @@ void density_alpha(int cubic, int flags, const Scenes& sc, const Nbr& nb, const 
 // nb.fr set: the coupled-scene variants (ref sums, G_ij evaluated for them with `cubic`)
 void pressure_eval(int cubic, int df, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel,
                    const float4* bpos, const float* bvol, const float4* bvel, const float* rho, const float* alpha,
-                   const float* pG_ff, const float* pG_fb, float* kappa, float* delta, const SolverDev* st, double* partials,
+                   const float* pG_ff, const float* pG_fb, float* kappa, float* delta, SolverDev* st, double* partials,
                    hipStream_t s);
 // joint: one decision for all scenes (coupled fluid objects)
 void fold_pressure(const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, uint32_t lmin,
                    int joint, hipStream_t s);
+// fold set: every workgroup of the apply folds its scene's errors (partials) itself and the scene's
+// first one does fold_pressure's part (not for coupled scenes)
+struct FoldPressure {
+    const double* partials;
+    uint32_t* active;
+    double tol;
+    uint32_t lmin;
+};
 void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, float4* vel, const float4* bpos,
-                    const float* bvol, const float* pG_ff, const float* pG_fb, const float* kappa, const SolverDev* st,
-                    hipStream_t s);
+                    const float* bvol, const float* pG_ff, const float* pG_fb, const float* kappa, SolverDev* st,
+                    const FoldPressure* fold, hipStream_t s);
+// Whether the consumers of a solver's sums fold them themselves (one launch less per sum).
+bool fold_in_consumer(uint32_t most_blocks);
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
                float4* cgx, hipStream_t s);
 // pair coefficients of the implicit operator: a_ij into ca, b_ij into cb (may be null)
@@ -240,9 +251,16 @@ struct CgOperator {
     const float* rho = nullptr;
     const float* irho = nullptr;
 };
+// fold set (mode 1, streamed operator): every workgroup first folds its scene's r.r of the last
+// update (fold->partials) itself, and the scene's first one does fold_cg(2)'s part.
+struct FoldCg {
+    const double* partials;
+    uint32_t* active;
+    double tol;
+};
 void cg_apply(int mode, const CgOperator& op, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos,
               const float4* x0, const dev::f3* rr, const dev::f3* pprev, dev::f3* pout, dev::f3* Ap, const float4* b,
-              dev::f3* r, dev::f3* x, const SolverDev* st, double* partials, hipStream_t s);
+              dev::f3* r, dev::f3* x, SolverDev* st, double* partials, const FoldCg* fold, hipStream_t s);
 // A.p (mode 1) and the update, each with its fold (k_fold_cg 1 / 2) done by the scene's last
 // workgroup to finish (the solver record's counter counts arrivals): two launches per CG
 // iteration instead of four, with the same bits. arrive: one counter per workgroup (zero, and
@@ -274,8 +292,10 @@ void fold_cg(int mode, const Scenes& sc, const double* partials, SolverDev* st, 
 void cg_update(const Scenes& sc, float4* x, float4* r, const float4* prec, const float4* Ap, const SolverDev* st,
                double* partials, hipStream_t s);
 // the same on packed triples (the forward solve), and its copy of x into the velocities
-void cg_update3(const Scenes& sc, dev::f3* x, dev::f3* r, const dev::f3* p, const dev::f3* Ap, const SolverDev* st,
-                double* partials, hipStream_t s);
+// pAp set: every workgroup folds its scene's p.Ap partials (pAp) itself, and the scene's first one
+// does fold_cg(1)'s part
+void cg_update3(const Scenes& sc, dev::f3* x, dev::f3* r, const dev::f3* p, const dev::f3* Ap, SolverDev* st,
+                const double* pAp, double* partials, hipStream_t s);
 void copy_vel_out3(const Scenes& sc, const dev::f3* x, float4* vel, hipStream_t s);
 // p = r + beta p in the records (the adjoint's solve; the forward forms p inside cg_apply)
 void cg_direction(const Scenes& sc, const float4* r, float4* prec, const SolverDev* st, hipStream_t s);

@@ -14,8 +14,8 @@
 // streams 4-8 bytes per pair instead of re-evaluating square roots and divisions.
 //
 // Convergence sums: each workgroup reduces its T-rounded terms in double and writes one
-// partial; a one-workgroup fold kernel adds the partials in index order (deterministic, no
-// FP64 atomics) and updates a SolverDev record on the device. Kernels of later iterations
+// partial; the workgroups that need the sum, or in large grids a one-workgroup fold kernel, add the
+// partials in index order (deterministic, no FP64 atomics) and update a SolverDev record on the device. Kernels of later iterations
 // read SolverDev::done first and exit at once, so the host can enqueue several iterations
 // before it looks at the result.
 #include "device_common.hpp"
@@ -70,7 +70,7 @@ __device__ __forceinline__ void walk_walls(const Nbr& nb, uint32_t i, uint32_t l
 template <bool COH = false>
 __device__ __forceinline__ void block_partial(double v, double* __restrict__ partials, uint32_t blk) {
     __shared__ double lds[kBlock / 64];
-    const double bs = block_sum_d(v, lds);
+    const double bs = block_total<kBlock / 64>(v, lds);
     if (threadIdx.x == 0) {
         if constexpr (COH) __hip_atomic_store(partials + blk, bs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         else partials[blk] = bs;
@@ -104,8 +104,8 @@ __device__ __forceinline__ void st3c(f3* p, f3 v) {
 __device__ __forceinline__ void block_partial(double v, double* __restrict__ partials) {
     block_partial(v, partials, blockIdx.x);
 }
-// Sum of partials[0..n) in index-strided order, valid in thread 0 (one workgroup of
-// kFoldThreads).
+// Sum of partials[0..n) in index-strided order, valid in every thread of a workgroup of
+// kFoldThreads (call it again only after a further barrier).
 constexpr int kFoldThreads = 1024;
 __device__ __forceinline__ double fold(const double* __restrict__ partials, uint32_t n) {
     __shared__ double lds[kFoldThreads / 64];
@@ -122,7 +122,69 @@ __device__ __forceinline__ double fold(const double* __restrict__ partials, uint
         for (uint32_t q = 0; q < R; q++)
             if (k0 + q * blockDim.x < n) s += v[q];
     }
-    return block_sum_d(s, lds);
+    return block_total<kFoldThreads / 64>(s, lds);
+}
+
+// The fold of the kFoldThreads-thread fold kernels, computed by one kBlock-thread workgroup in
+// exactly their order: thread t plays their threads t + kBlock v (v < kFoldThreads / kBlock);
+// each sums its strided partials left to right, each of their waves is reduced by the same
+// butterfly (the played threads of one of their waves all sit in one wave here, in the same
+// lanes), and every thread adds the wave totals in wave order. Valid in every thread; call it
+// again only after a further barrier.
+template <bool COH>
+__device__ __forceinline__ double fold_as_fold_kernel(const double* __restrict__ partials, uint32_t n) {
+    constexpr uint32_t V = kFoldThreads / kBlock;
+    constexpr uint32_t kWaves = kFoldThreads / 64;
+    constexpr uint32_t R = 4;  // strides of kFoldThreads loaded per batch: R * V loads in flight
+    __shared__ double wsum[kWaves];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    auto ld = [&](uint32_t k) -> double {
+        if constexpr (COH) return __hip_atomic_load(partials + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else return partials[k];
+    };
+    double s[V];
+#pragma unroll
+    for (uint32_t v = 0; v < V; v++) s[v] = 0.0;
+    for (uint32_t m0 = 0; m0 * kFoldThreads < n; m0 += R) {
+        double t[R][V];
+#pragma unroll
+        for (uint32_t r = 0; r < R; r++)
+#pragma unroll
+            for (uint32_t v = 0; v < V; v++) {
+                const uint32_t k = threadIdx.x + v * kBlock + (m0 + r) * kFoldThreads;
+                t[r][v] = k < n ? ld(k) : 0.0;
+            }
+#pragma unroll
+        for (uint32_t r = 0; r < R; r++)
+#pragma unroll
+            for (uint32_t v = 0; v < V; v++)
+                if (threadIdx.x + v * kBlock + (m0 + r) * kFoldThreads < n) s[v] += t[r][v];
+    }
+#pragma unroll
+    for (uint32_t v = 0; v < V; v++) {
+        const double x = wave_sum_d(s[v]);
+        if (lane == 0) wsum[wave + v * (kBlock / 64)] = x;
+    }
+    __syncthreads();
+    double w[kWaves];
+#pragma unroll
+    for (uint32_t q = 0; q < kWaves; q++) w[q] = wsum[q];
+    double t = 0.0;
+#pragma unroll
+    for (uint32_t q = 0; q < kWaves; q++) t += w[q];
+    return t;
+}
+
+// The same sum in a workgroup of Q * kBlock threads, valid in every thread (Q = 4: the fold kernels'
+// own thread count).
+template <int Q>
+__device__ __forceinline__ double fold_everywhere(const double* __restrict__ partials, uint32_t n) {
+    if constexpr (Q == 1) {
+        return fold_as_fold_kernel<false>(partials, n);
+    } else {
+        static_assert(Q * kBlock == kFoldThreads, "the quad forms have the fold kernels' size");
+        return fold(partials, n);
+    }
 }
 
 // Halo count of workgroup blk: > kHaloCap (not staged) when there are no halos (hl.n null: the
@@ -169,8 +231,8 @@ __device__ __forceinline__ T sub_lanes(T s, T t) {
     else return s - t;
 }
 // block_partial of a workgroup with a quad per slot (`v` counts in lane part 0): the slots'
-// values are put back one per lane of the first kBlock / 64 waves and reduced there in
-// block_sum_d's order, so the partial has the same bits.
+// values are put back one per lane and reduced by the first wave in block_total's order, so the
+// partial has the same bits.
 template <int Q, bool COH = false>
 __device__ __forceinline__ void slot_partial(double v, double* __restrict__ partials, uint32_t blk) {
     if constexpr (Q == 1) {
@@ -178,19 +240,15 @@ __device__ __forceinline__ void slot_partial(double v, double* __restrict__ part
     } else {
         static_assert(!COH, "the persistent solver runs one lane per slot");
         __shared__ double pv[kBlock];
-        __shared__ double ws[kBlock / 64];
         if (threadIdx.x % Q == 0) pv[threadIdx.x / Q] = v;
         __syncthreads();
-        if (threadIdx.x < kBlock) {
-            double s = pv[threadIdx.x];
-            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-            if ((threadIdx.x & 63u) == 0) ws[threadIdx.x >> 6] = s;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double s = 0.0;
-            for (int w = 0; w < kBlock / 64; w++) s += ws[w];
-            partials[blk] = s;
+        if (threadIdx.x < 64) {
+            double w[kBlock / 64], s = 0.0;
+#pragma unroll
+            for (int q = 0; q < kBlock / 64; q++) w[q] = wave_sum_d(pv[64 * q + threadIdx.x]);
+#pragma unroll
+            for (int q = 0; q < kBlock / 64; q++) s += w[q];
+            if (threadIdx.x == 0) partials[blk] = s;
         }
     }
 }
@@ -687,7 +745,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_eval(Scenes sc, Nbr nb,
                                                         const float* __restrict__ rho, const float* __restrict__ alpha,
                                                         const float* __restrict__ pG_ff, const float* __restrict__ pG_fb,
                                                         float* __restrict__ kappa, float* __restrict__ delta,
-                                                        const SolverDev* st, double* __restrict__ partials) {
+                                                        SolverDev* st, double* __restrict__ partials) {
     static_assert(Q == 1 || !(REF || BOBJ), "coupled scenes and wall objects run one lane per slot");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t N = sc.N;
@@ -705,6 +763,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_eval(Scenes sc, Nbr nb,
     if (st[sid].done) return;  // this scene's loop has finished
     const StepParams P = sc.P[sid];
     const bool live = i < P.end;
+    if (blk == P.blk0 && threadIdx.x == 0) st[sid].it = st[sid].l;  // for an apply that folds
     const f3 xi = mk(xi4);
     float df = 0.0f;
     using Val = GroupVal<Q>;
@@ -828,10 +887,20 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_eval(Scenes sc, Nbr nb,
 }
 
 // Mean positive error and the loop decision of the DF/CD drivers
-// (MPSSPHDFSPHUtil.cu:331-333,417-419): break when E < tol and l > lmin. Workgroup s folds
-// scene s's partials; a scene that finishes leaves the count of active scenes.
-// The iteration number is the record's l (1 after the reset, it + 1 after iteration it), so the
-// launches of a chunk do not depend on where the chunk starts.
+// (MPSSPHDFSPHUtil.cu:331-333,417-419): break when E < tol and l > lmin. `s` is the scene's sum of
+// errors in iteration `it`; a scene that finishes leaves the count of active scenes.
+__device__ __forceinline__ void record_pressure(SolverDev* sd, double E, bool ok, uint32_t it, uint32_t* active) {
+    if (it - 1 < MPS_MAX_ITER_LOG) sd->log[it - 1] = E;
+    if (ok) {
+        sd->done = 1u;
+        sd->l = it;
+        atomicSub(active, 1u);
+    } else {
+        sd->l = it + 1;
+    }
+}
+// Workgroup s folds scene s's partials. The iteration number is the record's l (1 after the reset,
+// it + 1 after iteration it), so the launches of a chunk do not depend on where the chunk starts.
 __global__ void __launch_bounds__(kFoldThreads) k_fold_pressure(Scenes sc, const double* __restrict__ partials,
                                                         SolverDev* st, uint32_t* active, double tol, uint32_t lmin) {
     const uint32_t sid = blockIdx.x;
@@ -842,14 +911,7 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_pressure(Scenes sc, const
     const double s = fold(partials + P.blk0, P.nblk);
     if (threadIdx.x == 0) {
         const double E = s / double(P.count);
-        if (it - 1 < MPS_MAX_ITER_LOG) sd->log[it - 1] = E;
-        if (E < tol && it > lmin) {
-            sd->done = 1u;
-            sd->l = it;
-            atomicSub(active, 1u);
-        } else {
-            sd->l = it + 1;
-        }
+        record_pressure(sd, E, E < tol && it > lmin, it, active);
     }
 }
 
@@ -885,12 +947,16 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_pressure_joint(Scenes sc,
 
 // ApplyDFSPH_kernel ff/fb + ApplyDFSPHFinal_kernel (MPSSPHDFSPHUtil.cuh:342-468) + UpdateVelocity.
 // The halo's (x_j, kappa_j) are staged in LDS (see k_cg_apply).
-template <bool REF, bool CUBIC, bool BOBJ, int Q>
+// FOLD: every workgroup folds its scene's errors itself, in the fold kernels' order, and takes the
+// loop decision of k_fold_pressure; the scene's first workgroup records it. The others read `done`
+// and `it`: `it` was copied by the evaluation, and a `done` that is already set says what they
+// would find. One launch less per iteration (4 us and its gap) for ~1 us in the apply.
+template <bool REF, bool CUBIC, bool BOBJ, int Q, bool FOLD>
 __global__ void __launch_bounds__(Q * kBlock) k_pressure_apply(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                          float4* __restrict__ vel, const float4* __restrict__ bpos,
                                                          const float* __restrict__ bvol, const float* __restrict__ pG_ff,
                                                          const float* __restrict__ pG_fb, const float* __restrict__ kappa,
-                                                         const SolverDev* st) {
+                                                         SolverDev* st, launch::FoldPressure fp) {
     static_assert(Q == 1 || !(REF || BOBJ), "coupled scenes and wall objects run one lane per slot");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t N = sc.N;
@@ -905,6 +971,13 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_apply(Scenes sc, Nbr nb
     const uint32_t sid = sc.blk_scene[blk];
     if (st[sid].done) return;
     const StepParams P = sc.P[sid];
+    if constexpr (FOLD) {
+        const uint32_t it = st[sid].it;
+        const double E = fold_everywhere<Q>(fp.partials + P.blk0, P.nblk) / double(P.count);
+        const bool ok = E < fp.tol && it > fp.lmin;
+        if (blk == P.blk0 && threadIdx.x == 0) record_pressure(st + sid, E, ok, it, fp.active);
+        if (ok) return;
+    }
     const bool live = i < P.end;
     const f3 xi = mk(xi4);
     f3 ff{0.f, 0.f, 0.f};
@@ -1406,7 +1479,26 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const 
     slot_partial<Q, PCOH>(part, partials, blk);
 }
 
-template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1>
+// What k_fold_cg<2> records of iteration `it`: `s` is the new r.r, `prev` the one before.
+__device__ __forceinline__ void record_cg(SolverDev* st, double s, double prev, bool done, uint32_t* active) {
+    const uint32_t it = st->l;
+    st->beta = float(s / prev);
+    st->rr = s;
+    if (it < MPS_MAX_ITER_LOG) st->log[it] = s;
+    st->l = it + 1;
+    if (done) {
+        st->done = 1u;
+        atomicSub(active, 1u);
+    }
+}
+__device__ __forceinline__ bool cg_done(double s, double thr, double tol) { return s < thr || (tol < 0.0 && s == 0.0); }
+
+// FOLD (MODE 1): every workgroup first folds its scene's r.r of the last update itself, in the fold
+// kernels' order, forms beta and takes the convergence test of k_fold_cg<2>; the scene's first
+// workgroup records them. The others read `done`, `thr` and `rr_prev` of the record, which that
+// workgroup does not write (`rr_prev` is kept by the update), or, for `done`, only sets to what
+// they find themselves.
+template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1, bool FOLD = false>
 __global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl, const float* __restrict__ cb,
                                                    const float* __restrict__ ca, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const float* __restrict__ rho,
@@ -1414,11 +1506,20 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo
                                                    const f3* __restrict__ rr, const f3* __restrict__ pprev,
                                                    f3* __restrict__ pout, f3* __restrict__ Ap,
                                                    const float4* __restrict__ b, f3* __restrict__ r, f3* __restrict__ x,
-                                                   const SolverDev* st, double* __restrict__ partials) {
+                                                   SolverDev* st, double* __restrict__ partials, launch::FoldCg fc) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     auto head = [&]() -> CgHead {
         const uint32_t sid = sc.blk_scene[blk];
         if (MODE == 0) return {sid, false, 0.0f};
+        if constexpr (FOLD) {
+            if (st[sid].done) return {sid, true, 0.0f};
+            const uint32_t blk0 = sc.P[sid].blk0;
+            const double prev = st[sid].rr_prev, thr = st[sid].thr;
+            const double s = fold_everywhere<Q>(fc.partials + blk0, sc.P[sid].nblk);
+            const bool done = cg_done(s, thr, fc.tol);
+            if (blk == blk0 && threadIdx.x == 0) record_cg(st + sid, s, prev, done, fc.active);
+            return {sid, done, float(s / prev)};
+        }
         return {sid, st[sid].done != 0u, st[sid].beta};
     };
     cg_apply_block<MODE, RECOMP, CUBIC, false, false, DEEP ? kHaloCap : kStageAp, Q>(
@@ -1435,7 +1536,6 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_cg(Scenes sc, const doubl
     const uint32_t sid = blockIdx.x;
     SolverDev* st = stv + sid;
     if (MODE != 0 && st->done) return;
-    const uint32_t it = st->l;
     const StepParams P = sc.P[sid];
     const double s = fold(partials + P.blk0, P.nblk);
     if (threadIdx.x != 0) return;
@@ -1452,14 +1552,7 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_cg(Scenes sc, const doubl
         st->pAp = s;
         st->alpha = float(st->rr / s);
     } else {
-        st->beta = float(s / st->rr);
-        st->rr = s;
-        if (it < MPS_MAX_ITER_LOG) st->log[it] = s;
-        st->l = it + 1;
-        if (s < st->thr || (tol < 0.0 && s == 0.0)) {
-            st->done = 1u;
-            atomicSub(active, 1u);
-        }
+        record_cg(st, s, st->rr, cg_done(s, st->thr, tol), active);
     }
 }
 
@@ -1513,66 +1606,34 @@ __device__ __forceinline__ void cg_update3_block(uint32_t blk, uint32_t end, flo
     }
     block_partial<PCOH>(part, partials, blk);
 }
+// FOLD: every workgroup first folds its scene's p.Ap itself and forms alpha (k_fold_cg<1>); the
+// scene's first workgroup records it and keeps the r.r that the next A.p needs as rr_prev, which no
+// workgroup of this launch reads.
+template <bool FOLD>
 __global__ void __launch_bounds__(kBlock) k_cg_update3(Scenes sc, f3* __restrict__ x, f3* __restrict__ r,
                                                      const f3* __restrict__ p, const f3* __restrict__ Ap,
-                                                     const SolverDev* st, double* __restrict__ partials) {
+                                                     SolverDev* st, const double* __restrict__ pAp,
+                                                     double* __restrict__ partials) {
     const uint32_t sid = sc.blk_scene[blockIdx.x];
     if (st[sid].done) return;
-    cg_update3_block(blockIdx.x, sc.P[sid].end, st[sid].alpha, x, r, p, Ap, partials);
+    float alpha;
+    if constexpr (FOLD) {
+        const uint32_t blk0 = sc.P[sid].blk0;
+        const double rr = st[sid].rr;
+        const double s = fold_as_fold_kernel<false>(pAp + blk0, sc.P[sid].nblk);
+        alpha = float(rr / s);
+        if (blockIdx.x == blk0 && threadIdx.x == 0) {
+            st[sid].pAp = s;
+            st[sid].alpha = alpha;
+            st[sid].rr_prev = rr;
+        }
+    } else {
+        alpha = st[sid].alpha;
+    }
+    cg_update3_block(blockIdx.x, sc.P[sid].end, alpha, x, r, p, Ap, partials);
 }
 
 // ----------------------------------------------------------------- persistent CG
-// The fold of the kFoldThreads-thread fold kernels, computed by one kBlock-thread workgroup in
-// exactly their order: thread t plays their threads t + kBlock v (v < kFoldThreads / kBlock);
-// each sums its strided partials left to right, each of their waves is reduced by the same
-// butterfly (the played threads of one of their waves all sit in one wave here, in the same
-// lanes), and thread 0 adds the wave totals in wave order. Valid in every thread.
-template <bool COH>
-__device__ __forceinline__ double fold_as_fold_kernel(const double* __restrict__ partials, uint32_t n) {
-    constexpr uint32_t V = kFoldThreads / kBlock;
-    constexpr uint32_t kWaves = kFoldThreads / 64;
-    constexpr uint32_t R = 4;  // strides of kFoldThreads loaded per batch: R * V loads in flight
-    __shared__ double wsum[kWaves];
-    __shared__ double total;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    auto ld = [&](uint32_t k) -> double {
-        if constexpr (COH) return __hip_atomic_load(partials + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else return partials[k];
-    };
-    double s[V];
-#pragma unroll
-    for (uint32_t v = 0; v < V; v++) s[v] = 0.0;
-    for (uint32_t m0 = 0; m0 * kFoldThreads < n; m0 += R) {
-        double t[R][V];
-#pragma unroll
-        for (uint32_t r = 0; r < R; r++)
-#pragma unroll
-            for (uint32_t v = 0; v < V; v++) {
-                const uint32_t k = threadIdx.x + v * kBlock + (m0 + r) * kFoldThreads;
-                t[r][v] = k < n ? ld(k) : 0.0;
-            }
-#pragma unroll
-        for (uint32_t r = 0; r < R; r++)
-#pragma unroll
-            for (uint32_t v = 0; v < V; v++)
-                if (threadIdx.x + v * kBlock + (m0 + r) * kFoldThreads < n) s[v] += t[r][v];
-    }
-#pragma unroll
-    for (uint32_t v = 0; v < V; v++) {
-        double x = s[v];
-        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-        if (lane == 0) wsum[wave + v * (kBlock / 64)] = x;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (uint32_t w = 0; w < kWaves; w++) t += wsum[w];
-        total = t;
-    }
-    __syncthreads();
-    return total;
-}
-
 // Grid-wide barrier of a co-resident grid (cooperative launch). The wait is bounded: after
 // `spin` polls, or when another workgroup gave up, it sets gs->gave_up and returns false, and
 // the caller leaves the kernel; every workgroup's wait then ends within `spin` polls.
@@ -1738,15 +1799,7 @@ __device__ __forceinline__ void fold_in_last_workgroup(const Scenes& sc, uint32_
         st->pAp = s;
         st->alpha = float(st->rr / s);
     } else {
-        const uint32_t it = st->l;
-        st->beta = float(s / st->rr);
-        st->rr = s;
-        if (it < MPS_MAX_ITER_LOG) st->log[it] = s;
-        st->l = it + 1;
-        if (s < st->thr || (tol < 0.0 && s == 0.0)) {
-            st->done = 1u;
-            atomicSub(active, 1u);
-        }
+        record_cg(st, s, st->rr, cg_done(s, st->thr, tol), active);
     }
 }
 // k_cg_apply<1> + k_fold_cg<1> in one launch
@@ -2105,7 +2158,7 @@ void density_alpha(int cubic, int flags, const Scenes& sc, const Nbr& nb, const 
 }
 void pressure_eval(int cubic, int df, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel,
                    const float4* bpos, const float* bvol, const float4* bvel, const float* rho, const float* alpha,
-                   const float* pG_ff, const float* pG_fb, float* kappa, float* delta, const SolverDev* st, double* partials,
+                   const float* pG_ff, const float* pG_fb, float* kappa, float* delta, SolverDev* st, double* partials,
                    hipStream_t s) {
     if (!sc.N) return;
     const unsigned g = nb_(sc.N);
@@ -2141,21 +2194,25 @@ void fold_pressure(const Scenes& sc, const double* partials, SolverDev* st, uint
     else launch_k(k_fold_pressure, sc.S, kFoldThreads, 0, s, sc, partials, st, active, tol, lmin);
 }
 void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, float4* vel, const float4* bpos,
-                    const float* bvol, const float* pG_ff, const float* pG_fb, const float* kappa, const SolverDev* st,
-                    hipStream_t s) {
+                    const float* bvol, const float* pG_ff, const float* pG_fb, const float* kappa, SolverDev* st,
+                    const FoldPressure* fold, hipStream_t s) {
     if (!sc.N) return;
-    using K = decltype(&k_pressure_apply<false, false, false, 1>);
-    static constexpr K tab[8] = {k_pressure_apply<false, false, false, 1>, k_pressure_apply<false, false, true, 1>,
-                                 k_pressure_apply<false, false, false, 1>, k_pressure_apply<false, false, true, 1>,
-                                 k_pressure_apply<true, false, false, 1>,  k_pressure_apply<true, false, true, 1>,
-                                 k_pressure_apply<true, true, false, 1>,   k_pressure_apply<true, true, true, 1>};
+    using K = decltype(&k_pressure_apply<false, false, false, 1, false>);
+    static constexpr K tab[8] = {k_pressure_apply<false, false, false, 1, false>, k_pressure_apply<false, false, true, 1, false>,
+                                 k_pressure_apply<false, false, false, 1, false>, k_pressure_apply<false, false, true, 1, false>,
+                                 k_pressure_apply<true, false, false, 1, false>,  k_pressure_apply<true, false, true, 1, false>,
+                                 k_pressure_apply<true, true, false, 1, false>,   k_pressure_apply<true, true, true, 1, false>};
     const K k = tab[(nb.fr ? 4 : 0) | (cubic ? 2 : 0) | (nb.fbo ? 1 : 0)];
     if (!nb.fr && !nb.fbo && quad(sc, kQuadOnePerCu)) {
-        launch_k(k_pressure_apply<false, false, false, 4>, nb_(sc.N), 4 * kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb,
-                 kappa, st);
+        launch_k(fold ? k_pressure_apply<false, false, false, 4, true> : k_pressure_apply<false, false, false, 4, false>, nb_(sc.N),
+                 4 * kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb, kappa, st, fold ? *fold : FoldPressure{});
         return;
     }
-    launch_k(k, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb, kappa, st);
+    if (fold && !nb.fr)
+        launch_k(nb.fbo ? k_pressure_apply<false, false, true, 1, true> : k_pressure_apply<false, false, false, 1, true>, nb_(sc.N),
+                 kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb, kappa, st, *fold);
+    else
+        launch_k(k, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb, kappa, st, FoldPressure{});
 }
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
                float4* cgx, hipStream_t s) {
@@ -2175,22 +2232,25 @@ void cg_pack(uint32_t N, const float4* pos, const float4* x0, float4* rec, hipSt
 }
 void cg_apply(int mode, const CgOperator& op, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos,
               const float4* x0, const f3* rr, const f3* pprev, f3* pout, f3* Ap, const float4* b, f3* r, f3* x,
-              const SolverDev* st, double* partials, hipStream_t s) {
+              SolverDev* st, double* partials, const FoldCg* fold, hipStream_t s) {
     if (!sc.N) return;
     const unsigned g = nb_(sc.N);
     const bool q = !op.recompute && quad(sc, kQuadOnePerCu);
     const unsigned threads = q ? 4 * kBlock : kBlock;
 #define MPS_CG_APPLY(M, R, C, ...)                                                                                   \
     launch_k(k_cg_apply<M, R, C, ##__VA_ARGS__>, g, threads, 0, s, sc, nb, hl, op.cb, op.ca, pos, op.vel, op.rho, op.irho, \
-             x0, rr, pprev, pout, Ap, b, r, x, st, partials)
+             x0, rr, pprev, pout, Ap, b, r, x, st, partials, fold ? *fold : FoldCg{})
     if (q) {
         if (mode == 0) MPS_CG_APPLY(0, false, true, true, 4);
+        else if (fold) MPS_CG_APPLY(1, false, true, true, 4, true);
         else MPS_CG_APPLY(1, false, true, true, 4);
     } else if (!op.recompute && op.deep) {
         if (mode == 0) MPS_CG_APPLY(0, false, true, true);
+        else if (fold) MPS_CG_APPLY(1, false, true, true, 1, true);
         else MPS_CG_APPLY(1, false, true, true);
     } else if (!op.recompute) {
         if (mode == 0) MPS_CG_APPLY(0, false, true);
+        else if (fold) MPS_CG_APPLY(1, false, true, false, 1, true);
         else MPS_CG_APPLY(1, false, true);
     } else if (op.cubic) {
         if (mode == 0) MPS_CG_APPLY(0, true, true);
@@ -2256,10 +2316,15 @@ void cg_update(const Scenes& sc, float4* x, float4* r, const float4* prec, const
                double* partials, hipStream_t s) {
     if (sc.N) launch_k(k_cg_update, nb_(sc.N), kBlock, 0, s, sc, x, r, prec, Ap, st, partials);
 }
-void cg_update3(const Scenes& sc, f3* x, f3* r, const f3* p, const f3* Ap, const SolverDev* st, double* partials,
+void cg_update3(const Scenes& sc, f3* x, f3* r, const f3* p, const f3* Ap, SolverDev* st, const double* pAp, double* partials,
                 hipStream_t s) {
-    if (sc.N) launch_k(k_cg_update3, nb_(sc.N), kBlock, 0, s, sc, x, r, p, Ap, st, partials);
+    if (sc.N) launch_k(pAp ? k_cg_update3<true> : k_cg_update3<false>, nb_(sc.N), kBlock, 0, s, sc, x, r, p, Ap, st, pAp, partials);
 }
+// Every consumer workgroup reads all partial sums of its scene, so the work grows with the square of
+// the workgroups. Whole passes (fold launches -> folds in the consumers): 128 workgroups 15.5 ->
+// 14.1 ms, 1006 24.5 -> 22.8, 2051 33.8 -> 34.3, 3907 65.7 -> 68.4 (there A.p 73.0 -> 79.8 us and
+// the update 11.4 -> 15.5, against two fold launches of 4.0).
+bool fold_in_consumer(uint32_t most_blocks) { return most_blocks <= 1536; }
 void copy_vel_out3(const Scenes& sc, const f3* x, float4* vel, hipStream_t s) {
     if (sc.N) launch_k(k_copy_vel_out3, nb_(sc.N), kBlock, 0, s, sc, x, vel);
 }
