@@ -298,6 +298,11 @@ struct mps_ctx {
     mps::GridSync* d_grid = nullptr;  // barrier words of the persistent solver (allocated at creation)
     uint32_t persist_cap[6] = {0, 0, 0, 0, 0, 0};  // co-resident workgroups per kernel variant (0 = not asked yet)
     uint32_t persist_fallbacks = 0;       // persistent solves that gave up and reran chunked
+    // The first pass takes its dense form when more than one workgroup in kSearchCrowded had more
+    // candidates than the usual form holds.
+    static constexpr uint32_t kSearchCrowded = 32;
+    int search_dense = 0;
+    uint32_t search_left = 0;             // workgroups that the last search's first pass left to the second
     uint32_t deep_halos = 0;              // workgroups of the last list build with halos over kHaloShallow
     uint32_t* d_flags = nullptr;  // [0] nonfinite, [1] sampling mismatch, [4..6] halo statistics of the step
     uint32_t* h_flags = nullptr;
@@ -831,10 +836,21 @@ struct mps_ctx {
             cff.reserve(std::max<uint32_t>(N, 1));
             nfb.reserve(size_t(Kfb) * std::max<uint32_t>(N, 1));
             cfb.reserve(std::max<uint32_t>(N, 1));
-            T_(K_NEI_FLUID, [&] {
-                mps::launch::neighbors_fluid(pos.p, scn(), uint32_t(cells()), g, fluid_view(), view(bh, B), nff.p, Kff, cff.p,
-                                             nfb.p, Kfb, cfb.p, nstat.p, d_ctr, stream);
-            });
+            reserve_halo();
+            auto search = [&](mps::launch::SearchPasses passes) {
+                T_(K_NEI_FLUID, [&] {
+                    mps::launch::neighbors_fluid(pos.p, scn(), uint32_t(cells()), g, fluid_view(), view(bh, B), nff.p, Kff, cff.p,
+                                                 nfb.p, Kfb, cfb.p, nstat.p,
+                                                 mps::launch::HaloOut{halo_idx.p, halo_n.p, nb16.p, cfg.halo_limit, d_flags + 4},
+                                                 passes, search_dense, d_ctr, stream);
+                });
+            };
+            auto counters = [&] {
+                HIPCHK(hipMemcpyAsync(h_ctr, d_ctr, sizeof(NbrCounters), hipMemcpyDeviceToHost, stream));
+                sync();
+            };
+            const bool both = search_left != 0;  // the last search left blocks to the second pass
+            search(both ? mps::launch::kSearchBoth : mps::launch::kSearchFirst);
             if (coupled()) {
                 nfr.reserve(size_t(Kfr) * std::max<uint32_t>(N, 1));
                 cfr.reserve(std::max<uint32_t>(N, 1));
@@ -843,8 +859,13 @@ struct mps_ctx {
                                                stream);
                 });
             }
-            HIPCHK(hipMemcpyAsync(h_ctr, d_ctr, sizeof(NbrCounters), hipMemcpyDeviceToHost, stream));
-            sync();
+            counters();
+            search_left = h_ctr->left;
+            search_dense = uint64_t(h_ctr->crowded) * kSearchCrowded > (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
+            if (h_ctr->left && !both) {
+                search(mps::launch::kSearchLeft);
+                counters();
+            }
             bool grow = false;
             if (coupled() && h_ctr->max_fr > Kfr) { Kfr = (h_ctr->max_fr + 15u) & ~15u; grow = true; }
             if (h_ctr->max_ff > Kff) { Kff = (h_ctr->max_ff + 15u) & ~15u; grow = true; }
@@ -867,7 +888,8 @@ struct mps_ctx {
                 nnz_ff = h_ctr->nnz_ff;
                 nnz_fb = h_ctr->nnz_fb;
                 pairs_valid = false;
-                halo_valid = false;
+                if (h_ctr->todo) build_halo(0);  // blocks that the search left out
+                halo_valid = true;
                 return;
             }
             nei_regrow++;
@@ -929,17 +951,24 @@ struct mps_ctx {
         const uint64_t nb = (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
         return cfg.cg_halo_depth == 2 || (cfg.cg_halo_depth == 0 && uint64_t(deep_halos) * 1000u > nb);
     }
-    void ensure_halo() {
-        if (halo_valid) return;
-        const size_t m = std::max<uint32_t>(N, 1);
+    void reserve_halo() {
+        const size_t nblk = std::max<size_t>((size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock, 1);
+        nb16.reserve(size_t(Kff) * std::max<uint32_t>(N, 1));
+        halo_idx.reserve(nblk * mps::kHaloCap);
+        halo_n.reserve(nblk);
+    }
+    void build_halo(int all) {
         const uint32_t nblk = uint32_t((size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock);
-        nb16.reserve(size_t(Kff) * m);
-        halo_idx.reserve(size_t(std::max<uint32_t>(nblk, 1)) * mps::kHaloCap);
-        halo_n.reserve(std::max<uint32_t>(nblk, 1));
         T_(K_HALO, [&] {
-            mps::launch::halo_build(scn(), nbr(), nblk, cfg.halo_limit, halo_idx.p, halo_n.p, nb16.p, d_flags + 4, stream);
+            mps::launch::halo_build(all, scn(), nbr(), nblk, cfg.halo_limit, halo_idx.p, halo_n.p, nb16.p, d_flags + 4, stream);
         });
         halo_valid = true;
+    }
+    // The halos of the lists in place when no search has just built them (positions were set since).
+    void ensure_halo() {
+        if (halo_valid) return;
+        reserve_halo();
+        build_halo(1);
     }
 
     // Workgroups of the largest scene: the number of partial sums that a fold adds.

@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "kernels.hpp"
+
 namespace mps {
 namespace dev {
 
@@ -211,6 +213,48 @@ __device__ __forceinline__ double block_sum_d(double v, double* lds /*[kBlock/64
     const double s = block_total<kBlock / 64>(v, lds);
     __syncthreads();
     return s;
+}
+
+// Statistics of the block halos by one workgroup of 1024 threads (no same-address atomics from every
+// workgroup of the build): stats[0] = largest halo staged, stats[1] = blocks not staged, stats[2] =
+// blocks with a halo or not staged, stats[3] = blocks whose halo is staged but deeper than
+// kHaloShallow.
+__device__ __forceinline__ void fold_halo_stats(const uint32_t* __restrict__ hn, uint32_t nblk, uint32_t* __restrict__ stats) {
+    __shared__ uint32_t wm[1024 / 64], ws[1024 / 64], wb[1024 / 64], wd[1024 / 64];
+    uint32_t mx = 0u, sp = 0u, bl = 0u, dp = 0u;
+    for (uint32_t b = threadIdx.x; b < nblk; b += blockDim.x) {
+        const uint32_t h = hn[b];
+        if (h > kHaloCap) sp++;
+        else mx = max(mx, h);
+        if (h) bl++;
+        if (h > kHaloShallow && h <= kHaloCap) dp++;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        mx = max(mx, (uint32_t)__shfl_xor((int)mx, off, 64));
+        sp += (uint32_t)__shfl_xor((int)sp, off, 64);
+        bl += (uint32_t)__shfl_xor((int)bl, off, 64);
+        dp += (uint32_t)__shfl_xor((int)dp, off, 64);
+    }
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    if (lane == 0) {
+        wm[wave] = mx;
+        ws[wave] = sp;
+        wb[wave] = bl;
+        wd[wave] = dp;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (uint32_t w = 1; w < blockDim.x / 64; w++) {
+            mx = max(mx, wm[w]);
+            sp += ws[w];
+            bl += wb[w];
+            dp += wd[w];
+        }
+        stats[0] = mx;
+        stats[1] = sp;
+        stats[2] = bl;
+        stats[3] = dp;
+    }
 }
 
 }  // namespace dev

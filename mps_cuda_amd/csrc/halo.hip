@@ -3,12 +3,16 @@
 // The implicit viscosity operator (A.p) is applied ~30 times per step over the same lists.
 // Gathering the 32-byte CG record of every neighbour from global memory costs most of its
 // time: a block of 256 slots touches ~7k list entries but only ~900 distinct records (its
-// halo), and the caches cannot keep the halos of all resident blocks. This pass, run once
-// per solve, lists for each 256-slot block the distinct neighbour slots in ascending order
-// (at most kHaloCap) and rewrites every list entry of the block as a 16-bit position in that
-// list. A.p then stages the halo's records into LDS with coalesced loads and gathers from
-// LDS. A block with more than kHaloCap distinct neighbours keeps the global path
-// (halo count > kHaloCap marks it).
+// halo), and the caches cannot keep the halos of all resident blocks. So each 256-slot block has
+// a list of the distinct neighbour slots in ascending order (at most kHaloCap), and every list entry
+// as a 16-bit position in that list. A.p then stages the halo's records into LDS with coalesced
+// loads and gathers from LDS. A block with more than kHaloCap distinct neighbours keeps the global
+// path (halo count > kHaloCap marks it).
+//
+// The fluid search writes the halos along with the lists (hash.hip). This pass builds them from the
+// lists: for the blocks whose candidates fit none of the search's staged forms, and for all blocks
+// when positions were set after a search. It hashes each entry and sorts the distinct ones, ~200 us
+// at 1M particles where the search pays ~80.
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -36,9 +40,10 @@ __device__ __forceinline__ uint32_t halo_find(const uint32_t* key, uint32_t j) {
 
 // Blocks with more than `limit` (<= kHaloCap) distinct neighbours are marked not staged
 // (n = kHaloCap + 1).
-__global__ void __launch_bounds__(kBlock) k_halo_build(Scenes sc, Nbr nb, uint32_t limit, uint32_t* __restrict__ hidx,
+__global__ void __launch_bounds__(kBlock) k_halo_build(Scenes sc, Nbr nb, int all, uint32_t limit, uint32_t* __restrict__ hidx,
                                                      uint32_t* __restrict__ hn, uint16_t* __restrict__ n16) {
     const uint32_t blk = blockIdx.x;
+    if (!all && hn[blk] != kHaloTodo) return;  // the search built it
     const uint32_t sid = sc.blk_scene[blk];
     const StepParams P = sc.P[sid];
     const uint32_t N = P.N;
@@ -159,59 +164,20 @@ __global__ void __launch_bounds__(kBlock) k_halo_build(Scenes sc, Nbr nb, uint32
     }
 }
 
-// stats[0] = largest halo staged, stats[1] = blocks not staged, stats[2] = blocks with a halo
-// or not staged, stats[3] = blocks whose halo is staged but deeper than kHaloShallow: one
-// workgroup folds the per-block counts (no same-address atomics from every workgroup of the
-// build).
 constexpr int kHaloStatThreads = 1024;
 __global__ void __launch_bounds__(kHaloStatThreads) k_halo_stats(const uint32_t* __restrict__ hn, uint32_t nblk,
                                                                 uint32_t* __restrict__ stats) {
-    __shared__ uint32_t wm[kHaloStatThreads / 64], ws[kHaloStatThreads / 64], wb[kHaloStatThreads / 64],
-        wd[kHaloStatThreads / 64];
-    uint32_t mx = 0u, sp = 0u, bl = 0u, dp = 0u;
-    for (uint32_t b = threadIdx.x; b < nblk; b += blockDim.x) {
-        const uint32_t h = hn[b];
-        if (h > kHaloCap) sp++;
-        else mx = max(mx, h);
-        if (h) bl++;
-        if (h > kHaloShallow && h <= kHaloCap) dp++;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, off, 64));
-        sp += (uint32_t)__shfl_xor((int)sp, off, 64);
-        bl += (uint32_t)__shfl_xor((int)bl, off, 64);
-        dp += (uint32_t)__shfl_xor((int)dp, off, 64);
-    }
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    if (lane == 0) {
-        wm[wave] = mx;
-        ws[wave] = sp;
-        wb[wave] = bl;
-        wd[wave] = dp;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (uint32_t w = 1; w < blockDim.x / 64; w++) {
-            mx = max(mx, wm[w]);
-            sp += ws[w];
-            bl += wb[w];
-            dp += wd[w];
-        }
-        stats[0] = mx;
-        stats[1] = sp;
-        stats[2] = bl;
-        stats[3] = dp;
-    }
+    fold_halo_stats(hn, nblk, stats);
 }
 
 }  // namespace dev
 
 namespace launch {
-void halo_build(const Scenes& sc, const Nbr& nb, uint32_t nblk, uint32_t limit, uint32_t* hidx, uint32_t* hn, uint16_t* n16,
-                uint32_t* stats, hipStream_t s) {
+void halo_build(int all, const Scenes& sc, const Nbr& nb, uint32_t nblk, uint32_t limit, uint32_t* hidx, uint32_t* hn,
+                uint16_t* n16, uint32_t* stats, hipStream_t s) {
     limit = limit == 0u || limit > kHaloCap ? kHaloCap : limit;
     if (!nblk) return;
-    launch_k(dev::k_halo_build, nblk, dev::kBlock, 0, s, sc, nb, limit, hidx, hn, n16);
+    launch_k(dev::k_halo_build, nblk, dev::kBlock, 0, s, sc, nb, all, limit, hidx, hn, n16);
     launch_k(dev::k_halo_stats, 1, dev::kHaloStatThreads, 0, s, hn, nblk, stats);
 }
 }  // namespace launch

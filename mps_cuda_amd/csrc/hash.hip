@@ -312,31 +312,24 @@ __device__ __forceinline__ bool within(const float4& xi, float ri, const float4&
     return __builtin_sqrtf(dd) < thr;
 }
 
-// within() for four candidates of one radius, as a bit mask (bit k: candidate k). The cut-off
-// thr = (h_i + h_j) * 0.5 (h = 4 r) is then the same for every pair, and it, t2lo = thr^2 * 0.9999
-// and t2hi = thr^2 * 1.0001 come precomputed with the same float operations. The squared distances decide first, and the square
-// root is taken only within 1e-4 of the cut-off. The two range tests are sign bits rather than
-// comparisons: for finite values dd - t2lo is negative exactly when dd < t2lo, and t2hi - dd
-// exactly when dd > t2hi (two unequal floats differ by a nonzero float; equal ones give +0).
-// A NaN distance sets both bits or neither, and is then no hit.
-__device__ __forceinline__ uint32_t hit_bits4(const float4& xi, float thr, float t2lo, float t2hi, const float4 (&q)[4]) {
-    uint32_t lo = 0u, hi = 0u;
-    float dd[4];
+// The neighbour test of one radius against squared distances: sqrt(dd) < thr exactly when
+// dd < cut_of(thr). The square root is monotone and correctly rounded, so the distances that pass are
+// those below one float, the smallest x with sqrt(x) >= thr; it lies within 2 ulp of the rounded
+// thr * thr (sqrt(x) rounds up to thr from (thr - ulp/2)^2 on), and the search for it starts above.
+__device__ __forceinline__ float cut_of(float thr) {
+    float x = thr * thr;
+    x = __uint_as_float(__float_as_uint(x) + (x < 3.0e38f ? 2u : 0u));
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float ddx = xi.x - q[k].x, ddy = xi.y - q[k].y, ddz = xi.z - q[k].z;
-        dd[k] = (ddx * ddx + ddy * ddy) + ddz * ddz;
-        lo |= (__float_as_uint(dd[k] - t2lo) >> 31) << k;
-        hi |= (__float_as_uint(t2hi - dd[k]) >> 31) << k;
+    for (int k = 0; k < 6; k++) {
+        const float y = __uint_as_float(__float_as_uint(x) - (x > 0.0f ? 1u : 0u));
+        if (__builtin_sqrtf(y) >= thr) x = y;
     }
-    uint32_t in = lo & ~hi;
-    const uint32_t near = ~(lo | hi) & 15u;
-    if (near) {
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if ((near >> k) & 1u) in |= static_cast<uint32_t>(__builtin_sqrtf(dd[k]) < thr) << k;
-    }
-    return in;
+    return x;
+}
+// m = 2 m + (dd < cut): the hits of a run collect from its first copy in the top bit down. A NaN
+// distance is no hit.
+__device__ __forceinline__ void push_hit(uint32_t& m, float dd, float cut) {
+    asm("v_cmp_lt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(dd), "v"(cut) : "vcc");
 }
 
 // Where a search puts its lists: rows of K slots (out[i*K + k]), columns (out[k*stride + i]) or
@@ -389,9 +382,9 @@ __device__ __forceinline__ uint32_t search_cells(float4 xi, uint32_t i, const Ha
 
 // Per-workgroup (largest count, sum of counts) of up to two lists, written to st[blk] and
 // st[n + blk]; k_count_fold reduces them (no same-address atomics from every wave).
-template <int L>
+template <int L, uint32_t NW = kBlock / 64>
 __device__ __forceinline__ void block_counts(const uint32_t (&c)[L], uint2* __restrict__ st, uint32_t n, uint32_t blk) {
-    __shared__ uint32_t wm[L][kBlock / 64], ws[L][kBlock / 64];
+    __shared__ uint32_t wm[L][NW], ws[L][NW];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int l = 0; l < L; l++) {
@@ -410,7 +403,7 @@ __device__ __forceinline__ void block_counts(const uint32_t (&c)[L], uint2* __re
 #pragma unroll
         for (int l = 0; l < L; l++) {
             uint32_t mx = 0u, sm = 0u;
-            for (uint32_t w = 0; w < kBlock / 64; w++) {
+            for (uint32_t w = 0; w < NW; w++) {
                 mx = max(mx, wm[l][w]);
                 sm += ws[l][w];
             }
@@ -419,17 +412,36 @@ __device__ __forceinline__ void block_counts(const uint32_t (&c)[L], uint2* __re
     }
 }
 
+// The counts of a search over its workgroups' records: workgroup l of the launch folds list l into
+// maxc[l] and nnz[l]. The fluid search's launch has a third workgroup, which counts its halos (hn):
+// stats[0] = largest staged, [1] = not staged, [2] = blocks with neighbours, [3] = staged but deeper
+// than kHaloShallow (blocks left to k_halo_build are counted after it).
 constexpr int kCountFoldThreads = 1024;
 __global__ void __launch_bounds__(kCountFoldThreads) k_count_fold(const uint2* __restrict__ st, uint32_t n, uint32_t* maxc,
-                                                                unsigned long long* nnz) {
+                                                                unsigned long long* nnz, const uint32_t* __restrict__ hn,
+                                                                uint32_t* __restrict__ stats) {
+    if (blockIdx.x == 2u) {
+        fold_halo_stats(hn, n, stats);
+        return;
+    }
     __shared__ uint32_t wm[kCountFoldThreads / 64];
     __shared__ unsigned long long ws[kCountFoldThreads / 64];
     uint32_t mx = 0u;
     unsigned long long sm = 0ull;
-    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) {
-        const uint2 v = st[k];
-        mx = max(mx, v.x);
-        sm += v.y;
+    st += size_t(blockIdx.x) * n;
+    constexpr uint32_t R = 4;  // records of a thread in flight
+    for (uint32_t k0 = threadIdx.x; k0 < n; k0 += R * blockDim.x) {
+        uint2 v[R];
+#pragma unroll
+        for (uint32_t q = 0; q < R; q++) {
+            const uint32_t k = k0 + q * blockDim.x;
+            v[q] = k < n ? st[k] : make_uint2(0u, 0u);
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < R; q++) {
+            mx = max(mx, v[q].x);
+            sm += v[q].y;
+        }
     }
     for (int off = 32; off > 0; off >>= 1) {
         mx = max(mx, (uint32_t)__shfl_xor((int)mx, off, 64));
@@ -446,8 +458,8 @@ __global__ void __launch_bounds__(kCountFoldThreads) k_count_fold(const uint2* _
             mx = max(mx, wm[w]);
             sm += ws[w];
         }
-        *maxc = mx;
-        *nnz = sm;
+        maxc[blockIdx.x] = mx;
+        nnz[blockIdx.x] = sm;
     }
 }
 
@@ -460,22 +472,44 @@ __global__ void __launch_bounds__(kCountFoldThreads) k_count_fold(const uint2* _
 // bounds are read once, and all fluid (then wall) particles of those cells are staged in LDS
 // in that order, each with its slot (a wall particle: its id) in place of the radius. So the
 // three cells x-1, x, x+1 of any row of a particle are one contiguous run of staged copies, and
-// every particle walks its 27 cells in the reference order as 9 row runs. A block with more
-// rows, cells or candidates than the LDS holds, or whose staged fluid (or wall) particles do
-// not all share one radius, searches the global tables for that set; the lists are the same
-// either way.
-constexpr uint32_t kSrchRowHash = 128;  // LDS hash slots for rows
-constexpr uint32_t kSrchRows = 96;      // rows per block
-constexpr uint32_t kSrchCells = 384;    // cells per block (the rows' x ranges)
-constexpr uint32_t kSrchCand = 1920;    // staged candidates (fluid, then walls)
-constexpr uint32_t kSrchPad = 4;        // a group of four read at the end of a run stays in the array
+// every particle walks its 27 cells in the reference order as 9 row runs: first a hit mask per
+// run, then the hits of all runs as list entries. The staged copies that are anybody's hit are the
+// block's halo (halo.hip): their slots in ascending order, and every list entry as a position
+// among them, are written by the same kernel, which has the lists and the copies at hand.
+//
+// Q = 4 shares a slot among a quad of lanes, which take the runs 0..8 in turn.
+//
+// A block may have more rows, cells or candidates than the LDS holds, staged fluid (or wall)
+// particles that do not all share one radius, or a run of more copies than a hit mask has bits. The
+// first pass over many blocks (LAST false) leaves such a block alone (n = kHaloTodo); a second one,
+// with room for more and a quad per slot, takes what is left. The LAST pass searches the global
+// tables for a set that does not fit even there, and leaves the halo of a block whose fluid was
+// searched so to k_halo_build. The lists are the same whichever way.
+//
+// Bound by its vector instructions and LDS latency: of the ~50 us that a workgroup takes (1M
+// particles, four workgroups per CU) the distance tests are 13, writing the lists 9, the halo 15,
+// registering rows and staging 14. Search and halos together, before (a search of its own and
+// k_halo_build) -> now: 250 particles 97 -> 48 us, 33k 207 -> 57, 45k near rest density 365 -> 75, 257k
+// 179 -> 110, 525k near rest density 630 -> 343, 1M 433 -> 330.
+template <uint32_t HASH_BITS, uint32_t ROWS, uint32_t CELLS, uint32_t CAND, uint32_t WORDS>
+struct SearchCaps {
+    static constexpr uint32_t kHashBits = HASH_BITS, kRowHash = 1u << HASH_BITS;
+    static constexpr uint32_t kRows = ROWS, kCells = CELLS, kCand = CAND;
+    static constexpr uint32_t kWords = WORDS, kRun = 32u * WORDS;  // a run's hit mask
+};
+// Near rest density a block has 1500-2700 candidates; particles in thin sheets give up to 200 rows
+// and 850 cells; a cell at the origin is two cells wide (coordinates are truncated towards 0), so
+// there a run can hold over 100 copies.
+using SearchStd = SearchCaps<7, 96, 384, 1920, 3>;     // 39 KB: four workgroups per CU
+using SearchDense = SearchCaps<7, 96, 384, 2752, 3>;   // 52 KB: three (525k near rest density: 437 -> 343 us)
+using SearchWide = SearchCaps<9, 224, 1024, 3328, 8>;  // 78 KB: two
+constexpr uint32_t kSrchPad = 4;                     // a group of four read at the end of a run stays in the array
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
-__device__ __forceinline__ uint32_t row_hash(uint32_t c) { return (c * 2654435761u) >> 25; }
-static_assert(kSrchRowHash == (1u << 7), "row_hash gives 7 bits");
-static_assert(kSrchRows <= kBlock && kSrchCells <= 2u * kBlock, "one row per thread, two cells per thread");
+constexpr uint32_t kHit = 0x80000000u;  // marks a staged fluid copy that is in a list (slots are below 2^31)
 
-// Inclusive scan of a 64-bit value over the kBlock threads; `ws` holds kBlock / 64 wave totals
+// Inclusive scan of a 64-bit value over the workgroup's NW waves; `ws` holds NW wave totals
 // (synchronise before reusing it). `total` receives the block's sum.
+template <uint32_t NW>
 __device__ __forceinline__ unsigned long long block_scan_u64(unsigned long long v, unsigned long long* ws,
                                                              unsigned long long& total) {
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
@@ -487,49 +521,125 @@ __device__ __forceinline__ unsigned long long block_scan_u64(unsigned long long 
     if (lane == 63u) ws[w] = v;
     __syncthreads();
     total = 0ull;
-    for (uint32_t q = 0; q < kBlock / 64u; q++) {
+    for (uint32_t q = 0; q < NW; q++) {
         if (q < w) v += ws[q];
         total += ws[q];
     }
     return v;
 }
 
-// The hits among staged candidates [lo, hi) in order: four candidates per step (hit_bits4,
-// the threshold of equal radii), a hit mask per 32 candidates, then the hits' ids (held in w) as
-// list entries cnt, cnt + 1, ... (entries past K are counted only).
-// `self` is the particle's own staged index, which is not a neighbour (any value >= hi: none).
-template <int LAYOUT>
-__device__ __forceinline__ void walk_run(const float4* cand, uint32_t lo, uint32_t hi, const float4& xi, float thr, float t2lo,
-                                         float t2hi, uint32_t self, uint32_t* __restrict__ out, uint32_t K, uint32_t N,
-                                         uint32_t i, uint32_t& cnt) {
-    for (uint32_t c0 = lo; c0 < hi; c0 += 32u) {
-        const uint32_t n = min(hi - c0, 32u);
-        uint32_t m = 0u;
-        for (uint32_t q = 0; q < n; q += 4u) {
-            float4 v[4];
-#pragma unroll
-            for (uint32_t k = 0; k < 4u; k++) v[k] = cand[c0 + q + k];  // <= hi + 2 < array size
-            m |= hit_bits4(xi, thr, t2lo, t2hi, v) << q;
-        }
-        m &= n < 32u ? (1u << n) - 1u : ~0u;  // the group of four read past hi
-        const uint32_t d = self - c0;
-        if (d < 32u) m &= ~(1u << d);
-        while (m) {
-            const uint32_t b = static_cast<uint32_t>(__builtin_ctz(m));
-            m &= m - 1u;
-            if (cnt < K) out[list_at<LAYOUT>(cnt, i, K, N)] = __float_as_uint(cand[c0 + b].w);
-            cnt++;
-        }
-    }
+template <int L>
+__device__ __forceinline__ uint32_t quad_u32(uint32_t v) {  // the value of lane L of the quad
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), L * 0x55, 0xF, 0xF, true));
+}
+__device__ __forceinline__ uint32_t quad_sum(uint32_t v) { return quad_u32<0>(v) + quad_u32<1>(v) + quad_u32<2>(v) + quad_u32<3>(v); }
+// Sum over the quad's lanes before lane l (every lane reads every other: no lane may be masked off).
+__device__ __forceinline__ uint32_t quad_before(uint32_t v, uint32_t l) {
+    const uint32_t a = quad_u32<0>(v), b = quad_u32<1>(v), c = quad_u32<2>(v);
+    return (l > 0u ? a : 0u) + (l > 1u ? b : 0u) + (l > 2u ? c : 0u);
 }
 
-__global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __restrict__ pos, Scenes sc, uint32_t C, HashGeom g,
+// The hits of one slot among its 9 row runs; with Q = 4 a lane holds the runs l, l + 4 and 8 (l = 0).
+template <int Q, uint32_t WORDS>
+struct RowHits {
+    static constexpr uint32_t kRuns = Q == 1 ? 9 : 3;
+    uint32_t lo[kRuns];             // first staged copy of each run
+    uint32_t m[kRuns][WORDS];       // its hits, one bit per copy
+    uint32_t at[kRuns];             // list position of its first hit
+    uint32_t count;                 // hits of all runs
+
+    // run(r) gives the [lo, hi) of run r; `self` is the slot's own staged copy (any other value:
+    // none); a copy is a hit when its squared distance is below `cut`. False if a run is too long for
+    // its mask (for the whole quad).
+    template <class Run>
+    __device__ __forceinline__ bool test(const float4* cand, uint32_t l, const float4& xi, float cut, uint32_t self, Run&& run) {
+        uint32_t over = 0u, n[kRuns];
+#pragma unroll
+        for (uint32_t q = 0; q < kRuns; q++) {
+            const uint32_t r = Q == 1 ? q : l + 4u * q;
+            uint32_t a = 0u, b = 0u;
+            if (r < 9u) run(r, a, b);
+            lo[q] = a;
+            over |= b - a > 32u * WORDS ? 1u : 0u;
+            n[q] = 0u;
+#pragma unroll
+            for (uint32_t w = 0; w < WORDS; w++) {
+                uint32_t mm = 0u;
+                const uint32_t c0 = a + 32u * w;
+                if (c0 < b) {
+                    const uint32_t len = min(b - c0, 32u);
+                    uint32_t k = 0;
+                    for (; k < len; k += 4u) {
+                        float4 v[4];
+#pragma unroll
+                        for (uint32_t e = 0; e < 4u; e++) v[e] = cand[c0 + k + e];  // <= hi + 2 < array size
+#pragma unroll
+                        for (uint32_t e = 0; e < 4u; e++) {
+                            const float dx = xi.x - v[e].x, dy = xi.y - v[e].y, dz = xi.z - v[e].z;
+                            push_hit(mm, (dx * dx + dy * dy) + dz * dz, cut);
+                        }
+                    }
+                    mm = __brev(mm) >> (32u - k);                // bit e: copy c0 + e
+                    mm &= len < 32u ? (1u << len) - 1u : ~0u;  // the group of four read past hi
+                    const uint32_t d = self - c0;
+                    if (d < 32u) mm &= ~(1u << d);
+                }
+                m[q][w] = mm;
+                n[q] += __popc(mm);
+            }
+        }
+        if constexpr (Q == 1) {
+            count = 0u;
+#pragma unroll
+            for (uint32_t q = 0; q < kRuns; q++) {
+                at[q] = count;
+                count += n[q];
+            }
+            return !over;
+        } else {
+            const uint32_t t0 = quad_sum(n[0]), t1 = quad_sum(n[1]);
+            at[0] = quad_before(n[0], l);
+            at[1] = t0 + quad_before(n[1], l);
+            at[2] = t0 + t1;
+            count = t0 + t1 + quad_sum(n[2]);
+            return quad_sum(over) == 0u;
+        }
+    }
+    // use(list position, staged copy) for every hit, in list order within a run
+    template <class Use>
+    __device__ __forceinline__ void each(Use&& use) const {
+#pragma unroll
+        for (uint32_t q = 0; q < kRuns; q++) {
+            uint32_t k = at[q];
+#pragma unroll
+            for (uint32_t w = 0; w < WORDS; w++) {
+                uint32_t b = m[q][w];
+                while (b) {
+                    const uint32_t t = lo[q] + 32u * w + static_cast<uint32_t>(__builtin_ctz(b));
+                    b &= b - 1u;
+                    use(k, t);
+                    k++;
+                }
+            }
+        }
+    }
+};
+
+template <int Q, class Caps, bool LAST>
+__global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __restrict__ pos, Scenes sc, uint32_t C, HashGeom g,
                                                           HashView fl, HashView bd, uint32_t* __restrict__ nff, uint32_t Kff,
                                                           uint32_t* __restrict__ cff, uint32_t* __restrict__ nfb, uint32_t Kfb,
-                                                          uint32_t* __restrict__ cfb, uint2* __restrict__ bstat) {
+                                                          uint32_t* __restrict__ cfb, uint2* __restrict__ bstat,
+                                                          launch::HaloOut ho, int left, NbrCounters* __restrict__ ctr) {
+    constexpr uint32_t kThreads = Q * kBlock, kWaves = kThreads / 64u;
+    constexpr uint32_t kRowHash = Caps::kRowHash, kRows = Caps::kRows, kCells = Caps::kCells, kCand = Caps::kCand;
+    constexpr uint32_t kCellsPer = (kCells + kThreads - 1u) / kThreads;  // cells per thread
+    static_assert(kRows <= kThreads && kRows <= 255u + 1u && kRows < kRowHash, "one row per thread");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    if (LAST && left && ho.n[blk] != kHaloTodo) return;  // the first pass did this block
     const uint32_t tid = threadIdx.x;
-    const uint32_t i = blk * kBlock + tid;
+    const uint32_t i = blk * kBlock + tid / Q;
+    const uint32_t l = tid % Q;
     const uint32_t N = sc.N;
     const uint32_t sid = sc.blk_scene[blk];
     const uint32_t end = sc.P[sid].end;
@@ -539,19 +649,21 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __rest
     const uint32_t* fend = fl.end + base;
     const uint32_t* bstart = bd.start + base;
     const uint32_t* bend = bd.end + base;
-    __shared__ uint32_t rkey[kSrchRowHash];      // row hash: wrapped key of the row's cell x = 0
-    __shared__ int rxlo[kSrchRowHash], rxhi[kSrchRowHash];  // the row's x range (unwrapped)
-    __shared__ uint16_t rbase[kSrchRowHash];     // the row's first cell
-    __shared__ uint8_t rslot[kSrchRows];         // hash slot of each row, in registration order
-    __shared__ uint32_t ecell[kSrchCells], efs[kSrchCells], ebs[kSrchCells];
-    __shared__ uint16_t efo[kSrchCells + 1], ebo[kSrchCells + 1];
-    __shared__ float4 cand[kSrchCand + kSrchPad];
-    __shared__ unsigned long long ws[kBlock / 64];
+    __shared__ uint32_t rkey[kRowHash];      // row hash: wrapped key of the row's cell x = 0
+    __shared__ int rxlo[kRowHash], rxhi[kRowHash];  // the row's x range (unwrapped)
+    __shared__ uint16_t rbase[kRowHash];     // the row's first cell
+    __shared__ uint16_t rslot[kRows];        // hash slot of each row, in registration order
+    static_assert(kCells % 8u == 0u, "the halo pass reads eight cells at a time");
+    __shared__ __align__(16) uint32_t ecell[kCells], efs[kCells], ebs[kCells];
+    __shared__ uint16_t efo[kCells + 1], ebo[kCells + 1];
+    __shared__ float4 cand[kCand + kSrchPad];
+    __shared__ unsigned long long ws[kWaves];
     __shared__ uint32_t nrow, mixed, first[2];  // first: first cell with fluid, with walls
-    if (tid < kSrchRowHash) {
-        rkey[tid] = kNoRow;
-        rxlo[tid] = 0x7FFFFFFF;
-        rxhi[tid] = -0x7FFFFFFF - 1;
+    auto row_hash = [](uint32_t c) -> uint32_t { return (c * 2654435761u) >> (32u - Caps::kHashBits); };
+    for (uint32_t t = tid; t < kRowHash; t += kThreads) {
+        rkey[t] = kNoRow;
+        rxlo[t] = 0x7FFFFFFF;
+        rxhi[t] = -0x7FFFFFFF - 1;
     }
     if (tid == 0) {
         nrow = 0u;
@@ -561,7 +673,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __rest
     const float4 xi = live ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     const i3 p = grid_pos(xi.x, xi.y, xi.z, g);
     bool leader = live;
-    if (live && tid > 0) {
+    if (live && tid >= Q) {
         const float4 xp = pos[i - 1];
         const i3 pp = grid_pos(xp.x, xp.y, xp.z, g);
         leader = pp.x != p.x || pp.y != p.y || pp.z != p.z;
@@ -570,40 +682,41 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __rest
     // 1. rows (inserts stop once the block is known to be over the cap, so the table never
     //    fills; every probe loop is bounded anyway)
     if (leader) {
-        for (int r = 0; r < 9; r++) {
-            if (*(volatile uint32_t*)&nrow > kSrchRows) break;
-            const uint32_t k = grid_index(0, p.y + r % 3 - 1, p.z + r / 3 - 1, g);
+        for (uint32_t r = l; r < 9u; r += Q) {
+            if (*(volatile uint32_t*)&nrow > kRows) break;
+            const uint32_t k = grid_index(0, p.y + int(r % 3u) - 1, p.z + int(r / 3u) - 1, g);
             uint32_t h = row_hash(k);
-            for (uint32_t probe = 0; probe < kSrchRowHash; probe++) {
+            for (uint32_t probe = 0; probe < kRowHash; probe++) {
                 const uint32_t prev = atomicCAS(&rkey[h], kNoRow, k);
                 if (prev == kNoRow) {
                     const uint32_t e = atomicAdd(&nrow, 1u);
-                    if (e < kSrchRows) rslot[e] = static_cast<uint8_t>(h);
+                    if (e < kRows) rslot[e] = static_cast<uint16_t>(h);
                 }
                 if (prev == kNoRow || prev == k) {
                     atomicMin(&rxlo[h], p.x - 1);
                     atomicMax(&rxhi[h], p.x + 1);
                     break;
                 }
-                h = (h + 1u) & (kSrchRowHash - 1u);
+                h = (h + 1u) & (kRowHash - 1u);
             }
         }
     }
     __syncthreads();
     const uint32_t nr = nrow;
-    bool staged = nr <= kSrchRows;
+    bool staged = nr <= kRows;
     uint32_t nc = 0u;
     // 2. number each row's cells over its x range (rows in registration order)
     if (staged) {
         const uint32_t h = tid < nr ? rslot[tid] : 0u;
-        const uint32_t len = tid < nr ? static_cast<uint32_t>(min(static_cast<long long>(rxhi[h]) - rxlo[h] + 1, 
-                                                                 static_cast<long long>(kSrchCells) + 1)) : 0u;
+        const uint32_t len = tid < nr ? static_cast<uint32_t>(min(static_cast<long long>(rxhi[h]) - rxlo[h] + 1,
+                                                                 static_cast<long long>(kCells) + 1)) : 0u;
         unsigned long long tot;
-        const uint32_t b0 = static_cast<uint32_t>(block_scan_u64(len, ws, tot)) - len;
+        const uint32_t b0 = static_cast<uint32_t>(block_scan_u64<kWaves>(len, ws, tot)) - len;
         nc = static_cast<uint32_t>(tot);
-        staged = nc <= kSrchCells;
+        staged = nc <= kCells;
         if (staged && tid < nr) {
             rbase[h] = static_cast<uint16_t>(b0);
+            if (len > g.hx) atomicOr(&mixed, 4u);  // the row wraps around: a cell is staged twice (see 6.)
             const uint32_t k0 = rkey[h];
             for (uint32_t q = 0; q < len; q++) ecell[b0 + q] = k0 + (static_cast<uint32_t>(rxlo[h] + static_cast<int>(q)) & (g.hx - 1u));
         }
@@ -613,10 +726,11 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __rest
     //    after all fluid
     uint32_t tf = 0u, tb = 0u;
     if (staged) {
-        uint32_t fc[2] = {0u, 0u}, bc[2] = {0u, 0u};
+        uint32_t fc[kCellsPer], bc[kCellsPer], fsum = 0u, bsum = 0u;
 #pragma unroll
-        for (uint32_t q = 0; q < 2; q++) {
-            const uint32_t e = 2u * tid + q;
+        for (uint32_t q = 0; q < kCellsPer; q++) {
+            const uint32_t e = kCellsPer * tid + q;
+            fc[q] = bc[q] = 0u;
             if (e < nc) {
                 const uint32_t c = ecell[e];
                 const uint32_t s0 = fstart[c], s1 = fend[c];
@@ -628,19 +742,22 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __rest
                     bc[q] = b0 < b1 ? b1 - b0 : 0u;
                 }
             }
+            fsum += fc[q];
+            bsum += bc[q];
         }
-        const unsigned long long mine = (static_cast<unsigned long long>(bc[0] + bc[1]) << 32) | (fc[0] + fc[1]);
+        const unsigned long long mine = (static_cast<unsigned long long>(bsum) << 32) | fsum;
         unsigned long long tot;
-        const unsigned long long ex = block_scan_u64(mine, ws, tot) - mine;
+        const unsigned long long ex = block_scan_u64<kWaves>(mine, ws, tot) - mine;
         tf = static_cast<uint32_t>(tot & 0xFFFFFFFFull);
         tb = static_cast<uint32_t>(tot >> 32);
-        staged = static_cast<unsigned long long>(tf) + tb <= kSrchCand;
+        staged = static_cast<unsigned long long>(tf) + tb <= kCand;
+        if (!LAST && tid == 0 && static_cast<unsigned long long>(tf) + tb > SearchStd::kCand) atomicAdd(&ctr->crowded, 1u);
         uint32_t fo = static_cast<uint32_t>(ex & 0xFFFFFFFFull), bo = static_cast<uint32_t>(ex >> 32);
         if (staged) {
             // each copy's w first holds its cell (read back by the staging pass)
 #pragma unroll
-            for (uint32_t q = 0; q < 2; q++) {
-                const uint32_t e = 2u * tid + q;
+            for (uint32_t q = 0; q < kCellsPer; q++) {
+                const uint32_t e = kCellsPer * tid + q;
                 if (e < nc) {
                     efo[e] = static_cast<uint16_t>(fo);
                     ebo[e] = static_cast<uint16_t>(tf + bo);
@@ -659,79 +776,195 @@ __global__ void __launch_bounds__(kBlock) k_neighbors_fluid(const float4* __rest
         }
         __syncthreads();
     }
-    // 4. stage the candidates with their ids (copy t of cell e is particle efs[e] + t - efo[e]).
-    //    `mixed` records whether some fluid (bit 0) or wall (bit 1) candidate has another radius
-    //    than the first staged candidate of its set.
+    // 4. stage the candidates with their ids (copy t of cell e is particle efs[e] + t - efo[e]),
+    //    kStage loads of a thread in flight. `mixed` records whether some fluid (bit 0) or wall (bit 1)
+    //    candidate has another radius than the first staged candidate of its set.
     float rw = 0.0f;  // the walls' common radius
     if (staged) {
+        constexpr uint32_t kStage = 4;
         uint32_t mx = 0u;
-        if (tf) {
-            const float rf = pos[efs[first[0]]].w;
-            for (uint32_t t = tid; t < tf; t += kBlock) {
-                const uint32_t e = __float_as_uint(cand[t].w);
-                const uint32_t s = efs[e] + (t - efo[e]);
-                const float4 v = pos[s];
-                cand[t] = make_float4(v.x, v.y, v.z, __uint_as_float(s));
-                mx |= v.w != rf ? 1u : 0u;
+        auto stage = [&](uint32_t t_lo, uint32_t t_hi, const uint32_t* es, const uint16_t* eo, const float4* from, const uint32_t* id,
+                         float r0, uint32_t bit) {
+            for (uint32_t t0 = t_lo + tid; t0 < t_hi; t0 += kStage * kThreads) {
+                float4 v[kStage];
+                uint32_t s[kStage];
+#pragma unroll
+                for (uint32_t q = 0; q < kStage; q++) {
+                    const uint32_t t = t0 + q * kThreads;
+                    if (t < t_hi) {
+                        const uint32_t e = __float_as_uint(cand[t].w);
+                        s[q] = es[e] + (t - eo[e]);
+                        v[q] = from[s[q]];
+                        if (id) s[q] = id[s[q]];
+                    }
+                }
+#pragma unroll
+                for (uint32_t q = 0; q < kStage; q++) {
+                    const uint32_t t = t0 + q * kThreads;
+                    if (t < t_hi) {
+                        cand[t] = make_float4(v[q].x, v[q].y, v[q].z, __uint_as_float(s[q]));
+                        mx |= v[q].w != r0 ? bit : 0u;
+                    }
+                }
             }
-        }
+        };
+        if (tf) stage(0u, tf, efs, efo, pos, nullptr, pos[efs[first[0]]].w, 1u);
         if (tb) {
             rw = bd.spos[ebs[first[1]]].w;
-            for (uint32_t t = tf + tid; t < tf + tb; t += kBlock) {
-                const uint32_t e = __float_as_uint(cand[t].w);
-                const uint32_t sb = ebs[e] + (t - ebo[e]);
-                const float4 v = bd.spos[sb];
-                cand[t] = make_float4(v.x, v.y, v.z, __uint_as_float(bd.id ? bd.id[sb] : sb));
-                mx |= v.w != rw ? 2u : 0u;
-            }
+            stage(tf, tf + tb, ebs, ebo, bd.spos, bd.id, rw, 2u);
         }
         if (mx) atomicOr(&mixed, mx);
         __syncthreads();
     }
     // 5. the search proper: 9 rows (z, then y offsets), each the run of cells x-1, x, x+1
     uint32_t a = 0u, b = 0u;
-    if (live) {
-        const uint32_t mix = staged ? mixed : 3u;
-        const float ri = xi.w * 4.0f;
-        // the particle's cell x + dx in row (y, z)
-        auto cell_of = [&](int dx, int y, int z) -> uint32_t {
-            const uint32_t k = grid_index(0, y, z, g);
-            uint32_t h = row_hash(k);
+    const uint32_t mix = staged ? mixed : 3u;
+    const float ri = xi.w * 4.0f;
+    // the particle's cell x + dx in row (y, z)
+    auto cell_of = [&](int dx, int y, int z) -> uint32_t {
+        const uint32_t k = grid_index(0, y, z, g);
+        uint32_t h = row_hash(k);
 #pragma unroll 1
-            for (uint32_t probe = 0; probe < kSrchRowHash && rkey[h] != k; probe++) h = (h + 1u) & (kSrchRowHash - 1u);
-            return rkey[h] == k ? rbase[h] + static_cast<uint32_t>(p.x + dx - rxlo[h]) : kNoRow;
-        };
-        auto rows = [&](auto layout, const uint16_t* eo, float thr, uint32_t self, uint32_t* out, uint32_t K, uint32_t& cnt) {
-            const float t2 = thr * thr, t2lo = t2 * 0.9999f, t2hi = t2 * 1.0001f;
-            for (int r = 0; r < 9; r++) {
-                const uint32_t e = cell_of(-1, p.y + r % 3 - 1, p.z + r / 3 - 1);
-                if (e == kNoRow) continue;  // not reached: every row of a run was registered
-                walk_run<decltype(layout)::value>(cand, eo[e], eo[e + 3u], xi, thr, t2lo, t2hi, self, out, K, N, i, cnt);
-            }
-        };
+        for (uint32_t probe = 0; probe < kRowHash && rkey[h] != k; probe++) h = (h + 1u) & (kRowHash - 1u);
+        return rkey[h] == k ? rbase[h] + static_cast<uint32_t>(p.x + dx - rxlo[h]) : kNoRow;
+    };
+    auto run_of = [&](const uint16_t* eo, uint32_t r, uint32_t& lo, uint32_t& hi) {
+        const uint32_t e = cell_of(-1, p.y + int(r % 3u) - 1, p.z + int(r / 3u) - 1);
+        if (e == kNoRow) return;  // not reached: every row of a run was registered
+        lo = eo[e];
+        hi = eo[e + 3u];
+    };
+    // a search of the global tables (one lane of the slot), its count in every lane
+    auto global = [&](auto&& search) -> uint32_t {
+        const uint32_t n = l == 0u ? search() : 0u;
+        if constexpr (Q == 1) return n;
+        else return quad_u32<0>(n);
+    };
+    RowHits<Q, Caps::kWords> hits;
+    bool have = false;  // `hits` are this slot's fluid neighbours
+    if (live) {
         if (!(mix & 1u)) {
             const uint32_t eh = cell_of(0, p.y, p.z);
             const uint32_t self = eh == kNoRow ? kNoRow : efo[eh] + (i - efs[eh]);
-            rows(std::integral_constant<int, kGroups>{}, efo, (ri + ri) * 0.5f, self, nff, Kff, a);
+            have = hits.test(cand, l, xi, cut_of((ri + ri) * 0.5f), self, [&](uint32_t r, uint32_t& lo, uint32_t& hi) { run_of(efo, r, lo, hi); });
+        }
+        if (have) {
+            a = hits.count;
+            hits.each([&](uint32_t k, uint32_t t) {
+                const uint32_t s = __float_as_uint(cand[t].w) & ~kHit;
+                cand[t].w = __uint_as_float(s | kHit);
+                if (k < Kff) nff[ell(k, i, N)] = s;
+            });
+        } else if constexpr (LAST) {
+            a = global([&] { return search_cells<true, kGroups>(xi, i, g, fstart, fend, fl.id, fl.spos, nff, Kff, N); });
+            if (!(mix & 1u)) atomicOr(&mixed, 4u);  // a run too long: the block's halo is left to k_halo_build
         } else {
-            a = search_cells<true, kGroups>(xi, i, g, fstart, fend, fl.id, fl.spos, nff, Kff, N);
+            atomicOr(&mixed, 4u);
         }
         if (bd.n) {
             if (staged && tb == 0u) {
                 b = 0u;  // no wall particle in any cell of the block
-            } else if (!(mix & 2u)) {
-                rows(std::integral_constant<int, kCols>{}, ebo, (ri + rw * 4.0f) * 0.5f, kNoRow, nfb, Kfb, b);
             } else {
-                b = search_cells<false, kCols>(xi, i, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N);
+                RowHits<Q, Caps::kWords> wh;
+                if (!(mix & 2u) && wh.test(cand, l, xi, cut_of((ri + rw * 4.0f) * 0.5f), kNoRow,
+                                           [&](uint32_t r, uint32_t& lo, uint32_t& hi) { run_of(ebo, r, lo, hi); })) {
+                    b = wh.count;
+                    wh.each([&](uint32_t k, uint32_t t) {
+                        if (k < Kfb) nfb[size_t(k) * N + i] = __float_as_uint(cand[t].w);
+                    });
+                } else if constexpr (LAST) {
+                    b = global([&] { return search_cells<false, kCols>(xi, i, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N); });
+                } else {
+                    atomicOr(&mixed, 4u);
+                }
             }
         }
     }
-    if (i < N) {
+    if (l == 0u && i < N) {
         cff[i] = a;
         cfb[i] = b;
     }
-    const uint32_t cnt[2] = {a, b};
-    block_counts<2>(cnt, bstat, gridDim.x, blk);
+    // 6. the block's halo: the marked copies, cells in order of their first slot (cells are disjoint
+    //    slot ranges, so that is ascending slot order; a block with a cell staged twice is left out)
+    __syncthreads();
+    if (!staged || (mixed & 5u)) {
+        if (tid == 0) {
+            ho.n[blk] = kHaloTodo;
+            atomicAdd(LAST ? &ctr->todo : &ctr->left, 1u);
+        }
+    } else {
+        // marked copies of each cell (in ecell, no longer needed), then their sum over the cells with
+        // smaller slots
+        uint32_t mine = 0u;
+#pragma unroll
+        for (uint32_t q = 0; q < kCellsPer; q++) {
+            const uint32_t e = kCellsPer * tid + q;
+            if (e < nc) {
+                uint32_t n = 0u;
+                for (uint32_t t = efo[e]; t < efo[e + 1u]; t++) n += __float_as_uint(cand[t].w) >> 31;
+                ecell[e] = n;
+                if (efo[e + 1u] == efo[e]) efs[e] = 0xFFFFFFFFu;
+                mine += n;
+            } else if (e < kCells) {
+                ecell[e] = 0u;
+            }
+        }
+        unsigned long long tot;
+        block_scan_u64<kWaves>(mine, ws, tot);  // (ends with every ecell written)
+        const uint32_t H = static_cast<uint32_t>(tot);
+        const bool fits = H <= ho.limit;
+        if (tid == 0) ho.n[blk] = fits ? H : kHaloCap + 1u;
+        if (fits) {
+            uint32_t* out = ho.idx + size_t(blk) * kHaloCap;
+            uint32_t from[kCellsPer];
+#pragma unroll
+            for (uint32_t q = 0; q < kCellsPer; q++) from[q] = 0u;
+            const uint32_t e0 = kCellsPer * tid;
+            if (e0 < nc) {
+                uint32_t s[kCellsPer];
+#pragma unroll
+                for (uint32_t q = 0; q < kCellsPer; q++) s[q] = e0 + q < nc ? efs[e0 + q] : 0u;
+                // four cells per read, two reads ahead (cells past nc count nothing)
+                for (uint32_t e = 0; e < nc; e += 8u) {
+                    uint4 se[2], n[2];
+#pragma unroll
+                    for (uint32_t h = 0; h < 2u; h++) {
+                        se[h] = reinterpret_cast<const uint4*>(efs)[e / 4u + h];
+                        n[h] = reinterpret_cast<const uint4*>(ecell)[e / 4u + h];
+                    }
+#pragma unroll
+                    for (uint32_t h = 0; h < 2u; h++)
+#pragma unroll
+                        for (uint32_t q = 0; q < kCellsPer; q++)
+                            from[q] += (se[h].x < s[q] ? n[h].x : 0u) + (se[h].y < s[q] ? n[h].y : 0u) +
+                                       (se[h].z < s[q] ? n[h].z : 0u) + (se[h].w < s[q] ? n[h].w : 0u);
+                }
+            }
+            __syncthreads();  // every position base is known before the copies' slots give way to positions
+#pragma unroll
+            for (uint32_t q = 0; q < kCellsPer; q++) {
+                const uint32_t e = e0 + q;
+                if (e < nc) {
+                    uint32_t at = from[q];
+                    for (uint32_t t = efo[e]; t < efo[e + 1u]; t++) {
+                        const uint32_t w = __float_as_uint(cand[t].w);
+                        if (w & kHit) {
+                            out[at] = w & ~kHit;
+                            cand[t].w = __uint_as_float(at);
+                            at++;
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            if (have)
+                hits.each([&](uint32_t k, uint32_t t) {
+                    if (k < Kff) ho.nb16[ell(k, i, N)] = static_cast<uint16_t>(__float_as_uint(cand[t].w));
+                });
+        }
+    }
+    const uint32_t cnt[2] = {l == 0u ? a : 0u, l == 0u ? b : 0u};
+    block_counts<2, kWaves>(cnt, bstat, gridDim.x, blk);
 }
 
 __global__ void __launch_bounds__(kBlock) k_neighbors_boundary(const float4* __restrict__ pos, uint32_t B,
@@ -876,26 +1109,42 @@ void cell_table(const uint32_t* key, const uint32_t* id, uint32_t n, uint32_t* s
 }
 void neighbors_fluid(const float4* pos, const Scenes& sc, uint32_t C, const HashGeom& g, const HashView& fl, const HashView& bd,
                      uint32_t* nff, uint32_t Kff, uint32_t* cff, uint32_t* nfb, uint32_t Kfb, uint32_t* cfb, uint2* bstat,
-                     NbrCounters* ctr, hipStream_t s) {
+                     HaloOut ho, SearchPasses passes, int dense, NbrCounters* ctr, hipStream_t s) {
     if (!sc.N) return;
     const uint32_t g_ = nb(sc.N);
-    launch_k(k_neighbors_fluid, g_, kBlock, 0, s, pos, sc, C, g, fl, bd, nff, Kff, cff, nfb, Kfb, cfb, bstat);
-    launch_k(k_count_fold, 1, kCountFoldThreads, 0, s, bstat, g_, &ctr->max_ff, &ctr->nnz_ff);
-    launch_k(k_count_fold, 1, kCountFoldThreads, 0, s, bstat + g_, g_, &ctr->max_fb, &ctr->nnz_fb);
+    ho.limit = ho.limit == 0u || ho.limit > kHaloCap ? kHaloCap : ho.limit;
+#define MPS_SEARCH(Q, CAPS, LAST, LEFT)                                                                                       \
+    launch_k(k_neighbors_fluid<Q, CAPS, LAST>, g_, Q * kBlock, 0, s, pos, sc, C, g, fl, bd, nff, Kff, cff, nfb, Kfb, cfb, bstat, \
+             ho, LEFT, ctr)
+    // Up to two workgroups per CU one pass of the quad form (its blocks have the chip to themselves:
+    // 128 workgroups 206 -> 72 us with the halos); beyond, the one-lane form and, where the last
+    // search left blocks (or this one did: passes = kSearchLeft), the quad form over those.
+    if (g_ <= 512u) {
+        MPS_SEARCH(4, SearchWide, true, 0);
+    } else {
+        if (passes != kSearchLeft) {
+            if (dense) MPS_SEARCH(1, SearchDense, false, 0);
+            else MPS_SEARCH(1, SearchStd, false, 0);
+        }
+        if (passes != kSearchFirst) MPS_SEARCH(4, SearchWide, true, 1);
+    }
+#undef MPS_SEARCH
+    // (max_ff, max_fb) and (nnz_ff, nnz_fb) are neighbours in the record
+    launch_k(k_count_fold, 3, kCountFoldThreads, 0, s, bstat, g_, &ctr->max_ff, &ctr->nnz_ff, ho.n, ho.stats);
 }
 void neighbors_ref(const float4* pos, const Scenes& sc, uint32_t C, const HashGeom& g, const HashView& fl, uint32_t* nfr,
                    uint32_t Kfr, uint32_t* cfr, uint2* bstat, NbrCounters* ctr, hipStream_t s) {
     if (!sc.N) return;
     const uint32_t g_ = nb(sc.N);
     launch_k(k_neighbors_ref, g_, kBlock, 0, s, pos, sc, C, g, fl, nfr, Kfr, cfr, bstat);
-    launch_k(k_count_fold, 1, kCountFoldThreads, 0, s, bstat, g_, &ctr->max_fr, &ctr->nnz_fr);
+    launch_k(k_count_fold, 1, kCountFoldThreads, 0, s, bstat, g_, &ctr->max_fr, &ctr->nnz_fr, nullptr, nullptr);
 }
 void neighbors_boundary(const float4* pos, uint32_t B, const uint32_t* scene, uint32_t C, const HashGeom& g, const HashView& bd,
                         uint32_t* nbb, uint32_t Kbb, uint32_t* cbb, uint2* bstat, NbrCounters* ctr, hipStream_t s) {
     if (!B) return;
     const uint32_t g_ = nb(B);
     launch_k(k_neighbors_boundary, g_, kBlock, 0, s, pos, B, scene, C, g, bd, nbb, Kbb, cbb, bstat);
-    launch_k(k_count_fold, 1, kCountFoldThreads, 0, s, bstat, g_, &ctr->max_bb, &ctr->nnz_bb);
+    launch_k(k_count_fold, 1, kCountFoldThreads, 0, s, bstat, g_, &ctr->max_bb, &ctr->nnz_bb, nullptr, nullptr);
 }
 void gather_f4(const uint32_t* perm, uint32_t n, const float4* in, float4* out, hipStream_t s) {
     if (n) launch_k(k_gather_f4, nb(n), kBlock, 0, s, perm, n, in, out);

@@ -31,6 +31,10 @@ struct HashView {
 // Neighbour statistics written by the search kernels.
 struct NbrCounters {
     uint32_t max_ff, max_fb, max_bb, max_fr;
+    uint32_t left;  // workgroups that the first pass of the fluid search left to the second
+    uint32_t crowded;  // workgroups of the first pass with more candidates than its usual form holds
+    uint32_t todo;  // workgroups of the fluid search whose halo is left to k_halo_build
+    uint32_t pad;
     unsigned long long nnz_ff, nnz_fb, nnz_bb, nnz_fr;
 };
 
@@ -106,6 +110,7 @@ constexpr uint32_t kMaxWallObjects = 4;
 // (four); the deep one pays once a few blocks in a thousand have halos over kHaloShallow.
 constexpr uint32_t kHaloCap = 1536;
 constexpr uint32_t kHaloShallow = 1264;
+constexpr uint32_t kHaloTodo = 0xFFFFFFFFu;  // n[b] after the search: this block's halo is still to be built
 struct Halo {
     const uint32_t* idx;
     const uint32_t* n;
@@ -175,11 +180,24 @@ void fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s);
 void clear_cells(const uint32_t* key, uint32_t n, uint32_t* start, uint32_t* end, hipStream_t s);
 void cell_table(const uint32_t* key, const uint32_t* id, uint32_t n, uint32_t* start, uint32_t* end, const float4* pos,
                 float4* spos, hipStream_t s);
+// Where the fluid search writes the block halos; limit: the largest one kept (0 or > kHaloCap:
+// kHaloCap).
+struct HaloOut {
+    uint32_t* idx;
+    uint32_t* n;
+    uint16_t* nb16;
+    uint32_t limit;
+    uint32_t* stats;  // 4 words: see k_count_fold
+};
+// The passes of a search over many blocks: the first alone, both, or the second for the blocks that
+// the first left (NbrCounters::left; both passes in one call do without the host's look at it).
+// dense: the first pass in its form with more candidates (and three workgroups per CU, not four).
+enum SearchPasses { kSearchFirst, kSearchBoth, kSearchLeft };
 // bstat: scratch of 2 * ceil(N / kBlock) (fluid) or ceil(B / kBlock) (walls) per-workgroup
 // count records, folded into ctr after the search
 void neighbors_fluid(const float4* pos, const Scenes& sc, uint32_t C, const dev::HashGeom& g, const HashView& fl,
                      const HashView& bd, uint32_t* nff, uint32_t Kff, uint32_t* cff, uint32_t* nfb, uint32_t Kfb, uint32_t* cfb,
-                     uint2* bstat, NbrCounters* ctr, hipStream_t s);
+                     uint2* bstat, HaloOut ho, SearchPasses passes, int dense, NbrCounters* ctr, hipStream_t s);
 // ref lists of coupled scenes (other scenes' fluid, ascending scene order)
 void neighbors_ref(const float4* pos, const Scenes& sc, uint32_t C, const dev::HashGeom& g, const HashView& fl, uint32_t* nfr,
                    uint32_t Kfr, uint32_t* cfr, uint2* bstat, NbrCounters* ctr, hipStream_t s);
@@ -284,8 +302,9 @@ void cg_persistent(const CgOperator& op, int coherent, const Scenes& sc, const N
 // ---- halo.hip
 // stats (3 words, accumulated): largest staged halo, blocks over kHaloCap, blocks with particles
 // limit: largest halo staged (0 or > kHaloCap: kHaloCap)
-void halo_build(const Scenes& sc, const Nbr& nb, uint32_t nblk, uint32_t limit, uint32_t* hidx, uint32_t* hn, uint16_t* n16,
-                uint32_t* stats, hipStream_t s);
+// all: every block, or only those with n = kHaloTodo
+void halo_build(int all, const Scenes& sc, const Nbr& nb, uint32_t nblk, uint32_t limit, uint32_t* hidx, uint32_t* hn,
+                uint16_t* n16, uint32_t* stats, hipStream_t s);
 // mode 0: initial r.r + test; 1: alpha; 2: new r.r, beta + test
 void fold_cg(int mode, const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, hipStream_t s);
 // x += alpha p, r -= alpha Ap, partial r.r (p from the records; the adjoint's solve)
