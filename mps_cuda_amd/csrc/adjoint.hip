@@ -294,112 +294,26 @@ __global__ void __launch_bounds__(kBlock) k_adj_dbar(Scenes sc, Nbr nb, const fl
 }
 
 // ----------------------------------------------------------------- implicit viscosity / ST solve
-// rev at entry k of slot i (ell()) = position of i in the list of its k-th neighbour (the lists are symmetric);
-// kEmpty (and *bad = 1) if it is missing.
-__global__ void __launch_bounds__(kBlock) k_adj_rev_index(Scenes sc, Nbr nb, uint32_t* __restrict__ rev, uint32_t* bad) {
-    const uint32_t sid = sc.blk_scene[blockIdx.x];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t N = sc.N;
-    if (i >= sc.P[sid].end) return;
-    const uint32_t c = nb.cff[i];
-    for (uint32_t k = 0; k < c; k++) {
-        const uint32_t j = nb.ff[ell(k, i, N)];
-        const uint32_t cj = nb.cff[j];
-        uint32_t m = kEmpty;
-        for (uint32_t q = 0; q < cj; q++)
-            if (nb.ff[ell(q, j, N)] == i) {
-                m = q;
-                break;
-            }
-        if (m == kEmpty) atomicOr(bad, 1u);
-        rev[ell(k, i, N)] = m;
-    }
-}
-// (caT, cbT) at entry k of slot i = the coefficients (a_ji, b_ji) of the pair seen from the neighbour j
-__global__ void __launch_bounds__(kBlock) k_adj_transpose_coeffs(Scenes sc, Nbr nb, const uint32_t* __restrict__ rev,
-                                                               const float* __restrict__ ca, const float* __restrict__ cb,
-                                                               float* __restrict__ caT, float* __restrict__ cbT) {
-    const uint32_t sid = sc.blk_scene[blockIdx.x];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t N = sc.N;
-    if (i >= sc.P[sid].end) return;
-    const uint32_t c = nb.cff[i];
-    for (uint32_t k = 0; k < c; k++) {
-        const size_t slot = ell(k, i, N);
-        const uint32_t m = rev[slot];
-        const size_t at = m == kEmpty ? 0 : ell(m, nb.ff[slot], N);
-        caT[slot] = m == kEmpty ? 0.0f : ca[at];
-        cbT[slot] = m == kEmpty ? 0.0f : cb[at];
-    }
-}
-
-__device__ __forceinline__ f3 rec_pv(float4 a, float4 b) { return {a.w, b.x, b.y}; }
 // Start of the transposed solve A_f^T lambda = b from lambda = 0: r = p = b, partial r.r.
-__global__ void __launch_bounds__(kBlock) k_adj_cg_init(Scenes sc, const float4* __restrict__ pos, const float4* __restrict__ b,
-                                                      float4* __restrict__ x, float4* __restrict__ r, float4* __restrict__ rec,
-                                                      double* __restrict__ partials) {
+__global__ void __launch_bounds__(kBlock) k_adj_cg_start(Scenes sc, const float4* __restrict__ b, f3* __restrict__ x,
+                                                       f3* __restrict__ r, f3* __restrict__ p, double* __restrict__ partials) {
     __shared__ double lds[kBlock / 64];
     const uint32_t sid = sc.blk_scene[blockIdx.x];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     double part = 0.0;
-    if (i < sc.N) {
-        const float4 p4 = pos[i];
-        float4 b4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (i < sc.P[sid].end) {
-            b4 = b[i];
-            part = double(b4.x * b4.x) + double(b4.y * b4.y) + double(b4.z * b4.z);
-        }
-        x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        r[i] = make_float4(b4.x, b4.y, b4.z, 0.f);
-        rec[2 * size_t(i)] = make_float4(p4.x, p4.y, p4.z, b4.x);
-        rec[2 * size_t(i) + 1] = make_float4(b4.y, b4.z, 0.f, 0.f);
+    if (i < sc.P[sid].end) {
+        const f3 bi = mk(b[i]);
+        part = double(bi.x * bi.x) + double(bi.y * bi.y) + double(bi.z * bi.z);
+        x[i] = f3z();
+        r[i] = bi;
+        p[i] = bi;
     }
     const double s = block_sum_d(part, lds);
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
-// Warm start: r = b - A_f^T x0 (x0 packed in recA), p = r into recB, x = x0; partials of r.r
-// at partials[blk] and of b.b at partials[nblk + blk].
-__global__ void __launch_bounds__(kBlock) k_adj_cg_init_warm(Scenes sc, Nbr nb, const float* __restrict__ ca,
-                                                           const float* __restrict__ cb, const float* __restrict__ caT,
-                                                           const float* __restrict__ cbT, const float4* __restrict__ recA,
-                                                           const float4* __restrict__ b, float4* __restrict__ x,
-                                                           float4* __restrict__ r, float4* __restrict__ recB,
-                                                           double* __restrict__ partials, uint32_t nblk) {
-    const uint32_t sid = sc.blk_scene[blockIdx.x];
-    const StepParams P = sc.P[sid];
+__global__ void __launch_bounds__(kBlock) k_adj_lambda(Scenes sc, const f3* __restrict__ x, float4* __restrict__ lam) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
-    double prr = 0.0, pbb = 0.0;
-    if (i < N) {
-        const float4 ra = recA[2 * size_t(i)], rb = recA[2 * size_t(i) + 1];
-        const f3 xi = mk(ra), x0 = rec_pv(ra, rb);
-        f3 ri = f3z();
-        if (i < P.end) {
-            f3 acc = f3z();
-            const uint32_t c = nb.cff[i];
-            for (uint32_t k = 0; k < c; k++) {
-                const size_t slot = ell(k, i, N);
-                const uint32_t j = nb.ff[slot];
-                const float2 ab = make_float2(ca[slot], cb[slot]), abT = make_float2(caT[slot], cbT[slot]);
-                const float4 ja = recA[2 * size_t(j)], jb = recA[2 * size_t(j) + 1];
-                const f3 xij = xi - mk(ja);
-                const f3 pj = rec_pv(ja, jb);
-                acc = acc + (ab.x * x0 - abT.x * pj) + (ab.y * dot3(x0, xij) - abT.y * dot3(pj, xij)) * xij;
-            }
-            const f3 Ax = x0 * (1.0f + P.cg_factor) + acc;
-            const f3 bi = mk(b[i]);
-            ri = bi - Ax;
-            prr = double(ri.x * ri.x) + double(ri.y * ri.y) + double(ri.z * ri.z);
-            pbb = double(bi.x * bi.x) + double(bi.y * bi.y) + double(bi.z * bi.z);
-            x[i] = make_float4(x0.x, x0.y, x0.z, 0.0f);
-        } else {
-            x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        r[i] = make_float4(ri.x, ri.y, ri.z, 0.0f);
-        recB[2 * size_t(i)] = make_float4(xi.x, xi.y, xi.z, ri.x);
-        recB[2 * size_t(i) + 1] = make_float4(ri.y, ri.z, 0.f, 0.f);
-    }
-    block_partial2(prr, pbb, partials, nblk);
+    if (i < sc.P[sc.blk_scene[blockIdx.x]].end) lam[i] = f4(x[i], 0.0f);
 }
 // Start of the transposed loop: r.r, and the stop threshold -tol * b.b (relative to the right-
 // hand side, so a good starting guess does not tighten it) or tol.
@@ -425,41 +339,6 @@ __global__ void __launch_bounds__(kBlock) k_adj_fold_start(Scenes sc, const doub
             atomicSub(active, 1u);
         }
     }
-}
-
-// (A_f^T p)_i = (1+f) p_i + sum_j [ (a_ij p_i - a_ji p_j) + (b_ij (p_i.x_ij) - b_ji (p_j.x_ij)) x_ij ]
-// and partials of p.Ap, for scenes whose solve is still running.
-__global__ void __launch_bounds__(kBlock) k_adj_cg_applyT(Scenes sc, Nbr nb, const float* __restrict__ ca,
-                                                        const float* __restrict__ cb, const float* __restrict__ caT,
-                                                        const float* __restrict__ cbT, const float4* __restrict__ rec,
-                                                        float4* __restrict__ Ap, const SolverDev* st, double* __restrict__ partials) {
-    __shared__ double lds[kBlock / 64];
-    const uint32_t sid = sc.blk_scene[blockIdx.x];
-    if (st[sid].done) return;
-    const StepParams P = sc.P[sid];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t N = P.N;
-    double part = 0.0;
-    if (i < P.end) {
-        const float4 ra = rec[2 * size_t(i)], rb = rec[2 * size_t(i) + 1];
-        const f3 xi = mk(ra), pi = rec_pv(ra, rb);
-        f3 acc = f3z();
-        const uint32_t c = nb.cff[i];
-        for (uint32_t k = 0; k < c; k++) {
-            const size_t slot = ell(k, i, N);
-            const uint32_t j = nb.ff[slot];
-            const float2 ab = make_float2(ca[slot], cb[slot]), abT = make_float2(caT[slot], cbT[slot]);
-            const float4 ja = rec[2 * size_t(j)], jb = rec[2 * size_t(j) + 1];
-            const f3 xij = xi - mk(ja);
-            const f3 pj = rec_pv(ja, jb);
-            acc = acc + (ab.x * pi - abT.x * pj) + (ab.y * dot3(pi, xij) - abT.y * dot3(pj, xij)) * xij;
-        }
-        const f3 o = pi * (1.0f + P.cg_factor) + acc;
-        Ap[i] = make_float4(o.x, o.y, o.z, 0.0f);
-        part = double(pi.x * o.x) + double(pi.y * o.y) + double(pi.z * o.z);
-    }
-    const double s = block_sum_d(part, lds);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
 // The pair term of the residual seen from particle "i" (self) with neighbour "j" (other):
@@ -824,20 +703,11 @@ void adj_dbar(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, con
                  bvel, pG_ff, pG_fb, dbar, L, it, av, ax);
     });
 }
-void adj_rev_index(const Scenes& sc, const Nbr& nb, uint32_t* rev, uint32_t* bad, hipStream_t s) {
-    if (sc.N) launch_k(k_adj_rev_index, nbk(sc.N), kBlock, 0, s, sc, nb, rev, bad);
+void adj_cg_start(const Scenes& sc, const float4* b, f3* x, f3* r, f3* p, double* partials, hipStream_t s) {
+    if (sc.N) launch_k(k_adj_cg_start, nbk(sc.N), kBlock, 0, s, sc, b, x, r, p, partials);
 }
-void adj_transpose_coeffs(const Scenes& sc, const Nbr& nb, const uint32_t* rev, const float* ca, const float* cb, float* caT, float* cbT,
-                          hipStream_t s) {
-    if (sc.N) launch_k(k_adj_transpose_coeffs, nbk(sc.N), kBlock, 0, s, sc, nb, rev, ca, cb, caT, cbT);
-}
-void adj_cg_init(const Scenes& sc, const float4* pos, const float4* b, float4* x, float4* r, float4* rec, double* partials,
-                 hipStream_t s) {
-    if (sc.N) launch_k(k_adj_cg_init, nbk(sc.N), kBlock, 0, s, sc, pos, b, x, r, rec, partials);
-}
-void adj_cg_applyT(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* rec, float4* Ap,
-                   const SolverDev* st, double* partials, hipStream_t s) {
-    if (sc.N) launch_k(k_adj_cg_applyT, nbk(sc.N), kBlock, 0, s, sc, nb, ca, cb, caT, cbT, rec, Ap, st, partials);
+void adj_lambda(const Scenes& sc, const f3* x, float4* lam, hipStream_t s) {
+    if (sc.N) launch_k(k_adj_lambda, nbk(sc.N), kBlock, 0, s, sc, x, lam);
 }
 void adj_cg_grad(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vin, const float4* vstar,
                  const float* rho, const float* fst, const float4* lam, float4* avin, float4* ax, float* rbar, float* fbar,
@@ -875,10 +745,6 @@ void adj_density(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, 
 void adj_unpermute(uint32_t n, const uint32_t* src, const float4* ax, const float4* av, const float4* al, float4* ax_out,
                    float4* av_out, float4* al_out, hipStream_t s) {
     if (n) launch_k(k_adj_unpermute, nbk(n), kBlock, 0, s, n, src, ax, av, al, ax_out, av_out, al_out);
-}
-void adj_cg_init_warm(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* recA,
-                      const float4* b, float4* x, float4* r, float4* recB, double* partials, hipStream_t s) {
-    if (sc.N) launch_k(k_adj_cg_init_warm, nbk(sc.N), kBlock, 0, s, sc, nb, ca, cb, caT, cbT, recA, b, x, r, recB, partials, nbk(sc.N));
 }
 void adj_fold_start(const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, hipStream_t s) {
     if (sc.N) launch_k(k_adj_fold_start, sc.S, kBlock, 0, s, sc, partials, nbk(sc.N), st, active, tol);

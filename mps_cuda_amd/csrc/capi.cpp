@@ -190,13 +190,15 @@ struct mps_ctx {
         uint32_t Kff = 0, Kfb = 0;
         DBuf<float4> pos, bpos;
         DBuf<float> bvol;
-        DBuf<uint32_t> src, nff, cff, nfb, cfb, perm_end;
+        DBuf<uint32_t> src, nff, cff, nfb, cfb, perm_end, halo_idx, halo_n;
+        DBuf<uint16_t> nb16;
+        bool deep = false;  // which staged forms the step's halos ask for
         std::vector<DBuf<float4>> snaps;
         uint32_t nsnap = 0, df_last = 0, cg_out = 0;
         std::vector<uint32_t> ldf, lcd;
         void release() {
             pos.release(); bpos.release(); bvol.release(); src.release(); nff.release(); cff.release();
-            nfb.release(); cfb.release(); perm_end.release();
+            nfb.release(); cfb.release(); perm_end.release(); halo_idx.release(); halo_n.release(); nb16.release();
             for (auto& b : snaps) b.release();
         }
     };
@@ -226,7 +228,7 @@ struct mps_ctx {
         adj_n = 0;
         lam_valid = false;
     }
-    DBuf<uint32_t> perm0, d_L, rev;
+    DBuf<uint32_t> perm0, d_L;
     DBuf<float> gobs;  // one observation's cotangents (Nref x 3 position, then velocity)
     DBuf<float4> adx, adv, adx2, adv2, aux4, gvec, avin, lam, lam2;
     bool lam_valid = false;  // lam holds the later step's transposed solution (warm start)
@@ -234,7 +236,7 @@ struct mps_ctx {
     DBuf<float> caT, cbT;  // (a_ji, b_ji) per list entry
     DBuf<double> acc_mu, acc_sig;
     // fluid: pos = (x, y, z, r), vel = (vx, vy, vz, m)
-    DBuf<float4> pos, vel, color, cgb, cgx, cgr, cgAp, jprev, jt[3], jcand, tmp4;
+    DBuf<float4> pos, vel, color, cgb, cgx, jprev, jt[3], jcand, tmp4;
     // the forward CG's vectors as packed triples: x, r, A p and two p buffers
     DBuf<mps::dev::f3> v3x, v3r, v3Ap, v3p, v3q;
     DBuf<float> rho, alpha, kappa, delta, fst, tmp1;
@@ -283,7 +285,6 @@ struct mps_ctx {
     DBuf<uint32_t> halo_idx, halo_n;
     DBuf<uint16_t> nb16;
     DBuf<uint2> nstat;  // per-workgroup neighbour-count records of the searches
-    DBuf<float4> cgrecA, cgrecB;  // 32-byte (position, vector) records for the CG gathers
     bool pairs_valid = false;
     bool halo_valid = false;  // block halos match the fluid lists
     uint32_t nei_regrow = 0;
@@ -1113,7 +1114,7 @@ struct mps_ctx {
         T_(K_ST_FACTOR, [&] { mps::launch::st_factor(P, nbr(), hl, pos.p, vel.p, pairG_ff.p, fst.p, cgx.p, stream); });
         T_(K_CG_SETUP, [&] {
             mps::launch::cg_setup(cubic(), P, nbr(), hl, pos.p, vel.p, rho.p, fst.p, pairA.p,
-                                  op.recompute ? nullptr : pairB.p, cgb.p, op.recompute ? irho.p : nullptr, stream);
+                                  op.recompute ? nullptr : pairB.p, nullptr, nullptr, cgb.p, op.recompute ? irho.p : nullptr, stream);
         });
         mps::launch::solver_reset(sd, S, act, stream);
         const double tol = cfg.cg_tol;
@@ -1394,42 +1395,56 @@ struct mps_ctx {
         adj_B = B;
         adj_S = S;
     }
-    // Transposed solve A_f^T lambda = adv (lambda in cgx), same chunked loop as the forward CG,
-    // started from the later step's solution when there is one.
-    void adj_solveT(const mps::Nbr& nb, const float4* p0) {
+    // Transposed solve A_f^T lambda = adv (lambda in lam), same chunked loop as the forward CG,
+    // started from the later step's solution (in lam) when there is one.
+    void adj_solveT(const mps::Nbr& nb, const mps::Halo& hl, const float4* p0) {
         const mps::Scenes P = scn();
         SolverDev* sd = d_solver + 2 * size_t(S);
         uint32_t* act = d_active + 2;
         const double tol = cfg.adj_cg_tol != 0.0 ? cfg.adj_cg_tol : -1.0e-12;
+        const size_t m = std::max<uint32_t>(N, 1);
+        const uint32_t nblk = uint32_t((size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock);
+        v3x.reserve(m); v3r.reserve(m); v3Ap.reserve(m); v3p.reserve(m); v3q.reserve(m);
+        auto pbuf = [&](uint32_t k) { return (k & 1u) ? v3q.p : v3p.p; };
+        mps::launch::CgOperator op;
+        op.ca = pairA.p;
+        op.cb = pairB.p;
+        op.caT = caT.p;
+        op.cbT = cbT.p;
         mps::launch::solver_reset(sd, S, act, stream);
         if (lam_valid) {
-            cgrecA.reserve(2 * std::max<uint32_t>(N, 1));
-            mps::launch::cg_pack(N, p0, lam.p, cgrecA.p, stream);
-            mps::launch::adj_cg_init_warm(P, nb, pairA.p, pairB.p, caT.p, cbT.p, cgrecA.p, adv.p, cgx.p, cgr.p, cgrecB.p, partials.p,
-                                          stream);
+            mps::launch::cg_apply(0, op, P, nb, hl, p0, lam.p, nullptr, nullptr, pbuf(0), nullptr, adv.p, v3r.p, v3x.p, sd, partials.p,
+                                  nullptr, stream);
             mps::launch::adj_fold_start(P, partials.p, sd, act, tol, stream);
         } else {
-            mps::launch::adj_cg_init(P, p0, adv.p, cgx.p, cgr.p, cgrecB.p, partials.p, stream);
+            mps::launch::adj_cg_start(P, adv.p, v3x.p, v3r.p, pbuf(0), partials.p, stream);
             mps::launch::fold_cg(0, P, partials.p, sd, act, tol, stream);
         }
         const uint32_t cap = cfg.adj_cg_max_iter ? cfg.adj_cg_max_iter : 300u;
         uint32_t it = 1;
         bool done = fetch_active(2) == 0;
+        // sums folded as in viscosity_cg
+        const bool fuse = mps::launch::fold_in_consumer(most_blocks());
+        double* part_rr = fuse ? partials.p + nblk : partials.p;
+        const mps::launch::FoldCg fc{part_rr, act, tol};
         while (it <= cap && !done) {
             const uint32_t chunk = chunk_len(it, pred_adj, cap - it + 1);
             std::vector<uint64_t> key = key_base(4, chunk, P, nb);
-            for (const void* q : {(const void*)pairA.p, (const void*)pairB.p, (const void*)caT.p, (const void*)cbT.p, (const void*)cgrecB.p, (const void*)cgAp.p,
-                                  (const void*)cgx.p, (const void*)cgr.p, (const void*)sd, (const void*)partials.p,
-                                  (const void*)act})
+            for (const void* q : {(const void*)op.ca, (const void*)op.cb, (const void*)op.caT, (const void*)op.cbT, (const void*)p0,
+                                  (const void*)pbuf(it - 1), (const void*)pbuf(it), (const void*)v3Ap.p, (const void*)v3r.p,
+                                  (const void*)v3x.p, (const void*)sd, (const void*)partials.p, (const void*)act, (const void*)hl.idx,
+                                  (const void*)hl.n, (const void*)hl.nb16})
                 key.push_back(u(q));
             key.push_back(u(tol));
+            key.push_back(fuse);
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
-                    mps::launch::adj_cg_applyT(P, nb, pairA.p, pairB.p, caT.p, cbT.p, cgrecB.p, cgAp.p, sd, partials.p, stream);
-                    mps::launch::fold_cg(1, P, partials.p, sd, act, tol, stream);
-                    mps::launch::cg_update(P, cgx.p, cgr.p, cgrecB.p, cgAp.p, sd, partials.p, stream);
-                    mps::launch::fold_cg(2, P, partials.p, sd, act, tol, stream);
-                    mps::launch::cg_direction(P, cgr.p, cgrecB.p, sd, stream);
+                    const uint32_t k = it + c;
+                    mps::launch::cg_apply(1, op, P, nb, hl, p0, nullptr, v3r.p, pbuf(k - 1), pbuf(k), v3Ap.p, nullptr, nullptr, nullptr,
+                                          sd, partials.p, fuse && c ? &fc : nullptr, stream);
+                    if (!fuse) mps::launch::fold_cg(1, P, partials.p, sd, act, tol, stream);
+                    mps::launch::cg_update3(P, v3x.p, v3r.p, pbuf(k), v3Ap.p, sd, fuse ? partials.p : nullptr, part_rr, stream);
+                    if (!fuse || c + 1 == chunk) mps::launch::fold_cg(2, P, part_rr, sd, act, tol, stream);
                 }
             });
             it += chunk;
@@ -1438,12 +1453,16 @@ struct mps_ctx {
         uint32_t l = 0;
         (void)fetch_records(2, cap, &l);
         pred_adj = std::max<uint32_t>(l, 1);
+        lam.reserve(m);
+        mps::launch::adj_lambda(P, v3x.p, lam.p, stream);
+        lam_valid = true;
     }
     // Reverse of one recorded step: (adx, adv) from the step's end state to its start, in the
     // slot order of the previous step.
     void reverse_step(TapeStep& T) {
         const mps::Scenes P = scn();
         const mps::Nbr nb{T.nff.p, T.cff.p, T.nfb.p, T.cfb.p};
+        const mps::Halo hl{T.halo_idx.p, T.halo_n.p, T.nb16.p, T.deep};
         const size_t m = std::max<uint32_t>(N, 1);
         pairG_ff.reserve(size_t(T.Kff) * m);
         pairG_fb.reserve(size_t(T.Kfb) * m);
@@ -1451,7 +1470,7 @@ struct mps_ctx {
         halo_valid = false;
         const mps::launch::AdjKind ak{cubic(), adj_eq ? 1 : 0};
         mps::launch::density_alpha(cubic(), mps::launch::kDoDensity | mps::launch::kDoAlpha | mps::launch::kDoPairs, P, nb,
-                                   mps::Halo{}, T.pos.p, T.snaps[0].p, T.bpos.p, T.bvol.p, rho.p, alpha.p, color.p, pairG_ff.p,
+                                   hl, T.pos.p, T.snaps[0].p, T.bpos.p, T.bvol.p, rho.p, alpha.p, color.p, pairG_ff.p,
                                    pairG_fb.p, stream);
         abar.reserve(m); rbar.reserve(m); dbar.reserve(m); fbar.reserve(m); fstr.reserve(m);
         aux4.reserve(m); gvec.reserve(m); avin.reserve(m); adx2.reserve(m); adv2.reserve(m);
@@ -1479,19 +1498,12 @@ struct mps_ctx {
             const float4* vin = T.snaps[T.df_last].p;
             const float4* vst = T.snaps[T.cg_out].p;
             pairA.reserve(size_t(T.Kff) * m); pairB.reserve(size_t(T.Kff) * m);
-            caT.reserve(size_t(T.Kff) * m); cbT.reserve(size_t(T.Kff) * m); rev.reserve(size_t(T.Kff) * m);
-            cgrecB.reserve(2 * m);
-            mps::launch::st_factor(P, nb, mps::Halo{}, T.pos.p, vin, pairG_ff.p, fstr.p, cgx.p, stream);
-            mps::launch::cg_setup(cubic(), P, nb, mps::Halo{}, T.pos.p, vin, rho.p, fstr.p, pairA.p, pairB.p, cgb.p, nullptr,
+            caT.reserve(size_t(T.Kff) * m); cbT.reserve(size_t(T.Kff) * m);
+            mps::launch::st_factor(P, nb, hl, T.pos.p, vin, pairG_ff.p, fstr.p, cgx.p, stream);
+            mps::launch::cg_setup(cubic(), P, nb, hl, T.pos.p, vin, rho.p, fstr.p, pairA.p, pairB.p, caT.p, cbT.p, cgb.p, nullptr,
                                   stream);
-            mps::launch::zero_words(d_flags + 2, 1, stream);
-            mps::launch::adj_rev_index(P, nb, rev.p, d_flags + 2, stream);
-            mps::launch::adj_transpose_coeffs(P, nb, rev.p, pairA.p, pairB.p, caT.p, cbT.p, stream);
-            adj_solveT(nb, T.pos.p);
-            lam.reserve(m);
-            HIPCHK(hipMemcpyAsync(lam.p, cgx.p, sizeof(float4) * N, hipMemcpyDeviceToDevice, stream));
-            lam_valid = true;
-            mps::launch::adj_cg_grad(ak, P, nb, T.pos.p, vin, vst, rho.p, fstr.p, cgx.p, avin.p, adx.p, rbar.p, fbar.p, partials.p,
+            adj_solveT(nb, hl, T.pos.p);
+            mps::launch::adj_cg_grad(ak, P, nb, T.pos.p, vin, vst, rho.p, fstr.p, lam.p, avin.p, adx.p, rbar.p, fbar.p, partials.p,
                                      stream);
             mps::launch::adj_fold2(P, partials.p, acc_mu.p, acc_sig.p, stream);
             mps::launch::adj_fst(ak, P, nb, T.pos.p, vin, pairG_ff.p, fbar.p, avin.p, adx.p, stream);
@@ -1564,9 +1576,6 @@ struct mps_ctx {
                 reverse_step(T);
             }
         }
-        HIPCHK(hipMemcpyAsync(h_flags + 2, d_flags + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        sync();
-        if (h_flags[2]) throw ApiError{MPS_ERR_STATE, "asymmetric neighbour lists in the adjoint"};
         std::vector<float4> hv = down(adv.p, N);
         std::vector<uint32_t> hp0 = down(perm0.p, N);
         for (uint32_t q = 0; q < N; q++) {
@@ -1742,6 +1751,11 @@ struct mps_ctx {
             dcopy(rec->cff, cff.p, N);
             dcopy(rec->nfb, nfb.p, size_t(Kfb) * N);
             dcopy(rec->cfb, cfb.p, N);
+            const size_t nblk = (size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
+            dcopy(rec->nb16, nb16.p, size_t(Kff) * N);
+            dcopy(rec->halo_idx, halo_idx.p, nblk * mps::kHaloCap);
+            dcopy(rec->halo_n, halo_n.p, nblk);
+            rec->deep = use_deep();
             dcopy(rec->bpos, bpos.p, B);
             dcopy(rec->bvol, bvol.p, B);
         }
@@ -1839,8 +1853,8 @@ struct mps_ctx {
     // ------------------------------------------------------------------ setup
     void alloc_fluid(uint32_t n) {
         const size_t m = std::max<uint32_t>(n, 1);
-        pos.reserve(m); vel.reserve(m); color.reserve(m); cgb.reserve(m); cgx.reserve(m); cgr.reserve(m);
-        cgAp.reserve(m); rho.reserve(m); alpha.reserve(m); kappa.reserve(m); delta.reserve(m); fst.reserve(m);
+        pos.reserve(m); vel.reserve(m); color.reserve(m); cgb.reserve(m); cgx.reserve(m);
+        rho.reserve(m); alpha.reserve(m); kappa.reserve(m); delta.reserve(m); fst.reserve(m);
         cff.reserve(m); cfb.reserve(m); perm.reserve(m); inv.reserve(m); mkey.reserve(m);
     }
     void require_single(const char* what) const {
@@ -2481,9 +2495,9 @@ struct mps_ctx {
     }
 
     ~mps_ctx() {
-        pos.release(); vel.release(); color.release(); cgb.release(); cgx.release(); cgr.release();
+        pos.release(); vel.release(); color.release(); cgb.release(); cgx.release();
         v3x.release(); v3r.release(); v3Ap.release(); v3p.release(); v3q.release();
-        cgAp.release(); jprev.release(); for (auto& t : jt) t.release(); jcand.release(); tmp4.release();
+        jprev.release(); for (auto& t : jt) t.release(); jcand.release(); tmp4.release();
         rho.release(); alpha.release(); kappa.release(); delta.release(); fst.release(); tmp1.release();
         pos_alt.release(); vel_alt.release(); color_alt.release(); cgb_alt.release(); rho_alt.release();
         alpha_alt.release(); kappa_alt.release(); delta_alt.release(); fst_alt.release();
@@ -2494,7 +2508,7 @@ struct mps_ctx {
         bobj.release(); bS4.release();
         partials.release();
         arrive.release();
-        pairG_ff.release(); pairG_fb.release(); pairA.release(); pairB.release(); irho.release(); halo_idx.release(); halo_n.release(); nb16.release(); nstat.release(); cgrecA.release(); cgrecB.release();
+        pairG_ff.release(); pairG_fb.release(); pairA.release(); pairB.release(); irho.release(); halo_idx.release(); halo_n.release(); nb16.release(); nstat.release();
         if (copy_stream) (void)hipStreamSynchronize(copy_stream);
         for (ReadbackSlot& sl : rb) {
             sl.buf.release();
@@ -2508,7 +2522,7 @@ struct mps_ctx {
         for (auto& t : tape) t.release();
         for (auto& c : ckpts) c.release();
         ck_end.release();
-        perm0.release(); d_L.release(); rev.release(); gobs.release(); adx.release(); adv.release(); adx2.release(); adv2.release();
+        perm0.release(); d_L.release(); gobs.release(); adx.release(); adv.release(); adx2.release(); adv2.release();
         aux4.release(); gvec.release(); avin.release(); abar.release(); rbar.release(); dbar.release(); fbar.release();
         fstr.release(); caT.release(); cbT.release(); acc_mu.release(); acc_sig.release(); lam.release(); lam2.release();
         if (d_active) (void)hipFree(d_active);

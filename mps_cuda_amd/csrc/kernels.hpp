@@ -247,13 +247,11 @@ void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, 
 bool fold_in_consumer(uint32_t most_blocks);
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
                float4* cgx, hipStream_t s);
-// pair coefficients of the implicit operator: a_ij into ca, b_ij into cb (may be null)
+// pair coefficients of the implicit operator: a_ij into ca, b_ij into cb (may be null); with caT and
+// cbT also the pair seen from the neighbour (a_ji, b_ji), for the transposed operator
 void cg_setup(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* rho,
-              const float* fst, float* ca, float* cb, float4* cgb, float* irho, hipStream_t s);
-// The adjoint's transposed solve keeps p in 32-byte records with the position:
-// rec[2i] = (x, y, z, p.x), rec[2i+1] = (p.y, p.z, 0, 0)
-void cg_pack(uint32_t N, const float4* pos, const float4* x0, float4* rec, hipStream_t s);
-// The forward solve's vectors are packed triples (dev::f3).
+              const float* fst, float* ca, float* cb, float* caT, float* cbT, float4* cgb, float* irho, hipStream_t s);
+// The solves' vectors are packed triples (dev::f3).
 // mode 0: A x0 with f = 0 (x0 from the float4 array x0), then r = b - A x0, pout = r, x = x0, partial r.r;
 // mode 1: p = r + beta pprev (r in rr, beta from the record), A p with f into Ap, p into pout,
 // partial p.Ap. Halo records are staged in LDS (kHaloCap).
@@ -265,6 +263,8 @@ struct CgOperator {
     int deep = 0;  // the streamed operator stages halos up to kHaloCap (else kHaloShallow)
     const float* ca = nullptr;
     const float* cb = nullptr;
+    const float* caT = nullptr;  // set, with cbT: the transposed operator (mode 0 then starts its solve from a
+    const float* cbT = nullptr;  // guess: r = b - A_f^T x0, partial sums of r.r and, nblk further, of b.b)
     const float4* vel = nullptr;
     const float* rho = nullptr;
     const float* irho = nullptr;
@@ -307,17 +307,12 @@ void halo_build(int all, const Scenes& sc, const Nbr& nb, uint32_t nblk, uint32_
                 uint16_t* n16, uint32_t* stats, hipStream_t s);
 // mode 0: initial r.r + test; 1: alpha; 2: new r.r, beta + test
 void fold_cg(int mode, const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, hipStream_t s);
-// x += alpha p, r -= alpha Ap, partial r.r (p from the records; the adjoint's solve)
-void cg_update(const Scenes& sc, float4* x, float4* r, const float4* prec, const float4* Ap, const SolverDev* st,
-               double* partials, hipStream_t s);
-// the same on packed triples (the forward solve), and its copy of x into the velocities
+// x += alpha p, r -= alpha Ap, partial r.r (the copy of x into the velocities: copy_vel_out3).
 // pAp set: every workgroup folds its scene's p.Ap partials (pAp) itself, and the scene's first one
 // does fold_cg(1)'s part
 void cg_update3(const Scenes& sc, dev::f3* x, dev::f3* r, const dev::f3* p, const dev::f3* Ap, SolverDev* st,
                 const double* pAp, double* partials, hipStream_t s);
 void copy_vel_out3(const Scenes& sc, const dev::f3* x, float4* vel, hipStream_t s);
-// p = r + beta p in the records (the adjoint's solve; the forward forms p inside cg_apply)
-void cg_direction(const Scenes& sc, const float4* r, float4* prec, const SolverDev* st, hipStream_t s);
 void copy_vel_out(const Scenes& sc, const float4* x, float4* vel, hipStream_t s);
 void jacobi_candidate(int cubic, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vel,
                       const float* rho, const float4* u, float4* out, hipStream_t s);
@@ -356,13 +351,10 @@ void adj_kbar(AdjKind k, int df, const Scenes& sc, const Nbr& nb, const float4* 
 void adj_dbar(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vel, const float4* bpos,
               const float* bvol, const float4* bvel, const float* pG_ff, const float* pG_fb, const float* dbar, const uint32_t* L, uint32_t it,
               float4* av, float4* ax, hipStream_t s);
-void adj_rev_index(const Scenes& sc, const Nbr& nb, uint32_t* rev, uint32_t* bad, hipStream_t s);
-void adj_transpose_coeffs(const Scenes& sc, const Nbr& nb, const uint32_t* rev, const float* ca, const float* cb, float* caT, float* cbT,
-                          hipStream_t s);
-void adj_cg_init(const Scenes& sc, const float4* pos, const float4* b, float4* x, float4* r, float4* rec, double* partials,
-                 hipStream_t s);
-void adj_cg_applyT(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* rec, float4* Ap,
-                   const SolverDev* st, double* partials, hipStream_t s);
+// start of the transposed solve from lambda = 0: x = 0, r = p = b, partial r.r
+void adj_cg_start(const Scenes& sc, const float4* b, dev::f3* x, dev::f3* r, dev::f3* p, double* partials, hipStream_t s);
+// lam = x as float4
+void adj_lambda(const Scenes& sc, const dev::f3* x, float4* lam, hipStream_t s);
 // partials: 2 * ceil(N / kBlock) doubles (mubar, sigmabar per workgroup)
 void adj_cg_grad(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vin, const float4* vstar, const float* rho,
                  const float* fst, const float4* lam, float4* avin, float4* ax, float* rbar, float* fbar, double* partials,
@@ -377,9 +369,7 @@ void adj_density(AdjKind k, const Scenes& sc, const Nbr& nb, const float4* pos, 
 // also carries the transposed solve's solution (al, may be null) back, as the next warm start
 void adj_unpermute(uint32_t n, const uint32_t* src, const float4* ax, const float4* av, const float4* al, float4* ax_out,
                    float4* av_out, float4* al_out, hipStream_t s);
-// warm start of A_f^T lambda = b from x0 (packed in recA with the positions): partials of r.r and b.b
-void adj_cg_init_warm(const Scenes& sc, const Nbr& nb, const float* ca, const float* cb, const float* caT, const float* cbT, const float4* recA,
-                      const float4* b, float4* x, float4* r, float4* recB, double* partials, hipStream_t s);
+// r.r and b.b of a solve started from a guess; the threshold is relative to b.b
 void adj_fold_start(const Scenes& sc, const double* partials, SolverDev* st, uint32_t* active, double tol, hipStream_t s);
 // adx[s] += gx[perm[s]], adv[s] += gv[perm[s]] (gx, gv: n_ref x 3 floats in reference order; gv may be
 // null): the cotangent of an observed state, added in the slot order that state was stored in

@@ -187,10 +187,6 @@ __device__ __forceinline__ double fold_everywhere(const double* __restrict__ par
     }
 }
 
-// Halo count of workgroup blk: > kHaloCap (not staged) when there are no halos (hl.n null: the
-// adjoint's kernels run on its taped lists).
-__device__ __forceinline__ uint32_t halo_count(const Halo& hl, uint32_t blk) { return hl.n ? hl.n[blk] : kHaloCap + 1u; }
-
 // ---- walks of the fluid lists
 // The fluid lists, and everything stored per list entry, keep the four entries 4g .. 4g+3 of a
 // slot side by side (ell(), device_common.hpp). With one lane per slot (Q = 1) a lane loads a group
@@ -216,6 +212,16 @@ __device__ __forceinline__ float add_quad(float s, float t) {
 }
 __device__ __forceinline__ f3 add_quad(f3 s, f3 t) { return {add_quad(s.x, t.x), add_quad(s.y, t.y), add_quad(s.z, t.z)}; }
 
+// two terms per lane: t0 + u0 + t1 + u1 + ...
+__device__ __forceinline__ float add_quad(float s, float t, float u) {
+    s = (s + quad_lane<0>(t)) + quad_lane<0>(u);
+    s = (s + quad_lane<1>(t)) + quad_lane<1>(u);
+    s = (s + quad_lane<2>(t)) + quad_lane<2>(u);
+    return (s + quad_lane<3>(t)) + quad_lane<3>(u);
+}
+__device__ __forceinline__ f3 add_quad(f3 s, f3 t, f3 u) {
+    return {add_quad(s.x, t.x, u.x), add_quad(s.y, t.y, u.y), add_quad(s.z, t.z, u.z)};
+}
 __device__ __forceinline__ float sub_quad(float s, float t) {
     return (((s - quad_lane<0>(t)) - quad_lane<1>(t)) - quad_lane<2>(t)) - quad_lane<3>(t);
 }
@@ -282,17 +288,21 @@ struct GroupIdx<4, STAGED> {
     }
     __device__ __forceinline__ uint32_t at(int) const { return w; }
 };
-// A float stored per entry, streamed with non-temporal loads; GroupAB: two such arrays. (The
+// The arrays of values per list entry that a walk streams with non-temporal loads. (The
 // coefficients a_ij and b_ij are two arrays and not pairs, so that each of a lane's 16-byte loads
 // belongs to a contiguous kilobyte of the wave: with pairs, two loads touch every line, and the
 // line is fetched twice.)
+struct Streams {
+    const float *a = nullptr, *b = nullptr, *aT = nullptr, *bT = nullptr;
+};
 template <int Q>
 struct GroupVal {
     typename std::conditional<Q == 1, v4f, float>::type v;
-    __device__ __forceinline__ void load(const float* p, const float*, size_t group, uint32_t l) {
+    __device__ __forceinline__ void load(const float* p, size_t group, uint32_t l) {
         if constexpr (Q == 1) v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p) + group);
         else v = __builtin_nontemporal_load(p + 4 * group + l);
     }
+    __device__ __forceinline__ void load(const Streams& s, size_t group, uint32_t l) { load(s.a, group, l); }
     __device__ __forceinline__ float at(int e) const {
         if constexpr (Q == 1) return v[e];
         else return v;
@@ -301,13 +311,23 @@ struct GroupVal {
 template <int Q>
 struct GroupAB {
     GroupVal<Q> a, b;
-    __device__ __forceinline__ void load(const float* pa, const float* pb, size_t group, uint32_t l) {
-        a.load(pa, nullptr, group, l);
-        b.load(pb, nullptr, group, l);
+    __device__ __forceinline__ void load(const Streams& s, size_t group, uint32_t l) {
+        a.load(s.a, group, l);
+        b.load(s.b, group, l);
+    }
+};
+template <int Q>
+struct GroupABT {
+    GroupVal<Q> a, b, aT, bT;
+    __device__ __forceinline__ void load(const Streams& s, size_t group, uint32_t l) {
+        a.load(s.a, group, l);
+        b.load(s.b, group, l);
+        aT.load(s.aT, group, l);
+        bT.load(s.bT, group, l);
     }
 };
 struct NoVal {
-    __device__ __forceinline__ void load(const float*, const float*, size_t, uint32_t) {}
+    __device__ __forceinline__ void load(const Streams&, size_t, uint32_t) {}
 };
 
 // Groups requested before the halo staging, and halo records that a thread stages per pass. A.p
@@ -330,11 +350,10 @@ struct Walk {
     Val vp[PRE], vr;
     const Nbr& nb;
     const Halo& hl;
-    const float *val, *val2;  // the arrays that Val reads
+    const Streams val;  // the arrays that Val reads
     uint32_t i, l, N, gf, nr;
-    __device__ __forceinline__ Walk(const Nbr& nb, const Halo& hl, const float* val, const float* val2, uint32_t i, uint32_t l,
-                                    uint32_t N, uint32_t c)
-        : nb(nb), hl(hl), val(val), val2(val2), i(i), l(l), N(N), gf(c >> 2), nr(c & 3u) {
+    __device__ __forceinline__ Walk(const Nbr& nb, const Halo& hl, const Streams& val, uint32_t i, uint32_t l, uint32_t N, uint32_t c)
+        : nb(nb), hl(hl), val(val), i(i), l(l), N(N), gf(c >> 2), nr(c & 3u) {
 #pragma unroll
         for (uint32_t g = 0; g < PRE; g++)
             if (g < gf) get(g, ip[g], vp[g]);
@@ -343,7 +362,7 @@ struct Walk {
     __device__ __forceinline__ void get(uint32_t g, Idx& x, Val& v) const {
         const size_t group = size_t(g) * N + i;
         x.load(nb, hl, group, l);
-        v.load(val, val2, group, l);
+        v.load(val, group, l);
     }
     template <class Full, class Rest>
     __device__ __forceinline__ void run(Full&& full, Rest&& rest) {
@@ -377,12 +396,12 @@ struct BlockHead {
         i = blk * kBlock + threadIdx.x / Q;
         l = threadIdx.x % Q;
         c = i < N ? cff[i] : 0u;
-        H = halo_count(hl, blk);
+        H = hl.n[blk];
         hs = hl.idx + size_t(blk) * kHaloCap;
 #pragma unroll
         for (uint32_t q = 0; q < R; q++) {
             const uint32_t t = threadIdx.x + q * kThreads;
-            sh[q] = hl.n && t < kHaloCap ? hs[t] : 0u;
+            sh[q] = t < kHaloCap ? hs[t] : 0u;
         }
     }
     // store(t, load(s)) for every halo record t < H (s = its slot): R records per thread and
@@ -550,7 +569,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_density_alpha(int flags, Scenes 
     };
     auto walk_fluid = [&](auto staged) {
         constexpr bool STAGED = decltype(staged)::value;
-        Walk<Q, STAGED, NoVal, 1> wk(nb, hl, nullptr, nullptr, i, l, N, live ? c : 0u);
+        Walk<Q, STAGED, NoVal, 1> wk(nb, hl, Streams{}, i, l, N, live ? c : 0u);
         if constexpr (STAGED) {
             hd.stage([&](uint32_t j) { return pos[j]; }, [&](uint32_t t, const float4& x) { la[t] = x; });
             __syncthreads();
@@ -769,7 +788,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_eval(Scenes sc, Nbr nb,
     using Val = GroupVal<Q>;
     auto walk_fluid = [&](auto staged) {
         constexpr bool STAGED = decltype(staged)::value;
-        Walk<Q, STAGED, Val, Q == 1 ? kPreEval : kPreQuad> wk(nb, hl, pG_ff, nullptr, i, l, N, hd.c);
+        Walk<Q, STAGED, Val, Q == 1 ? kPreEval : kPreQuad> wk(nb, hl, Streams{pG_ff}, i, l, N, hd.c);
         struct Rec {
             f3 x, v;
         };
@@ -984,7 +1003,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_apply(Scenes sc, Nbr nb
     using Val = GroupVal<Q>;
     auto walk_fluid = [&](auto staged) {
         constexpr bool STAGED = decltype(staged)::value;
-        Walk<Q, STAGED, Val, Q == 1 ? kPrePressure : kPreQuad> wk(nb, hl, pG_ff, nullptr, i, l, N, hd.c);
+        Walk<Q, STAGED, Val, Q == 1 ? kPrePressure : kPreQuad> wk(nb, hl, Streams{pG_ff}, i, l, N, hd.c);
         auto rec = [&](uint32_t j) {
             const float4 x = pos[j];
             return make_float4(x.x, x.y, x.z, kappa[j]);
@@ -1104,7 +1123,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_st_factor(Scenes sc, Nbr nb, Hal
     using Val = GroupVal<Q>;
     auto walk_fluid = [&](auto staged) {
         constexpr bool STAGED = decltype(staged)::value;
-        Walk<Q, STAGED, Val, 1> wk(nb, hl, pG_ff, nullptr, i, l, N, hd.c);
+        Walk<Q, STAGED, Val, 1> wk(nb, hl, Streams{pG_ff}, i, l, N, hd.c);
         struct Rec {
             float4 x, v;
         };
@@ -1173,17 +1192,21 @@ __device__ __forceinline__ float st_g(const StepParams& P, f3 vij, f3 xij, float
 //   cs_i = dt sigma/m_i, cx = XSPH/dt, cv_i = 10 rho0 mu/rho_i.
 // Writes a_ij (ca), b_ij (cb, unless null), and 1/rho_i per slot (irho, unless null) for the A.p
 // that recomputes b_ij.
-template <bool CUBIC, int Q>
+// T: also the coefficients (a_ji, b_ji) of the pair seen from the neighbour, which the adjoint's
+// transposed operator streams: the same expressions with the ends exchanged. (The lists are
+// symmetric; what the neighbour's own entry holds has the same bits, since every factor that depends
+// on the pair is even in x_ij.)
+template <bool CUBIC, int Q, bool T>
 __global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const float* __restrict__ rho,
-                                                   const float* __restrict__ fst, float* __restrict__ ca, float* __restrict__ cb, float4* __restrict__ cgb,
-                                                   float* __restrict__ irho) {
+                                                   const float* __restrict__ fst, float* __restrict__ ca, float* __restrict__ cb, float* __restrict__ caT,
+                                                   float* __restrict__ cbT, float4* __restrict__ cgb, float* __restrict__ irho) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t N = sc.N;
     // the block's halo (x_j, v_j, m_j, rho_j, f_j) in LDS (see k_cg_apply)
     constexpr uint32_t kDepth = Q == 1 ? kStageSetup : kHaloCap;
     __shared__ float4 la[kDepth], lb[kDepth];
-    __shared__ float lc[kDepth];
+    __shared__ typename std::conditional<T, float2, float>::type lc[kDepth];  // f_j; T: (f_j, r_j)
     BlockHead<Q, kHaloLoads<Q>> hd(blk, N, nb.cff, hl);
     const uint32_t i = hd.i, l = hd.l;
     const bool in = i < N;
@@ -1207,7 +1230,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo
         float rho, f;
     };
     struct Term {
-        float a, b;
+        float a, b, aT, bT;
         f3 s;
     };
     auto term = [&](const Rec& r) -> Term {
@@ -1220,31 +1243,45 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo
         const float wij = mj / dj * Wk<CUBIC>(dist, invHi);
         Term t;
         t.a = P.dt * (cs * sij + cx * wij);
-        t.b = 0.0f;
-        if (cb) {
+        t.b = t.aT = t.bT = 0.0f;
+        if (T || cb) {
             const float irhoj = 1.0f / dj;
             const float cij = 0.5f * (mi + mj) * irhoj * Phik<CUBIC>(dist, invHi, onePercentHSq);
             t.b = -P.dt * cv * cij;
         }
         t.s = sij * xij;
+        if constexpr (T) {
+            const float hj = r.x.w * 4.0f, invHj = 1.0f / hj;
+            float mji;
+            const float gji = st_g(P, vi - mk(r.v), xij, dist, invHj, mj, mi, dj, di, r.f, fi, mji);
+            const float sji = mji * gji;
+            const float wji = mi / di * Wk<CUBIC>(dist, invHj);
+            t.aT = P.dt * (P.dt * P.sigma / mj * sji + cx * wji);
+            const float cvj = 10.0f * P.rho0 * P.mu / dj;
+            const float cji = 0.5f * (mj + mi) * (1.0f / di) * Phik<CUBIC>(dist, invHj, 0.01f * hj * hj);
+            t.bT = -P.dt * cvj * cji;
+        }
         return t;
     };
     auto walk_fluid = [&](auto staged) {
         constexpr bool STAGED = decltype(staged)::value;
-        Walk<Q, STAGED, NoVal, 1> wk(nb, hl, nullptr, nullptr, i, l, N, hd.c);
+        Walk<Q, STAGED, NoVal, 1> wk(nb, hl, Streams{}, i, l, N, hd.c);
         if constexpr (STAGED) {
             hd.stage([&](uint32_t j) { return Rec{pos[j], vel[j], rho[j], fst[j]}; },
                      [&](uint32_t t, const Rec& r) {
                          la[t] = make_float4(r.x.x, r.x.y, r.x.z, r.v.x);
                          lb[t] = make_float4(r.v.y, r.v.z, r.v.w, r.rho);
-                         lc[t] = r.f;
+                         if constexpr (T) lc[t] = make_float2(r.f, r.x.w);
+                         else lc[t] = r.f;
                      });
             __syncthreads();
         }
         auto at = [&](uint32_t j) -> Rec {
             if constexpr (STAGED) {
                 const float4 e = la[j], g = lb[j];
-                return {e, make_float4(e.w, g.x, g.y, g.z), g.w, lc[j]};
+                const auto f = lc[j];
+                if constexpr (T) return {make_float4(e.x, e.y, e.z, f.y), make_float4(e.w, g.x, g.y, g.z), g.w, f.x};
+                else return {e, make_float4(e.w, g.x, g.y, g.z), g.w, f};
             } else {
                 return {pos[j], vel[j], rho[j], fst[j]};
             }
@@ -1252,7 +1289,11 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo
         // one entry's coefficients at its place in the list
         auto put = [&](size_t entry, const Term& t) {
             ca[entry] = t.a;
-            if (cb) cb[entry] = t.b;
+            if (T || cb) cb[entry] = t.b;
+            if constexpr (T) {
+                caT[entry] = t.aT;
+                cbT[entry] = t.bT;
+            }
         };
         wk.run(
             [&](uint32_t g, const auto& x, const NoVal&) {
@@ -1265,7 +1306,11 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo
                         bi = bi - t[e].s;
                     }
                     reinterpret_cast<v4f*>(ca)[group] = v4f{t[0].a, t[1].a, t[2].a, t[3].a};
-                    if (cb) reinterpret_cast<v4f*>(cb)[group] = v4f{t[0].b, t[1].b, t[2].b, t[3].b};
+                    if (T || cb) reinterpret_cast<v4f*>(cb)[group] = v4f{t[0].b, t[1].b, t[2].b, t[3].b};
+                    if constexpr (T) {
+                        reinterpret_cast<v4f*>(caT)[group] = v4f{t[0].aT, t[1].aT, t[2].aT, t[3].aT};
+                        reinterpret_cast<v4f*>(cbT)[group] = v4f{t[0].bT, t[1].bT, t[2].bT, t[3].bT};
+                    }
                 } else {
                     const Term t = term(at(x.at(0)));
                     put(4 * group + l, t);
@@ -1282,7 +1327,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo
                         bi = bi - t.s;
                     }
                 } else {
-                    Term t{0.f, 0.f, {0.f, 0.f, 0.f}};
+                    Term t{0.f, 0.f, 0.f, 0.f, {0.f, 0.f, 0.f}};
                     if (l < n) {
                         t = term(at(x.at(0)));
                         put(4 * group + l, t);
@@ -1297,20 +1342,6 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_setup(Scenes sc, Nbr nb, Halo
     if (irho) irho[i] = 1.0f / di;
     const f3 b = (P.dt * P.sigma / mi) * bi + vi;
     cgb[i] = make_float4(b.x, b.y, b.z, 0.0f);
-}
-
-// CG vectors that neighbours read are kept in 32-byte records with the position, so one
-// gather per pair brings both x_j and p_j (one 32-byte sector): rec[2j] = (x, y, z, p.x),
-// rec[2j+1] = (p.y, p.z, 0, 0).
-__device__ __forceinline__ f3 rec_p(float4 a, float4 b) { return {a.w, b.x, b.y}; }
-__device__ __forceinline__ f3 rec_p(float4 a, float2 b) { return {a.w, b.x, b.y}; }
-__global__ void __launch_bounds__(kBlock) k_cg_pack(uint32_t N, const float4* __restrict__ pos, const float4* __restrict__ x0,
-                                                  float4* __restrict__ rec) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const float4 x = pos[i], v = x0[i];
-    rec[2 * size_t(i)] = make_float4(x.x, x.y, x.z, v.x);
-    rec[2 * size_t(i) + 1] = make_float4(v.y, v.z, 0.0f, 0.0f);
 }
 
 // (A p)_i = (1+f) p_i + sum_j [ a_ij p_ij + (b_ij (p_ij . x_ij)) x_ij ].
@@ -1335,15 +1366,21 @@ __global__ void __launch_bounds__(kBlock) k_cg_pack(uint32_t N, const float4* __
 // One workgroup's share of A.p: block `blk`. head() gives its scene, whether that scene's loop has
 // finished, and the search-direction factor; it is called once the loads that need none of these
 // are on their way.
+// TRANS: the adjoint's A_f^T p, (1+f) p_i + sum_j [ (a_ij p_i - a_ji p_j) + (b_ij (p_i.x_ij) -
+// b_ji (p_j.x_ij)) x_ij ], with the neighbour's coefficients streamed beside the own ones; its MODE 0
+// starts a solve from a guess x0 (r = b - A_f^T x0, f included; partial sums of r.r and, gridDim.x
+// further, of b.b). At 64k particles (256 workgroups, 28 neighbours each) an iteration of the
+// transposed solve took five launches and 44 us with one entry per load and its records gathered from
+// L2 (24 us of it A^T.p); staged, in groups, with the direction and the folds inside: two and 17 us.
 // PCOH: the partial sum is stored device-coherently (a workgroup of the same launch folds it).
 struct CgHead {
     uint32_t sid;
     bool done;
     float beta;
 };
-template <int MODE, bool RECOMP, bool CUBIC, bool COH = false, bool PCOH = COH, uint32_t DEPTH = kStageAp, int Q = 1, class Head>
+template <int MODE, bool RECOMP, bool CUBIC, bool COH = false, bool PCOH = COH, uint32_t DEPTH = kStageAp, int Q = 1, bool TRANS = false, class Head>
 __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const Scenes& sc, const Nbr& nb,
-                                               const Halo& hl, const float* __restrict__ cb, const float* __restrict__ ca,
+                                               const Halo& hl, const Streams& coef,
                                                const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                const float* __restrict__ rho, const float* __restrict__ irho,
                                                const float4* __restrict__ x0, const f3* __restrict__ rr,
@@ -1387,12 +1424,12 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const 
             return a * pij + (bb * dot3(pij, xij)) * xij;
         }
     };
-    using Val = typename std::conditional<RECOMP, GroupVal<Q>, GroupAB<Q>>::type;
+    using Val = typename std::conditional<TRANS, GroupABT<Q>, typename std::conditional<RECOMP, GroupVal<Q>, GroupAB<Q>>::type>::type;
     auto walk_fluid = [&](auto staged) {
         constexpr bool STAGED = decltype(staged)::value;
         // the first groups are loaded before the halo staging: their stream overlaps the
         // staging's gathers instead of following them
-        Walk<Q, STAGED, Val, Q == 1 ? kPreApply : kPreQuad> wk(nb, hl, ca, cb, i, l, N, hd.c);
+        Walk<Q, STAGED, Val, Q == 1 ? kPreApply : kPreQuad> wk(nb, hl, coef, i, l, N, hd.c);
         auto rec = [&](uint32_t j) -> Rec {
             const float4 xj = pos[j];
             if constexpr (RECOMP) return {mk(xj), vec(j), vel[j].w, irho[j]};
@@ -1429,9 +1466,29 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const 
                 return rec(j);
             }
         };
-        auto entry = [&](const Val& v, int e, const Rec& q) -> f3 {
-            if constexpr (RECOMP) return term(v.at(e), 0.0f, q);
-            else return term(v.a.at(e), v.b.at(e), q);
+        // the terms of one entry, added to the sum one after the other (one term, or two if TRANS)
+        struct Terms {
+            f3 a, b;
+        };
+        auto entry = [&](const Val& v, int e, const Rec& q) -> Terms {
+            if constexpr (TRANS) {
+                const f3 xij = xi - q.x;
+                return {v.a.at(e) * pi - v.aT.at(e) * q.p, (v.b.at(e) * dot3(pi, xij) - v.bT.at(e) * dot3(q.p, xij)) * xij};
+            } else if constexpr (RECOMP) {
+                return {term(v.at(e), 0.0f, q), {}};
+            } else {
+                return {term(v.a.at(e), v.b.at(e), q), {}};
+            }
+        };
+        auto add = [&](const Terms& t) {
+            if constexpr (Q == 1) {
+                acc = acc + t.a;
+                if constexpr (TRANS) acc = acc + t.b;
+            } else if constexpr (TRANS) {
+                acc = add_quad(acc, t.a, t.b);
+            } else {
+                acc = add_quad(acc, t.a);
+            }
         };
         wk.run(
             [&](uint32_t, const auto& jx, const Val& v) {
@@ -1440,28 +1497,28 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const 
 #pragma unroll
                     for (int e = 0; e < 4; e++) q[e] = at(jx.at(e));
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc = acc + entry(v, e, q[e]);
+                    for (int e = 0; e < 4; e++) add(entry(v, e, q[e]));
                 } else {
-                    acc = add_quad(acc, entry(v, 0, at(jx.at(0))));
+                    add(entry(v, 0, at(jx.at(0))));
                 }
             },
             [&](uint32_t, const auto& jx, const Val& v, uint32_t n) {
                 if constexpr (Q == 1) {
 #pragma unroll
                     for (int e = 0; e < 3; e++)
-                        if (e < int(n)) acc = acc + entry(v, e, at(jx.at(e)));
+                        if (e < int(n)) add(entry(v, e, at(jx.at(e))));
                 } else {
-                    f3 t{0.f, 0.f, 0.f};
+                    Terms t{};
                     if (l < n) t = entry(v, 0, at(jx.at(0)));
-                    acc = add_quad(acc, t);
+                    add(t);
                 }
             });
     };
     if (hd.H <= DEPTH) walk_fluid(std::true_type{});  // the same for the whole block
     else walk_fluid(std::false_type{});               // halo over the limit: gather from global memory
-    double part = 0.0;
+    double part = 0.0, part_b = 0.0;
     if (live && l == 0) {
-        const float f = MODE == 0 ? 0.0f : P.cg_factor;
+        const float f = MODE == 0 && !TRANS ? 0.0f : P.cg_factor;
         const f3 o = pi * (1.0f + f) + acc;
         if (MODE == 0) {
             const float4 bi = b[i];
@@ -1470,6 +1527,7 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const 
             pout[i] = ri;
             x[i] = pi;
             part = double(ri.x * ri.x) + double(ri.y * ri.y) + double(ri.z * ri.z);
+            if constexpr (TRANS) part_b = double(bi.x * bi.x) + double(bi.y * bi.y) + double(bi.z * bi.z);
         } else {
             st3c<COH>(pout + i, pi);
             Ap[i] = o;
@@ -1477,6 +1535,10 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const 
         }
     }
     slot_partial<Q, PCOH>(part, partials, blk);
+    if constexpr (TRANS && MODE == 0) {
+        __syncthreads();
+        slot_partial<Q>(part_b, partials + gridDim.x, blk);
+    }
 }
 
 // What k_fold_cg<2> records of iteration `it`: `s` is the new r.r, `prev` the one before.
@@ -1498,9 +1560,8 @@ __device__ __forceinline__ bool cg_done(double s, double thr, double tol) { retu
 // workgroup records them. The others read `done`, `thr` and `rr_prev` of the record, which that
 // workgroup does not write (`rr_prev` is kept by the update), or, for `done`, only sets to what
 // they find themselves.
-template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1, bool FOLD = false>
-__global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl, const float* __restrict__ cb,
-                                                   const float* __restrict__ ca, const float4* __restrict__ pos,
+template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1, bool FOLD = false, bool TRANS = false>
+__global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl, Streams coef, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const float* __restrict__ rho,
                                                    const float* __restrict__ irho, const float4* __restrict__ x0,
                                                    const f3* __restrict__ rr, const f3* __restrict__ pprev,
@@ -1522,8 +1583,8 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo
         }
         return {sid, st[sid].done != 0u, st[sid].beta};
     };
-    cg_apply_block<MODE, RECOMP, CUBIC, false, false, DEEP ? kHaloCap : kStageAp, Q>(
-        blk, head, sc, nb, hl, cb, ca, pos, vel, rho, irho, x0, rr, pprev, pout, Ap, b, r, x, partials);
+    cg_apply_block<MODE, RECOMP, CUBIC, false, false, DEEP ? kHaloCap : kStageAp, Q, TRANS>(
+        blk, head, sc, nb, hl, coef, pos, vel, rho, irho, x0, rr, pprev, pout, Ap, b, r, x, partials);
 }
 
 // Scalars of CGSolver (MPSSolver.cuh:31-65). MODE 0: r.r of the initial residual and the
@@ -1556,35 +1617,8 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_cg(Scenes sc, const doubl
     }
 }
 
-// UpdateCGResidual_kernel + the r.r half of ComputeCGBetaParam_kernel (MPSCGKernel.cuh:69-121).
-// p in the 32-byte records (the adjoint's transposed solve).
-__global__ void __launch_bounds__(kBlock) k_cg_update(Scenes sc, float4* __restrict__ x, float4* __restrict__ r,
-                                                    const float4* __restrict__ prec, const float4* __restrict__ Ap,
-                                                    const SolverDev* st, double* __restrict__ partials) {
-    const uint32_t sid = sc.blk_scene[blockIdx.x];
-    if (st[sid].done) return;
-    const uint32_t end = sc.P[sid].end;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const float a = st[sid].alpha;
-    double part = 0.0;
-    if (i < end) {
-        const f3 pi = rec_p(prec[2 * size_t(i)], prec[2 * size_t(i) + 1]);
-        const float4 api = Ap[i];
-        float4 xi = x[i], ri = r[i];
-        xi.x = xi.x + a * pi.x;
-        xi.y = xi.y + a * pi.y;
-        xi.z = xi.z + a * pi.z;
-        ri.x = ri.x - a * api.x;
-        ri.y = ri.y - a * api.y;
-        ri.z = ri.z - a * api.z;
-        x[i] = xi;
-        r[i] = ri;
-        part = double(ri.x * ri.x) + double(ri.y * ri.y) + double(ri.z * ri.z);
-    }
-    block_partial(part, partials);
-}
-
-// The update on packed triples (the forward solve): same expressions as k_cg_update.
+// UpdateCGResidual_kernel + the r.r half of ComputeCGBetaParam_kernel (MPSCGKernel.cuh:69-121), on
+// packed triples.
 template <bool COH = false, bool PCOH = COH>
 __device__ __forceinline__ void cg_update3_block(uint32_t blk, uint32_t end, float a, f3* __restrict__ x,
                                                  f3* __restrict__ r, const f3* __restrict__ p, const f3* __restrict__ Ap,
@@ -1700,8 +1734,7 @@ __device__ __forceinline__ bool grid_barrier(GridSync* gs, uint32_t nwg, uint32_
 // after iteration cap. Partial sums alternate between two buffers, so a fold never reads a
 // buffer that the next phase writes. Results are those of the chunked launches bit for bit.
 template <bool RECOMP, bool CUBIC, bool COH>
-__global__ void __launch_bounds__(kBlock) k_cg_persistent(Scenes sc, Nbr nb, Halo hl, const float* __restrict__ cb,
-                                                        const float* __restrict__ ca, const float4* __restrict__ pos,
+__global__ void __launch_bounds__(kBlock) k_cg_persistent(Scenes sc, Nbr nb, Halo hl, Streams coef, const float4* __restrict__ pos,
                                                         const float4* __restrict__ vel, const float* __restrict__ rho,
                                                         const float* __restrict__ irho, f3* __restrict__ r,
                                                         f3* __restrict__ pbuf0, f3* __restrict__ pbuf1, f3* __restrict__ Ap,
@@ -1723,7 +1756,7 @@ __global__ void __launch_bounds__(kBlock) k_cg_persistent(Scenes sc, Nbr nb, Hal
         f3* pprev = (k & 1u) ? pbuf0 : pbuf1;  // p of iteration k - 1 (p_0 = r in pbuf0)
         f3* pout = (k & 1u) ? pbuf1 : pbuf0;
         if (!done)
-            cg_apply_block<1, RECOMP, CUBIC, COH>(blk, [&]() -> CgHead { return {sid, false, beta}; }, sc, nb, hl, cb, ca, pos, vel, rho, irho, nullptr, r, pprev,
+            cg_apply_block<1, RECOMP, CUBIC, COH>(blk, [&]() -> CgHead { return {sid, false, beta}; }, sc, nb, hl, coef, pos, vel, rho, irho, nullptr, r, pprev,
                                                   pout, Ap, nullptr, nullptr, nullptr, partA);
         if (!grid_barrier<COH>(gs, nwg, spin)) return;
         if (threadIdx.x == 0) running_s = __hip_atomic_load(active, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1804,8 +1837,7 @@ __device__ __forceinline__ void fold_in_last_workgroup(const Scenes& sc, uint32_
 }
 // k_cg_apply<1> + k_fold_cg<1> in one launch
 template <bool RECOMP, bool CUBIC>
-__global__ void __launch_bounds__(kBlock) k_cg_apply_fold(Scenes sc, Nbr nb, Halo hl, const float* __restrict__ cb,
-                                                        const float* __restrict__ ca, const float4* __restrict__ pos,
+__global__ void __launch_bounds__(kBlock) k_cg_apply_fold(Scenes sc, Nbr nb, Halo hl, Streams coef, const float4* __restrict__ pos,
                                                         const float4* __restrict__ vel, const float* __restrict__ rho,
                                                         const float* __restrict__ irho, const f3* __restrict__ rr,
                                                         const f3* __restrict__ pprev, f3* __restrict__ pout,
@@ -1814,7 +1846,7 @@ __global__ void __launch_bounds__(kBlock) k_cg_apply_fold(Scenes sc, Nbr nb, Hal
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t sid = sc.blk_scene[blk];
     if (st[sid].done) return;
-    cg_apply_block<1, RECOMP, CUBIC, false, true>(blk, [&]() -> CgHead { return {sid, false, st[sid].beta}; }, sc, nb, hl, cb, ca, pos, vel, rho, irho, nullptr, rr,
+    cg_apply_block<1, RECOMP, CUBIC, false, true>(blk, [&]() -> CgHead { return {sid, false, st[sid].beta}; }, sc, nb, hl, coef, pos, vel, rho, irho, nullptr, rr,
                                                   pprev, pout, Ap, nullptr, nullptr, nullptr, partials);
     fold_in_last_workgroup<1>(sc, sid, blk, partials, st, nullptr, 0.0, arrive);
 }
@@ -1827,23 +1859,6 @@ __global__ void __launch_bounds__(kBlock) k_cg_update3_fold(Scenes sc, f3* __res
     if (st[sid].done) return;
     cg_update3_block<false, true>(blockIdx.x, sc.P[sid].end, st[sid].alpha, x, r, p, Ap, partials);
     fold_in_last_workgroup<2>(sc, sid, blockIdx.x, partials, st, active, tol, arrive);
-}
-
-// UpdateCGDirection_kernel (MPSCGKernel.cuh:123-133), p kept in the position records
-__global__ void __launch_bounds__(kBlock) k_cg_direction(Scenes sc, const float4* __restrict__ r, float4* __restrict__ prec,
-                                                       const SolverDev* st) {
-    const uint32_t sid = sc.blk_scene[blockIdx.x];
-    if (st[sid].done) return;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= sc.P[sid].end) return;
-    const float bta = st[sid].beta;
-    const float4 ri = r[i];
-    float4 a = prec[2 * size_t(i)], b = prec[2 * size_t(i) + 1];
-    a.w = ri.x + bta * a.w;
-    b.x = ri.y + bta * b.x;
-    b.y = ri.z + bta * b.y;
-    prec[2 * size_t(i)] = a;
-    prec[2 * size_t(i) + 1] = b;
 }
 
 __global__ void __launch_bounds__(kBlock) k_copy_vel_out3(Scenes sc, const f3* __restrict__ x, float4* __restrict__ vel) {
@@ -2149,7 +2164,7 @@ void density_alpha(int cubic, int flags, const Scenes& sc, const Nbr& nb, const 
                                  k_density_alpha<true, false, false, 1>,  k_density_alpha<true, false, true, 1>,
                                  k_density_alpha<true, true, false, 1>,   k_density_alpha<true, true, true, 1>};
     const K k = tab[(cubic ? 4 : 0) | (nb.fr ? 2 : 0) | (nb.fbo ? 1 : 0)];
-    if (!nb.fr && !nb.fbo && hl.n && quad(sc, kQuadTwoPerCu)) {
+    if (!nb.fr && !nb.fbo && quad(sc, kQuadTwoPerCu)) {
         launch_k(cubic ? k_density_alpha<true, false, false, 4> : k_density_alpha<false, false, false, 4>, nb_(sc.N), 4 * kBlock, 0, s,
                  flags, sc, nb, hl, pos, vel, bpos, bvol, rho, alpha, color, pG_ff, pG_fb);
         return;
@@ -2217,18 +2232,19 @@ void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, 
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
                float4* cgx, hipStream_t s) {
     if (!sc.N) return;
-    if (hl.n && quad(sc, kQuadOnePerCu)) launch_k(k_st_factor<4>, nb_(sc.N), 4 * kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
+    if (quad(sc, kQuadOnePerCu)) launch_k(k_st_factor<4>, nb_(sc.N), 4 * kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
     else launch_k(k_st_factor<1>, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
 }
 void cg_setup(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* rho,
-              const float* fst, float* ca, float* cb, float4* cgb, float* irho, hipStream_t s) {
+              const float* fst, float* ca, float* cb, float* caT, float* cbT, float4* cgb, float* irho, hipStream_t s) {
     if (!sc.N) return;
-    const bool q = hl.n && (hl.deep || quad(sc, kQuadTwoPerCu));
-    if (cubic) launch_k(q ? k_cg_setup<true, 4> : k_cg_setup<true, 1>, nb_(sc.N), q ? 4 * kBlock : kBlock, 0, s, sc, nb, hl, pos, vel, rho, fst, ca, cb, cgb, irho);
-    else launch_k(q ? k_cg_setup<false, 4> : k_cg_setup<false, 1>, nb_(sc.N), q ? 4 * kBlock : kBlock, 0, s, sc, nb, hl, pos, vel, rho, fst, ca, cb, cgb, irho);
-}
-void cg_pack(uint32_t N, const float4* pos, const float4* x0, float4* rec, hipStream_t s) {
-    if (N) launch_k(k_cg_pack, nb_(N), kBlock, 0, s, N, pos, x0, rec);
+    const bool q = hl.deep || quad(sc, kQuadTwoPerCu);
+    using K = decltype(&k_cg_setup<true, 1, false>);
+    static constexpr K tab[8] = {k_cg_setup<false, 1, false>, k_cg_setup<false, 1, true>, k_cg_setup<false, 4, false>,
+                                 k_cg_setup<false, 4, true>,  k_cg_setup<true, 1, false>, k_cg_setup<true, 1, true>,
+                                 k_cg_setup<true, 4, false>,  k_cg_setup<true, 4, true>};
+    launch_k(tab[(cubic ? 4 : 0) | (q ? 2 : 0) | (caT ? 1 : 0)], nb_(sc.N), q ? 4 * kBlock : kBlock, 0, s, sc, nb, hl, pos, vel, rho,
+             fst, ca, cb, caT, cbT, cgb, irho);
 }
 void cg_apply(int mode, const CgOperator& op, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos,
               const float4* x0, const f3* rr, const f3* pprev, f3* pout, f3* Ap, const float4* b, f3* r, f3* x,
@@ -2237,10 +2253,21 @@ void cg_apply(int mode, const CgOperator& op, const Scenes& sc, const Nbr& nb, c
     const unsigned g = nb_(sc.N);
     const bool q = !op.recompute && quad(sc, kQuadOnePerCu);
     const unsigned threads = q ? 4 * kBlock : kBlock;
+    const Streams coef{op.ca, op.cb, op.caT, op.cbT};
 #define MPS_CG_APPLY(M, R, C, ...)                                                                                   \
-    launch_k(k_cg_apply<M, R, C, ##__VA_ARGS__>, g, threads, 0, s, sc, nb, hl, op.cb, op.ca, pos, op.vel, op.rho, op.irho, \
+    launch_k(k_cg_apply<M, R, C, ##__VA_ARGS__>, g, threads, 0, s, sc, nb, hl, coef, pos, op.vel, op.rho, op.irho, \
              x0, rr, pprev, pout, Ap, b, r, x, st, partials, fold ? *fold : FoldCg{})
-    if (q) {
+    if (op.caT) {  // transposed (deep staging: its registers allow four workgroups per CU anyway)
+        if (q) {
+            if (mode == 0) MPS_CG_APPLY(0, false, true, true, 4, false, true);
+            else if (fold) MPS_CG_APPLY(1, false, true, true, 4, true, true);
+            else MPS_CG_APPLY(1, false, true, true, 4, false, true);
+        } else {
+            if (mode == 0) MPS_CG_APPLY(0, false, true, true, 1, false, true);
+            else if (fold) MPS_CG_APPLY(1, false, true, true, 1, true, true);
+            else MPS_CG_APPLY(1, false, true, true, 1, false, true);
+        }
+    } else if (q) {
         if (mode == 0) MPS_CG_APPLY(0, false, true, true, 4);
         else if (fold) MPS_CG_APPLY(1, false, true, true, 4, true);
         else MPS_CG_APPLY(1, false, true, true, 4);
@@ -2265,8 +2292,9 @@ void cg_apply_fold(const CgOperator& op, const Scenes& sc, const Nbr& nb, const 
                    const f3* pprev, f3* pout, f3* Ap, SolverDev* st, double* partials, uint32_t* arrive, hipStream_t s) {
     if (!sc.N) return;
     const unsigned g = nb_(sc.N);
+    const Streams coef{op.ca, op.cb};
 #define MPS_CG_APPLY_FOLD(R, C)                                                                                    \
-    launch_k(k_cg_apply_fold<R, C>, g, kBlock, 0, s, sc, nb, hl, op.cb, op.ca, pos, op.vel, op.rho, op.irho, rr, pprev, \
+    launch_k(k_cg_apply_fold<R, C>, g, kBlock, 0, s, sc, nb, hl, coef, pos, op.vel, op.rho, op.irho, rr, pprev, \
              pout, Ap, st, partials, arrive)
     if (!op.recompute) MPS_CG_APPLY_FOLD(false, true);
     else if (op.cubic) MPS_CG_APPLY_FOLD(true, true);
@@ -2299,8 +2327,9 @@ void cg_persistent(const CgOperator& op, int coherent, const Scenes& sc, const N
                    double* partB, GridSync* gs, uint32_t cap, double tol, uint32_t spin, hipStream_t s) {
     if (!sc.N) return;
     const uint32_t nblk = nb_(sc.N);
-    void* args[] = {const_cast<Scenes*>(&sc), const_cast<Nbr*>(&nb), const_cast<Halo*>(&hl), const_cast<float**>(&op.cb),
-                    const_cast<float**>(&op.ca), const_cast<float4**>(&pos), const_cast<float4**>(&op.vel),
+    Streams coef{op.ca, op.cb};
+    void* args[] = {const_cast<Scenes*>(&sc), const_cast<Nbr*>(&nb), const_cast<Halo*>(&hl), &coef,
+                    const_cast<float4**>(&pos), const_cast<float4**>(&op.vel),
                     const_cast<float**>(&op.rho), const_cast<float**>(&op.irho), &r, &pbuf0, &pbuf1, &Ap, &x, &st, &active,
                     &partA, &partB, &gs, &cap, &tol, &spin};
     const hipError_t rc = hipLaunchCooperativeKernel(persistent_fn(op, coherent), dim3(nblk), dim3(kBlock), args, 0, s);
@@ -2311,10 +2340,6 @@ void fold_cg(int mode, const Scenes& sc, const double* partials, SolverDev* st, 
     if (mode == 0) launch_k(k_fold_cg<0>, sc.S, kFoldThreads, 0, s, sc, partials, st, active, tol);
     else if (mode == 1) launch_k(k_fold_cg<1>, sc.S, kFoldThreads, 0, s, sc, partials, st, active, tol);
     else launch_k(k_fold_cg<2>, sc.S, kFoldThreads, 0, s, sc, partials, st, active, tol);
-}
-void cg_update(const Scenes& sc, float4* x, float4* r, const float4* prec, const float4* Ap, const SolverDev* st,
-               double* partials, hipStream_t s) {
-    if (sc.N) launch_k(k_cg_update, nb_(sc.N), kBlock, 0, s, sc, x, r, prec, Ap, st, partials);
 }
 void cg_update3(const Scenes& sc, f3* x, f3* r, const f3* p, const f3* Ap, SolverDev* st, const double* pAp, double* partials,
                 hipStream_t s) {
@@ -2327,9 +2352,6 @@ void cg_update3(const Scenes& sc, f3* x, f3* r, const f3* p, const f3* Ap, Solve
 bool fold_in_consumer(uint32_t most_blocks) { return most_blocks <= 1536; }
 void copy_vel_out3(const Scenes& sc, const f3* x, float4* vel, hipStream_t s) {
     if (sc.N) launch_k(k_copy_vel_out3, nb_(sc.N), kBlock, 0, s, sc, x, vel);
-}
-void cg_direction(const Scenes& sc, const float4* r, float4* prec, const SolverDev* st, hipStream_t s) {
-    if (sc.N) launch_k(k_cg_direction, nb_(sc.N), kBlock, 0, s, sc, r, prec, st);
 }
 void copy_vel_out(const Scenes& sc, const float4* x, float4* vel, hipStream_t s) {
     if (sc.N) launch_k(k_copy_vel_out, nb_(sc.N), kBlock, 0, s, sc, x, vel);
