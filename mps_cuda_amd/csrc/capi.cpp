@@ -734,16 +734,23 @@ struct mps_ctx {
                 mps::launch::fill_u32(h.end.p, C, mps::dev::kEmpty, stream);
             });
             h.cells_init = true;
-        } else {
-            T_(K_CELLS, [&] { mps::launch::clear_cells_m(mkey.p, lkey.p, h.n_valid, h.start.p, h.end.p, stream); });
         }
+        const uint32_t n_old = h.n_valid;
+        const int mb = morton_bits();
+        // every buffer first, so nothing is cleared or moved unless the whole hash can run
+        if (const size_t m = N) {
+            keyref.reserve(m); vals.reserve(m); src.reserve(m); lkey.reserve(m); hash_perm.reserve(m);
+            h.key.reserve(m); h.id.reserve(m); h.key2.reserve(m); h.id2.reserve(m);
+            h.temp.reserve(mps::launch::radix_temp_words(N));
+            pos_alt.reserve(m); vel_alt.reserve(m); color_alt.reserve(m); cgb_alt.reserve(m);
+            rho_alt.reserve(m); alpha_alt.reserve(m); kappa_alt.reserve(m); delta_alt.reserve(m); fst_alt.reserve(m);
+        }
+        T_(K_KEYS, [&] {
+            mps::launch::fluid_keys(pos.p, perm.p, N, g, blk_scene.p, mb, keyref.p, vals.p, mkey.p, lkey.p, n_old, h.start.p, h.end.p,
+                                    stream);
+        });
         h.n_valid = 0;
         if (N == 0) return;
-        keyref.reserve(N); vals.reserve(N); src.reserve(N); lkey.reserve(N); hash_perm.reserve(N);
-        h.key.reserve(N); h.id.reserve(N); h.key2.reserve(N); h.id2.reserve(N);
-        h.temp.reserve(mps::launch::radix_temp_words(N));
-        const int mb = morton_bits();
-        T_(K_KEYS, [&] { mps::launch::cell_morton_slots(pos.p, perm.p, N, g, blk_scene.p, mb, keyref.p, vals.p, stream); });
         const int bits = mb + scene_bits();
         uint32_t *k = keyref.p, *v = vals.p, *k2 = h.key2.p, *v2 = h.id2.p;
         T_(K_SORT, [&] { mps::launch::radix_sort(k, v, k2, v2, h.temp.p, Nref, bits, stream); });
@@ -755,27 +762,17 @@ struct mps_ctx {
             std::swap(h.id, h.id2);
         }
         T_(K_REORDER, [&] {
-            // sorted position q -> slot; perm, src (old slot) and the key per slot
-            mps::launch::place(h.key.p, h.id.p, Nref, mb, d_delta.p, inv.p, perm.p, src.p, mkey.p, stream);
-            auto mv4 = [&](DBuf<float4>& a, DBuf<float4>& alt) {
-                alt.reserve(N);
-                mps::launch::gather_f4(src.p, N, a.p, alt.p, stream);
-                std::swap(a, alt);
-            };
-            auto mv1 = [&](DBuf<float>& a, DBuf<float>& alt) {
-                alt.reserve(N);
-                mps::launch::gather_f1(src.p, N, a.p, alt.p, stream);
-                std::swap(a, alt);
-            };
-            mv4(pos, pos_alt); mv4(vel, vel_alt); mv4(color, color_alt); mv4(cgb, cgb_alt);
-            mv1(rho, rho_alt); mv1(alpha, alpha_alt); mv1(kappa, kappa_alt); mv1(delta, delta_alt); mv1(fst, fst_alt);
-            HIPCHK(hipMemcpyAsync(hash_perm.p, h.id.p, sizeof(uint32_t) * Nref, hipMemcpyDeviceToDevice, stream));
-            mps::launch::invert(perm.p, N, inv.p, stream);
+            mps::launch::FluidMove mv{{pos.p, vel.p, color.p, cgb.p},
+                                      {pos_alt.p, vel_alt.p, color_alt.p, cgb_alt.p},
+                                      {rho.p, alpha.p, kappa.p, delta.p, fst.p},
+                                      {rho_alt.p, alpha_alt.p, kappa_alt.p, delta_alt.p, fst_alt.p}};
+            mps::launch::fluid_reorder(h.key.p, h.id.p, Nref, g, mb, uint32_t(cells()), d_delta.p, inv.p, perm.p, src.p, mkey.p,
+                                       lkey.p, hash_perm.p, h.start.p, h.end.p, mv, stream);
+            std::swap(pos, pos_alt); std::swap(vel, vel_alt); std::swap(color, color_alt); std::swap(cgb, cgb_alt);
+            std::swap(rho, rho_alt); std::swap(alpha, alpha_alt); std::swap(kappa, kappa_alt);
+            std::swap(delta, delta_alt); std::swap(fst, fst_alt);
         });
         if (rec) dcopy(rec->src, src.p, N);
-        T_(K_CELLS, [&] {
-            mps::launch::cell_table_m(mkey.p, pos.p, N, g, mb, uint32_t(cells()), h.start.p, h.end.p, lkey.p, stream);
-        });
         h.n_valid = N;
         pairs_valid = false;
         halo_valid = false;

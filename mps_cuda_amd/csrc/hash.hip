@@ -14,6 +14,7 @@
 //     so the host can grow the capacity and search again;
 //   * the fluid search stages a workgroup's candidates in LDS, row by row, so that each
 //     particle walks its 27 cells as 9 contiguous runs (k_neighbors_fluid).
+#include <algorithm>
 #include <type_traits>
 
 #include "device_common.hpp"
@@ -25,125 +26,243 @@ namespace mps {
 namespace dev {
 
 // ===================================================================== radix sort
+// Stable LSD radix sort of (key, value) pairs. Two ways by size:
+//   * up to kSortOne items, one workgroup keeps them in registers and trades them through LDS
+//     between the passes: one launch for all passes;
+//   * beyond, tiles of kSortTile items, a histogram and a scatter per pass. Up to kSortSelf tiles
+//     every scatter workgroup sums the histograms of the tiles before its own (and of all, for the
+//     digits' totals) by itself; with more tiles a scan in between does it once.
+// In a tile every wave owns a contiguous strip and counts its digits in its own LDS counters, so
+// ranking needs no barrier: equal digits of a round are ranked by ballots, rounds by the counter.
+// What bounds it: launches and their latency up to some 100 k items (15 launches of 3-5 us with
+// 8-bit digits, a scan of three launches and a barrier per round: 250 particles 65 -> 9.5 us, 33 k
+// 74 -> 23), then the scattered 4-byte stores (1 M: 95 -> 45 us).
 constexpr int kSortThreads = 256;
 constexpr int kSortRounds = 8;
 constexpr int kSortTile = kSortThreads * kSortRounds;
+constexpr int kSortWaves = kSortThreads / 64;
+constexpr int kOneThreads = 1024;
+constexpr int kOneWaves = kOneThreads / 64;
+constexpr int kOneRounds = 8;
+constexpr uint32_t kSortOne = kOneThreads * kOneRounds;
+constexpr uint32_t kSortSelf = 32;
+constexpr int kOneDigit = 8;
 
-__global__ void __launch_bounds__(kSortThreads) k_radix_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
-                                                           uint32_t* __restrict__ hist, uint32_t nblk) {
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0u;
-    __syncthreads();
-    const uint32_t base = blockIdx.x * kSortTile;
-#pragma unroll
-    for (int r = 0; r < kSortRounds; r++) {
-        const uint32_t i = base + r * kSortThreads + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    hist[threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
-}
-
-// Exclusive scan of the digit histogram (length L = 256 * tiles), reduce-then-scan over
-// 1024-element chunks: chunk sums, one-block scan of the sums, chunk scans.
-constexpr int kScanChunk = 1024;
-__device__ __forceinline__ uint32_t block_incl_scan_1024(uint32_t v, uint32_t* lds /*[16]*/, uint32_t* total) {
+// Inclusive scan of one value per thread over W waves (every thread calls it; ws: W + 1 words).
+template <int W>
+__device__ __forceinline__ uint32_t block_incl_scan(uint32_t v, uint32_t* ws) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int off = 1; off < 64; off <<= 1) {
         const uint32_t t = __shfl_up(v, off, 64);
         if (lane >= off) v += t;
     }
-    if (lane == 63) lds[w] = v;
+    if (lane == 63) ws[w] = v;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); q++) {
-            const uint32_t t = lds[q];
-            lds[q] = run;
-            run += t;
-        }
-        lds[16] = run;
+    uint32_t before = 0u;
+#pragma unroll
+    for (int q = 0; q < W; q++) before += q < w ? ws[q] : 0u;
+    __syncthreads();
+    return v + before;
+}
+// Rank of this lane's digit among the wave's items so far; cnt: the wave's own 2^D counters.
+template <int D>
+__device__ __forceinline__ uint32_t wave_rank(uint32_t d, bool valid, uint32_t* cnt) {
+    const uint64_t lt = (1ull << (threadIdx.x & 63)) - 1ull;
+    uint64_t m = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < D; b++) {
+        const bool bit = (d >> b) & 1u;
+        const uint64_t bb = __ballot(bit);
+        m &= bit ? bb : ~bb;
     }
-    __syncthreads();
-    v += lds[w];
-    *total = lds[16];
-    __syncthreads();
-    return v;
-}
-__global__ void __launch_bounds__(kScanChunk) k_scan_sums(const uint32_t* __restrict__ a, uint32_t L, uint32_t* __restrict__ sums) {
-    __shared__ uint32_t lds[17];
-    const uint32_t i = blockIdx.x * kScanChunk + threadIdx.x;
-    uint32_t tot;
-    block_incl_scan_1024(i < L ? a[i] : 0u, lds, &tot);
-    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
-}
-__global__ void __launch_bounds__(kScanChunk) k_scan_top(uint32_t* __restrict__ sums, uint32_t n) {
-    __shared__ uint32_t lds[17];
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < n; base += kScanChunk) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t v = i < n ? sums[i] : 0u;
-        uint32_t tot;
-        const uint32_t inc = block_incl_scan_1024(v, lds, &tot);
-        if (i < n) sums[i] = carry + inc - v;
-        carry += tot;
-    }
-}
-__global__ void __launch_bounds__(kScanChunk) k_scan_apply(uint32_t* __restrict__ a, uint32_t L, const uint32_t* __restrict__ sums) {
-    __shared__ uint32_t lds[17];
-    const uint32_t i = blockIdx.x * kScanChunk + threadIdx.x;
-    const uint32_t v = i < L ? a[i] : 0u;
-    uint32_t tot;
-    const uint32_t inc = block_incl_scan_1024(v, lds, &tot);
-    if (i < L) a[i] = sums[blockIdx.x] + inc - v;
+    const uint32_t before = __popcll(m & lt);
+    const uint32_t base = cnt[d];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (valid && before == 0u) cnt[d] = base + __popcll(m);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return base + before;
 }
 
-// Stable scatter: items are ranked round by round (256 per round, wave-major, lane-minor),
-// which preserves input order among equal digits.
+__global__ void __launch_bounds__(kOneThreads) k_radix_one(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                         uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n,
+                                                         int bits) {
+    constexpr uint32_t kDigits = 1u << kOneDigit;
+    __shared__ uint32_t cnt[kOneWaves][kDigits];
+    __shared__ uint32_t ws[kOneWaves];
+    __shared__ uint2 item[kSortOne];
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const uint32_t rounds = (n + kOneThreads - 1u) / kOneThreads;
+    const uint32_t first = w * 64u * rounds + lane;
+    uint2 it[kOneRounds];
+#pragma unroll
+    for (uint32_t r = 0; r < kOneRounds; r++) {
+        const uint32_t i = first + 64u * r;
+        const bool valid = r < rounds && i < n;
+        it[r] = valid ? make_uint2(kin[i], vin[i]) : make_uint2(0u, 0u);
+    }
+    for (int shift = 0; shift < bits; shift += kOneDigit) {
+        for (uint32_t c = t; c < kOneWaves * kDigits; c += kOneThreads) cnt[0][c] = 0u;
+        __syncthreads();
+        uint32_t rank[kOneRounds];
+#pragma unroll
+        for (uint32_t r = 0; r < kOneRounds; r++)
+            if (r < rounds) rank[r] = wave_rank<kOneDigit>((it[r].x >> shift) & (kDigits - 1u), first + 64u * r < n, cnt[w]);
+        __syncthreads();
+        // a digit's counters become the position of each wave's first item of it
+        uint32_t tot = 0u;
+        if (t < kDigits)
+            for (int q = 0; q < kOneWaves; q++) {
+                const uint32_t c = cnt[q][t];
+                cnt[q][t] = tot;
+                tot += c;
+            }
+        const uint32_t before = block_incl_scan<kOneWaves>(tot, ws) - tot;
+        if (t < kDigits)
+            for (int q = 0; q < kOneWaves; q++) cnt[q][t] += before;
+        __syncthreads();
+        const bool last = shift + kOneDigit >= bits;
+#pragma unroll
+        for (uint32_t r = 0; r < kOneRounds; r++)
+            if (r < rounds && first + 64u * r < n) {
+                const uint32_t at = cnt[w][(it[r].x >> shift) & (kDigits - 1u)] + rank[r];
+                if (last) {
+                    kout[at] = it[r].x;
+                    vout[at] = it[r].y;
+                } else {
+                    item[at] = it[r];
+                }
+            }
+        if (last) break;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < kOneRounds; r++)
+            if (r < rounds && first + 64u * r < n) it[r] = item[first + 64u * r];
+    }
+}
+
+// hist[tile][digit]
+template <int D>
+__global__ void __launch_bounds__(kSortThreads) k_radix_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
+                                                           uint32_t* __restrict__ hist) {
+    constexpr uint32_t kDigits = 1u << D;
+    __shared__ uint32_t h[kDigits];
+    for (uint32_t d = threadIdx.x; d < kDigits; d += kSortThreads) h[d] = 0u;
+    __syncthreads();
+    const uint32_t base = blockIdx.x * kSortTile;
+#pragma unroll
+    for (int r = 0; r < kSortRounds; r++) {
+        const uint32_t i = base + r * kSortThreads + threadIdx.x;
+        if (i < n) atomicAdd(&h[(keys[i] >> shift) & (kDigits - 1u)], 1u);
+    }
+    __syncthreads();
+    for (uint32_t d = threadIdx.x; d < kDigits; d += kSortThreads) hist[size_t(blockIdx.x) * kDigits + d] = h[d];
+}
+
+// Exclusive scan of the histograms over the tiles, in place, and the digits' totals: 16 digits
+// (a 64-byte line of every tile) per workgroup, a run of tiles per thread.
+constexpr uint32_t kScanDigits = 16;
+constexpr uint32_t kScanRuns = 64;
+__global__ void __launch_bounds__(kScanDigits* kScanRuns) k_radix_scan(uint32_t* __restrict__ hist, uint32_t digits,
+                                                                        uint32_t tiles, uint32_t* __restrict__ total) {
+    __shared__ uint32_t run[kScanRuns][kScanDigits];
+    const uint32_t d = blockIdx.x * kScanDigits + threadIdx.x % kScanDigits, r = threadIdx.x / kScanDigits;
+    const uint32_t per = (tiles + kScanRuns - 1u) / kScanRuns;
+    const uint32_t t0 = min(r * per, tiles), t1 = min(t0 + per, tiles);
+    uint32_t sum = 0u;
+#pragma unroll 8
+    for (uint32_t t = t0; t < t1; t++) sum += hist[size_t(t) * digits + d];
+    run[r][threadIdx.x % kScanDigits] = sum;
+    __syncthreads();
+    uint32_t before = 0u, all = 0u;
+#pragma unroll 8
+    for (uint32_t q = 0; q < kScanRuns; q++) {
+        const uint32_t v = run[q][threadIdx.x % kScanDigits];
+        before += q < r ? v : 0u;
+        all += v;
+    }
+    if (r == 0u) total[d] = all;
+#pragma unroll 8
+    for (uint32_t t = t0; t < t1; t++) {
+        const uint32_t v = hist[size_t(t) * digits + d];
+        hist[size_t(t) * digits + d] = before;
+        before += v;
+    }
+}
+
+// SELF: hist holds the tiles' counts; otherwise their exclusive scan, with the totals beside it.
+template <int D, bool SELF>
 __global__ void __launch_bounds__(kSortThreads) k_radix_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                               uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n,
-                                                              int shift, const uint32_t* __restrict__ offs, uint32_t nblk) {
-    __shared__ uint32_t base[256];
-    __shared__ uint32_t wcnt[4][256];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    base[threadIdx.x] = offs[threadIdx.x * nblk + blockIdx.x];
-    const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+                                                              int shift, const uint32_t* __restrict__ hist, uint32_t tiles,
+                                                              const uint32_t* __restrict__ total) {
+    constexpr uint32_t kDigits = 1u << D;
+    constexpr uint32_t kPer = (kDigits + kSortThreads - 1u) / kSortThreads;  // digits per thread, neighbours
+    __shared__ uint32_t cnt[kSortWaves][kDigits];
+    __shared__ uint32_t ws[kSortWaves];
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const uint32_t first = blockIdx.x * kSortTile + w * (64u * kSortRounds) + lane;
+    uint32_t key[kSortRounds], val[kSortRounds], rank[kSortRounds];
+#pragma unroll
     for (int r = 0; r < kSortRounds; r++) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) wcnt[k][threadIdx.x] = 0u;
-        __syncthreads();
-        const uint32_t i = blockIdx.x * kSortTile + r * kSortThreads + threadIdx.x;
-        const bool valid = i < n;
-        const uint32_t key = valid ? kin[i] : 0u;
-        const uint32_t d = (key >> shift) & 255u;
-        uint64_t m = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t bb = __ballot(bit);
-            m &= bit ? bb : ~bb;
-        }
-        const uint32_t rank = __popcll(m & lt);
-        if (valid && rank == 0u) wcnt[w][d] = __popcll(m);
-        __syncthreads();
-        {
-            const uint32_t t = threadIdx.x;
-            const uint32_t c0 = wcnt[0][t], c1 = wcnt[1][t], c2 = wcnt[2][t], c3 = wcnt[3][t];
-            const uint32_t b0 = base[t];
-            wcnt[0][t] = b0;
-            wcnt[1][t] = b0 + c0;
-            wcnt[2][t] = b0 + c0 + c1;
-            wcnt[3][t] = b0 + c0 + c1 + c2;
-            base[t] = b0 + c0 + c1 + c2 + c3;
-        }
-        __syncthreads();
-        if (valid) {
-            const uint32_t pos = wcnt[w][d] + rank;
-            kout[pos] = key;
-            vout[pos] = vin[i];
-        }
-        __syncthreads();
+        const uint32_t i = first + 64u * r;
+        key[r] = i < n ? kin[i] : 0u;
+        val[r] = i < n ? vin[i] : 0u;
     }
+    const uint32_t d0 = t * kPer;
+    uint32_t before[kPer], tot[kPer], sum = 0u;
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; q++) before[q] = tot[q] = 0u;
+    if (d0 < kDigits) {
+        if constexpr (SELF) {
+#pragma unroll 8
+            for (uint32_t b = 0; b < tiles; b++)
+#pragma unroll
+                for (uint32_t q = 0; q < kPer; q++) {
+                    const uint32_t h = hist[size_t(b) * kDigits + d0 + q];
+                    before[q] += b < blockIdx.x ? h : 0u;
+                    tot[q] += h;
+                }
+        } else {
+#pragma unroll
+            for (uint32_t q = 0; q < kPer; q++) {
+                before[q] = hist[size_t(blockIdx.x) * kDigits + d0 + q];
+                tot[q] = total[d0 + q];
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; q++) {
+        before[q] += sum;
+        sum += tot[q];
+    }
+    for (uint32_t c = t; c < kSortWaves * kDigits; c += kSortThreads) cnt[0][c] = 0u;
+    const uint32_t base = block_incl_scan<kSortWaves>(sum, ws) - sum;  // (its barriers follow the clearing)
+#pragma unroll
+    for (int r = 0; r < kSortRounds; r++)
+        rank[r] = wave_rank<D>((key[r] >> shift) & (kDigits - 1u), first + 64u * r < n, cnt[w]);
+    __syncthreads();
+    if (d0 < kDigits) {
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; q++) {
+            uint32_t at = base + before[q];
+#pragma unroll
+            for (int v = 0; v < kSortWaves; v++) {
+                const uint32_t c = cnt[v][d0 + q];
+                cnt[v][d0 + q] = at;
+                at += c;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRounds; r++)
+        if (first + 64u * r < n) {
+            const uint32_t at = cnt[w][(key[r] >> shift) & (kDigits - 1u)] + rank[r];
+            kout[at] = key[r];
+            vout[at] = val[r];
+        }
 }
 
 // ===================================================================== hashing
@@ -184,10 +303,17 @@ __device__ __forceinline__ uint32_t cell_morton(i3 c, const HashGeom& g) {
     const uint32_t z = static_cast<uint32_t>(c.z) & (g.hz - 1u);
     return split_by3(x) | (split_by3(y) << 1u) | (split_by3(z) << 2u);
 }
-__global__ void __launch_bounds__(kBlock) k_cell_morton_slots(const float4* __restrict__ pos, const uint32_t* __restrict__ perm,
-                                                            uint32_t n, HashGeom g, const uint32_t* __restrict__ blk_scene,
-                                                            int shift, uint32_t* __restrict__ keyref, uint32_t* __restrict__ iota) {
+// First launch of the fluid hash: empties the cell table of the last one and writes the new keys.
+__global__ void __launch_bounds__(kBlock) k_fluid_keys(const float4* __restrict__ pos, const uint32_t* __restrict__ perm, uint32_t n,
+                                                     HashGeom g, const uint32_t* __restrict__ blk_scene, int shift,
+                                                     uint32_t* __restrict__ keyref, uint32_t* __restrict__ iota,
+                                                     const uint32_t* __restrict__ mkey, const uint32_t* __restrict__ lkey,
+                                                     uint32_t n_old, uint32_t* __restrict__ start, uint32_t* __restrict__ end) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < n_old) {
+        const uint32_t m = mkey[s];
+        if (m != kEmpty && (s == 0 || mkey[s - 1] != m)) start[lkey[s]] = end[lkey[s]] = kEmpty;
+    }
     if (s >= n) return;
     iota[s] = s;
     const uint32_t ref = perm[s];
@@ -195,61 +321,52 @@ __global__ void __launch_bounds__(kBlock) k_cell_morton_slots(const float4* __re
     const float4 p = pos[s];
     keyref[ref] = (blk_scene[blockIdx.x] << shift) | cell_morton(grid_pos(p.x, p.y, p.z, g), g);
 }
-// Sorted position q (key[q], reference id id[q]) -> slot q + delta[scene]: scene s's sorted
-// range [cum_s, cum_s + count_s) lands on its slots [begin_s, end_s). Writes the new perm, the
-// old slot of each particle (src, for the gathers) and the key per slot.
-__global__ void __launch_bounds__(kBlock) k_place(const uint32_t* __restrict__ key, const uint32_t* __restrict__ id, uint32_t nref,
-                                                int shift, const uint32_t* __restrict__ delta, const uint32_t* __restrict__ inv,
-                                                uint32_t* __restrict__ perm, uint32_t* __restrict__ src,
-                                                uint32_t* __restrict__ mkey) {
+// Last launch of the fluid hash: sorted position q (key[q], reference id id[q]) -> slot
+// q + delta[scene], where scene s's sorted range [cum_s, cum_s + count_s) lands on its slots
+// [begin_s, end_s). A thread takes its particle's whole state from the old slot (src) to the new
+// one, relabels it (perm, inv; no other thread reads or writes this particle's inv) and enters the
+// bounds of its run in the cell table, which is indexed by scene * C + the reference's linear cell
+// key (lkey keeps that index for clearing and for exporting the hash). Padding slots keep
+// kEmpty in perm, src and mkey. One pass for what were twelve launches (the labels, a gather per array,
+// the inverse, the table), each of which read src again: 250 particles 45 -> 5 us, 33 k 53 -> 12; 1 M
+// 81 -> 44, 4 TB/s of the 176 bytes per particle, whose loads follow inv in groups of a cell.
+__global__ void __launch_bounds__(kBlock) k_fluid_reorder(const uint32_t* __restrict__ key, const uint32_t* __restrict__ id,
+                                                        uint32_t nref, HashGeom g, int shift, uint32_t C,
+                                                        const uint32_t* __restrict__ delta, uint32_t* __restrict__ inv,
+                                                        uint32_t* __restrict__ perm, uint32_t* __restrict__ src,
+                                                        uint32_t* __restrict__ mkey, uint32_t* __restrict__ lkey,
+                                                        uint32_t* __restrict__ hash_perm, uint32_t* __restrict__ start,
+                                                        uint32_t* __restrict__ end, launch::FluidMove mv) {
     const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= nref) return;
-    const uint32_t k = key[q];
+    const uint32_t k = key[q], ref = id[q];
+    const uint32_t o = inv[ref];
     const uint32_t slot = q + delta[k >> shift];
-    const uint32_t ref = id[q];
+    float4 a[4];
+    float b[5];
+#pragma unroll
+    for (int v = 0; v < 4; v++) a[v] = mv.from4[v][o];
+#pragma unroll
+    for (int v = 0; v < 5; v++) b[v] = mv.from1[v][o];
     perm[slot] = ref;
-    src[slot] = inv[ref];
+    inv[ref] = slot;
+    src[slot] = o;
     mkey[slot] = k;
-}
-// Cell table over Morton-sorted slots: start/end are indexed by scene * C + the reference's
-// linear cell key; lkey[s] keeps that index (for clearing and for exporting the hash). mkey
-// is kEmpty on padding slots, which therefore end every run.
-__global__ void __launch_bounds__(kBlock) k_cell_table_m(const uint32_t* __restrict__ mkey, const float4* __restrict__ pos,
-                                                       uint32_t n, HashGeom g, int shift, uint32_t C,
-                                                       uint32_t* __restrict__ start, uint32_t* __restrict__ end,
-                                                       uint32_t* __restrict__ lkey) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const uint32_t m = mkey[s];
-    if (m == kEmpty) return;
-    const float4 p = pos[s];
-    const i3 c = grid_pos(p.x, p.y, p.z, g);
-    const uint32_t t = (m >> shift) * C + grid_index(c.x, c.y, c.z, g);
-    lkey[s] = t;
-    if (s == 0 || mkey[s - 1] != m) start[t] = s;
-    if (s == n - 1 || mkey[s + 1] != m) end[t] = s + 1;
-}
-__global__ void __launch_bounds__(kBlock) k_clear_cells_m(const uint32_t* __restrict__ mkey, const uint32_t* __restrict__ lkey,
-                                                        uint32_t n, uint32_t* __restrict__ start, uint32_t* __restrict__ end) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const uint32_t m = mkey[s];
-    if (m == kEmpty) return;
-    if (s == 0 || mkey[s - 1] != m) {
-        start[lkey[s]] = kEmpty;
-        end[lkey[s]] = kEmpty;
-    }
+    hash_perm[q] = ref;
+#pragma unroll
+    for (int v = 0; v < 4; v++) mv.to4[v][slot] = a[v];
+#pragma unroll
+    for (int v = 0; v < 5; v++) mv.to1[v][slot] = b[v];
+    const i3 c = grid_pos(a[0].x, a[0].y, a[0].z, g);
+    const uint32_t t = (k >> shift) * C + grid_index(c.x, c.y, c.z, g);
+    lkey[slot] = t;
+    if (q == 0 || key[q - 1] != k) start[t] = slot;
+    if (q == nref - 1 || key[q + 1] != k) end[t] = slot + 1;
 }
 // inv[perm[s]] = s (padding slots skipped)
 __global__ void __launch_bounds__(kBlock) k_invert(const uint32_t* __restrict__ perm, uint32_t n, uint32_t* __restrict__ inv) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s < n && perm[s] != kEmpty) inv[perm[s]] = s;
-}
-// src[s'] = inv[perm_new[s']]: old slot of the particle that moves to slot s'
-__global__ void __launch_bounds__(kBlock) k_compose(const uint32_t* __restrict__ perm_new, const uint32_t* __restrict__ inv,
-                                                  uint32_t n, uint32_t* __restrict__ src) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n) src[s] = inv[perm_new[s]];
 }
 // perm[s] = map[perm[s]]  (relabel reference ids after a Z-sort)
 __global__ void __launch_bounds__(kBlock) k_relabel(uint32_t* __restrict__ perm, const uint32_t* __restrict__ map, uint32_t n) {
@@ -1038,24 +1155,51 @@ using namespace dev;
 
 static inline unsigned nb(size_t n, unsigned b = kBlock) { return unsigned((n + b - 1) / b); }
 
+// Fewest passes of at most 11 bits: a 64^3 grid takes two passes of 9 bits, a 128^3 grid two of 11
+// (with at most 8 bits, three each: 1 M particles 45 against 60 us, 257 k 34 against 49, 33 k 23
+// against 28).
+constexpr int kMaxDigit = 11;
+
 size_t radix_temp_words(uint32_t n) {
-    const size_t L = size_t(256) * ((n + kSortTile - 1) / kSortTile);
-    return L + (L + kScanChunk - 1) / kScanChunk + 1;
+    return (size_t((n + kSortTile - 1) / kSortTile) + 1) << kMaxDigit;
 }
 
 int radix_sort(uint32_t*& keys, uint32_t*& vals, uint32_t*& keys_alt, uint32_t*& vals_alt, uint32_t* temp, uint32_t n,
                int key_bits, hipStream_t s) {
-    if (n == 0) return 0;
-    const uint32_t nblk = (n + kSortTile - 1) / kSortTile;
-    const uint32_t L = 256u * nblk;
-    for (int shift = 0; shift < key_bits; shift += 8) {
-        launch_k(k_radix_hist, nblk, kSortThreads, 0, s, keys, n, shift, temp, nblk);
-        const uint32_t nch = (L + kScanChunk - 1) / kScanChunk;
-        uint32_t* sums = temp + L;
-        launch_k(k_scan_sums, nch, kScanChunk, 0, s, temp, L, sums);
-        launch_k(k_scan_top, 1, kScanChunk, 0, s, sums, nch);
-        launch_k(k_scan_apply, nch, kScanChunk, 0, s, temp, L, sums);
-        launch_k(k_radix_scatter, nblk, kSortThreads, 0, s, keys, vals, keys_alt, vals_alt, n, shift, temp, nblk);
+    if (n == 0 || key_bits <= 0) return 0;
+    if (n <= kSortOne) {
+        launch_k(k_radix_one, 1, kOneThreads, 0, s, keys, vals, keys_alt, vals_alt, n, key_bits);
+        std::swap(keys, keys_alt);
+        std::swap(vals, vals_alt);
+        return 0;
+    }
+    const uint32_t tiles = (n + kSortTile - 1) / kSortTile;
+    const int passes = (key_bits + kMaxDigit - 1) / kMaxDigit;
+    const int digit = std::max((key_bits + passes - 1) / passes, 4);  // 16 digits per scanning workgroup
+    uint32_t* total = temp + (size_t(tiles) << digit);
+    auto pass = [&](auto d, int shift) {
+        constexpr int D = decltype(d)::value;
+        launch_k(k_radix_hist<D>, tiles, kSortThreads, 0, s, keys, n, shift, temp);
+        if (tiles <= kSortSelf) {
+            launch_k(k_radix_scatter<D, true>, tiles, kSortThreads, 0, s, keys, vals, keys_alt, vals_alt, n, shift, temp, tiles,
+                     total);
+        } else {
+            launch_k(k_radix_scan, (1u << D) / kScanDigits, kScanDigits * kScanRuns, 0, s, temp, 1u << D, tiles, total);
+            launch_k(k_radix_scatter<D, false>, tiles, kSortThreads, 0, s, keys, vals, keys_alt, vals_alt, n, shift, temp, tiles,
+                     total);
+        }
+    };
+    for (int shift = 0; shift < key_bits; shift += digit) {
+        switch (digit) {
+            case 11: pass(std::integral_constant<int, 11>{}, shift); break;
+            case 10: pass(std::integral_constant<int, 10>{}, shift); break;
+            case 9: pass(std::integral_constant<int, 9>{}, shift); break;
+            case 8: pass(std::integral_constant<int, 8>{}, shift); break;
+            case 7: pass(std::integral_constant<int, 7>{}, shift); break;
+            case 6: pass(std::integral_constant<int, 6>{}, shift); break;
+            case 5: pass(std::integral_constant<int, 5>{}, shift); break;
+            default: pass(std::integral_constant<int, 4>{}, shift); break;
+        }
         std::swap(keys, keys_alt);
         std::swap(vals, vals_alt);
     }
@@ -1070,26 +1214,21 @@ void cell_keys_slots(const float4* pos, const uint32_t* perm, uint32_t n, const 
                      const uint32_t* blk_scene, int shift, uint32_t* keyref, uint32_t* iota, hipStream_t s) {
     if (n) launch_k(k_cell_keys_slots, nb(n), kBlock, 0, s, pos, perm, n, g, morton, blk_scene, shift, keyref, iota);
 }
-void cell_morton_slots(const float4* pos, const uint32_t* perm, uint32_t n, const HashGeom& g, const uint32_t* blk_scene,
-                       int shift, uint32_t* keyref, uint32_t* iota, hipStream_t s) {
-    if (n) launch_k(k_cell_morton_slots, nb(n), kBlock, 0, s, pos, perm, n, g, blk_scene, shift, keyref, iota);
+void fluid_keys(const float4* pos, const uint32_t* perm, uint32_t n, const HashGeom& g, const uint32_t* blk_scene, int shift,
+                uint32_t* keyref, uint32_t* iota, const uint32_t* mkey, const uint32_t* lkey, uint32_t n_old, uint32_t* start,
+                uint32_t* end, hipStream_t s) {
+    const uint32_t m = std::max(n, n_old);
+    if (m) launch_k(k_fluid_keys, nb(m), kBlock, 0, s, pos, perm, n, g, blk_scene, shift, keyref, iota, mkey, lkey, n_old,
+                    start, end);
 }
-void place(const uint32_t* key, const uint32_t* id, uint32_t nref, int shift, const uint32_t* delta, const uint32_t* inv,
-           uint32_t* perm, uint32_t* src, uint32_t* mkey, hipStream_t s) {
-    if (nref) launch_k(k_place, nb(nref), kBlock, 0, s, key, id, nref, shift, delta, inv, perm, src, mkey);
-}
-void cell_table_m(const uint32_t* mkey, const float4* pos, uint32_t n, const HashGeom& g, int shift, uint32_t C, uint32_t* start,
-                  uint32_t* end, uint32_t* lkey, hipStream_t s) {
-    if (n) launch_k(k_cell_table_m, nb(n), kBlock, 0, s, mkey, pos, n, g, shift, C, start, end, lkey);
-}
-void clear_cells_m(const uint32_t* mkey, const uint32_t* lkey, uint32_t n, uint32_t* start, uint32_t* end, hipStream_t s) {
-    if (n) launch_k(k_clear_cells_m, nb(n), kBlock, 0, s, mkey, lkey, n, start, end);
+void fluid_reorder(const uint32_t* key, const uint32_t* id, uint32_t nref, const HashGeom& g, int shift, uint32_t C,
+                   const uint32_t* delta, uint32_t* inv, uint32_t* perm, uint32_t* src, uint32_t* mkey, uint32_t* lkey,
+                   uint32_t* hash_perm, uint32_t* start, uint32_t* end, const FluidMove& mv, hipStream_t s) {
+    if (nref) launch_k(k_fluid_reorder, nb(nref), kBlock, 0, s, key, id, nref, g, shift, C, delta, inv, perm, src, mkey, lkey,
+                       hash_perm, start, end, mv);
 }
 void invert(const uint32_t* perm, uint32_t n, uint32_t* inv, hipStream_t s) {
     if (n) launch_k(k_invert, nb(n), kBlock, 0, s, perm, n, inv);
-}
-void compose(const uint32_t* perm_new, const uint32_t* inv, uint32_t n, uint32_t* src, hipStream_t s) {
-    if (n) launch_k(k_compose, nb(n), kBlock, 0, s, perm_new, inv, n, src);
 }
 void relabel(uint32_t* perm, const uint32_t* map, uint32_t n, hipStream_t s) {
     if (n) launch_k(k_relabel, nb(n), kBlock, 0, s, perm, map, n);

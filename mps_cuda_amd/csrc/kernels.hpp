@@ -164,16 +164,23 @@ void cell_keys(const float4* pos, uint32_t n, const dev::HashGeom& g, int morton
                uint32_t* key, uint32_t* id, hipStream_t s);
 void cell_keys_slots(const float4* pos, const uint32_t* perm, uint32_t n, const dev::HashGeom& g, int morton,
                      const uint32_t* blk_scene, int shift, uint32_t* keyref, uint32_t* iota, hipStream_t s);
-void cell_morton_slots(const float4* pos, const uint32_t* perm, uint32_t n, const dev::HashGeom& g, const uint32_t* blk_scene,
-                       int shift, uint32_t* keyref, uint32_t* iota, hipStream_t s);
-// sorted position q -> slot q + delta[key[q] >> shift]: new perm, src (old slot) and key per slot
-void place(const uint32_t* key, const uint32_t* id, uint32_t nref, int shift, const uint32_t* delta, const uint32_t* inv,
-           uint32_t* perm, uint32_t* src, uint32_t* mkey, hipStream_t s);
-void cell_table_m(const uint32_t* mkey, const float4* pos, uint32_t n, const dev::HashGeom& g, int shift, uint32_t C,
-                  uint32_t* start, uint32_t* end, uint32_t* lkey, hipStream_t s);
-void clear_cells_m(const uint32_t* mkey, const uint32_t* lkey, uint32_t n, uint32_t* start, uint32_t* end, hipStream_t s);
+// Fluid hash, before the sort: empties the cell table (n_old slots of the last hash; 0: it is empty)
+// and writes the Morton keys at the reference ids.
+void fluid_keys(const float4* pos, const uint32_t* perm, uint32_t n, const dev::HashGeom& g, const uint32_t* blk_scene, int shift,
+                uint32_t* keyref, uint32_t* iota, const uint32_t* mkey, const uint32_t* lkey, uint32_t n_old, uint32_t* start,
+                uint32_t* end, hipStream_t s);
+// The per-particle arrays a fluid hash moves, from the old order to the new; the first is the positions.
+struct FluidMove {
+    const float4* from4[4];
+    float4* to4[4];
+    const float* from1[5];
+    float* to1[5];
+};
+// Fluid hash, after the sort: labels, state and cell table in the new slot order.
+void fluid_reorder(const uint32_t* key, const uint32_t* id, uint32_t nref, const dev::HashGeom& g, int shift, uint32_t C,
+                   const uint32_t* delta, uint32_t* inv, uint32_t* perm, uint32_t* src, uint32_t* mkey, uint32_t* lkey,
+                   uint32_t* hash_perm, uint32_t* start, uint32_t* end, const FluidMove& mv, hipStream_t s);
 void invert(const uint32_t* perm, uint32_t n, uint32_t* inv, hipStream_t s);
-void compose(const uint32_t* perm_new, const uint32_t* inv, uint32_t n, uint32_t* src, hipStream_t s);
 void relabel(uint32_t* perm, const uint32_t* map, uint32_t n, hipStream_t s);
 void iota(uint32_t* p, uint32_t n, hipStream_t s);
 void fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s);
