@@ -237,6 +237,9 @@ struct mps_ctx {
     DBuf<double> acc_mu, acc_sig;
     // fluid: pos = (x, y, z, r), vel = (vx, vy, vz, m)
     DBuf<float4> pos, vel, color, cgb, cgx, jprev, jt[3], jcand, tmp4;
+    // device side of fluid arrays that come from or go to the host, kStagePart particles at a time
+    static constexpr size_t kStagePart = size_t(1) << 20;
+    DBuf<float> stage;
     // the forward CG's vectors as packed triples: x, r, A p and two p buffers
     DBuf<mps::dev::f3> v3x, v3r, v3Ap, v3p, v3q;
     DBuf<float> rho, alpha, kappa, delta, fst, tmp1;
@@ -1853,6 +1856,7 @@ struct mps_ctx {
         pos.reserve(m); vel.reserve(m); color.reserve(m); cgb.reserve(m); cgx.reserve(m);
         rho.reserve(m); alpha.reserve(m); kappa.reserve(m); delta.reserve(m); fst.reserve(m);
         cff.reserve(m); cfb.reserve(m); perm.reserve(m); inv.reserve(m); mkey.reserve(m);
+        stage.reserve(8 * std::min(m, kStagePart));  // here, so that no read or write of an array allocates
     }
     void require_single(const char* what) const {
         if (!scenes.empty()) throw ApiError{MPS_ERR_STATE, std::string(what) + ": the context holds a batch of scenes"};
@@ -1860,19 +1864,10 @@ struct mps_ctx {
     // Zero the derived fluid state of slots [0, n) and start at frame 0.
     void reset_fluid_state(uint32_t n) {
         if (n) {
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(rho.p), n, stream);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(alpha.p), n, stream);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(kappa.p), n, stream);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(delta.p), n, stream);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(fst.p), n, stream);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(cgb.p), 4 * size_t(n), stream);
-            mps::launch::zero_words(cff.p, n, stream);
-            mps::launch::zero_words(cfb.p, n, stream);
             // Padding slots between scenes keep kEmpty in mkey and src for good: the hash
-            // writes both only at live slots, and the reorder gathers skip kEmpty sources.
-            mps::launch::fill_u32(mkey.p, n, mps::dev::kEmpty, stream);
+            // writes both only at live slots.
             src.reserve(n);
-            mps::launch::fill_u32(src.p, n, mps::dev::kEmpty, stream);
+            mps::launch::fluid_reset(n, rho.p, alpha.p, kappa.p, delta.p, fst.p, cgb.p, cff.p, cfb.p, mkey.p, src.p, stream);
         }
         fh.cells_init = false;
         fh.n_valid = 0;
@@ -1893,18 +1888,21 @@ struct mps_ctx {
         if (n > 0x7FFFFFFFu) throw ApiError{MPS_ERR_INVALID, "too many particles"};
         require_single("mps_upload_fluid");
         alloc_fluid(uint32_t(n));
-        std::vector<float4> hp(n), hv(n), hc(n, make_float4(0.f, 0.f, 1.f, 1.f));
-        for (size_t i = 0; i < n; i++) {
-            hp[i] = make_float4(p[3 * i], p[3 * i + 1], p[3 * i + 2], r[i]);
-            hv[i] = make_float4(v ? v[3 * i] : 0.f, v ? v[3 * i + 1] : 0.f, v ? v[3 * i + 2] : 0.f, m ? m[i] : float(mMass));
-        }
         N = Nref = uint32_t(n);
-        if (n) {
-            HIPCHK(hipMemcpyAsync(pos.p, hp.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
-            HIPCHK(hipMemcpyAsync(vel.p, hv.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
-            HIPCHK(hipMemcpyAsync(color.p, hc.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
-            mps::launch::iota(perm.p, uint32_t(n), stream);
-            mps::launch::iota(inv.p, uint32_t(n), stream);
+        // the caller's arrays as they are, packed on the device, a bounded part at a time
+        const size_t part = std::min(n, kStagePart);
+        for (size_t i = 0; i < n; i += part) {
+            const size_t k = std::min(part, n - i);
+            float* at = stage.p;
+            auto put = [&](const float* a, size_t w) -> const float* {
+                if (!a) return nullptr;
+                HIPCHK(hipMemcpyAsync(at, a + i * w, k * w * sizeof(float), hipMemcpyHostToDevice, stream));
+                at += k * w;
+                return at - k * w;
+            };
+            const float *dp = put(p, 3), *dr = put(r, 1), *dv = put(v, 3), *dm = put(m, 1);
+            mps::launch::fluid_upload(uint32_t(k), uint32_t(i), dp, dr, dv, dm, float(mMass), pos.p, vel.p, color.p, perm.p, inv.p,
+                                      stream);
         }
         reset_fluid_state(uint32_t(n));
         sync();
@@ -2318,58 +2316,28 @@ struct mps_ctx {
     }
     // returns (count, elem_bytes) and optionally the data as bytes
     void array_io(int32_t id, size_t* count, size_t* eb, void* dst, const void* src, size_t bytes) {
-        // fluid arrays live in slot order; the API shows reference order (out[perm[s]] = a[s])
-        std::vector<uint32_t> hperm;
-        auto get_perm = [&]() -> const std::vector<uint32_t>& {
-            if (hperm.empty() && N) hperm = down(perm.p, N);
-            return hperm;
-        };
-        auto fl4 = [&](DBuf<float4>& a, int comp /* -1 = xyz, 3 = w, 4 = all */) {
-            const size_t w = comp == -1 ? 3 : (comp == 4 ? 4 : 1);
+        // fluid arrays live in slot order; the API shows reference order (out[ref] = a[inv[ref]]): w
+        // floats at `off` of each slot's `stride`, a bounded part at a time
+        auto fl = [&](float* a, uint32_t w, uint32_t stride, uint32_t off) {
             *count = Nref;
-            *eb = 4 * w;
+            *eb = 4 * size_t(w);
             if (!(dst || src)) return;
             if (bytes != size_t(Nref) * 4 * w) throw ApiError{MPS_ERR_INVALID, "size mismatch"};
-            const auto& P = get_perm();
-            std::vector<float4> h = down(a.p, N);
-            if (dst) {
-                float* d = static_cast<float*>(dst);
-                for (uint32_t s = 0; s < N; s++) {
-                    if (P[s] == mps::dev::kEmpty) continue;
-                    const float q[4] = {h[s].x, h[s].y, h[s].z, h[s].w};
-                    if (comp == -1) for (int k = 0; k < 3; k++) d[3 * size_t(P[s]) + k] = q[k];
-                    else if (comp == 4) for (int k = 0; k < 4; k++) d[4 * size_t(P[s]) + k] = q[k];
-                    else d[P[s]] = q[3];
-                }
-            } else {
-                const float* q = static_cast<const float*>(src);
-                for (uint32_t s = 0; s < N; s++) {
-                    if (P[s] == mps::dev::kEmpty) continue;
-                    if (comp == -1) { h[s].x = q[3 * size_t(P[s])]; h[s].y = q[3 * size_t(P[s]) + 1]; h[s].z = q[3 * size_t(P[s]) + 2]; }
-                    else if (comp == 4) { h[s].x = q[4 * size_t(P[s])]; h[s].y = q[4 * size_t(P[s]) + 1]; h[s].z = q[4 * size_t(P[s]) + 2]; h[s].w = q[4 * size_t(P[s]) + 3]; }
-                    else h[s].w = q[P[s]];
-                }
-                up(a.p, h);
+            const size_t part = std::min<size_t>(Nref, kStagePart);
+            for (size_t i = 0; i < Nref; i += part) {
+                const uint32_t k = uint32_t(std::min(part, Nref - i));
+                const size_t at = i * w, len = size_t(k) * w * sizeof(float);
+                if (!dst)
+                    HIPCHK(hipMemcpyAsync(stage.p, static_cast<const float*>(src) + at, len, hipMemcpyHostToDevice, stream));
+                mps::launch::array_move(dst != nullptr, k, uint32_t(i), w, stride, off, inv.p, a, stage.p, stream);
+                if (dst) HIPCHK(hipMemcpyAsync(static_cast<float*>(dst) + at, stage.p, len, hipMemcpyDeviceToHost, stream));
             }
+            sync();
         };
-        auto fl1 = [&](DBuf<float>& a) {
-            *count = Nref;
-            *eb = 4;
-            if (!(dst || src)) return;
-            if (bytes != size_t(Nref) * 4) throw ApiError{MPS_ERR_INVALID, "size mismatch"};
-            const auto& P = get_perm();
-            std::vector<float> h = down(a.p, N);
-            if (dst) {
-                float* d = static_cast<float*>(dst);
-                for (uint32_t s = 0; s < N; s++)
-                    if (P[s] != mps::dev::kEmpty) d[P[s]] = h[s];
-            } else {
-                const float* q = static_cast<const float*>(src);
-                for (uint32_t s = 0; s < N; s++)
-                    if (P[s] != mps::dev::kEmpty) h[s] = q[P[s]];
-                up(a.p, h);
-            }
+        auto fl4 = [&](DBuf<float4>& a, int comp /* -1 = xyz, 3 = w, 4 = all */) {
+            fl(reinterpret_cast<float*>(a.p), comp == -1 ? 3 : comp == 4 ? 4 : 1, 4, comp == 3 ? 3 : 0);
         };
+        auto fl1 = [&](DBuf<float>& a) { fl(a.p, 1, 1, 0); };
         auto f4xyz = [&](DBuf<float4>& a, uint32_t n) {
             *count = n;
             *eb = 12;
@@ -2494,7 +2462,7 @@ struct mps_ctx {
     ~mps_ctx() {
         pos.release(); vel.release(); color.release(); cgb.release(); cgx.release();
         v3x.release(); v3r.release(); v3Ap.release(); v3p.release(); v3q.release();
-        jprev.release(); for (auto& t : jt) t.release(); jcand.release(); tmp4.release();
+        jprev.release(); for (auto& t : jt) t.release(); jcand.release(); tmp4.release(); stage.release();
         rho.release(); alpha.release(); kappa.release(); delta.release(); fst.release(); tmp1.release();
         pos_alt.release(); vel_alt.release(); color_alt.release(); cgb_alt.release(); rho_alt.release();
         alpha_alt.release(); kappa_alt.release(); delta_alt.release(); fst_alt.release();

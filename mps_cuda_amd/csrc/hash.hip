@@ -373,11 +373,6 @@ __global__ void __launch_bounds__(kBlock) k_relabel(uint32_t* __restrict__ perm,
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s < n && perm[s] != kEmpty) perm[s] = map[perm[s]];
 }
-__global__ void __launch_bounds__(kBlock) k_iota(uint32_t* __restrict__ p, uint32_t n) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n) p[s] = s;
-}
-
 __global__ void __launch_bounds__(kBlock) k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v) {
     const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -1232,9 +1227,6 @@ void invert(const uint32_t* perm, uint32_t n, uint32_t* inv, hipStream_t s) {
 }
 void relabel(uint32_t* perm, const uint32_t* map, uint32_t n, hipStream_t s) {
     if (n) launch_k(k_relabel, nb(n), kBlock, 0, s, perm, map, n);
-}
-void iota(uint32_t* p, uint32_t n, hipStream_t s) {
-    if (n) launch_k(k_iota, nb(n), kBlock, 0, s, p, n);
 }
 void fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s) {
     if (n) launch_k(k_fill_u32, unsigned((n + kBlock - 1) / kBlock), kBlock, 0, s, p, n, v);

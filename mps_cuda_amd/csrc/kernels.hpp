@@ -182,7 +182,6 @@ void fluid_reorder(const uint32_t* key, const uint32_t* id, uint32_t nref, const
                    uint32_t* hash_perm, uint32_t* start, uint32_t* end, const FluidMove& mv, hipStream_t s);
 void invert(const uint32_t* perm, uint32_t n, uint32_t* inv, hipStream_t s);
 void relabel(uint32_t* perm, const uint32_t* map, uint32_t n, hipStream_t s);
-void iota(uint32_t* p, uint32_t n, hipStream_t s);
 void fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s);
 void clear_cells(const uint32_t* key, uint32_t n, uint32_t* start, uint32_t* end, hipStream_t s);
 void cell_table(const uint32_t* key, const uint32_t* id, uint32_t n, uint32_t* start, uint32_t* end, const float4* pos,
@@ -336,6 +335,14 @@ void calib_copy(const float4* a, float4* b, size_t n, hipStream_t s);
 // STREAM-style copy (one 16-byte vector per thread, non-temporal): the in-run copy rate
 void stream_copy(const float4* a, float4* b, size_t n, hipStream_t s);
 void zero_words(uint32_t* p, size_t nwords, hipStream_t s);
+// w floats at `off` of each slot's `stride` (slots) to or from elements [first, first + n) in
+// reference order (staged)
+void array_move(bool out, uint32_t n, uint32_t first, uint32_t w, uint32_t stride, uint32_t off, const uint32_t* inv, float* slots,
+                float* staged, hipStream_t s);
+void fluid_upload(uint32_t n, uint32_t first, const float* xyz, const float* rad, const float* vxyz, const float* mass,
+                  float one_mass, float4* pos, float4* vel, float4* color, uint32_t* perm, uint32_t* inv, hipStream_t s);
+void fluid_reset(uint32_t n, float* rho, float* alpha, float* kappa, float* delta, float* fst, float4* cgb, uint32_t* cff,
+                 uint32_t* cfb, uint32_t* mkey, uint32_t* src, hipStream_t s);
 void pack_readback(uint32_t n, const float4* pos, const float4* color, const uint32_t* perm, float* xyz, float* rad,
                    float* rgba, hipStream_t s);
 void pack_readback_f64(uint32_t n, const float4* pos, const float4* color, const uint32_t* perm, double* xyz, double* rad,
