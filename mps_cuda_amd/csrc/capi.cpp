@@ -298,7 +298,6 @@ struct mps_ctx {
     SolverDev* h_solver = nullptr;
     uint32_t solver_cap = 0;        // scenes the two arrays above hold
     uint32_t* d_active = nullptr;   // [3]: scenes whose DF / CD / CG loop is still running
-    uint32_t* h_active = nullptr;
     mps::GridSync* d_grid = nullptr;  // barrier words of the persistent solver (allocated at creation)
     uint32_t persist_cap[6] = {0, 0, 0, 0, 0, 0};  // co-resident workgroups per kernel variant (0 = not asked yet)
     uint32_t persist_fallbacks = 0;       // persistent solves that gave up and reran chunked
@@ -360,6 +359,7 @@ struct mps_ctx {
         rb_seq++;
     }
     uint32_t pred[3] = {2, 3, 8};
+    uint32_t pred_prev[3] = {0, 0, 0};  // the solves before those
     uint32_t pred_adj = 8;  // iterations of the last transposed solve of the adjoint
     // Iterations enqueued before the next host poll: the predicted count first (the previous
     // solve's), then small chunks, so a solve that runs a little longer than predicted does not
@@ -583,7 +583,7 @@ struct mps_ctx {
         HIPCHK(hipMalloc(reinterpret_cast<void**>(&d_solver), 3 * size_t(S) * sizeof(SolverDev)));
         HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&h_solver), 3 * size_t(S) * sizeof(SolverDev)));
         solver_cap = S;
-        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, stream);
+        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, {}, stream);
     }
     mps::Scenes scn() const { return mps::Scenes{d_params.p, blk_scene.p, N, S}; }
     // bits of the scene index placed above the cell bits of a sort key
@@ -978,18 +978,21 @@ struct mps_ctx {
         for (const SceneHost& h : scenes) n = std::max(n, h.nf);
         return ((scenes.empty() ? N : n) + mps::dev::kBlock - 1) / mps::dev::kBlock;
     }
-    // number of scenes whose loop `idx` is still running
-    uint32_t fetch_active(int idx) {
-        HIPCHK(hipMemcpyAsync(&h_active[idx], &d_active[idx], sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+    // Wait for the records of the loops [first, first + n) and copy them to h_solver.
+    void fetch_records(int first, int n) {
+        HIPCHK(hipMemcpyAsync(h_solver + size_t(first) * S, d_solver + size_t(first) * S, n * size_t(S) * sizeof(SolverDev),
+                              hipMemcpyDeviceToHost, stream));
         sync();
-        return h_active[idx];
     }
-    // Copy the S records of loop `idx` back and return the reference loop variable of each
-    // scene (cap + 1 when it hit the cap), the largest one in *lmax.
-    std::vector<uint32_t> fetch_records(int idx, uint32_t cap, uint32_t* lmax) {
-        SolverDev* h = h_solver + size_t(idx) * S;
-        HIPCHK(hipMemcpyAsync(h, d_solver + size_t(idx) * S, S * sizeof(SolverDev), hipMemcpyDeviceToHost, stream));
-        sync();
+    // Whether loop `idx` has ended in every scene, by the fetched records.
+    bool loop_done(int idx) const {
+        for (uint32_t q = 0; q < S; q++)
+            if (h_solver[size_t(idx) * S + q].done != 1u) return false;
+        return true;
+    }
+    // The reference loop variable of each scene (cap + 1 when it hit the cap), the largest one in *lmax.
+    std::vector<uint32_t> loop_counts(int idx, uint32_t cap, uint32_t* lmax) const {
+        const SolverDev* h = h_solver + size_t(idx) * S;
         std::vector<uint32_t> l(S);
         *lmax = 0;
         for (uint32_t q = 0; q < S; q++) {
@@ -998,26 +1001,44 @@ struct mps_ctx {
         }
         return l;
     }
+    uint32_t loop_it[3] = {1, 1, 1};  // the loops' next iteration to enqueue (DF, CD, CG)
+    void set_pred(int idx, uint32_t l) {
+        pred_prev[idx] = pred[idx];
+        pred[idx] = std::max<uint32_t>(l, 1);
+    }
     // DF / CD loop (MPSSPHDFSPHUtil.cu:270-441)
-    uint32_t pressure_solve(bool df, mps_step_stats* st) {
+    void pressure_solve(bool df, mps_step_stats* st) {
+        if (N == 0) return;
         const int idx = df ? 0 : 1;
-        if (N == 0) return 0;
-        SolverDev* sd = d_solver + size_t(idx) * S;
-        mps::launch::solver_reset(sd, S, d_active + idx, stream);
+        pressure_begin(df, {});
+        do {
+            pressure_chunk(df, pred[idx]);
+            fetch_records(idx, 1);
+        } while (loop_it[idx] <= cfg.max_iter && !loop_done(idx));
+        pressure_end(df, st);
+    }
+    void pressure_begin(bool df, const mps::launch::Gate& gate) {
+        const int idx = df ? 0 : 1;
+        mps::launch::solver_reset(d_solver + size_t(idx) * S, S, d_active + idx, gate, stream);
         ensure_partials();
         ensure_pairs();
         ensure_halo();
+        loop_it[idx] = 1;
+    }
+    void pressure_chunk(bool df, uint32_t predicted) {
+        const int idx = df ? 0 : 1;
+        SolverDev* sd = d_solver + size_t(idx) * S;
         const mps::Scenes P = scn();
         const mps::Halo hl = halo();
         const double tol = df ? cfg.df_tol : cfg.cd_tol;
         const uint32_t lmin = df ? cfg.df_min_iter : cfg.cd_min_iter;
         const uint32_t cap = cfg.max_iter;
-        uint32_t it = 1;
-        bool done = false;
+        uint32_t& it = loop_it[idx];
         const bool fuse = !coupled() && mps::launch::fold_in_consumer(most_blocks());
         const mps::launch::FoldPressure fp{partials.p, d_active + idx, tol, lmin};
-        while (it <= cap && !done) {
-            const uint32_t chunk = chunk_len(it, std::max<uint32_t>(pred[idx], lmin + 1), cap - it + 1);
+        if (it > cap) return;
+        {
+            const uint32_t chunk = chunk_len(it, std::max<uint32_t>(predicted, lmin + 1), cap - it + 1);
             std::vector<uint64_t> key = key_base(df ? 1 : 2, chunk, P, nbr());
             for (const void* q : {(const void*)pos.p, (const void*)vel.p, (const void*)bpos.p, (const void*)bvol.p,
                                   (const void*)bvel.p, (const void*)rho.p, (const void*)alpha.p, (const void*)pairG_ff.p,
@@ -1045,11 +1066,15 @@ struct mps_ctx {
                 }
             });
             it += chunk;
-            done = fetch_active(idx) == 0;
         }
+    }
+    void pressure_end(bool df, mps_step_stats* st) {
+        const int idx = df ? 0 : 1;
+        const uint32_t cap = cfg.max_iter;
+        const bool fuse = !coupled() && mps::launch::fold_in_consumer(most_blocks());
         uint32_t l = 0;
-        const std::vector<uint32_t> ls = fetch_records(idx, cap, &l);
-        pred[idx] = std::max<uint32_t>(l, 1);
+        const std::vector<uint32_t> ls = loop_counts(idx, cap, &l);
+        set_pred(idx, l);
         if (rec) {
             if (df) {
                 rec->ldf = ls;
@@ -1081,17 +1106,26 @@ struct mps_ctx {
                 std::memcpy(log, src, sizeof(double) * MPS_MAX_ITER_LOG);
             }
         }
-        return l;
     }
     // ApplyImplicitViscosityNSurfaceTension + CGSolver (MPSSPHNonPressureUtil.cu:127-188,
     // MPSSolver.cuh:12-73)
-    uint32_t viscosity_cg(mps_step_stats* st) {
-        if (N == 0) return 0;
-        SolverDev* sd = d_solver + 2 * size_t(S);
-        uint32_t* act = d_active + 2;
-        ensure_partials();
-        ensure_pairs();
-        const mps::Scenes P = scn();
+    void viscosity_cg(mps_step_stats* st) {
+        if (N == 0) return;
+        cg_begin({});
+        if (!cg_persistent_run(st)) {
+            do {
+                cg_chunk(pred[2]);
+                fetch_records(2, 1);
+            } while (loop_it[2] <= cfg.cg_max_iter && !loop_done(2));
+        } else {
+            fetch_records(2, 1);
+        }
+        T_(K_COPY_OUT, [&] { mps::launch::copy_vel_out3(scn(), v3x.p, vel.p, {}, stream); });
+        cg_end(st);
+    }
+    // p of iteration k is written to pbuf(k) while pbuf(k - 1) is read; p_0 = r
+    mps::dev::f3* pbuf(uint32_t k) { return (k & 1u) ? v3q.p : v3p.p; }
+    mps::launch::CgOperator cg_operator() {
         const size_t m = std::max<uint32_t>(N, 1);
         mps::launch::CgOperator op;
         op.recompute = cfg.cg_stream_coeffs ? 0 : 1;
@@ -1108,6 +1142,16 @@ struct mps_ctx {
             pairB.reserve(size_t(Kff) * m);
             op.cb = pairB.p;
         }
+        return op;
+    }
+    void cg_begin(const mps::launch::Gate& gate) {
+        SolverDev* sd = d_solver + 2 * size_t(S);
+        uint32_t* act = d_active + 2;
+        ensure_partials();
+        ensure_pairs();
+        const mps::Scenes P = scn();
+        const mps::launch::CgOperator op = cg_operator();
+        const size_t m = std::max<uint32_t>(N, 1);
         v3x.reserve(m); v3r.reserve(m); v3Ap.reserve(m); v3p.reserve(m); v3q.reserve(m);
         ensure_halo();
         const mps::Halo hl = halo();
@@ -1116,23 +1160,33 @@ struct mps_ctx {
             mps::launch::cg_setup(cubic(), P, nbr(), hl, pos.p, vel.p, rho.p, fst.p, pairA.p,
                                   op.recompute ? nullptr : pairB.p, nullptr, nullptr, cgb.p, op.recompute ? irho.p : nullptr, stream);
         });
-        mps::launch::solver_reset(sd, S, act, stream);
-        const double tol = cfg.cg_tol;
-        // p of iteration k is written to pbuf(k) while pbuf(k - 1) is read; p_0 = r
-        auto pbuf = [&](uint32_t k) { return (k & 1u) ? v3q.p : v3p.p; };
+        mps::launch::solver_reset(sd, S, act, gate, stream);
+        cg_start(op, P, hl);
+        loop_it[2] = 1;
+    }
+    void cg_start(const mps::launch::CgOperator& op, const mps::Scenes& P, const mps::Halo& hl) {
+        SolverDev* sd = d_solver + 2 * size_t(S);
         T_(K_CG_INIT, [&] {
             mps::launch::cg_apply(0, op, P, nbr(), hl, pos.p, cgx.p, nullptr, nullptr, pbuf(0), nullptr, cgb.p, v3r.p,
                                   v3x.p, sd, partials.p, nullptr, stream);
         });
-        T_(K_FOLD, [&] { mps::launch::fold_cg(0, P, partials.p, sd, act, tol, stream); });
+        T_(K_FOLD, [&] { mps::launch::fold_cg(0, P, partials.p, sd, d_active + 2, cfg.cg_tol, stream); });
+    }
+    // The whole loop in one cooperative launch; false: not taken, or given up and started again.
+    bool cg_persistent_run(mps_step_stats* st) {
+        if (!cfg.persistent_solver || prof_on) return false;
+        SolverDev* sd = d_solver + 2 * size_t(S);
+        uint32_t* act = d_active + 2;
+        const mps::Scenes P = scn();
+        const mps::Halo hl = halo();
+        const mps::launch::CgOperator op = cg_operator();
+        const double tol = cfg.cg_tol;
         const uint32_t cap = cfg.cg_max_iter;
-        uint32_t it = 1;
-        bool done = false;
         // all iterations in one cooperative launch when every workgroup fits the device at once
         const uint32_t nblk = uint32_t((size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock);
         const int coh = cfg.persistent_solver == 2 ? 1 : 0;
         const int variant = (op.recompute ? (op.cubic ? 1 : 2) : 0) + 3 * coh;
-        if (cfg.persistent_solver && !prof_on && nblk > 0) {
+        if (nblk > 0) {
             if (!persist_cap[variant]) persist_cap[variant] = std::max<uint32_t>(mps::launch::cg_persistent_capacity(op, coh), 1u);
             if (nblk <= persist_cap[variant] && nblk <= mps::kGridGroup * mps::kGridGroups) {
                 mps::launch::zero_words(reinterpret_cast<uint32_t*>(d_grid), sizeof(mps::GridSync) / 4, stream);
@@ -1142,23 +1196,32 @@ struct mps_ctx {
                 mps::GridSync g{};
                 HIPCHK(hipMemcpyAsync(&g, d_grid, sizeof(g), hipMemcpyDeviceToHost, stream));
                 sync();
-                if (!g.gave_up) {
-                    it = cap + 1;  // the launch ran every iteration the loop needed
+                if (!g.gave_up) {  // the launch ran every iteration the loop needed
                     if (st) st->cg_persistent = 1;
-                } else {  // a barrier wait gave up: the whole solve again with chunked launches
-                    persist_fallbacks++;
-                    if (st) st->cg_persistent = 2;
-                    mps::launch::solver_reset(sd, S, act, stream);
-                    T_(K_CG_INIT, [&] {
-                        mps::launch::cg_apply(0, op, P, nbr(), hl, pos.p, cgx.p, nullptr, nullptr, pbuf(0), nullptr, cgb.p,
-                                              v3r.p, v3x.p, sd, partials.p, nullptr, stream);
-                    });
-                    T_(K_FOLD, [&] { mps::launch::fold_cg(0, P, partials.p, sd, act, tol, stream); });
+                    return true;
                 }
+                // a barrier wait gave up: the whole solve again with chunked launches
+                persist_fallbacks++;
+                if (st) st->cg_persistent = 2;
+                mps::launch::solver_reset(sd, S, act, {}, stream);
+                cg_start(op, P, hl);
             }
         }
-        while (it <= cap && !done) {
-            const uint32_t chunk = chunk_len(it, pred[2], cap - it + 1);
+        return false;
+    }
+    void cg_chunk(uint32_t predicted) {
+        SolverDev* sd = d_solver + 2 * size_t(S);
+        uint32_t* act = d_active + 2;
+        const mps::Scenes P = scn();
+        const mps::Halo hl = halo();
+        const mps::launch::CgOperator op = cg_operator();
+        const uint32_t nblk = uint32_t((size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock);
+        const double tol = cfg.cg_tol;
+        const uint32_t cap = cfg.cg_max_iter;
+        uint32_t& it = loop_it[2];
+        if (it > cap) return;
+        {
+            const uint32_t chunk = chunk_len(it, predicted, cap - it + 1);
             std::vector<uint64_t> key = key_base(3, chunk, P, nbr());
             for (const void* q : {(const void*)op.cb, (const void*)op.ca, (const void*)op.vel, (const void*)op.rho,
                                   (const void*)op.irho, (const void*)pos.p, (const void*)pbuf(it - 1), (const void*)pbuf(it),
@@ -1205,18 +1268,19 @@ struct mps_ctx {
                 }
             });
             it += chunk;
-            done = fetch_active(2) == 0;
         }
+    }
+    void cg_end(mps_step_stats* st) {
+        const uint32_t cap = cfg.cg_max_iter;
         uint32_t l = 0;
-        const std::vector<uint32_t> ls = fetch_records(2, cap, &l);
-        pred[2] = std::max<uint32_t>(l, 1);
+        const std::vector<uint32_t> ls = loop_counts(2, cap, &l);
+        set_pred(2, l);
         if (prof_on) {  // A.p (with the direction) and the update ran for iterations 1..l-1
             kuse[K_CG_APPLY] += std::min(l - 1, cap);
             kuse[K_CG_UPDATE] += std::min(l - 1, cap);
-            if ((!cfg.cg_fold_in_kernel || g_no_alloc) && (op.recompute || !mps::launch::fold_in_consumer(most_blocks())))
+            if ((!cfg.cg_fold_in_kernel || g_no_alloc) && (!cfg.cg_stream_coeffs || !mps::launch::fold_in_consumer(most_blocks())))
                 kuse[K_FOLD] += 2 * std::min(l - 1, cap);
         }
-        T_(K_COPY_OUT, [&] { mps::launch::copy_vel_out3(P, v3x.p, vel.p, stream); });
         for (uint32_t q = 0; q < S && q < sstats.size(); q++) {
             mps_step_stats& o = sstats[q];
             const SolverDev& r = h_solver[2 * size_t(S) + q];
@@ -1230,11 +1294,10 @@ struct mps_ctx {
             st->l_cg = l;
             st->hit_cap_cg = l > cap;
         }
-        return l;
     }
     // ApplyImplicitJacobiViscosity (SPHUtil.cu:344-453, commented out in the reference)
-    uint32_t viscosity_jacobi(mps_step_stats* st) {
-        if (N == 0) return 0;
+    void viscosity_jacobi(mps_step_stats* st) {
+        if (N == 0) return;
         if (S > 1) throw ApiError{MPS_ERR_STATE, "the Jacobi viscosity solve runs one scene per context"};
         ensure_partials();
         const mps::Scenes P = scn();
@@ -1300,14 +1363,52 @@ struct mps_ctx {
             st->l_cg = l;
             st->hit_cap_cg = conv ? 0u : 1u;
         }
-        return l;
     }
     void viscosity(mps_step_stats* st) {
         if (cfg.visc_solver == MPS_VISC_CG) viscosity_cg(st);
         else if (cfg.visc_solver == MPS_VISC_JACOBI) viscosity_jacobi(st);
     }
-    void advect() {
-        T_(K_ADVECT, [&] { mps::launch::advect(scn(), pos.p, vel.p, d_flags, stream); });
+    void advect(const mps::launch::Gate& gate = {}) {
+        T_(K_ADVECT, [&] { mps::launch::advect(scn(), pos.p, vel.p, d_flags, gate, stream); });
+    }
+    void fetch_flags() { HIPCHK(hipMemcpyAsync(h_flags, d_flags, 8 * sizeof(uint32_t), hipMemcpyDeviceToHost, stream)); }
+    // The three solves and the advection of a step, enqueued as one with predicted iteration counts and
+    // one wait at the end. Each loop's start and the launches that change the state for good (the
+    // velocities' copy, the advection) are gated on the loop before them having ended; where one had
+    // not, everything after it did nothing, and the host goes on from there. The counts are the larger
+    // of the last two solves': an iteration too many costs launches that exit at once, one too few
+    // the gated rest of the step. A wait per solve leaves the GPU idle for some 10 us each
+    // (33 k particles: 7 waits a step before, 2 now).
+    bool can_run_ahead() const {
+        return N && !rec && cfg.visc_solver == MPS_VISC_CG && !cfg.persistent_solver && !cfg.host_sync_every;
+    }
+    void solve_ahead(mps_step_stats* st) {
+        static constexpr int kOrder[3] = {0, 2, 1};
+        const uint32_t caps[3] = {cfg.max_iter, cfg.max_iter, cfg.cg_max_iter};
+        int first = 0;
+        for (bool begun = false; first < 3; begun = true) {
+            mps::launch::Gate gate;
+            for (int q = first; q < 3; q++) {
+                const int idx = kOrder[q];
+                const uint32_t predicted = std::max(pred[idx], pred_prev[idx]);
+                if (idx == 2) {
+                    if (q > first || !begun) cg_begin(gate);
+                    cg_chunk(predicted);
+                } else {
+                    if (q > first || !begun) pressure_begin(idx == 0, gate);
+                    pressure_chunk(idx == 0, predicted);
+                }
+                gate = {d_solver + size_t(idx) * S, loop_it[idx] <= caps[idx] ? d_active + idx : nullptr};
+                if (idx == 2) T_(K_COPY_OUT, [&] { mps::launch::copy_vel_out3(scn(), v3x.p, vel.p, gate, stream); });
+            }
+            advect(gate);
+            fetch_flags();
+            fetch_records(0, 3);
+            while (first < 3 && (loop_done(kOrder[first]) || loop_it[kOrder[first]] > caps[kOrder[first]])) first++;
+        }
+        pressure_end(true, st);
+        cg_end(st);
+        pressure_end(false, st);
     }
 
     template <class T>
@@ -1405,13 +1506,12 @@ struct mps_ctx {
         const size_t m = std::max<uint32_t>(N, 1);
         const uint32_t nblk = uint32_t((size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock);
         v3x.reserve(m); v3r.reserve(m); v3Ap.reserve(m); v3p.reserve(m); v3q.reserve(m);
-        auto pbuf = [&](uint32_t k) { return (k & 1u) ? v3q.p : v3p.p; };
         mps::launch::CgOperator op;
         op.ca = pairA.p;
         op.cb = pairB.p;
         op.caT = caT.p;
         op.cbT = cbT.p;
-        mps::launch::solver_reset(sd, S, act, stream);
+        mps::launch::solver_reset(sd, S, act, {}, stream);
         if (lam_valid) {
             mps::launch::cg_apply(0, op, P, nb, hl, p0, lam.p, nullptr, nullptr, pbuf(0), nullptr, adv.p, v3r.p, v3x.p, sd, partials.p,
                                   nullptr, stream);
@@ -1422,8 +1522,8 @@ struct mps_ctx {
         }
         const uint32_t cap = cfg.adj_cg_max_iter ? cfg.adj_cg_max_iter : 300u;
         uint32_t it = 1;
-        bool done = fetch_active(2) == 0;
-        // sums folded as in viscosity_cg
+        bool done = false;
+        // sums folded as in cg_chunk
         const bool fuse = mps::launch::fold_in_consumer(most_blocks());
         double* part_rr = fuse ? partials.p + nblk : partials.p;
         const mps::launch::FoldCg fc{part_rr, act, tol};
@@ -1448,10 +1548,11 @@ struct mps_ctx {
                 }
             });
             it += chunk;
-            done = fetch_active(2) == 0;
+            fetch_records(2, 1);
+            done = loop_done(2);
         }
         uint32_t l = 0;
-        (void)fetch_records(2, cap, &l);
+        (void)loop_counts(2, cap, &l);
         pred_adj = std::max<uint32_t>(l, 1);
         lam.reserve(m);
         mps::launch::adj_lambda(P, v3x.p, lam.p, stream);
@@ -1734,8 +1835,7 @@ struct mps_ctx {
         st->n_fluid = Nref;
         st->n_boundary = B;
         const uint32_t regrow0 = nei_regrow;
-        mps::launch::zero_words(d_flags, 1, stream);
-        mps::launch::zero_words(d_flags + 4, 4, stream);
+        mps::launch::zero_words(d_flags, 8, stream);
         if (cfg.zsort_interval && (frame % cfg.zsort_interval) == 1u) {
             zsort();
             st->zsorted = 1;
@@ -1761,17 +1861,21 @@ struct mps_ctx {
         }
         density_alpha(mps::launch::kDoDensity | mps::launch::kDoAlpha | mps::launch::kDoGravity);
         rec_snap();
-        pressure_solve(true, st);
-        viscosity(st);
-        if (rec) {
-            rec_snap();
-            rec->cg_out = rec->nsnap - 1;
+        if (can_run_ahead()) {
+            solve_ahead(st);
+        } else {
+            pressure_solve(true, st);
+            viscosity(st);
+            if (rec) {
+                rec_snap();
+                rec->cg_out = rec->nsnap - 1;
+            }
+            pressure_solve(false, st);
+            advect();
+            if (rec) dcopy(rec->perm_end, perm.p, N);
+            fetch_flags();
+            sync();
         }
-        pressure_solve(false, st);
-        advect();
-        if (rec) dcopy(rec->perm_end, perm.p, N);
-        HIPCHK(hipMemcpyAsync(h_flags, d_flags, 8 * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        sync();
         st->nonfinite = h_flags[0] ? 1u : 0u;
         st->halo_max = h_flags[4];
         st->halo_spill = h_flags[5];
@@ -1846,7 +1950,7 @@ struct mps_ctx {
         solver_cap = kNoAllocScenes;
         d_active = reinterpret_cast<uint32_t*>(base + kScrOffActive);
         // the records keep the last call's contents: start them as a fresh context would
-        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, stream);
+        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, {}, stream);
         step(st);
     }
 
@@ -1876,6 +1980,7 @@ struct mps_ctx {
         drop_rollout();
         frame = 0;
         pred[0] = 2; pred[1] = 3; pred[2] = 8; pred_adj = 8;
+        pred_prev[0] = pred_prev[1] = pred_prev[2] = 0;
         params_dirty = true;
     }
     void alloc_boundary(uint32_t n) {
@@ -2491,7 +2596,6 @@ struct mps_ctx {
         aux4.release(); gvec.release(); avin.release(); abar.release(); rbar.release(); dbar.release(); fbar.release();
         fstr.release(); caT.release(); cbT.release(); acc_mu.release(); acc_sig.release(); lam.release(); lam2.release();
         if (d_active) (void)hipFree(d_active);
-        if (h_active) (void)hipHostFree(h_active);
         for (const Rec& r : recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
         for (hipEvent_t e : evpool) (void)hipEventDestroy(e);
         if (d_ctr) (void)hipFree(d_ctr);
@@ -2654,7 +2758,6 @@ int mps_create(const mps_config* cfg, mps_ctx** out) {
         HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         HIPCHK(hipMalloc(reinterpret_cast<void**>(&c->d_ctr), sizeof(NbrCounters)));
         HIPCHK(hipMalloc(reinterpret_cast<void**>(&c->d_active), 4 * sizeof(uint32_t)));
-        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->h_active), 4 * sizeof(uint32_t)));
         HIPCHK(hipMalloc(reinterpret_cast<void**>(&c->d_flags), 8 * sizeof(uint32_t)));
         HIPCHK(hipMalloc(reinterpret_cast<void**>(&c->d_grid), sizeof(mps::GridSync)));
         HIPCHK(hipMalloc(reinterpret_cast<void**>(&c->d_err3), 4 * sizeof(double)));

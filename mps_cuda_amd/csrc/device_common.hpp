@@ -161,6 +161,11 @@ __device__ __forceinline__ uint32_t grid_zindex(i3 p, const HashGeom& g) {
     return split_by3(x) | (split_by3(y) << 1u) | (split_by3(z) << 2u);
 }
 
+// Whether a launch that was enqueued ahead of its predecessor's end has to do nothing.
+__device__ __forceinline__ bool shut(const launch::Gate& g) {
+    return (g.rec && g.rec->done == kSkipped) || (g.running && *g.running != 0u);
+}
+
 // --------------------------------------------------------------------- wave/block reductions
 // Sum of a double over the wave in every lane, in the order of the butterfly v += v[lane ^ off],
 // off = 32, 16, 8, 4, 2, 1. The first two steps swap half waves and rows of 16 lanes; after them

@@ -48,8 +48,9 @@ struct GridSync {
 };
 // Device-resident state of one iterative solve. The fold kernels finalise the sums here,
 // so the host only needs to look at `done`/`l`.
+constexpr uint32_t kSkipped = 2;  // SolverDev::done of a loop whose predecessor had not finished
 struct SolverDev {
-    uint32_t done;     // loop finished (converged); later kernels of the chunk exit at once
+    uint32_t done;     // loop finished (converged) or skipped; later kernels of the chunk exit at once
     uint32_t l;        // reference loop variable when the loop ended (or next iteration)
     uint32_t counter;  // workgroups of the current launch that arrived (folds in the last workgroup)
     uint32_t it;       // pressure loop: the iteration whose evaluation ran last (folds in the consumer)
@@ -154,6 +155,13 @@ inline void launch_k(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t shm, 
                              : hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, ptrs, shm, s);
     if (rc != hipSuccess) throw LaunchError{rc};  // faults while running surface at the next synchronisation
 }
+
+// What a launch enqueued ahead waits for: it does nothing if the loop before it still runs somewhere
+// (running, null: that loop ends here in any case) or was skipped itself (rec: its first record).
+struct Gate {
+    const SolverDev* rec = nullptr;
+    const uint32_t* running = nullptr;
+};
 
 // ---- hash.hip
 size_t radix_temp_words(uint32_t n);
@@ -318,7 +326,7 @@ void fold_cg(int mode, const Scenes& sc, const double* partials, SolverDev* st, 
 // does fold_cg(1)'s part
 void cg_update3(const Scenes& sc, dev::f3* x, dev::f3* r, const dev::f3* p, const dev::f3* Ap, SolverDev* st,
                 const double* pAp, double* partials, hipStream_t s);
-void copy_vel_out3(const Scenes& sc, const dev::f3* x, float4* vel, hipStream_t s);
+void copy_vel_out3(const Scenes& sc, const dev::f3* x, float4* vel, const Gate& gate, hipStream_t s);
 void copy_vel_out(const Scenes& sc, const float4* x, float4* vel, hipStream_t s);
 void jacobi_candidate(int cubic, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vel,
                       const float* rho, const float4* u, float4* out, hipStream_t s);
@@ -328,9 +336,9 @@ void jacobi_relax(uint32_t N, const float4* cand, const float4* cur, const float
 void jacobi_error(int cubic, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vel,
                   const float* rho, const float4* u0, const float4* u1, const float4* u2, int ncand, double* partials,
                   double* err3, hipStream_t s);
-void advect(const Scenes& sc, float4* pos, float4* vel, uint32_t* nonfinite, hipStream_t s);
+void advect(const Scenes& sc, float4* pos, float4* vel, uint32_t* nonfinite, const Gate& gate, hipStream_t s);
 // resets the S solver records st[0..S) and sets *active = S
-void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, hipStream_t s);
+void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, const Gate& gate, hipStream_t s);
 void calib_copy(const float4* a, float4* b, size_t n, hipStream_t s);
 // STREAM-style copy (one 16-byte vector per thread, non-temporal): the in-run copy rate
 void stream_copy(const float4* a, float4* b, size_t n, hipStream_t s);

@@ -1596,7 +1596,7 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_cg(Scenes sc, const doubl
                                                   uint32_t* active, double tol) {
     const uint32_t sid = blockIdx.x;
     SolverDev* st = stv + sid;
-    if (MODE != 0 && st->done) return;
+    if (st->done) return;
     const StepParams P = sc.P[sid];
     const double s = fold(partials + P.blk0, P.nblk);
     if (threadIdx.x != 0) return;
@@ -1861,7 +1861,9 @@ __global__ void __launch_bounds__(kBlock) k_cg_update3_fold(Scenes sc, f3* __res
     fold_in_last_workgroup<2>(sc, sid, blockIdx.x, partials, st, active, tol, arrive);
 }
 
-__global__ void __launch_bounds__(kBlock) k_copy_vel_out3(Scenes sc, const f3* __restrict__ x, float4* __restrict__ vel) {
+__global__ void __launch_bounds__(kBlock) k_copy_vel_out3(Scenes sc, const f3* __restrict__ x, float4* __restrict__ vel,
+                                                        launch::Gate gate) {
+    if (shut(gate)) return;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= sc.P[sc.blk_scene[blockIdx.x]].end) return;
     const f3 xi = x[i];
@@ -2018,7 +2020,8 @@ __global__ void __launch_bounds__(kBlock) k_fold_partials(const double* __restri
 // ----------------------------------------------------------------- advection
 // BoundaryCollision_kernel + UpdatePosition_kernel (MPSAdvectUtil.cuh:36-77)
 __global__ void __launch_bounds__(kBlock) k_advect(Scenes sc, float4* __restrict__ pos, float4* __restrict__ vel,
-                                                 uint32_t* __restrict__ nonfinite) {
+                                                 uint32_t* __restrict__ nonfinite, launch::Gate gate) {
+    if (shut(gate)) return;
     const uint32_t sid = sc.blk_scene[blockIdx.x];
     const StepParams P = sc.P[sid];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2047,11 +2050,11 @@ __global__ void __launch_bounds__(kBlock) k_advect(Scenes sc, float4* __restrict
 }
 
 // One workgroup per scene: st[blockIdx.x] starts a new loop; *active = S.
-__global__ void k_solver_reset(SolverDev* stv, uint32_t S, uint32_t* active) {
+__global__ void k_solver_reset(SolverDev* stv, uint32_t S, uint32_t* active, launch::Gate gate) {
     SolverDev* st = stv + blockIdx.x;
     const uint32_t t = threadIdx.x;
     if (t == 0) {
-        st->done = 0u;
+        st->done = shut(gate) ? kSkipped : 0u;
         st->l = 1u;
         st->counter = 0u;
         st->rr = 0.0;
@@ -2402,8 +2405,8 @@ void cg_update3(const Scenes& sc, f3* x, f3* r, const f3* p, const f3* Ap, Solve
 // 14.1 ms, 1006 24.5 -> 22.8, 2051 33.8 -> 34.3, 3907 65.7 -> 68.4 (there A.p 73.0 -> 79.8 us and
 // the update 11.4 -> 15.5, against two fold launches of 4.0).
 bool fold_in_consumer(uint32_t most_blocks) { return most_blocks <= 1536; }
-void copy_vel_out3(const Scenes& sc, const f3* x, float4* vel, hipStream_t s) {
-    if (sc.N) launch_k(k_copy_vel_out3, nb_(sc.N), kBlock, 0, s, sc, x, vel);
+void copy_vel_out3(const Scenes& sc, const f3* x, float4* vel, const Gate& gate, hipStream_t s) {
+    if (sc.N) launch_k(k_copy_vel_out3, nb_(sc.N), kBlock, 0, s, sc, x, vel, gate);
 }
 void copy_vel_out(const Scenes& sc, const float4* x, float4* vel, hipStream_t s) {
     if (sc.N) launch_k(k_copy_vel_out, nb_(sc.N), kBlock, 0, s, sc, x, vel);
@@ -2427,11 +2430,11 @@ void jacobi_error(int cubic, const Scenes& sc, const Nbr& nb, const float4* pos,
     else launch_k(k_jacobi_error<false>, g, kBlock, 0, s, sc, nb, pos, vel, rho, u0, u1, u2, ncand, partials);
     launch_k(k_fold_partials, 1, kBlock, 0, s, partials, g, ncand, err3);
 }
-void advect(const Scenes& sc, float4* pos, float4* vel, uint32_t* nonfinite, hipStream_t s) {
-    if (sc.N) launch_k(k_advect, nb_(sc.N), kBlock, 0, s, sc, pos, vel, nonfinite);
+void advect(const Scenes& sc, float4* pos, float4* vel, uint32_t* nonfinite, const Gate& gate, hipStream_t s) {
+    if (sc.N) launch_k(k_advect, nb_(sc.N), kBlock, 0, s, sc, pos, vel, nonfinite, gate);
 }
-void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, hipStream_t s) {
-    if (S) launch_k(k_solver_reset, S, kBlock, 0, s, st, S, active);
+void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, const Gate& gate, hipStream_t s) {
+    if (S) launch_k(k_solver_reset, S, kBlock, 0, s, st, S, active, gate);
 }
 void calib_copy(const float4* a, float4* b, size_t n, hipStream_t s) {
     if (n) launch_k(k_calib_copy, 4096, kBlock, 0, s, a, b, n);
