@@ -173,8 +173,12 @@ struct mps_ctx {
     };
     struct StagedScene {
         SceneHost h;
-        std::vector<float> pos, vel, rad, mass, bpos, brad, bmass;
+        mps::launch::SceneSource src;
     };
+    // the added scenes' arrays, back to back; the memory stays for the next batch up to kArenaKeep floats
+    static constexpr size_t kArenaKeep = size_t(1) << 24;
+    std::vector<float> arena;
+    DBuf<mps::launch::SceneSource> d_source;
     std::vector<SceneHost> scenes;      // batch layout; empty = one scene made of everything uploaded
     std::vector<StagedScene> staged;    // scenes added since the last commit
     std::vector<mps_step_stats> sstats; // per-scene statistics of the last step
@@ -2018,6 +2022,7 @@ struct mps_ctx {
         sync();
         drop_rollout();
         staged.clear();
+        arena.clear();
         scenes.clear();
         sstats.clear();
         N = Nref = B = 0;
@@ -2041,14 +2046,21 @@ struct mps_ctx {
         sc.h.mass = mt.density * sc.h.V;
         sc.h.nf = uint32_t(nf);
         sc.h.nb = uint32_t(nb);
-        sc.pos.assign(p, p + 3 * nf);
-        sc.rad.assign(r, r + nf);
-        sc.vel = v ? std::vector<float>(v, v + 3 * nf) : std::vector<float>(3 * nf, 0.0f);
-        sc.mass = m ? std::vector<float>(m, m + nf) : std::vector<float>(nf, float(sc.h.mass));
+        auto put = [&](const float* a, size_t n) -> uint64_t {
+            if (!a) return mps::launch::kNoArray;
+            const uint64_t at = arena.size();
+            arena.insert(arena.end(), a, a + n);
+            return at;
+        };
+        sc.src.pos = put(p, 3 * nf);
+        sc.src.rad = put(r, nf);
+        sc.src.vel = put(v, 3 * nf);
+        sc.src.mass = put(m, nf);
+        sc.src.one_mass = float(sc.h.mass);
         if (nb) {
-            sc.bpos.assign(bp, bp + 3 * nb);
-            sc.brad.assign(br, br + nb);
-            sc.bmass = bm ? std::vector<float>(bm, bm + nb) : std::vector<float>(nb, 0.0f);
+            sc.src.bpos = put(bp, 3 * nb);
+            sc.src.brad = put(br, nb);
+            sc.src.bmass = put(bm, nb);
         }
         staged.push_back(std::move(sc));
     }
@@ -2084,43 +2096,32 @@ struct mps_ctx {
         nbobj = 1;
         alloc_fluid(N);
         alloc_boundary(B);
-        std::vector<float4> hp(N, make_float4(0.f, 0.f, 0.f, 0.f)), hv(N, make_float4(0.f, 0.f, 0.f, 0.f));
-        std::vector<float4> hc(N, make_float4(0.f, 0.f, 1.f, 1.f));
-        std::vector<uint32_t> hperm(N, mps::dev::kEmpty), hinv(std::max<uint32_t>(Nref, 1)), hbs(std::max<uint32_t>(B, 1), 0u);
-        std::vector<float4> hbp(std::max<uint32_t>(B, 1)), hbv(std::max<uint32_t>(B, 1));
         const size_t nblk = std::max<size_t>((size_t(N) + blk - 1) / blk, 1);
         std::vector<uint32_t> hblk(nblk, 0u), hdelta(nsc);
+        std::vector<mps::launch::SceneSource> hsrc(nsc);
         for (uint32_t q = 0; q < nsc; q++) {
             const SceneHost& h = lay[q];
-            const StagedScene& sc = staged[q];
-            for (uint32_t i = 0; i < h.nf; i++) {
-                const uint32_t sl = h.begin + i;
-                hp[sl] = make_float4(sc.pos[3 * i], sc.pos[3 * i + 1], sc.pos[3 * i + 2], sc.rad[i]);
-                hv[sl] = make_float4(sc.vel[3 * i], sc.vel[3 * i + 1], sc.vel[3 * i + 2], sc.mass[i]);
-                hperm[sl] = h.ref0 + i;
-                hinv[h.ref0 + i] = sl;
-            }
+            hsrc[q] = staged[q].src;
+            hsrc[q].begin = h.begin;
+            hsrc[q].nf = h.nf;
+            hsrc[q].ref0 = h.ref0;
+            hsrc[q].b0 = h.b0;
             for (uint32_t b = h.begin / blk; b < (h.begin + h.nf + blk - 1) / blk; b++) hblk[b] = q;
             hdelta[q] = h.begin - h.ref0;
-            for (uint32_t i = 0; i < h.nb; i++) {
-                hbp[h.b0 + i] = make_float4(sc.bpos[3 * i], sc.bpos[3 * i + 1], sc.bpos[3 * i + 2], sc.brad[i]);
-                hbv[h.b0 + i] = make_float4(0.f, 0.f, 0.f, sc.bmass[i]);
-                hbs[h.b0 + i] = q;
-            }
         }
         blk_scene.reserve(nblk);
         d_delta.reserve(nsc);
+        d_source.reserve(nsc);
         bscene.reserve(std::max<uint32_t>(B, 1));
-        up(pos.p, hp); up(vel.p, hv); up(color.p, hc); up(perm.p, hperm); up(inv.p, hinv);
-        up(blk_scene.p, hblk); up(d_delta.p, hdelta);
-        if (B) {
-            up(bpos.p, hbp); up(bvel.p, hbv); up(bscene.p, hbs);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(bcolor.p), 4 * size_t(B), stream);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(bvol.p), B, stream);
-            mps::launch::zero_words(bface.p, B, stream);
-            mps::launch::zero_words(reinterpret_cast<uint32_t*>(bbcc.p), 2 * size_t(B), stream);
-            mps::launch::zero_words(cbb.p, B, stream);
-        }
+        stage.reserve(arena.size());
+        auto put = [&](void* d, const void* a, size_t bytes) { HIPCHK(hipMemcpyAsync(d, a, bytes, hipMemcpyHostToDevice, stream)); };
+        put(blk_scene.p, hblk.data(), nblk * sizeof(uint32_t));
+        put(d_delta.p, hdelta.data(), nsc * sizeof(uint32_t));
+        put(d_source.p, hsrc.data(), nsc * sizeof(mps::launch::SceneSource));
+        put(stage.p, arena.data(), arena.size() * sizeof(float));
+        mps::launch::batch_upload(N, stage.p, d_source.p, blk_scene.p, pos.p, vel.p, color.p, perm.p, inv.p, stream);
+        mps::launch::batch_upload_walls(B, nsc, stage.p, d_source.p, bpos.p, bvel.p, bscene.p, bcolor.p, bvol.p, bface.p, bbcc.p, cbb.p,
+                                        stream);
         scenes = lay;
         S = nsc;
         staged.clear();
@@ -2130,6 +2131,12 @@ struct mps_ctx {
         reset_fluid_state(N);
         sstats.clear();
         sync();
+        arena.clear();
+        if (arena.capacity() > kArenaKeep) std::vector<float>().swap(arena);
+        if (stage.cap > 8 * kStagePart) {
+            stage.release();
+            stage.reserve(8 * std::min<size_t>(N, kStagePart));
+        }
     }
     void upload_boundary(size_t n, const float* p, const float* r, const float* m) {
         if (n > 0x7FFFFFFFu) throw ApiError{MPS_ERR_INVALID, "too many particles"};
@@ -2567,7 +2574,7 @@ struct mps_ctx {
     ~mps_ctx() {
         pos.release(); vel.release(); color.release(); cgb.release(); cgx.release();
         v3x.release(); v3r.release(); v3Ap.release(); v3p.release(); v3q.release();
-        jprev.release(); for (auto& t : jt) t.release(); jcand.release(); tmp4.release(); stage.release();
+        jprev.release(); for (auto& t : jt) t.release(); jcand.release(); tmp4.release(); stage.release(); d_source.release();
         rho.release(); alpha.release(); kappa.release(); delta.release(); fst.release(); tmp1.release();
         pos_alt.release(); vel_alt.release(); color_alt.release(); cgb_alt.release(); rho_alt.release();
         alpha_alt.release(); kappa_alt.release(); delta_alt.release(); fst_alt.release();

@@ -349,6 +349,17 @@ void array_move(bool out, uint32_t n, uint32_t first, uint32_t w, uint32_t strid
                 float* staged, hipStream_t s);
 void fluid_upload(uint32_t n, uint32_t first, const float* xyz, const float* rad, const float* vxyz, const float* mass,
                   float one_mass, float4* pos, float4* vel, float4* color, uint32_t* perm, uint32_t* inv, hipStream_t s);
+// Where a scene's arrays lie in the staged floats (kNoArray: not given), and its place in the batch.
+constexpr uint64_t kNoArray = ~uint64_t(0);
+struct SceneSource {
+    uint64_t pos = kNoArray, rad = kNoArray, vel = kNoArray, mass = kNoArray, bpos = kNoArray, brad = kNoArray, bmass = kNoArray;
+    uint32_t begin = 0, nf = 0, ref0 = 0, b0 = 0;
+    float one_mass = 0.0f;
+};
+void batch_upload(uint32_t N, const float* staged, const SceneSource* src, const uint32_t* blk_scene, float4* pos, float4* vel,
+                  float4* color, uint32_t* perm, uint32_t* inv, hipStream_t s);
+void batch_upload_walls(uint32_t B, uint32_t S, const float* staged, const SceneSource* src, float4* bpos, float4* bvel,
+                        uint32_t* bscene, float4* bcolor, float* bvol, uint32_t* bface, float2* bbcc, uint32_t* cbb, hipStream_t s);
 void fluid_reset(uint32_t n, float* rho, float* alpha, float* kappa, float* delta, float* fst, float4* cgb, uint32_t* cff,
                  uint32_t* cfb, uint32_t* mkey, uint32_t* src, hipStream_t s);
 void pack_readback(uint32_t n, const float4* pos, const float4* color, const uint32_t* perm, float* xyz, float* rad,

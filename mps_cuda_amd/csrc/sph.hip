@@ -2122,6 +2122,62 @@ __global__ void __launch_bounds__(kBlock) k_fluid_upload(uint32_t n, uint32_t fi
     perm[i] = i;
     inv[i] = i;
 }
+// The fluid of a batch of scenes from their staged arrays: slot s of scene q is its particle s - begin;
+// the slots from a scene's end to its last workgroup's are padding (perm kEmpty). Packing the records
+// on the host and copying 56 bytes per particle took 12 scenes of 370 k particles 2.0 ms.
+__global__ void __launch_bounds__(kBlock) k_batch_upload(uint32_t N, const float* __restrict__ staged,
+                                                       const launch::SceneSource* __restrict__ src,
+                                                       const uint32_t* __restrict__ blk_scene, float4* __restrict__ pos,
+                                                       float4* __restrict__ vel, float4* __restrict__ color,
+                                                       uint32_t* __restrict__ perm, uint32_t* __restrict__ inv) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    if (s >= N) return;
+    const launch::SceneSource q = src[blk_scene[blockIdx.x]];
+    const uint32_t i = s - q.begin;
+    float4 p = make_float4(0.f, 0.f, 0.f, 0.f), v = p;
+    uint32_t ref = kEmpty;
+    if (i < q.nf) {
+        const float* a = staged + q.pos + 3 * size_t(i);
+        p = make_float4(a[0], a[1], a[2], staged[q.rad + i]);
+        if (q.vel != launch::kNoArray) {
+            const float* u = staged + q.vel + 3 * size_t(i);
+            v = make_float4(u[0], u[1], u[2], 0.f);
+        }
+        v.w = q.mass != launch::kNoArray ? staged[q.mass + i] : q.one_mass;
+        ref = q.ref0 + i;
+        inv[ref] = s;
+    }
+    pos[s] = p;
+    vel[s] = v;
+    color[s] = make_float4(0.f, 0.f, 1.f, 1.f);
+    perm[s] = ref;
+}
+// Their walls: wall b belongs to the last scene whose walls start at or before b.
+__global__ void __launch_bounds__(kBlock) k_batch_upload_walls(uint32_t B, uint32_t S, const float* __restrict__ staged,
+                                                             const launch::SceneSource* __restrict__ src, float4* __restrict__ bpos,
+                                                             float4* __restrict__ bvel, uint32_t* __restrict__ bscene,
+                                                             float4* __restrict__ bcolor, float* __restrict__ bvol,
+                                                             uint32_t* __restrict__ bface, float2* __restrict__ bbcc,
+                                                             uint32_t* __restrict__ cbb) {
+    const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
+    if (b >= B) return;
+    uint32_t lo = 0, hi = S;  // src[lo].b0 <= b < src[hi].b0
+    while (hi - lo > 1u) {
+        const uint32_t mid = (lo + hi) / 2u;
+        if (src[mid].b0 <= b) lo = mid;
+        else hi = mid;
+    }
+    const launch::SceneSource q = src[lo];
+    const uint32_t i = b - q.b0;
+    const float* a = staged + q.bpos + 3 * size_t(i);
+    bpos[b] = make_float4(a[0], a[1], a[2], staged[q.brad + i]);
+    bvel[b] = make_float4(0.f, 0.f, 0.f, q.bmass != launch::kNoArray ? staged[q.bmass + i] : 0.f);
+    bscene[b] = lo;
+    bcolor[b] = make_float4(0.f, 0.f, 0.f, 0.f);
+    bvol[b] = 0.f;
+    bface[b] = cbb[b] = 0u;
+    bbcc[b] = make_float2(0.f, 0.f);
+}
 // Derived state of a new fluid: zero; mkey and src kEmpty.
 __global__ void __launch_bounds__(kBlock) k_fluid_reset(uint32_t n, float* __restrict__ rho, float* __restrict__ alpha,
                                                       float* __restrict__ kappa, float* __restrict__ delta,
@@ -2454,6 +2510,14 @@ void array_move(bool out, uint32_t n, uint32_t first, uint32_t w, uint32_t strid
 void fluid_upload(uint32_t n, uint32_t first, const float* xyz, const float* rad, const float* vxyz, const float* mass,
                   float one_mass, float4* pos, float4* vel, float4* color, uint32_t* perm, uint32_t* inv, hipStream_t s) {
     if (n) launch_k(k_fluid_upload, nb_(n), kBlock, 0, s, n, first, xyz, rad, vxyz, mass, one_mass, pos, vel, color, perm, inv);
+}
+void batch_upload(uint32_t N, const float* staged, const SceneSource* src, const uint32_t* blk_scene, float4* pos, float4* vel,
+                  float4* color, uint32_t* perm, uint32_t* inv, hipStream_t s) {
+    if (N) launch_k(k_batch_upload, nb_(N), kBlock, 0, s, N, staged, src, blk_scene, pos, vel, color, perm, inv);
+}
+void batch_upload_walls(uint32_t B, uint32_t S, const float* staged, const SceneSource* src, float4* bpos, float4* bvel,
+                        uint32_t* bscene, float4* bcolor, float* bvol, uint32_t* bface, float2* bbcc, uint32_t* cbb, hipStream_t s) {
+    if (B) launch_k(k_batch_upload_walls, nb_(B), kBlock, 0, s, B, S, staged, src, bpos, bvel, bscene, bcolor, bvol, bface, bbcc, cbb);
 }
 void fluid_reset(uint32_t n, float* rho, float* alpha, float* kappa, float* delta, float* fst, float4* cgb, uint32_t* cff,
                  uint32_t* cfb, uint32_t* mkey, uint32_t* src, hipStream_t s) {
