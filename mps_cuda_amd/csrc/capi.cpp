@@ -596,7 +596,7 @@ struct mps_ctx {
         HIPCHK(hipMalloc(reinterpret_cast<void**>(&d_solver), 3 * size_t(S) * sizeof(SolverDev)));
         HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&h_solver), 3 * size_t(S) * sizeof(SolverDev)));
         solver_cap = S;
-        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, {}, stream);
+        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, stream);
     }
     mps::Scenes scn() const { return mps::Scenes{d_params.p, blk_scene.p, N, S}; }
     // bits of the scene index placed above the cell bits of a sort key
@@ -827,7 +827,7 @@ struct mps_ctx {
 
     void reset_counters() { mps::launch::zero_words(reinterpret_cast<uint32_t*>(d_ctr), sizeof(NbrCounters) / 4, stream); }
 
-    void neighbors() {
+    void neighbors(bool cleared = false) {  // cleared: the counters are zero
         const HashGeom g = geom();
         // capacities rounded to a multiple of 4
         if (Kff == 0) Kff = (std::max<uint32_t>(cfg.nei_capacity, 8) + 3u) & ~3u;
@@ -835,7 +835,7 @@ struct mps_ctx {
         if (Kbb == 0) Kbb = (std::max<uint32_t>(cfg.nei_capacity / 2, 8) + 3u) & ~3u;
         if (Kfr == 0) Kfr = (std::max<uint32_t>(cfg.nei_capacity / 2, 8) + 3u) & ~3u;
         for (int attempt = 0; attempt < 8; attempt++) {
-            reset_counters();
+            if (attempt || !cleared) reset_counters();
             nstat.reserve(2 * ((size_t(std::max(N, B)) + mps::dev::kBlock - 1) / mps::dev::kBlock) + 2);
             const bool do_b = bnd_dirty;
             if (do_b && B) {
@@ -1023,16 +1023,17 @@ struct mps_ctx {
     void pressure_solve(bool df, mps_step_stats* st) {
         if (N == 0) return;
         const int idx = df ? 0 : 1;
-        pressure_begin(df, {});
+        pressure_begin(df, false);
         do {
             pressure_chunk(df, pred[idx]);
             fetch_records(idx, 1);
         } while (loop_it[idx] <= cfg.max_iter && !loop_done(idx));
         pressure_end(df, st);
     }
-    void pressure_begin(bool df, const mps::launch::Gate& gate) {
+    // `reset`: an earlier launch has reset the records
+    void pressure_begin(bool df, bool reset) {
         const int idx = df ? 0 : 1;
-        mps::launch::solver_reset(d_solver + size_t(idx) * S, S, d_active + idx, gate, stream);
+        if (!reset) mps::launch::solver_reset(d_solver + size_t(idx) * S, S, d_active + idx, stream);
         ensure_partials();
         ensure_pairs();
         ensure_halo();
@@ -1133,7 +1134,7 @@ struct mps_ctx {
         } else {
             fetch_records(2, 1);
         }
-        T_(K_COPY_OUT, [&] { mps::launch::copy_vel_out3(scn(), v3x.p, vel.p, {}, stream); });
+        T_(K_COPY_OUT, [&] { mps::launch::copy_vel_out3(scn(), v3x.p, vel.p, {}, {}, stream); });
         cg_end(st);
     }
     // p of iteration k is written to pbuf(k) while pbuf(k - 1) is read; p_0 = r
@@ -1168,12 +1169,13 @@ struct mps_ctx {
         v3x.reserve(m); v3r.reserve(m); v3Ap.reserve(m); v3p.reserve(m); v3q.reserve(m);
         ensure_halo();
         const mps::Halo hl = halo();
-        T_(K_ST_FACTOR, [&] { mps::launch::st_factor(P, nbr(), hl, pos.p, vel.p, pairG_ff.p, fst.p, cgx.p, stream); });
+        T_(K_ST_FACTOR, [&] {
+            mps::launch::st_factor(P, nbr(), hl, pos.p, vel.p, pairG_ff.p, fst.p, cgx.p, {sd, act, gate}, stream);
+        });
         T_(K_CG_SETUP, [&] {
             mps::launch::cg_setup(cubic(), P, nbr(), hl, pos.p, vel.p, rho.p, fst.p, pairA.p,
                                   op.recompute ? nullptr : pairB.p, nullptr, nullptr, cgb.p, op.recompute ? irho.p : nullptr, stream);
         });
-        mps::launch::solver_reset(sd, S, act, gate, stream);
         cg_start(op, P, hl);
         loop_it[2] = 1;
     }
@@ -1216,7 +1218,7 @@ struct mps_ctx {
                 // a barrier wait gave up: the whole solve again with chunked launches
                 persist_fallbacks++;
                 if (st) st->cg_persistent = 2;
-                mps::launch::solver_reset(sd, S, act, {}, stream);
+                mps::launch::solver_reset(sd, S, act, stream);
                 cg_start(op, P, hl);
             }
         }
@@ -1408,11 +1410,15 @@ struct mps_ctx {
                     if (q > first || !begun) cg_begin(gate);
                     cg_chunk(predicted);
                 } else {
-                    if (q > first || !begun) pressure_begin(idx == 0, gate);
+                    // (the density solve's records: by the velocities' copy, the first loop's by the step's start)
+                    if (q > first || !begun) pressure_begin(idx == 0, true);
                     pressure_chunk(idx == 0, predicted);
                 }
                 gate = {d_solver + size_t(idx) * S, loop_it[idx] <= caps[idx] ? d_active + idx : nullptr};
-                if (idx == 2) T_(K_COPY_OUT, [&] { mps::launch::copy_vel_out3(scn(), v3x.p, vel.p, gate, stream); });
+                if (idx == 2)
+                    T_(K_COPY_OUT, [&] {
+                        mps::launch::copy_vel_out3(scn(), v3x.p, vel.p, gate, {d_solver + size_t(S), d_active + 1, gate}, stream);
+                    });
             }
             advect(gate);
             fetch_flags();
@@ -1543,7 +1549,7 @@ struct mps_ctx {
         op.cb = pairB.p;
         op.caT = caT.p;
         op.cbT = cbT.p;
-        mps::launch::solver_reset(sd, S, act, {}, stream);
+        mps::launch::solver_reset(sd, S, act, stream);
         if (lam_valid) {
             mps::launch::cg_apply(0, op, P, nb, hl, p0, lam.p, nullptr, nullptr, pbuf(0), nullptr, adv.p, v3r.p, v3x.p, sd, partials.p,
                                   nullptr, stream);
@@ -1632,7 +1638,7 @@ struct mps_ctx {
             const float4* vst = T.snaps[T.cg_out].p;
             pairA.reserve(size_t(T.Kff) * m); pairB.reserve(size_t(T.Kff) * m);
             caT.reserve(size_t(T.Kff) * m); cbT.reserve(size_t(T.Kff) * m);
-            mps::launch::st_factor(P, nb, hl, T.pos.p, vin, pairG_ff.p, fstr.p, cgx.p, stream);
+            mps::launch::st_factor(P, nb, hl, T.pos.p, vin, pairG_ff.p, fstr.p, cgx.p, {}, stream);
             mps::launch::cg_setup(cubic(), P, nb, hl, T.pos.p, vin, rho.p, fstr.p, pairA.p, pairB.p, caT.p, cbT.p, cgb.p, nullptr,
                                   stream);
             adj_solveT(nb, hl, T.pos.p);
@@ -1864,13 +1870,13 @@ struct mps_ctx {
         st->n_fluid = Nref;
         st->n_boundary = B;
         const uint32_t regrow0 = nei_regrow;
-        mps::launch::zero_words(d_flags, 8, stream);
+        mps::launch::step_begin(d_solver, S, d_active, d_flags, 8, d_ctr, stream);
         if (cfg.zsort_interval && (frame % cfg.zsort_interval) == 1u) {
             zsort();
             st->zsorted = 1;
         }
         hash();
-        neighbors();
+        neighbors(true);
         boundary_volume();
         if (rec) {
             rec->Kff = Kff;
@@ -1979,7 +1985,7 @@ struct mps_ctx {
         solver_cap = kNoAllocScenes;
         d_active = reinterpret_cast<uint32_t*>(base + kScrOffActive);
         // the records keep the last call's contents: start them as a fresh context would
-        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, {}, stream);
+        for (int k = 0; k < 3; k++) mps::launch::solver_reset(d_solver + size_t(k) * S, S, d_active + k, stream);
         step(st);
     }
 

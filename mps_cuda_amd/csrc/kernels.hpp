@@ -163,6 +163,13 @@ struct Gate {
     const uint32_t* running = nullptr;
 };
 
+// A loop whose records a launch before it resets (rec null: none), gated on the loop before that.
+struct LoopStart {
+    SolverDev* rec = nullptr;
+    uint32_t* active = nullptr;
+    Gate gate;
+};
+
 // ---- hash.hip
 size_t radix_temp_words(uint32_t n);
 int radix_sort(uint32_t*& keys, uint32_t*& vals, uint32_t*& keys_alt, uint32_t*& vals_alt, uint32_t* temp, uint32_t n,
@@ -260,7 +267,7 @@ void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, 
 // Whether the consumers of a solver's sums fold them themselves (one launch less per sum).
 bool fold_in_consumer(uint32_t most_blocks);
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
-               float4* cgx, hipStream_t s);
+               float4* cgx, const LoopStart& ls, hipStream_t s);
 // pair coefficients of the implicit operator: a_ij into ca, b_ij into cb (may be null); with caT and
 // cbT also the pair seen from the neighbour (a_ji, b_ji), for the transposed operator
 void cg_setup(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* rho,
@@ -326,7 +333,7 @@ void fold_cg(int mode, const Scenes& sc, const double* partials, SolverDev* st, 
 // does fold_cg(1)'s part
 void cg_update3(const Scenes& sc, dev::f3* x, dev::f3* r, const dev::f3* p, const dev::f3* Ap, SolverDev* st,
                 const double* pAp, double* partials, hipStream_t s);
-void copy_vel_out3(const Scenes& sc, const dev::f3* x, float4* vel, const Gate& gate, hipStream_t s);
+void copy_vel_out3(const Scenes& sc, const dev::f3* x, float4* vel, const Gate& gate, const LoopStart& ls, hipStream_t s);
 void copy_vel_out(const Scenes& sc, const float4* x, float4* vel, hipStream_t s);
 void jacobi_candidate(int cubic, const Scenes& sc, const Nbr& nb, const float4* pos, const float4* vel,
                       const float* rho, const float4* u, float4* out, hipStream_t s);
@@ -338,7 +345,9 @@ void jacobi_error(int cubic, const Scenes& sc, const Nbr& nb, const float4* pos,
                   double* err3, hipStream_t s);
 void advect(const Scenes& sc, float4* pos, float4* vel, uint32_t* nonfinite, const Gate& gate, hipStream_t s);
 // resets the S solver records st[0..S) and sets *active = S
-void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, const Gate& gate, hipStream_t s);
+// flags: nf <= 256 words
+void step_begin(SolverDev* st, uint32_t S, uint32_t* active, uint32_t* flags, uint32_t nf, NbrCounters* ctr, hipStream_t s);
+void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, hipStream_t s);
 void calib_copy(const float4* a, float4* b, size_t n, hipStream_t s);
 // STREAM-style copy (one 16-byte vector per thread, non-temporal): the in-run copy rate
 void stream_copy(const float4* a, float4* b, size_t n, hipStream_t s);

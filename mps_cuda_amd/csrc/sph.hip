@@ -752,6 +752,28 @@ __global__ void __launch_bounds__(Q * kBlock) k_density_alpha(int flags, Scenes 
 }
 
 // ----------------------------------------------------------------- pressure solves
+// The start of a loop: its record, by all threads of a workgroup. skip: the loop before it has not ended.
+__device__ __forceinline__ void reset_record(SolverDev* st, bool skip) {
+    if (threadIdx.x == 0) {
+        st->done = skip ? kSkipped : 0u;
+        st->l = 1u;
+        st->counter = 0u;
+        st->rr = 0.0;
+        st->pAp = 0.0;
+        st->thr = 0.0;
+        st->alpha = 0.0f;
+        st->beta = 0.0f;
+    }
+    for (uint32_t k = threadIdx.x; k < MPS_MAX_ITER_LOG; k += blockDim.x) st->log[k] = 0.0;
+}
+// The same by a launch over the fluid's workgroups that runs before the loop: each scene's first
+// workgroup resets the scene's record (a launch of its own took 2.5 us and a gap, four a step).
+__device__ __forceinline__ void reset_records(const launch::LoopStart& ls, const Scenes& sc, uint32_t blk, uint32_t sid) {
+    if (!ls.rec || blk != sc.P[sid].blk0) return;
+    reset_record(ls.rec + sid, shut(ls.gate));
+    if (blk == 0u && threadIdx.x == 0) *ls.active = sc.S;
+}
+
 // ComputeDensityDelta_kernel ff/fb (MPSSPHDFSPHUtil.cuh:139-257) fused with
 // ComputeDFStiffness_kernel / ComputeCDStiffness_kernel (:259-340); G_ij comes from the
 // alpha pass. Each workgroup publishes its sum of positive errors for k_fold_pressure.
@@ -1107,7 +1129,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_apply(Scenes sc, Nbr nb
 template <int Q>
 __global__ void __launch_bounds__(Q * kBlock) k_st_factor(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                     const float4* __restrict__ vel, const float* __restrict__ pG_ff,
-                                                    float* __restrict__ fst, float4* __restrict__ cgx) {
+                                                    float* __restrict__ fst, float4* __restrict__ cgx, launch::LoopStart ls) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t N = sc.N;
     // the block's halo (x_j, v_j, m_j) in LDS (see k_cg_apply)
@@ -1117,7 +1139,9 @@ __global__ void __launch_bounds__(Q * kBlock) k_st_factor(Scenes sc, Nbr nb, Hal
     const bool in = i < N;
     const float4 xi4 = in ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float4 vi4 = in ? vel[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const bool live = i < sc.P[sc.blk_scene[blk]].end;
+    const uint32_t sid = sc.blk_scene[blk];
+    reset_records(ls, sc, blk, sid);
+    const bool live = i < sc.P[sid].end;
     const f3 xi = mk(xi4), vi = mk(vi4);
     float d = 0.0f;
     using Val = GroupVal<Q>;
@@ -1862,10 +1886,12 @@ __global__ void __launch_bounds__(kBlock) k_cg_update3_fold(Scenes sc, f3* __res
 }
 
 __global__ void __launch_bounds__(kBlock) k_copy_vel_out3(Scenes sc, const f3* __restrict__ x, float4* __restrict__ vel,
-                                                        launch::Gate gate) {
+                                                        launch::Gate gate, launch::LoopStart ls) {
+    const uint32_t sid = sc.blk_scene[blockIdx.x];
+    reset_records(ls, sc, blockIdx.x, sid);
     if (shut(gate)) return;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= sc.P[sc.blk_scene[blockIdx.x]].end) return;
+    if (i >= sc.P[sid].end) return;
     const f3 xi = x[i];
     float4 v = vel[i];
     v.x = xi.x;
@@ -2050,21 +2076,17 @@ __global__ void __launch_bounds__(kBlock) k_advect(Scenes sc, float4* __restrict
 }
 
 // One workgroup per scene: st[blockIdx.x] starts a new loop; *active = S.
-__global__ void k_solver_reset(SolverDev* stv, uint32_t S, uint32_t* active, launch::Gate gate) {
-    SolverDev* st = stv + blockIdx.x;
-    const uint32_t t = threadIdx.x;
-    if (t == 0) {
-        st->done = shut(gate) ? kSkipped : 0u;
-        st->l = 1u;
-        st->counter = 0u;
-        st->rr = 0.0;
-        st->pAp = 0.0;
-        st->thr = 0.0;
-        st->alpha = 0.0f;
-        st->beta = 0.0f;
-        if (blockIdx.x == 0) *active = S;
-    }
-    for (uint32_t k = t; k < MPS_MAX_ITER_LOG; k += blockDim.x) st->log[k] = 0.0;
+__global__ void k_solver_reset(SolverDev* stv, uint32_t S, uint32_t* active) {
+    reset_record(stv + blockIdx.x, false);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *active = S;
+}
+// The start of a step: the first loop's records, the step's flags, the search's counters.
+__global__ void k_step_begin(SolverDev* stv, uint32_t S, uint32_t* active, uint32_t* flags, uint32_t nf, uint32_t* ctr, uint32_t nc) {
+    reset_record(stv + blockIdx.x, false);
+    if (blockIdx.x) return;
+    if (threadIdx.x == 0) *active = S;
+    if (threadIdx.x < nf) flags[threadIdx.x] = 0u;
+    if (threadIdx.x < nc) ctr[threadIdx.x] = 0u;
 }
 // Plain streaming copy (16-byte vectors), used only to calibrate byte counters.
 __global__ void __launch_bounds__(kBlock) k_calib_copy(const float4* __restrict__ a, float4* __restrict__ b, size_t n) {
@@ -2341,10 +2363,10 @@ void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, 
         launch_k(k, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, bpos, bvol, pG_ff, pG_fb, kappa, st, FoldPressure{});
 }
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
-               float4* cgx, hipStream_t s) {
+               float4* cgx, const LoopStart& ls, hipStream_t s) {
     if (!sc.N) return;
-    if (quad(sc, kQuadOnePerCu)) launch_k(k_st_factor<4>, nb_(sc.N), 4 * kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
-    else launch_k(k_st_factor<1>, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx);
+    if (quad(sc, kQuadOnePerCu)) launch_k(k_st_factor<4>, nb_(sc.N), 4 * kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx, ls);
+    else launch_k(k_st_factor<1>, nb_(sc.N), kBlock, 0, s, sc, nb, hl, pos, vel, pG_ff, fst, cgx, ls);
 }
 void cg_setup(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* rho,
               const float* fst, float* ca, float* cb, float* caT, float* cbT, float4* cgb, float* irho, hipStream_t s) {
@@ -2461,8 +2483,8 @@ void cg_update3(const Scenes& sc, f3* x, f3* r, const f3* p, const f3* Ap, Solve
 // 14.1 ms, 1006 24.5 -> 22.8, 2051 33.8 -> 34.3, 3907 65.7 -> 68.4 (there A.p 73.0 -> 79.8 us and
 // the update 11.4 -> 15.5, against two fold launches of 4.0).
 bool fold_in_consumer(uint32_t most_blocks) { return most_blocks <= 1536; }
-void copy_vel_out3(const Scenes& sc, const f3* x, float4* vel, const Gate& gate, hipStream_t s) {
-    if (sc.N) launch_k(k_copy_vel_out3, nb_(sc.N), kBlock, 0, s, sc, x, vel, gate);
+void copy_vel_out3(const Scenes& sc, const f3* x, float4* vel, const Gate& gate, const LoopStart& ls, hipStream_t s) {
+    if (sc.N) launch_k(k_copy_vel_out3, nb_(sc.N), kBlock, 0, s, sc, x, vel, gate, ls);
 }
 void copy_vel_out(const Scenes& sc, const float4* x, float4* vel, hipStream_t s) {
     if (sc.N) launch_k(k_copy_vel_out, nb_(sc.N), kBlock, 0, s, sc, x, vel);
@@ -2489,8 +2511,12 @@ void jacobi_error(int cubic, const Scenes& sc, const Nbr& nb, const float4* pos,
 void advect(const Scenes& sc, float4* pos, float4* vel, uint32_t* nonfinite, const Gate& gate, hipStream_t s) {
     if (sc.N) launch_k(k_advect, nb_(sc.N), kBlock, 0, s, sc, pos, vel, nonfinite, gate);
 }
-void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, const Gate& gate, hipStream_t s) {
-    if (S) launch_k(k_solver_reset, S, kBlock, 0, s, st, S, active, gate);
+void step_begin(SolverDev* st, uint32_t S, uint32_t* active, uint32_t* flags, uint32_t nf, NbrCounters* ctr, hipStream_t s) {
+    static_assert(sizeof(NbrCounters) / 4 <= kBlock, "one word per thread");
+    launch_k(k_step_begin, S, kBlock, 0, s, st, S, active, flags, nf, reinterpret_cast<uint32_t*>(ctr), sizeof(NbrCounters) / 4);
+}
+void solver_reset(SolverDev* st, uint32_t S, uint32_t* active, hipStream_t s) {
+    if (S) launch_k(k_solver_reset, S, kBlock, 0, s, st, S, active);
 }
 void calib_copy(const float4* a, float4* b, size_t n, hipStream_t s) {
     if (n) launch_k(k_calib_copy, 4096, kBlock, 0, s, a, b, n);
