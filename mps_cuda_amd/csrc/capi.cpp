@@ -375,12 +375,17 @@ struct mps_ctx {
     uint32_t pred_prev[3] = {0, 0, 0};  // the solves before those
     uint32_t pred_adj = 8;  // iterations of the last transposed solve of the adjoint
     // Iterations enqueued before the next host poll: the predicted count first (the previous
-    // solve's), then small chunks, so a solve that runs a little longer than predicted does not
-    // enqueue a whole second prediction of launches that would exit at once.
-    static constexpr uint32_t kFollowChunk = 2;
+    // solve's), then a power of two up to a quarter of those done, so that a solve that runs a
+    // little longer than predicted does not enqueue a whole second prediction of launches that
+    // would exit at once (5 us for the two of an iteration), and one that runs far longer does not
+    // wait 20 us for the host after every two (a transposed solve takes up to four times as many
+    // iterations as the one before it).
     uint32_t chunk_len(uint32_t it, uint32_t predicted, uint32_t left) const {
         if (cfg.host_sync_every) return std::min(cfg.host_sync_every, left);
-        return std::min(it == 1 ? std::max<uint32_t>(predicted, 1) : kFollowChunk, left);
+        if (it == 1) return std::min(std::max<uint32_t>(predicted, 1), left);
+        uint32_t n = 2;
+        while (8 * n < it) n *= 2;
+        return std::min(n, left);
     }
 
     // ------------------------------------------------------------------ kernel timing
@@ -488,7 +493,7 @@ struct mps_ctx {
         }
         auto it = graphs.find(key);
         if (it == graphs.end()) {
-            if (graphs.size() >= 64) clear_graphs();
+            if (graphs.size() >= 256) clear_graphs();
             GraphEntry e;
             HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
             try {
