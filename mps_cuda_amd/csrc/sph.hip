@@ -203,39 +203,6 @@ __device__ __forceinline__ double fold_everywhere(const double* __restrict__ par
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
-template <int L>
-__device__ __forceinline__ float quad_lane(float v) {  // the value of lane L of the quad, by DPP
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), L * 0x55, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float add_quad(float s, float t) {
-    return (((s + quad_lane<0>(t)) + quad_lane<1>(t)) + quad_lane<2>(t)) + quad_lane<3>(t);
-}
-__device__ __forceinline__ f3 add_quad(f3 s, f3 t) { return {add_quad(s.x, t.x), add_quad(s.y, t.y), add_quad(s.z, t.z)}; }
-
-// two terms per lane: t0 + u0 + t1 + u1 + ...
-__device__ __forceinline__ float add_quad(float s, float t, float u) {
-    s = (s + quad_lane<0>(t)) + quad_lane<0>(u);
-    s = (s + quad_lane<1>(t)) + quad_lane<1>(u);
-    s = (s + quad_lane<2>(t)) + quad_lane<2>(u);
-    return (s + quad_lane<3>(t)) + quad_lane<3>(u);
-}
-__device__ __forceinline__ f3 add_quad(f3 s, f3 t, f3 u) {
-    return {add_quad(s.x, t.x, u.x), add_quad(s.y, t.y, u.y), add_quad(s.z, t.z, u.z)};
-}
-__device__ __forceinline__ float sub_quad(float s, float t) {
-    return (((s - quad_lane<0>(t)) - quad_lane<1>(t)) - quad_lane<2>(t)) - quad_lane<3>(t);
-}
-__device__ __forceinline__ f3 sub_quad(f3 s, f3 t) { return {sub_quad(s.x, t.x), sub_quad(s.y, t.y), sub_quad(s.z, t.z)}; }
-template <int Q, class T>
-__device__ __forceinline__ T add_lanes(T s, T t) {
-    if constexpr (Q == 4) return add_quad(s, t);
-    else return s + t;
-}
-template <int Q, class T>
-__device__ __forceinline__ T sub_lanes(T s, T t) {
-    if constexpr (Q == 4) return sub_quad(s, t);
-    else return s - t;
-}
 // block_partial of a workgroup with a quad per slot (`v` counts in lane part 0): the slots'
 // values are put back one per lane and reduced by the first wave in block_total's order, so the
 // partial has the same bits.
