@@ -963,7 +963,11 @@ struct mps_ctx {
         if (!pairs_valid) density_alpha(mps::launch::kDoPairs);
     }
     // Block halos of the fluid lists for the halo-staged kernels (pressure solves, A.p)
-    mps::Halo halo() const { return mps::Halo{halo_idx.p, halo_n.p, nb16.p, use_deep()}; }
+    // Whether what an iteration streams per list entry (A.p: 10 bytes, the transposed one 18) stays in
+    // the 256 MB memory-side cache until the next iteration, beside the vectors and the halos (A.p gains
+    // up to some 200 MB of stream and loses from 250).
+    bool keep_streams(uint32_t bytes) const { return nnz_ff * bytes <= 210000000ull; }
+    mps::Halo halo() const { return mps::Halo{halo_idx.p, halo_n.p, nb16.p, use_deep(), keep_streams(10)}; }
     // Whether the staged kernels run their deep forms: when the last list build had more than one
     // workgroup in a thousand with a halo over the shallow depth (or as cfg.cg_halo_depth says).
     bool use_deep() const {
@@ -1066,7 +1070,7 @@ struct mps_ctx {
                 key.push_back(u(q));
             key.push_back(u(tol));
             key.push_back(lmin);
-            key.push_back(uint64_t(hl.deep) | (uint64_t(fuse) << 1));
+            key.push_back(uint64_t(hl.deep) | (uint64_t(fuse) << 1) | (uint64_t(hl.keep) << 2));
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
                     T_(df ? K_EVAL_DF : K_EVAL_CD, [&] {
@@ -1260,7 +1264,7 @@ struct mps_ctx {
             uint32_t* arr = fold_in ? arrive_counters() : nullptr;
             key.push_back(fold_in);
             key.push_back(u(arr));
-            key.push_back(uint64_t(op.deep) | (uint64_t(fuse) << 1));
+            key.push_back(uint64_t(op.deep) | (uint64_t(fuse) << 1) | (uint64_t(hl.keep) << 2));
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
                     const uint32_t k = it + c;
@@ -1579,7 +1583,7 @@ struct mps_ctx {
                                   (const void*)hl.n, (const void*)hl.nb16})
                 key.push_back(u(q));
             key.push_back(u(tol));
-            key.push_back(fuse);
+            key.push_back(uint64_t(fuse) | (uint64_t(hl.keep) << 1));
             launch_chunk(std::move(key), [&] {
                 for (uint32_t c = 0; c < chunk; c++) {
                     const uint32_t k = it + c;
@@ -1606,7 +1610,7 @@ struct mps_ctx {
     void reverse_step(TapeStep& T) {
         const mps::Scenes P = scn();
         const mps::Nbr nb{T.nff.p, T.cff.p, T.nfb.p, T.cfb.p};
-        const mps::Halo hl{T.halo_idx.p, T.halo_n.p, T.nb16.p, T.deep};
+        const mps::Halo hl{T.halo_idx.p, T.halo_n.p, T.nb16.p, T.deep, keep_streams(18)};
         const size_t m = std::max<uint32_t>(N, 1);
         pairG_ff.reserve(size_t(T.Kff) * m);
         pairG_fb.reserve(size_t(T.Kfb) * m);

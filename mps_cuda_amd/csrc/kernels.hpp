@@ -117,6 +117,7 @@ struct Halo {
     const uint32_t* n;
     const uint16_t* nb16;
     bool deep = false;  // enough halos are over kHaloShallow for the kernels' deep forms
+    bool keep = false;  // what A.p streams per iteration stays in the memory-side cache (GroupVal)
 };
 
 namespace launch {

@@ -255,19 +255,26 @@ struct GroupIdx<4, STAGED> {
     }
     __device__ __forceinline__ uint32_t at(int) const { return w; }
 };
-// The arrays of values per list entry that a walk streams with non-temporal loads. (The
+// The arrays of values per list entry that a walk streams, with non-temporal loads where they are over the
+// caches (GroupVal). (The
 // coefficients a_ij and b_ij are two arrays and not pairs, so that each of a lane's 16-byte loads
 // belongs to a contiguous kilobyte of the wave: with pairs, two loads touch every line, and the
 // line is fetched twice.)
 struct Streams {
     const float *a = nullptr, *b = nullptr, *aT = nullptr, *bT = nullptr;
 };
-template <int Q>
+// KEEP: without the hint, for arrays that a solve streams again and again and that stay in a cache from
+// one launch to the next. The grids with a quad per slot always do (their 2 MB per XCD in its L2: A.p at
+// 45k particles, 66 neighbours each, 14.8 -> 12.1 us); with one lane per slot A.p does while its stream
+// fits the 256 MB memory-side cache (Halo::keep; at spacing 0.6 of rest: 257k 22.7 -> 21.2 us, 405k 35.1 ->
+// 30.8, 512k 39.3 -> 36.7, 636k and 197 MB 50.0 -> 48.2, 804k and 250 MB 63.4 -> 68.0, 1M 71 -> 82).
+template <int Q, bool KEEP = false>
 struct GroupVal {
     typename std::conditional<Q == 1, v4f, float>::type v;
     __device__ __forceinline__ void load(const float* p, size_t group, uint32_t l) {
-        if constexpr (Q == 1) v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p) + group);
-        else v = __builtin_nontemporal_load(p + 4 * group + l);
+        if constexpr (Q != 1) v = p[4 * group + l];
+        else if constexpr (KEEP) v = reinterpret_cast<const v4f*>(p)[group];
+        else v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p) + group);
     }
     __device__ __forceinline__ void load(const Streams& s, size_t group, uint32_t l) { load(s.a, group, l); }
     __device__ __forceinline__ float at(int e) const {
@@ -275,17 +282,17 @@ struct GroupVal {
         else return v;
     }
 };
-template <int Q>
+template <int Q, bool KEEP>
 struct GroupAB {
-    GroupVal<Q> a, b;
+    GroupVal<Q, KEEP> a, b;
     __device__ __forceinline__ void load(const Streams& s, size_t group, uint32_t l) {
         a.load(s.a, group, l);
         b.load(s.b, group, l);
     }
 };
-template <int Q>
+template <int Q, bool KEEP>
 struct GroupABT {
-    GroupVal<Q> a, b, aT, bT;
+    GroupVal<Q, KEEP> a, b, aT, bT;
     __device__ __forceinline__ void load(const Streams& s, size_t group, uint32_t l) {
         a.load(s.a, group, l);
         b.load(s.b, group, l);
@@ -1369,7 +1376,7 @@ struct CgHead {
     bool done;
     float beta;
 };
-template <int MODE, bool RECOMP, bool CUBIC, bool COH = false, bool PCOH = COH, uint32_t DEPTH = kStageAp, int Q = 1, bool TRANS = false, class Head>
+template <int MODE, bool RECOMP, bool CUBIC, bool COH = false, bool PCOH = COH, uint32_t DEPTH = kStageAp, int Q = 1, bool TRANS = false, bool KEEP = false, class Head>
 __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const Scenes& sc, const Nbr& nb,
                                                const Halo& hl, const Streams& coef,
                                                const float4* __restrict__ pos, const float4* __restrict__ vel,
@@ -1415,7 +1422,8 @@ __device__ __forceinline__ void cg_apply_block(uint32_t blk, Head&& head, const 
             return a * pij + (bb * dot3(pij, xij)) * xij;
         }
     };
-    using Val = typename std::conditional<TRANS, GroupABT<Q>, typename std::conditional<RECOMP, GroupVal<Q>, GroupAB<Q>>::type>::type;
+    using Val = typename std::conditional<TRANS, GroupABT<Q, KEEP>,
+                                          typename std::conditional<RECOMP, GroupVal<Q>, GroupAB<Q, KEEP>>::type>::type;
     auto walk_fluid = [&](auto staged) {
         constexpr bool STAGED = decltype(staged)::value;
         // the first groups are loaded before the halo staging: their stream overlaps the
@@ -1551,7 +1559,7 @@ __device__ __forceinline__ bool cg_done(double s, double thr, double tol) { retu
 // workgroup records them. The others read `done`, `thr` and `rr_prev` of the record, which that
 // workgroup does not write (`rr_prev` is kept by the update), or, for `done`, only sets to what
 // they find themselves.
-template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1, bool FOLD = false, bool TRANS = false>
+template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1, bool FOLD = false, bool TRANS = false, bool KEEP = false>
 __global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl, Streams coef, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const float* __restrict__ rho,
                                                    const float* __restrict__ irho, const float4* __restrict__ x0,
@@ -1574,7 +1582,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo
         }
         return {sid, st[sid].done != 0u, st[sid].beta};
     };
-    cg_apply_block<MODE, RECOMP, CUBIC, false, false, DEEP ? kHaloCap : kStageAp, Q, TRANS>(
+    cg_apply_block<MODE, RECOMP, CUBIC, false, false, DEEP ? kHaloCap : kStageAp, Q, TRANS, KEEP>(
         blk, head, sc, nb, hl, coef, pos, vel, rho, irho, x0, rr, pprev, pout, Ap, b, r, x, partials);
 }
 
@@ -2364,7 +2372,9 @@ void cg_apply(int mode, const CgOperator& op, const Scenes& sc, const Nbr& nb, c
             else MPS_CG_APPLY(1, false, true, true, 4, false, true);
         } else {
             if (mode == 0) MPS_CG_APPLY(0, false, true, true, 1, false, true);
+            else if (fold && hl.keep) MPS_CG_APPLY(1, false, true, true, 1, true, true, true);
             else if (fold) MPS_CG_APPLY(1, false, true, true, 1, true, true);
+            else if (hl.keep) MPS_CG_APPLY(1, false, true, true, 1, false, true, true);
             else MPS_CG_APPLY(1, false, true, true, 1, false, true);
         }
     } else if (q) {
@@ -2373,11 +2383,15 @@ void cg_apply(int mode, const CgOperator& op, const Scenes& sc, const Nbr& nb, c
         else MPS_CG_APPLY(1, false, true, true, 4);
     } else if (!op.recompute && op.deep) {
         if (mode == 0) MPS_CG_APPLY(0, false, true, true);
+        else if (fold && hl.keep) MPS_CG_APPLY(1, false, true, true, 1, true, false, true);
         else if (fold) MPS_CG_APPLY(1, false, true, true, 1, true);
+        else if (hl.keep) MPS_CG_APPLY(1, false, true, true, 1, false, false, true);
         else MPS_CG_APPLY(1, false, true, true);
     } else if (!op.recompute) {
         if (mode == 0) MPS_CG_APPLY(0, false, true);
+        else if (fold && hl.keep) MPS_CG_APPLY(1, false, true, false, 1, true, false, true);
         else if (fold) MPS_CG_APPLY(1, false, true, false, 1, true);
+        else if (hl.keep) MPS_CG_APPLY(1, false, true, false, 1, false, false, true);
         else MPS_CG_APPLY(1, false, true);
     } else if (op.cubic) {
         if (mode == 0) MPS_CG_APPLY(0, true, true);
