@@ -3,7 +3,7 @@
 // Replaces SpatialHash::UpdateHash / ZSort / BuildNeighorhood (MPSSpatialHash.cu:53-218,
 // MPSSpatialHash.cuh:83-271). Design:
 //   * cell keys computed in double exactly like GetGridPos (trunc(x*(1/cell)) + H/2);
-//   * a stable LSD radix sort written here (8-bit digits, wave64 ballot ranking), so ties
+//   * a stable LSD radix sort written here (digits of up to 11 bits, wave64 ballot ranking), so ties
 //     keep ascending particle id — the order the reference's neighbour lists depend on;
 //   * cell start/end tables cleared incrementally (only cells occupied last step), plus a
 //     copy of the positions in key order so the 27-cell scan reads contiguous memory;
