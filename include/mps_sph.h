@@ -205,9 +205,9 @@ typedef struct mps_config {
                                     workgroup of the A.p and update launches (two launches per
                                     iteration; arrivals counted with device-scope atomics); 0 =
                                     (the default) folds by the workgroups that need the sums (two
-                                    launches, scenes of up to 1536 workgroups) or separate
-                                    one-workgroup fold launches (four). Same results; mps_autotune may change it. The allocation-free step
-                                    always uses 0. */
+                                    launches, grids of up to 1536 workgroups) or separate
+                                    one-workgroup fold launches (four). Same results; mps_autotune
+                                    may change it. The allocation-free step always uses 0. */
     uint32_t cg_halo_depth;      /* HIP library: LDS depth of the streamed viscosity operator's block
                                     halos. 0 = chosen each step from the previous list build (the
                                     deep form once more than 1 in 1000 workgroups have halos over

@@ -994,11 +994,9 @@ struct mps_ctx {
         build_halo(1);
     }
 
-    // Workgroups of the largest scene: the number of partial sums that a fold adds.
-    uint32_t most_blocks() const {
-        uint32_t n = 0;
-        for (const SceneHost& h : scenes) n = std::max(n, h.nf);
-        return ((scenes.empty() ? N : n) + mps::dev::kBlock - 1) / mps::dev::kBlock;
+    // Whether the workgroups that need a sum fold it themselves.
+    bool fold_in_consumers() const {
+        return mps::launch::fold_in_consumer(uint32_t((size_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock));
     }
     // Wait for the records of the loops [first, first + n) and copy them to h_solver.
     void fetch_records(int first, int n) {
@@ -1057,7 +1055,7 @@ struct mps_ctx {
         const uint32_t lmin = df ? cfg.df_min_iter : cfg.cd_min_iter;
         const uint32_t cap = cfg.max_iter;
         uint32_t& it = loop_it[idx];
-        const bool fuse = !coupled() && mps::launch::fold_in_consumer(most_blocks());
+        const bool fuse = !coupled() && fold_in_consumers();
         const mps::launch::FoldPressure fp{partials.p, d_active + idx, tol, lmin};
         if (it > cap) return;
         {
@@ -1094,7 +1092,7 @@ struct mps_ctx {
     void pressure_end(bool df, mps_step_stats* st) {
         const int idx = df ? 0 : 1;
         const uint32_t cap = cfg.max_iter;
-        const bool fuse = !coupled() && mps::launch::fold_in_consumer(most_blocks());
+        const bool fuse = !coupled() && fold_in_consumers();
         uint32_t l = 0;
         const std::vector<uint32_t> ls = loop_counts(idx, cap, &l);
         set_pred(idx, l);
@@ -1258,7 +1256,7 @@ struct mps_ctx {
             const bool fold_in = cfg.cg_fold_in_kernel != 0 && !g_no_alloc;
             // the sums folded by the launches that need them: p.Ap in `partials`, r.r in the next
             // nblk of them; a chunk ends with a fold launch of its last r.r
-            const bool fuse = !fold_in && !op.recompute && mps::launch::fold_in_consumer(most_blocks());
+            const bool fuse = !fold_in && !op.recompute && fold_in_consumers();
             double* part_rr = fuse ? partials.p + nblk : partials.p;
             const mps::launch::FoldCg fc{part_rr, act, tol};
             uint32_t* arr = fold_in ? arrive_counters() : nullptr;
@@ -1302,7 +1300,7 @@ struct mps_ctx {
         if (prof_on) {  // A.p (with the direction) and the update ran for iterations 1..l-1
             kuse[K_CG_APPLY] += std::min(l - 1, cap);
             kuse[K_CG_UPDATE] += std::min(l - 1, cap);
-            if ((!cfg.cg_fold_in_kernel || g_no_alloc) && (!cfg.cg_stream_coeffs || !mps::launch::fold_in_consumer(most_blocks())))
+            if ((!cfg.cg_fold_in_kernel || g_no_alloc) && (!cfg.cg_stream_coeffs || !fold_in_consumers()))
                 kuse[K_FOLD] += 2 * std::min(l - 1, cap);
         }
         for (uint32_t q = 0; q < S && q < sstats.size(); q++) {
@@ -1571,7 +1569,7 @@ struct mps_ctx {
         uint32_t it = 1;
         bool done = false;
         // sums folded as in cg_chunk
-        const bool fuse = mps::launch::fold_in_consumer(most_blocks());
+        const bool fuse = fold_in_consumers();
         double* part_rr = fuse ? partials.p + nblk : partials.p;
         const mps::launch::FoldCg fc{part_rr, act, tol};
         while (it <= cap && !done) {

@@ -266,7 +266,7 @@ void pressure_apply(int cubic, const Scenes& sc, const Nbr& nb, const Halo& hl, 
                     const float* bvol, const float* pG_ff, const float* pG_fb, const float* kappa, SolverDev* st,
                     const FoldPressure* fold, hipStream_t s);
 // Whether the consumers of a solver's sums fold them themselves (one launch less per sum).
-bool fold_in_consumer(uint32_t most_blocks);
+bool fold_in_consumer(uint32_t blocks);
 void st_factor(const Scenes& sc, const Nbr& nb, const Halo& hl, const float4* pos, const float4* vel, const float* pG_ff, float* fst,
                float4* cgx, const LoopStart& ls, hipStream_t s);
 // pair coefficients of the implicit operator: a_ij into ca, b_ij into cb (may be null); with caT and

@@ -2462,8 +2462,10 @@ void cg_update3(const Scenes& sc, f3* x, f3* r, const f3* p, const f3* Ap, Solve
 // Every consumer workgroup reads all partial sums of its scene, so the work grows with the square of
 // the workgroups. Whole passes (fold launches -> folds in the consumers): 128 workgroups 15.5 ->
 // 14.1 ms, 1006 24.5 -> 22.8, 2051 33.8 -> 34.3, 3907 65.7 -> 68.4 (there A.p 73.0 -> 79.8 us and
-// the update 11.4 -> 15.5, against two fold launches of 4.0).
-bool fold_in_consumer(uint32_t most_blocks) { return most_blocks <= 1536; }
+// the update 11.4 -> 15.5, against two fold launches of 4.0). The line is on the whole grid's
+// workgroups: in a batch each folds its own scene's sums only, but each pays the round trip (64 scenes,
+// 17.5 k workgroups, scenes of up to 1024: 22.3 ms per step with fold launches, 22.7 without).
+bool fold_in_consumer(uint32_t blocks) { return blocks <= 1536; }
 void copy_vel_out3(const Scenes& sc, const f3* x, float4* vel, const Gate& gate, const LoopStart& ls, hipStream_t s) {
     if (sc.N) launch_k(k_copy_vel_out3, nb_(sc.N), kBlock, 0, s, sc, x, vel, gate, ls);
 }
