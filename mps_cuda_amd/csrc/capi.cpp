@@ -1398,8 +1398,8 @@ struct mps_ctx {
     // one wait at the end. Each loop's start and the launches that change the state for good (the
     // velocities' copy, the advection) are gated on the loop before them having ended; where one had
     // not, everything after it did nothing, and the host goes on from there. The counts are the last
-    // solve's, and one more if the solve before it was longer: an iteration too many costs launches
-    // that exit at once (5 us each at 1 M particles), one too few the gated rest of the step. A wait per solve leaves the GPU idle for some 10 us each
+    // solve's, and one more if the solve before it took another number: an iteration too many costs
+    // launches that exit at once (5 us each at 1 M particles), one too few the gated rest of the step. A wait per solve leaves the GPU idle for some 10 us each
     // (33 k particles: 7 waits a step before, 2 now).
     bool can_run_ahead() const {
         return N && !rec && cfg.visc_solver == MPS_VISC_CG && !cfg.persistent_solver && !cfg.host_sync_every;
@@ -1412,7 +1412,7 @@ struct mps_ctx {
             mps::launch::Gate gate;
             for (int q = first; q < 3; q++) {
                 const int idx = kOrder[q];
-                const uint32_t predicted = std::min(std::max(pred[idx], pred_prev[idx]), pred[idx] + 1);
+                const uint32_t predicted = pred[idx] + (pred[idx] != pred_prev[idx] && pred_prev[idx] ? 1 : 0);
                 if (idx == 2) {
                     if (q > first || !begun) cg_begin(gate);
                     cg_chunk(predicted);
