@@ -53,7 +53,8 @@ struct SolverDev {
     uint32_t done;     // loop finished (converged) or skipped; later kernels of the chunk exit at once
     uint32_t l;        // reference loop variable when the loop ended (or next iteration)
     uint32_t counter;  // workgroups of the current launch that arrived (folds in the last workgroup)
-    uint32_t it;       // pressure loop: the iteration whose evaluation ran last (folds in the consumer)
+    uint32_t it;       // the iteration that the last evaluation or CG update worked on, 0 if the loop had ended
+                       // (folds in the consumer: what their launch reads of the loop's state before it folds)
     double rr;         // CG: r.r of the current residual
     double rr_prev;    // CG: r.r before the last update (folds in the consumer)
     double pAp;        // CG: p.Ap

@@ -732,6 +732,7 @@ __device__ __forceinline__ void reset_record(SolverDev* st, bool skip) {
         st->done = skip ? kSkipped : 0u;
         st->l = 1u;
         st->counter = 0u;
+        st->it = 0u;
         st->rr = 0.0;
         st->pAp = 0.0;
         st->thr = 0.0;
@@ -775,10 +776,11 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_eval(Scenes sc, Nbr nb,
     const f3 vi = in ? mk(vel[i]) : f3{0.f, 0.f, 0.f};
     const float rhoi = in ? rho[i] : 0.0f, alphai = in ? alpha[i] : 0.0f;
     const uint32_t sid = sc.blk_scene[blk];
-    if (st[sid].done) return;  // this scene's loop has finished
+    const bool done = st[sid].done != 0u;  // this scene's loop has finished
     const StepParams P = sc.P[sid];
+    if (blk == P.blk0 && threadIdx.x == 0) st[sid].it = done ? 0u : st[sid].l;  // for an apply that folds
+    if (done) return;
     const bool live = i < P.end;
-    if (blk == P.blk0 && threadIdx.x == 0) st[sid].it = st[sid].l;  // for an apply that folds
     const f3 xi = mk(xi4);
     float df = 0.0f;
     using Val = GroupVal<Q>;
@@ -963,9 +965,11 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_pressure_joint(Scenes sc,
 // ApplyDFSPH_kernel ff/fb + ApplyDFSPHFinal_kernel (MPSSPHDFSPHUtil.cuh:342-468) + UpdateVelocity.
 // The halo's (x_j, kappa_j) are staged in LDS (see k_cg_apply).
 // FOLD: every workgroup folds its scene's errors itself, in the fold kernels' order, and takes the
-// loop decision of k_fold_pressure; the scene's first workgroup records it. The others read `done`
-// and `it`: `it` was copied by the evaluation, and a `done` that is already set says what they
-// would find. One launch less per iteration (4 us and its gap) for ~1 us in the apply.
+// loop decision of k_fold_pressure; the scene's first workgroup records it (`done`, `l`). That may
+// happen while the waves of another workgroup are still to start, so nobody looks at what it writes:
+// whether the loop runs at all is read from `it`, which the evaluation wrote and this launch does
+// not, and is therefore the same for every wave that goes through the fold's barriers. One launch
+// less per iteration (4 us and its gap) for ~1 us in the apply.
 template <bool REF, bool CUBIC, bool BOBJ, int Q, bool FOLD>
 __global__ void __launch_bounds__(Q * kBlock) k_pressure_apply(Scenes sc, Nbr nb, Halo hl, const float4* __restrict__ pos,
                                                          float4* __restrict__ vel, const float4* __restrict__ bpos,
@@ -984,14 +988,16 @@ __global__ void __launch_bounds__(Q * kBlock) k_pressure_apply(Scenes sc, Nbr nb
     const float4 vi4 = in ? vel[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float pi = in ? kappa[i] : 0.0f;
     const uint32_t sid = sc.blk_scene[blk];
-    if (st[sid].done) return;
     const StepParams P = sc.P[sid];
     if constexpr (FOLD) {
         const uint32_t it = st[sid].it;
+        if (it == 0u) return;
         const double E = fold_everywhere<Q>(fp.partials + P.blk0, P.nblk) / double(P.count);
         const bool ok = E < fp.tol && it > fp.lmin;
         if (blk == P.blk0 && threadIdx.x == 0) record_pressure(st + sid, E, ok, it, fp.active);
         if (ok) return;
+    } else {
+        if (st[sid].done) return;
     }
     const bool live = i < P.end;
     const f3 xi = mk(xi4);
@@ -1556,9 +1562,9 @@ __device__ __forceinline__ bool cg_done(double s, double thr, double tol) { retu
 
 // FOLD (MODE 1): every workgroup first folds its scene's r.r of the last update itself, in the fold
 // kernels' order, forms beta and takes the convergence test of k_fold_cg<2>; the scene's first
-// workgroup records them. The others read `done`, `thr` and `rr_prev` of the record, which that
-// workgroup does not write (`rr_prev` is kept by the update), or, for `done`, only sets to what
-// they find themselves.
+// workgroup records them, possibly before the waves of another workgroup start. Before the fold
+// every wave therefore reads only words of the record that this launch does not write: `thr`, and
+// `it` (0: the loop has ended) and `rr_prev`, which the update keeps.
 template <int MODE, bool RECOMP, bool CUBIC, bool DEEP = false, int Q = 1, bool FOLD = false, bool TRANS = false, bool KEEP = false>
 __global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo hl, Streams coef, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const float* __restrict__ rho,
@@ -1572,7 +1578,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_cg_apply(Scenes sc, Nbr nb, Halo
         const uint32_t sid = sc.blk_scene[blk];
         if (MODE == 0) return {sid, false, 0.0f};
         if constexpr (FOLD) {
-            if (st[sid].done) return {sid, true, 0.0f};
+            if (st[sid].it == 0u) return {sid, true, 0.0f};
             const uint32_t blk0 = sc.P[sid].blk0;
             const double prev = st[sid].rr_prev, thr = st[sid].thr;
             const double s = fold_everywhere<Q>(fc.partials + blk0, sc.P[sid].nblk);
@@ -1640,22 +1646,26 @@ __device__ __forceinline__ void cg_update3_block(uint32_t blk, uint32_t end, flo
     block_partial<PCOH>(part, partials, blk);
 }
 // FOLD: every workgroup first folds its scene's p.Ap itself and forms alpha (k_fold_cg<1>); the
-// scene's first workgroup records it and keeps the r.r that the next A.p needs as rr_prev, which no
-// workgroup of this launch reads.
+// scene's first workgroup records it and keeps what the next A.p reads before its own fold: the r.r
+// as rr_prev, and the iteration, or 0 once the loop has ended, as `it`. No workgroup of this launch
+// reads either, and none writes `done`.
 template <bool FOLD>
 __global__ void __launch_bounds__(kBlock) k_cg_update3(Scenes sc, f3* __restrict__ x, f3* __restrict__ r,
                                                      const f3* __restrict__ p, const f3* __restrict__ Ap,
                                                      SolverDev* st, const double* __restrict__ pAp,
                                                      double* __restrict__ partials) {
     const uint32_t sid = sc.blk_scene[blockIdx.x];
-    if (st[sid].done) return;
+    const bool done = st[sid].done != 0u;
+    const bool first = FOLD && blockIdx.x == sc.P[sid].blk0 && threadIdx.x == 0;  // keeps the record
+    if (first) st[sid].it = done ? 0u : st[sid].l;
+    if (done) return;
     float alpha;
     if constexpr (FOLD) {
         const uint32_t blk0 = sc.P[sid].blk0;
         const double rr = st[sid].rr;
         const double s = fold_as_fold_kernel<false>(pAp + blk0, sc.P[sid].nblk);
         alpha = float(rr / s);
-        if (blockIdx.x == blk0 && threadIdx.x == 0) {
+        if (first) {
             st[sid].pAp = s;
             st[sid].alpha = alpha;
             st[sid].rr_prev = rr;
