@@ -868,8 +868,7 @@ struct mps_ctx {
                 HIPCHK(hipMemcpyAsync(h_ctr, d_ctr, sizeof(NbrCounters), hipMemcpyDeviceToHost, stream));
                 sync();
             };
-            const bool both = search_left != 0;  // the last search left blocks to the second pass
-            search(both ? mps::launch::kSearchBoth : mps::launch::kSearchFirst);
+            // before the fluid search, whose count records have to stay in nstat until its last pass
             if (coupled()) {
                 nfr.reserve(size_t(Kfr) * std::max<uint32_t>(N, 1));
                 cfr.reserve(std::max<uint32_t>(N, 1));
@@ -878,6 +877,8 @@ struct mps_ctx {
                                                stream);
                 });
             }
+            const bool both = search_left != 0;  // the last search left blocks to the second pass
+            search(both ? mps::launch::kSearchBoth : mps::launch::kSearchFirst);
             counters();
             search_left = h_ctr->left;
             search_dense = uint64_t(h_ctr->crowded) * kSearchCrowded > (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
