@@ -476,6 +476,7 @@ struct mps_ctx {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
     };
+    static constexpr size_t kGraphs = 256;
     std::map<std::vector<uint64_t>, GraphEntry> graphs;
     bool graphs_on() const { return cfg.use_graphs && !prof_on && !rec && !g_no_alloc; }
     void clear_graphs() {
@@ -493,7 +494,10 @@ struct mps_ctx {
         }
         auto it = graphs.find(key);
         if (it == graphs.end()) {
-            if (graphs.size() >= 256) clear_graphs();
+            if (graphs.size() >= kGraphs) {
+                sync();  // chunks of this step that replay one of them may still be running
+                clear_graphs();
+            }
             GraphEntry e;
             HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
             try {
