@@ -591,12 +591,20 @@ __global__ void __launch_bounds__(kCountFoldThreads) k_count_fold(const uint2* _
 //
 // Q = 4 shares a slot among a quad of lanes, which take the runs 0..8 in turn.
 //
-// A block may have more rows, cells or candidates than the LDS holds, staged fluid (or wall)
-// particles that do not all share one radius, or a run of more copies than a hit mask has bits. The
-// first pass over many blocks (LAST false) leaves such a block alone (n = kHaloTodo); a second one,
-// with room for more and a quad per slot, takes what is left. The LAST pass searches the global
-// tables for a set that does not fit even there, and leaves the halo of a block whose fluid was
-// searched so to k_halo_build. The lists are the same whichever way.
+// Staged fluid particles of several radii: a run's mask is made with the cut-off of the widest pair
+// that the block can hold, then the radii of its hits are read and each is tested with its own.
+// (1M particles of two radii, hash, search and density: 2110 us with such blocks left to the tables of a
+// second pass, 985 with one lane per slot over the tables in the only pass, now 653.)
+//
+// A block may have more rows, cells or candidates than the LDS holds, or a run of more copies than a
+// hit mask has bits. The first pass over many blocks (LAST false) leaves such a block alone
+// (n = kHaloLeft); a second one, with room for more and a quad per slot, takes what is left, and
+// searches the global tables for a set that does not fit even there. The first pass does so itself
+// where waiting would not help: walls of several radii, more candidates than the second pass holds, or
+// cells far wider than the support (kWideCell), whose tables one lane per slot of a full grid walks
+// faster than the second pass its copies: 257k particles, cells of two supports 581 us against 778, of
+// three 1599 against 1994. The halo of a block whose fluid was searched in the tables is left to
+// k_halo_build. The lists are the same whichever way.
 //
 // Bound by its vector instructions and LDS latency: of the ~50 us that a workgroup takes (1M
 // particles, four workgroups per CU) the distance tests are 13, writing the lists 9, the halo 15,
@@ -615,6 +623,7 @@ struct SearchCaps {
 using SearchStd = SearchCaps<7, 96, 384, 1920, 3>;     // 39 KB: four workgroups per CU
 using SearchDense = SearchCaps<7, 96, 384, 2752, 3>;   // 52 KB: three (525k near rest density: 437 -> 343 us)
 using SearchWide = SearchCaps<9, 224, 1024, 3328, 8>;  // 78 KB: two
+constexpr uint32_t kWideCell = 32;                   // a cell with more fluid is a wide one (one support wide: up to 20)
 constexpr uint32_t kSrchPad = 4;                     // a group of four read at the end of a run stays in the array
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
 constexpr uint32_t kHit = 0x80000000u;  // marks a staged fluid copy that is in a list (slots are below 2^31)
@@ -651,6 +660,42 @@ __device__ __forceinline__ uint32_t quad_before(uint32_t v, uint32_t l) {
     return (l > 0u ? a : 0u) + (l > 1u ? b : 0u) + (l > 2u ? c : 0u);
 }
 
+// search_cells by a quad of lanes: every lane takes a candidate of each four (two fours in flight), and
+// the hits of a four enter the list in candidate order. The count is valid in every lane.
+template <bool SELF, int LAYOUT>
+__device__ __forceinline__ uint32_t search_cells_quad(float4 xi, uint32_t i, uint32_t l, const HashGeom& g,
+                                                      const uint32_t* __restrict__ start, const uint32_t* __restrict__ end,
+                                                      const uint32_t* __restrict__ ids, const float4* __restrict__ spos,
+                                                      uint32_t* __restrict__ out, uint32_t K, uint32_t stride) {
+    const i3 p = grid_pos(xi.x, xi.y, xi.z, g);
+    const float ri = xi.w * 4.0f;
+    uint32_t k = 0u;
+#pragma unroll 1
+    for (int t = 0; t < 27; t++) {
+        const uint32_t c = grid_index(p.x + (t % 3) - 1, p.y + (t / 3) % 3 - 1, p.z + t / 9 - 1, g);
+        const uint32_t s0 = start[c], e = end[c];
+        const uint32_t n = s0 < e ? e - s0 : 0u;  // (the same in the four lanes, as are all counts)
+        for (uint32_t o = 0; o < n; o += 8u) {
+            float4 q[2];
+#pragma unroll
+            for (uint32_t h = 0; h < 2u; h++) q[h] = spos[s0 + min(o + 4u * h + l, n - 1u)];
+#pragma unroll
+            for (uint32_t h = 0; h < 2u; h++) {
+                const uint32_t at = o + 4u * h + l;
+                bool hit = at < n && within(xi, ri, q[h]);
+                uint32_t j = s0 + at;
+                if (hit && ids) j = ids[j];
+                if (SELF && j == i) hit = false;
+                const uint32_t one = hit ? 1u : 0u;
+                const uint32_t pl = k + quad_before(one, l);
+                if (hit && pl < K) out[list_at<LAYOUT>(pl, i, K, stride)] = j;
+                k += quad_sum(one);
+            }
+        }
+    }
+    return k;
+}
+
 // The hits of one slot among its 9 row runs; with Q = 4 a lane holds the runs l, l + 4 and 8 (l = 0).
 template <int Q, uint32_t WORDS>
 struct RowHits {
@@ -661,10 +706,11 @@ struct RowHits {
     uint32_t count;                 // hits of all runs
 
     // run(r) gives the [lo, hi) of run r; `self` is the slot's own staged copy (any other value:
-    // none); a copy is a hit when its squared distance is below `cut`. False if a run is too long for
-    // its mask (for the whole quad).
-    template <class Run>
-    __device__ __forceinline__ bool test(const float4* cand, uint32_t l, const float4& xi, float cut, uint32_t self, Run&& run) {
+    // none); a copy is a hit when its squared distance is below `cut` and, with `sift` set, the copy
+    // passes drop() too. False if a run is too long for its mask (for the whole quad).
+    template <class Run, class Drop>
+    __device__ __forceinline__ bool test(const float4* cand, uint32_t l, const float4& xi, float cut, uint32_t self, Run&& run,
+                                         bool sift, Drop&& drop) {
         uint32_t over = 0u, n[kRuns];
 #pragma unroll
         for (uint32_t q = 0; q < kRuns; q++) {
@@ -695,6 +741,7 @@ struct RowHits {
                     mm &= len < 32u ? (1u << len) - 1u : ~0u;  // the group of four read past hi
                     const uint32_t d = self - c0;
                     if (d < 32u) mm &= ~(1u << d);
+                    if (sift) mm = sifted(mm, c0, drop);
                 }
                 m[q][w] = mm;
                 n[q] += __popc(mm);
@@ -716,6 +763,24 @@ struct RowHits {
             count = t0 + t1 + quad_sum(n[2]);
             return quad_sum(over) == 0u;
         }
+    }
+    // The bits e of mm whose copy c0 + e is kept: drop(copies) takes four at a time (a copy again where
+    // fewer are left) and gives the set of those to drop.
+    template <class Drop>
+    static __device__ __forceinline__ uint32_t sifted(uint32_t mm, uint32_t c0, Drop&& drop) {
+        for (uint32_t left = mm; left;) {
+            uint32_t b[4], t[4];
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; e++) {
+                b[e] = left & (0u - left);  // the lowest bit
+                left ^= b[e];
+                t[e] = c0 + (b[e] ? static_cast<uint32_t>(__builtin_ctz(b[e])) : 0u);
+            }
+            const uint32_t out = drop(t);
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; e++) mm &= (out >> e) & 1u ? ~b[e] : ~0u;
+        }
+        return mm;
     }
     // use(list position, staged copy) for every hit, in list order within a run
     template <class Use>
@@ -748,7 +813,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     constexpr uint32_t kCellsPer = (kCells + kThreads - 1u) / kThreads;  // cells per thread
     static_assert(kRows <= kThreads && kRows <= 255u + 1u && kRows < kRowHash, "one row per thread");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    if (LAST && left && ho.n[blk] != kHaloTodo) return;  // the first pass did this block
+    if (LAST && left && ho.n[blk] != kHaloLeft) return;  // the first pass did this block
     const uint32_t tid = threadIdx.x;
     const uint32_t i = blk * kBlock + tid / Q;
     const uint32_t l = tid % Q;
@@ -771,6 +836,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     __shared__ float4 cand[kCand + kSrchPad];
     __shared__ unsigned long long ws[kWaves];
     __shared__ uint32_t nrow, mixed, first[2];  // first: first cell with fluid, with walls
+    __shared__ uint32_t widest;  // largest |radius| of the fluid copies that differ from the first, as bits
     auto row_hash = [](uint32_t c) -> uint32_t { return (c * 2654435761u) >> (32u - Caps::kHashBits); };
     for (uint32_t t = tid; t < kRowHash; t += kThreads) {
         rkey[t] = kNoRow;
@@ -778,6 +844,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
         rxhi[t] = -0x7FFFFFFF - 1;
     }
     if (tid == 0) {
+        widest = 0u;
         nrow = 0u;
         mixed = 0u;
         first[0] = first[1] = kNoRow;
@@ -816,6 +883,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     __syncthreads();
     const uint32_t nr = nrow;
     bool staged = nr <= kRows;
+    bool tables = LAST;  // what cannot be walked in LDS here searches the global tables
     uint32_t nc = 0u;
     // 2. number each row's cells over its x range (rows in registration order)
     if (staged) {
@@ -856,6 +924,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
             }
             fsum += fc[q];
             bsum += bc[q];
+            if (!LAST && fc[q] > kWideCell) atomicOr(&mixed, 8u);
         }
         const unsigned long long mine = (static_cast<unsigned long long>(bsum) << 32) | fsum;
         unsigned long long tot;
@@ -863,7 +932,8 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
         tf = static_cast<uint32_t>(tot & 0xFFFFFFFFull);
         tb = static_cast<uint32_t>(tot >> 32);
         staged = static_cast<unsigned long long>(tf) + tb <= kCand;
-        if (!LAST && tid == 0 && static_cast<unsigned long long>(tf) + tb > SearchStd::kCand) atomicAdd(&ctr->crowded, 1u);
+        tables = LAST || static_cast<unsigned long long>(tf) + tb > SearchWide::kCand || (mixed & 8u);
+        if (!LAST && tid == 0 && !tables && static_cast<unsigned long long>(tf) + tb > SearchStd::kCand) atomicAdd(&ctr->crowded, 1u);
         uint32_t fo = static_cast<uint32_t>(ex & 0xFFFFFFFFull), bo = static_cast<uint32_t>(ex >> 32);
         if (staged) {
             // each copy's w first holds its cell (read back by the staging pass)
@@ -890,11 +960,13 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     }
     // 4. stage the candidates with their ids (copy t of cell e is particle efs[e] + t - efo[e]),
     //    kStage loads of a thread in flight. `mixed` records whether some fluid (bit 0) or wall (bit 1)
-    //    candidate has another radius than the first staged candidate of its set.
-    float rw = 0.0f;  // the walls' common radius
+    //    candidate has another radius than the first staged candidate of its set (bit 2: the block's halo
+    //    cannot be written here, bit 3: a wide cell).
+    float rf = 0.0f, rw = 0.0f;  // the first fluid's radius, the walls' common one
     if (staged) {
         constexpr uint32_t kStage = 4;
         uint32_t mx = 0u;
+        float rmax = 0.0f;
         auto stage = [&](uint32_t t_lo, uint32_t t_hi, const uint32_t* es, const uint16_t* eo, const float4* from, const uint32_t* id,
                          float r0, uint32_t bit) {
             for (uint32_t t0 = t_lo + tid; t0 < t_hi; t0 += kStage * kThreads) {
@@ -916,11 +988,16 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
                     if (t < t_hi) {
                         cand[t] = make_float4(v[q].x, v[q].y, v[q].z, __uint_as_float(s[q]));
                         mx |= v[q].w != r0 ? bit : 0u;
+                        rmax = fmaxf(rmax, fabsf(v[q].w));  // (a NaN is nobody's neighbour)
                     }
                 }
             }
         };
-        if (tf) stage(0u, tf, efs, efo, pos, nullptr, pos[efs[first[0]]].w, 1u);
+        if (tf) {
+            rf = pos[efs[first[0]]].w;
+            stage(0u, tf, efs, efo, pos, nullptr, rf, 1u);
+            if (mx) atomicMax(&widest, __float_as_uint(rmax));
+        }
         if (tb) {
             rw = bd.spos[ebs[first[1]]].w;
             stage(tf, tf + tb, ebs, ebo, bd.spos, bd.id, rw, 2u);
@@ -946,19 +1023,30 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
         lo = eo[e];
         hi = eo[e + 3u];
     };
-    // a search of the global tables (one lane of the slot), its count in every lane
-    auto global = [&](auto&& search) -> uint32_t {
-        const uint32_t n = l == 0u ? search() : 0u;
-        if constexpr (Q == 1) return n;
-        else return quad_u32<0>(n);
+    // a fluid copy of another radius is a neighbour by the pair's own cut-off: its radius is read for the
+    // hits of the widest pair only
+    auto drop = [&](const uint32_t (&t)[4]) -> uint32_t {
+        float4 q[4];
+        float r[4];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) q[e] = cand[t[e]];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) r[e] = pos[__float_as_uint(q[e].w) & ~kHit].w;
+        uint32_t out = 0u;
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) out |= within(xi, ri, make_float4(q[e].x, q[e].y, q[e].z, r[e])) ? 0u : 1u << e;
+        return out;
     };
     RowHits<Q, Caps::kWords> hits;
     bool have = false;  // `hits` are this slot's fluid neighbours
     if (live) {
-        if (!(mix & 1u)) {
+        if (staged) {
             const uint32_t eh = cell_of(0, p.y, p.z);
             const uint32_t self = eh == kNoRow ? kNoRow : efo[eh] + (i - efs[eh]);
-            have = hits.test(cand, l, xi, cut_of((ri + ri) * 0.5f), self, [&](uint32_t r, uint32_t& lo, uint32_t& hi) { run_of(efo, r, lo, hi); });
+            const bool sift = mix & 1u;
+            const float rj = fmaxf(fabsf(rf), __uint_as_float(widest)) * 4.0f;
+            have = hits.test(cand, l, xi, cut_of(sift ? (fabsf(ri) + rj) * 0.5f : (ri + ri) * 0.5f), self,
+                             [&](uint32_t r, uint32_t& lo, uint32_t& hi) { run_of(efo, r, lo, hi); }, sift, drop);
         }
         if (have) {
             a = hits.count;
@@ -967,9 +1055,10 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
                 cand[t].w = __uint_as_float(s | kHit);
                 if (k < Kff) nff[ell(k, i, N)] = s;
             });
-        } else if constexpr (LAST) {
-            a = global([&] { return search_cells<true, kGroups>(xi, i, g, fstart, fend, fl.id, fl.spos, nff, Kff, N); });
-            if (!(mix & 1u)) atomicOr(&mixed, 4u);  // a run too long: the block's halo is left to k_halo_build
+        } else if (tables) {
+            if constexpr (Q == 1) a = search_cells<true, kGroups>(xi, i, g, fstart, fend, fl.id, fl.spos, nff, Kff, N);
+            else a = search_cells_quad<true, kGroups>(xi, i, l, g, fstart, fend, fl.id, fl.spos, nff, Kff, N);
+            atomicOr(&mixed, 4u);  // the block's halo is left to k_halo_build
         } else {
             atomicOr(&mixed, 4u);
         }
@@ -979,13 +1068,15 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
             } else {
                 RowHits<Q, Caps::kWords> wh;
                 if (!(mix & 2u) && wh.test(cand, l, xi, cut_of((ri + rw * 4.0f) * 0.5f), kNoRow,
-                                           [&](uint32_t r, uint32_t& lo, uint32_t& hi) { run_of(ebo, r, lo, hi); })) {
+                                           [&](uint32_t r, uint32_t& lo, uint32_t& hi) { run_of(ebo, r, lo, hi); }, false,
+                                           [](const uint32_t (&)[4]) -> uint32_t { return 0u; })) {
                     b = wh.count;
                     wh.each([&](uint32_t k, uint32_t t) {
                         if (k < Kfb) nfb[size_t(k) * N + i] = __float_as_uint(cand[t].w);
                     });
-                } else if constexpr (LAST) {
-                    b = global([&] { return search_cells<false, kCols>(xi, i, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N); });
+                } else if (tables || (staged && (mix & 2u))) {  // (no form stages walls of several radii)
+                    if constexpr (Q == 1) b = search_cells<false, kCols>(xi, i, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N);
+                    else b = search_cells_quad<false, kCols>(xi, i, l, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N);
                 } else {
                     atomicOr(&mixed, 4u);
                 }
@@ -999,10 +1090,10 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     // 6. the block's halo: the marked copies, cells in order of their first slot (cells are disjoint
     //    slot ranges, so that is ascending slot order; a block with a cell staged twice is left out)
     __syncthreads();
-    if (!staged || (mixed & 5u)) {
+    if (!staged || (mixed & 4u)) {
         if (tid == 0) {
-            ho.n[blk] = kHaloTodo;
-            atomicAdd(LAST ? &ctr->todo : &ctr->left, 1u);
+            ho.n[blk] = tables ? kHaloTodo : kHaloLeft;
+            atomicAdd(tables ? &ctr->todo : &ctr->left, 1u);
         }
     } else {
         // marked copies of each cell (in ecell, no longer needed), then their sum over the cells with

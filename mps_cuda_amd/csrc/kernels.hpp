@@ -32,7 +32,7 @@ struct HashView {
 struct NbrCounters {
     uint32_t max_ff, max_fb, max_bb, max_fr;
     uint32_t left;  // workgroups that the first pass of the fluid search left to the second
-    uint32_t crowded;  // workgroups of the first pass with more candidates than its usual form holds
+    uint32_t crowded;  // workgroups of the first pass with more candidates than its usual form holds (and not searched in the tables)
     uint32_t todo;  // workgroups of the fluid search whose halo is left to k_halo_build
     uint32_t pad;
     unsigned long long nnz_ff, nnz_fb, nnz_bb, nnz_fr;
@@ -113,6 +113,7 @@ constexpr uint32_t kMaxWallObjects = 4;
 constexpr uint32_t kHaloCap = 1536;
 constexpr uint32_t kHaloShallow = 1264;
 constexpr uint32_t kHaloTodo = 0xFFFFFFFFu;  // n[b] after the search: this block's halo is still to be built
+constexpr uint32_t kHaloLeft = 0xFFFFFFFEu;  // n[b] between the search's passes: this block is left to the second
 struct Halo {
     const uint32_t* idx;
     const uint32_t* n;
