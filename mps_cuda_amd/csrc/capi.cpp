@@ -391,7 +391,7 @@ struct mps_ctx {
     // ------------------------------------------------------------------ kernel timing
     enum KId {
         K_KEYS, K_SORT, K_CELLS, K_NEI_FLUID, K_NEI_BND, K_BSUM, K_BVOL, K_DENSITY, K_EVAL_DF, K_EVAL_CD,
-        K_APPLY, K_ST_FACTOR, K_CG_SETUP, K_CG_INIT, K_CG_APPLY, K_CG_UPDATE, K_CG_DIR, K_COPY_OUT, K_ADVECT,
+        K_APPLY, K_ST_FACTOR, K_CG_SETUP, K_CG_INIT, K_CG_APPLY, K_CG_UPDATE, K_COPY_OUT, K_ADVECT,
         K_ZSORT, K_JACOBI, K_FOLD, K_REORDER, K_HALO, K_CALIB, K_STREAM, K_COUNT
     };
     static const char* kname(int k) {
@@ -399,7 +399,7 @@ struct mps_ctx {
             "k_cell_keys", "radix_sort", "k_cell_table", "k_neighbors_fluid", "k_neighbors_boundary",
             "k_boundary_sum", "k_boundary_volume", "k_density_alpha", "k_pressure_eval<DF>", "k_pressure_eval<CD>",
             "k_pressure_apply", "k_st_factor", "k_cg_setup", "k_cg_apply<0>", "k_cg_apply<1>", "k_cg_update",
-            "k_cg_direction", "k_copy_vel_out", "k_advect", "zsort", "jacobi", "k_fold", "reorder", "k_halo_build",
+            "k_copy_vel_out", "k_advect", "zsort", "jacobi", "k_fold", "reorder", "k_halo_build",
             "k_calib_copy", "k_stream_copy"};
         return names[k];
     }
@@ -2460,14 +2460,6 @@ struct mps_ctx {
         std::vector<uint32_t> c = down(cnt, n), idx(size_t(n) + 1, 0u);
         for (uint32_t i = 0; i < n; i++) idx[i + 1] = idx[i] + c[i];
         return idx;
-    }
-    std::vector<uint32_t> csr_nei(const uint32_t* nbrs, const uint32_t* cnt, uint32_t n, uint32_t K) {
-        std::vector<uint32_t> c = down(cnt, n);
-        std::vector<uint32_t> ell = down(nbrs, size_t(K) * n);
-        std::vector<uint32_t> out;
-        for (uint32_t i = 0; i < n; i++)
-            for (uint32_t k = 0; k < c[i]; k++) out.push_back(ell[size_t(k) * n + i]);
-        return out;
     }
     // returns (count, elem_bytes) and optionally the data as bytes
     void array_io(int32_t id, size_t* count, size_t* eb, void* dst, const void* src, size_t bytes) {
