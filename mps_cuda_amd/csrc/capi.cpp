@@ -314,10 +314,14 @@ struct mps_ctx {
     mps::GridSync* d_grid = nullptr;  // barrier words of the persistent solver (allocated at creation)
     uint32_t persist_cap[6] = {0, 0, 0, 0, 0, 0};  // co-resident workgroups per kernel variant (0 = not asked yet)
     uint32_t persist_fallbacks = 0;       // persistent solves that gave up and reran chunked
-    // The first pass takes its dense form when more than one workgroup in kSearchCrowded had more
-    // candidates than the usual form holds.
-    static constexpr uint32_t kSearchCrowded = 32;
+    // The first pass takes its dense form when more than one workgroup in kSearchMany had more
+    // candidates than the usual form holds, and leaves nothing to a second one when as many had more rows
+    // or cells than it holds; where fewer had, it leaves those too. (A second pass costs some 50 us and
+    // its longest block; one block in the tables costs nothing beside a full grid, but a halo build for
+    // it 60 us, which the second pass saves.)
+    static constexpr uint32_t kSearchMany = 32;
     int search_dense = 0;
+    mps::launch::SearchLeave search_leave = mps::launch::kLeaveCrowded;
     uint32_t search_left = 0;             // workgroups that the last search's first pass left to the second
     uint32_t deep_halos = 0;              // workgroups of the last list build with halos over kHaloShallow
     uint32_t* d_flags = nullptr;  // [0] nonfinite, [1] sampling mismatch, [4..6] halo statistics of the step
@@ -865,7 +869,7 @@ struct mps_ctx {
                     mps::launch::neighbors_fluid(pos.p, scn(), uint32_t(cells()), g, fluid_view(), view(bh, B), nff.p, Kff, cff.p,
                                                  nfb.p, Kfb, cfb.p, nstat.p,
                                                  mps::launch::HaloOut{halo_idx.p, halo_n.p, nb16.p, cfg.halo_limit, d_flags + 4},
-                                                 passes, search_dense, d_ctr, stream);
+                                                 passes, search_leave, search_dense, d_ctr, stream);
                 });
             };
             auto counters = [&] {
@@ -884,12 +888,14 @@ struct mps_ctx {
             const bool both = search_left != 0;  // the last search left blocks to the second pass
             search(both ? mps::launch::kSearchBoth : mps::launch::kSearchFirst);
             counters();
+            const uint64_t blocks = (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
             search_left = h_ctr->left;
-            search_dense = uint64_t(h_ctr->crowded) * kSearchCrowded > (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
+            search_dense = uint64_t(h_ctr->crowded) * kSearchMany > blocks;
             if (h_ctr->left && !both) {
                 search(mps::launch::kSearchLeft);
                 counters();
             }
+            search_leave = uint64_t(h_ctr->spread) * kSearchMany > blocks ? mps::launch::kLeaveNone : mps::launch::kLeaveAll;
             bool grow = false;
             if (coupled() && h_ctr->max_fr > Kfr) { Kfr = (h_ctr->max_fr + 15u) & ~15u; grow = true; }
             if (h_ctr->max_ff > Kff) { Kff = (h_ctr->max_ff + 15u) & ~15u; grow = true; }

@@ -598,13 +598,14 @@ __global__ void __launch_bounds__(kCountFoldThreads) k_count_fold(const uint2* _
 //
 // A block may have more rows, cells or candidates than the LDS holds, or a run of more copies than a
 // hit mask has bits. The first pass over many blocks (LAST false) leaves such a block alone
-// (n = kHaloLeft); a second one, with room for more and a quad per slot, takes what is left, and
-// searches the global tables for a set that does not fit even there. The first pass does so itself
-// where waiting would not help: walls of several radii, more candidates than the second pass holds, or
-// cells far wider than the support (kWideCell), whose tables one lane per slot of a full grid walks
-// faster than the second pass its copies: 257k particles, cells of two supports 581 us against 778, of
-// three 1599 against 1994. The halo of a block whose fluid was searched in the tables is left to
-// k_halo_build. The lists are the same whichever way.
+// (n = kHaloLeft); a second one, with room for more and a quad per slot, takes it, and searches the
+// global tables for a set that does not fit even there. The first pass does so itself where waiting
+// would not help: walls of several radii, more candidates than the second pass holds, cells far wider
+// than the support (kWideCell; 257k particles, cells of two supports 581 us against 778, of three 1599
+// against 1994), and, where many blocks have too many rows or cells (scattered particles, a hash that
+// wraps the scene around), whatever does not fit (1M scattered particles, one to a cell: 944 us for hash,
+// search and density with a second pass, 568 without). The halo of a block whose fluid was searched in
+// the tables is left to k_halo_build. The lists are the same whichever way.
 //
 // Bound by its vector instructions and LDS latency: of the ~50 us that a workgroup takes (1M
 // particles, four workgroups per CU) the distance tests are 13, writing the lists 9, the halo 15,
@@ -626,6 +627,9 @@ using SearchWide = SearchCaps<9, 224, 1024, 3328, 8>;  // 78 KB: two
 constexpr uint32_t kWideCell = 32;                   // a cell with more fluid is a wide one (one support wide: up to 20)
 constexpr uint32_t kSrchPad = 4;                     // a group of four read at the end of a run stays in the array
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
+// Bits of a block's `mixed` beside 1 and 2 (fluid, walls of several radii): k_halo_build has to do its
+// halo; it has a wide cell; the first pass leaves it to the second.
+constexpr uint32_t kNoHalo = 4u, kWideCells = 8u, kLeave = 16u;
 constexpr uint32_t kHit = 0x80000000u;  // marks a staged fluid copy that is in a list (slots are below 2^31)
 
 // Inclusive scan of a 64-bit value over the workgroup's NW waves; `ws` holds NW wave totals
@@ -802,18 +806,20 @@ struct RowHits {
     }
 };
 
+//
+// mode: of the first pass which blocks it leaves (SearchLeave); of the last 1 if it takes only those.
 template <int Q, class Caps, bool LAST>
 __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __restrict__ pos, Scenes sc, uint32_t C, HashGeom g,
                                                           HashView fl, HashView bd, uint32_t* __restrict__ nff, uint32_t Kff,
                                                           uint32_t* __restrict__ cff, uint32_t* __restrict__ nfb, uint32_t Kfb,
                                                           uint32_t* __restrict__ cfb, uint2* __restrict__ bstat,
-                                                          launch::HaloOut ho, int left, NbrCounters* __restrict__ ctr) {
+                                                          launch::HaloOut ho, int mode, NbrCounters* __restrict__ ctr) {
     constexpr uint32_t kThreads = Q * kBlock, kWaves = kThreads / 64u;
     constexpr uint32_t kRowHash = Caps::kRowHash, kRows = Caps::kRows, kCells = Caps::kCells, kCand = Caps::kCand;
     constexpr uint32_t kCellsPer = (kCells + kThreads - 1u) / kThreads;  // cells per thread
     static_assert(kRows <= kThreads && kRows <= 255u + 1u && kRows < kRowHash, "one row per thread");
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    if (LAST && left && ho.n[blk] != kHaloLeft) return;  // the first pass did this block
+    if (LAST && mode && ho.n[blk] != kHaloLeft) return;  // the first pass did this block
     const uint32_t tid = threadIdx.x;
     const uint32_t i = blk * kBlock + tid / Q;
     const uint32_t l = tid % Q;
@@ -866,6 +872,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
             const uint32_t k = grid_index(0, p.y + int(r % 3u) - 1, p.z + int(r / 3u) - 1, g);
             uint32_t h = row_hash(k);
             for (uint32_t probe = 0; probe < kRowHash; probe++) {
+                if (probe > 7u && *(volatile uint32_t*)&nrow > kRows) break;  // (a probe of a full table is long)
                 const uint32_t prev = atomicCAS(&rkey[h], kNoRow, k);
                 if (prev == kNoRow) {
                     const uint32_t e = atomicAdd(&nrow, 1u);
@@ -883,7 +890,8 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     __syncthreads();
     const uint32_t nr = nrow;
     bool staged = nr <= kRows;
-    bool tables = LAST;  // what cannot be walked in LDS here searches the global tables
+    // whether what cannot be walked in LDS searches the global tables here, and is not left to a second pass
+    bool tables = LAST || mode == launch::kLeaveNone || (mode != launch::kLeaveAll && !staged);
     uint32_t nc = 0u;
     // 2. number each row's cells over its x range (rows in registration order)
     if (staged) {
@@ -894,14 +902,16 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
         const uint32_t b0 = static_cast<uint32_t>(block_scan_u64<kWaves>(len, ws, tot)) - len;
         nc = static_cast<uint32_t>(tot);
         staged = nc <= kCells;
+        tables |= mode != launch::kLeaveAll && !staged;
         if (staged && tid < nr) {
             rbase[h] = static_cast<uint16_t>(b0);
-            if (len > g.hx) atomicOr(&mixed, 4u);  // the row wraps around: a cell is staged twice (see 6.)
+            if (len > g.hx) atomicOr(&mixed, kNoHalo);  // the row wraps around: a cell is staged twice (see 6.)
             const uint32_t k0 = rkey[h];
             for (uint32_t q = 0; q < len; q++) ecell[b0 + q] = k0 + (static_cast<uint32_t>(rxlo[h] + static_cast<int>(q)) & (g.hx - 1u));
         }
         __syncthreads();
     }
+    if (!LAST && !staged && tid == 0) atomicAdd(&ctr->spread, 1u);
     // 3. bounds of each cell (read once) and offsets of its staged copies: fluid from 0, walls
     //    after all fluid
     uint32_t tf = 0u, tb = 0u;
@@ -924,7 +934,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
             }
             fsum += fc[q];
             bsum += bc[q];
-            if (!LAST && fc[q] > kWideCell) atomicOr(&mixed, 8u);
+            if (!LAST && fc[q] > kWideCell) atomicOr(&mixed, kWideCells);
         }
         const unsigned long long mine = (static_cast<unsigned long long>(bsum) << 32) | fsum;
         unsigned long long tot;
@@ -932,7 +942,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
         tf = static_cast<uint32_t>(tot & 0xFFFFFFFFull);
         tb = static_cast<uint32_t>(tot >> 32);
         staged = static_cast<unsigned long long>(tf) + tb <= kCand;
-        tables = LAST || static_cast<unsigned long long>(tf) + tb > SearchWide::kCand || (mixed & 8u);
+        tables |= static_cast<unsigned long long>(tf) + tb > SearchWide::kCand || (mixed & kWideCells);
         if (!LAST && tid == 0 && !tables && static_cast<unsigned long long>(tf) + tb > SearchStd::kCand) atomicAdd(&ctr->crowded, 1u);
         uint32_t fo = static_cast<uint32_t>(ex & 0xFFFFFFFFull), bo = static_cast<uint32_t>(ex >> 32);
         if (staged) {
@@ -960,8 +970,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     }
     // 4. stage the candidates with their ids (copy t of cell e is particle efs[e] + t - efo[e]),
     //    kStage loads of a thread in flight. `mixed` records whether some fluid (bit 0) or wall (bit 1)
-    //    candidate has another radius than the first staged candidate of its set (bit 2: the block's halo
-    //    cannot be written here, bit 3: a wide cell).
+    //    candidate has another radius than the first staged candidate of its set.
     float rf = 0.0f, rw = 0.0f;  // the first fluid's radius, the walls' common one
     if (staged) {
         constexpr uint32_t kStage = 4;
@@ -1058,9 +1067,9 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
         } else if (tables) {
             if constexpr (Q == 1) a = search_cells<true, kGroups>(xi, i, g, fstart, fend, fl.id, fl.spos, nff, Kff, N);
             else a = search_cells_quad<true, kGroups>(xi, i, l, g, fstart, fend, fl.id, fl.spos, nff, Kff, N);
-            atomicOr(&mixed, 4u);  // the block's halo is left to k_halo_build
+            atomicOr(&mixed, kNoHalo);
         } else {
-            atomicOr(&mixed, 4u);
+            atomicOr(&mixed, kLeave);
         }
         if (bd.n) {
             if (staged && tb == 0u) {
@@ -1078,7 +1087,7 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
                     if constexpr (Q == 1) b = search_cells<false, kCols>(xi, i, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N);
                     else b = search_cells_quad<false, kCols>(xi, i, l, g, bstart, bend, bd.id, bd.spos, nfb, Kfb, N);
                 } else {
-                    atomicOr(&mixed, 4u);
+                    atomicOr(&mixed, kLeave);
                 }
             }
         }
@@ -1090,10 +1099,11 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     // 6. the block's halo: the marked copies, cells in order of their first slot (cells are disjoint
     //    slot ranges, so that is ascending slot order; a block with a cell staged twice is left out)
     __syncthreads();
-    if (!staged || (mixed & 4u)) {
+    const bool leave = (!staged && !tables) || (mixed & kLeave);
+    if (leave || !staged || (mixed & kNoHalo)) {
         if (tid == 0) {
-            ho.n[blk] = tables ? kHaloTodo : kHaloLeft;
-            atomicAdd(tables ? &ctr->todo : &ctr->left, 1u);
+            ho.n[blk] = leave ? kHaloLeft : kHaloTodo;
+            atomicAdd(leave ? &ctr->left : &ctr->todo, 1u);
         }
     } else {
         // marked copies of each cell (in ecell, no longer needed), then their sum over the cells with
@@ -1331,13 +1341,13 @@ void cell_table(const uint32_t* key, const uint32_t* id, uint32_t n, uint32_t* s
 }
 void neighbors_fluid(const float4* pos, const Scenes& sc, uint32_t C, const HashGeom& g, const HashView& fl, const HashView& bd,
                      uint32_t* nff, uint32_t Kff, uint32_t* cff, uint32_t* nfb, uint32_t Kfb, uint32_t* cfb, uint2* bstat,
-                     HaloOut ho, SearchPasses passes, int dense, NbrCounters* ctr, hipStream_t s) {
+                     HaloOut ho, SearchPasses passes, SearchLeave leave, int dense, NbrCounters* ctr, hipStream_t s) {
     if (!sc.N) return;
     const uint32_t g_ = nb(sc.N);
     ho.limit = ho.limit == 0u || ho.limit > kHaloCap ? kHaloCap : ho.limit;
-#define MPS_SEARCH(Q, CAPS, LAST, LEFT)                                                                                       \
+#define MPS_SEARCH(Q, CAPS, LAST, MODE)                                                                                       \
     launch_k(k_neighbors_fluid<Q, CAPS, LAST>, g_, Q * kBlock, 0, s, pos, sc, C, g, fl, bd, nff, Kff, cff, nfb, Kfb, cfb, bstat, \
-             ho, LEFT, ctr)
+             ho, MODE, ctr)
     // Up to two workgroups per CU one pass of the quad form (its blocks have the chip to themselves:
     // 128 workgroups 206 -> 72 us with the halos); beyond, the one-lane form and, where the last
     // search left blocks (or this one did: passes = kSearchLeft), the quad form over those.
@@ -1345,8 +1355,8 @@ void neighbors_fluid(const float4* pos, const Scenes& sc, uint32_t C, const Hash
         MPS_SEARCH(4, SearchWide, true, 0);
     } else {
         if (passes != kSearchLeft) {
-            if (dense) MPS_SEARCH(1, SearchDense, false, 0);
-            else MPS_SEARCH(1, SearchStd, false, 0);
+            if (dense) MPS_SEARCH(1, SearchDense, false, leave);
+            else MPS_SEARCH(1, SearchStd, false, leave);
         }
         if (passes != kSearchFirst) MPS_SEARCH(4, SearchWide, true, 1);
     }

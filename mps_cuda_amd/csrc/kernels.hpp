@@ -34,7 +34,7 @@ struct NbrCounters {
     uint32_t left;  // workgroups that the first pass of the fluid search left to the second
     uint32_t crowded;  // workgroups of the first pass with more candidates than its usual form holds (and not searched in the tables)
     uint32_t todo;  // workgroups of the fluid search whose halo is left to k_halo_build
-    uint32_t pad;
+    uint32_t spread;  // workgroups of the first pass with more rows or cells than it holds
     unsigned long long nnz_ff, nnz_fb, nnz_bb, nnz_fr;
 };
 
@@ -217,11 +217,14 @@ struct HaloOut {
 // the first left (NbrCounters::left; both passes in one call do without the host's look at it).
 // dense: the first pass in its form with more candidates (and three workgroups per CU, not four).
 enum SearchPasses { kSearchFirst, kSearchBoth, kSearchLeft };
+// What the first pass leaves: nothing, blocks with too many candidates or too long a run of them, or
+// those with too many rows or cells too.
+enum SearchLeave { kLeaveNone, kLeaveCrowded, kLeaveAll };
 // bstat: scratch of 2 * ceil(N / kBlock) (fluid) or ceil(B / kBlock) (walls) per-workgroup
 // count records, folded into ctr after the search
 void neighbors_fluid(const float4* pos, const Scenes& sc, uint32_t C, const dev::HashGeom& g, const HashView& fl,
                      const HashView& bd, uint32_t* nff, uint32_t Kff, uint32_t* cff, uint32_t* nfb, uint32_t Kfb, uint32_t* cfb,
-                     uint2* bstat, HaloOut ho, SearchPasses passes, int dense, NbrCounters* ctr, hipStream_t s);
+                     uint2* bstat, HaloOut ho, SearchPasses passes, SearchLeave leave, int dense, NbrCounters* ctr, hipStream_t s);
 // ref lists of coupled scenes (other scenes' fluid, ascending scene order)
 void neighbors_ref(const float4* pos, const Scenes& sc, uint32_t C, const dev::HashGeom& g, const HashView& fl, uint32_t* nfr,
                    uint32_t Kfr, uint32_t* cfr, uint2* bstat, NbrCounters* ctr, hipStream_t s);
