@@ -2442,14 +2442,19 @@ struct mps_ctx {
     std::vector<uint32_t> csr_nei_fluid(const uint32_t* nbrs, const uint32_t* cnt, uint32_t K, bool groups) {
         std::vector<uint32_t> c = down(cnt, N), iv = down(inv.p, Nref), pm = down(perm.p, N);
         std::vector<uint32_t> ell = down(nbrs, size_t(K) * N);
-        std::vector<uint32_t> out;
+        size_t total = 0;
+        for (uint32_t i = 0; i < Nref; i++) total += c[iv[i]];
+        std::vector<uint32_t> out(total);
+        uint32_t* o = out.data();
         for (uint32_t i = 0; i < Nref; i++) {
-            const uint32_t sl = iv[i];
-            for (uint32_t k = 0; k < c[sl]; k++) {
-                // fluid lists keep four entries of a slot side by side (ell()), wall lists are columns
-                const size_t at = groups ? (size_t(k >> 2) * N + sl) * 4 + (k & 3u) : size_t(k) * N + sl;
-                const uint32_t j = ell[at];
-                out.push_back(groups ? pm[j] : j);
+            const uint32_t sl = iv[i], n = c[sl];
+            if (groups) {  // fluid lists keep four entries of a slot side by side (ell())
+                for (uint32_t k = 0; k < n; k += 4) {
+                    const uint32_t* e = &ell[(size_t(k >> 2) * N + sl) * 4];
+                    for (uint32_t q = 0; q < std::min(n - k, 4u); q++) *o++ = pm[e[q]];
+                }
+            } else {  // wall lists are columns
+                for (uint32_t k = 0; k < n; k++) *o++ = ell[size_t(k) * N + sl];
             }
         }
         return out;
