@@ -4,7 +4,8 @@ initial velocities and of each scene's viscosity and surface-tension coefficient
 The forward pass steps the library (mps_adj_rollout_traj, checkpoints every `checkpoint_every`
 steps) and returns the positions after the observed steps; the backward pass calls the
 library's hand-written adjoint (mps_adj_backward_traj), which recomputes each segment from its
-checkpoint and adds each observation's cotangent where that state was produced. Tensors cross
+checkpoint (the last one only if the rollout has not recorded it: it does where the context's rollout
+before was differentiated) and adds each observation's cotangent where that state was produced. Tensors cross
 the C ABI as host arrays.
 
 The library keeps one recorded rollout per context. A backward pass whose rollout has since been

@@ -327,7 +327,8 @@ void cg_persistent(const CgOperator& op, int coherent, const Scenes& sc, const N
                    dev::f3* pbuf0, dev::f3* pbuf1, dev::f3* Ap, dev::f3* x, SolverDev* st, uint32_t* active, double* partA,
                    double* partB, GridSync* gs, uint32_t cap, double tol, uint32_t spin, hipStream_t s);
 // ---- halo.hip
-// stats (3 words, accumulated): largest staged halo, blocks over kHaloCap, blocks with particles
+// stats (4 words, stored): largest staged halo, blocks not staged, blocks with a halo or not staged, blocks
+// staged but deeper than kHaloShallow
 // limit: largest halo staged (0 or > kHaloCap: kHaloCap)
 // all: every block, or only those with n = kHaloTodo
 void halo_build(int all, const Scenes& sc, const Nbr& nb, uint32_t nblk, uint32_t limit, uint32_t* hidx, uint32_t* hn,

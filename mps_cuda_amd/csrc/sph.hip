@@ -16,8 +16,8 @@
 // Convergence sums: each workgroup reduces its T-rounded terms in double and writes one
 // partial; the workgroups that need the sum, or in large grids a one-workgroup fold kernel, add the
 // partials in index order (deterministic, no FP64 atomics) and update a SolverDev record on the device. Kernels of later iterations
-// read SolverDev::done first and exit at once, so the host can enqueue several iterations
-// before it looks at the result.
+// read SolverDev::done first (those that fold: SolverDev::it) and exit at once, so the host can
+// enqueue several iterations before it looks at the result.
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -194,7 +194,7 @@ __device__ __forceinline__ double fold_everywhere(const double* __restrict__ par
 // entry per load (columns, two entries in flight) a walk waits for a quarter of the round trips and
 // issues a quarter of the loads and addresses: A.p 25 -> 15 us at 45k particles (66 neighbours each),
 // 85 -> 70 us at 525k (61), 76 -> 73 us at 1M (31; there the stream itself is the bound, and the
-// unused entries of the last groups cost 5 % more bytes). With a quad per slot
+// unused entries of the last groups cost 10 % more bytes: 482 -> 530 MB). With a quad per slot
 // (Q = 4) lane part l of the quad takes entry 4g + l of every group, and the group's four terms
 // are added to the running sum one after the other, in list order, by every lane of the quad
 // (add_quad): a sum has the same bits in both forms. An entry past the end of the list
