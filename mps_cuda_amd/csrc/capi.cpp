@@ -890,12 +890,14 @@ struct mps_ctx {
             counters();
             const uint64_t blocks = (uint64_t(N) + mps::dev::kBlock - 1) / mps::dev::kBlock;
             search_left = h_ctr->left;
-            search_dense = uint64_t(h_ctr->crowded) * kSearchMany > blocks;
             if (h_ctr->left && !both) {
                 search(mps::launch::kSearchLeft);
                 counters();
             }
-            search_leave = uint64_t(h_ctr->spread) * kSearchMany > blocks ? mps::launch::kLeaveNone : mps::launch::kLeaveAll;
+            if (blocks > mps::launch::kSearchOnePass) {  // (a search of one pass says nothing about the first's)
+                search_dense = uint64_t(h_ctr->crowded) * kSearchMany > blocks;
+                search_leave = uint64_t(h_ctr->spread) * kSearchMany > blocks ? mps::launch::kLeaveNone : mps::launch::kLeaveAll;
+            }
             bool grow = false;
             if (coupled() && h_ctr->max_fr > Kfr) { Kfr = (h_ctr->max_fr + 15u) & ~15u; grow = true; }
             if (h_ctr->max_ff > Kff) { Kff = (h_ctr->max_ff + 15u) & ~15u; grow = true; }

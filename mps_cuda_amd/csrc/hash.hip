@@ -1351,7 +1351,7 @@ void neighbors_fluid(const float4* pos, const Scenes& sc, uint32_t C, const Hash
     // Up to two workgroups per CU one pass of the quad form (its blocks have the chip to themselves:
     // 128 workgroups 206 -> 72 us with the halos); beyond, the one-lane form and, where the last
     // search left blocks (or this one did: passes = kSearchLeft), the quad form over those.
-    if (g_ <= 512u) {
+    if (g_ <= kSearchOnePass) {
         MPS_SEARCH(4, SearchWide, true, 0);
     } else {
         if (passes != kSearchLeft) {

@@ -220,6 +220,7 @@ enum SearchPasses { kSearchFirst, kSearchBoth, kSearchLeft };
 // What the first pass leaves: nothing, blocks with too many candidates or too long a run of them, or
 // those with too many rows or cells too.
 enum SearchLeave { kLeaveNone, kLeaveCrowded, kLeaveAll };
+constexpr uint32_t kSearchOnePass = 512;  // workgroups up to which there is only the last pass, over all of them
 // bstat: scratch of 2 * ceil(N / kBlock) (fluid) or ceil(B / kBlock) (walls) per-workgroup
 // count records, folded into ctr after the search
 void neighbors_fluid(const float4* pos, const Scenes& sc, uint32_t C, const dev::HashGeom& g, const HashView& fl,
