@@ -889,7 +889,8 @@ __global__ void __launch_bounds__(Q * kBlock) k_neighbors_fluid(const float4* __
     }
     __syncthreads();
     const uint32_t nr = nrow;
-    bool staged = nr <= kRows;
+    // (in a grid one cell wide a run holds the particle's own cell three times, but `self` is one copy of it)
+    bool staged = nr <= kRows && g.hx > 1u;
     // whether what cannot be walked in LDS searches the global tables here, and is not left to a second pass
     bool tables = LAST || mode == launch::kLeaveNone || (mode != launch::kLeaveAll && !staged);
     uint32_t nc = 0u;
